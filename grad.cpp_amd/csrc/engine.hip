@@ -5,13 +5,12 @@
 #include "checkpoint.h"
 #include "tokenizer.h"
 #include "kernels_attn.h"
+#include "kernel_tables.h"
 #include "kernels_common.h"
 #include "kernels_gemm.h"
-#include "kernels_gemm_big.h"
 #include "kernels_gemv.h"
-#include "kernels_persist.h"
 #include "kernels_pick.h"
-#include "kernels_xcd.h"
+#include "rows.h"
 
 #include <algorithm>
 #include <cmath>
@@ -122,6 +121,7 @@ struct LayerWeights {
     float *w1, *b1;      // GPT-2: (F, d), F.  Modern: (2F, d) rows (gate_p, up_p) interleaved
     float *w2, *b2;      // (d, F), d (GPT-2 only)
     float *g1, *be1, *g2, *be2;
+    char *s_wqkv, *s_wo, *s_w1, *s_w2;  // split forms for passes over many rows (kernels_split.h)
 };
 
 // Where tensor i of the file lives on the device.
@@ -142,6 +142,8 @@ struct Model {
     float *gf = nullptr, *bf = nullptr;
     float *rope_cos = nullptr, *rope_sin = nullptr;  // (max_len, head_size/2)
     std::vector<Placement> place;                    // file order
+    char* split_blob = nullptr;  // split forms of the matrices; null for shapes without a prompt pass
+    char* s_E = nullptr;
 
     // The XCD-sharded persistent kernel reads the weights from a second copy laid
     // out as one contiguous stream per workgroup (kernels_xcd.h); built by the
@@ -152,6 +154,7 @@ struct Model {
 
     ~Model() {
         if (blob) (void)hipFree(blob);
+        if (split_blob) (void)hipFree(split_blob);
         if (xcd_stream) (void)hipFree(xcd_stream);
     }
 };
@@ -206,7 +209,7 @@ static void plan_model(Model& m) {
         LayerWeights& w = m.layers[l];
         w = {B + lo[l].wqkv, B + lo[l].bqkv, B + lo[l].wo, B + lo[l].bo, B + lo[l].w1,
              B + lo[l].b1,   B + lo[l].w2,   B + lo[l].b2, B + lo[l].g1, B + lo[l].be1,
-             B + lo[l].g2,   B + lo[l].be2};
+             B + lo[l].g2,   B + lo[l].be2,  nullptr,      nullptr,      nullptr,      nullptr};
         for (int q = 0; q < 3; q++) m.place.push_back({w.wqkv + q * d * d, true, 1, 0});
         m.place.push_back({w.wo, true, 1, 0});
         for (int q = 0; q < 3; q++) m.place.push_back({w.bqkv + q * d, false, 1, 0});
@@ -232,6 +235,38 @@ static void plan_model(Model& m) {
     m.place.push_back({m.bf, false, 1, 0});
     m.rope_cos = B + ocos;
     m.rope_sin = B + osin;
+}
+
+// Shapes whose prompts go through each layer in one pass: head size 64, rows of whole
+// 64-column runs (four sets of wavefronts share K in blocks of 16) that norm_split keeps
+// in registers.
+static bool rows_shape_ok(const Shape& sh) {
+    return sh.head_size() == 64 && sh.d_model % 64 == 0 && sh.d_ff() % 64 == 0 && sh.d_model <= 4096;
+}
+
+// The second form of every matrix that passes over many rows read: six bytes per weight,
+// written once, here.
+static void split_model(Model& m) {
+    const Shape& sh = m.shape;
+    if (!rows_shape_ok(sh)) return;
+    const int d = sh.d_model, F = sh.d_ff(), up = sh.modern() ? 2 : 1;
+    const size_t per_layer = split_bytes(3 * d, d) + split_bytes(d, d) + split_bytes(up * F, d) + split_bytes(d, F);
+    HIP_CHECK(hipMalloc(&m.split_blob, sh.layers * per_layer + split_bytes(sh.vocab, d)));
+    char* at = m.split_blob;
+    const auto place = [&](const float* src, int N, int K, bool gate_up) {
+        split_weights(src, N, K, gate_up, at, nullptr);
+        char* const here = at;
+        at += split_bytes(N, K);
+        return here;
+    };
+    for (LayerWeights& w : m.layers) {
+        w.s_wqkv = place(w.wqkv, 3 * d, d, false);
+        w.s_wo = place(w.wo, d, d, false);
+        w.s_w1 = place(w.w1, up * F, d, sh.modern());
+        w.s_w2 = place(w.w2, d, F, false);
+    }
+    m.s_E = place(m.E, sh.vocab, d, false);
+    HIP_CHECK(hipDeviceSynchronize());
 }
 
 static std::unique_ptr<Model> upload_model(const Shape& shape, const std::vector<const float*>& t,
@@ -290,6 +325,7 @@ static std::unique_ptr<Model> upload_model(const Shape& shape, const std::vector
             HIP_CHECK(hipMemcpy(m->rope_sin, sn.data(), sn.size() * 4, hipMemcpyHostToDevice));
         }
     }
+    split_model(*m);
     return m;
 }
 
@@ -370,9 +406,11 @@ struct Session {
 
     // prompt pass (all prompt tokens at once): row-major [rows][width] activations
     float *pp_x = nullptr, *pp_q = nullptr, *pp_attn = nullptr, *pp_norm = nullptr, *pp_hidden = nullptr;
+    char *pp_split = nullptr, *pp_split_hidden = nullptr;  // split rows of d_model and of d_ff columns
     size_t pp_rows = 0;
-    float* score_logits = nullptr;  // [score_rows][vocab] logits of a block of rows being scored
-    size_t score_rows = 0;
+    float2* nll_part = nullptr;  // [pp_rows][split_nll_stride(vocab)] of rows being scored
+    float* nll_target = nullptr;  // [pp_rows]
+    size_t nll_rows = 0;
 
     // persistent engine
     Cell* cells = nullptr;  // xa, xb, q, kn, vn, at (d each), hid (F), token (1)
@@ -412,7 +450,7 @@ struct Session {
 #ifdef GH_PICK_TICKS
         {
             unsigned long long t[32] = {};
-            if (hipMemcpyFromSymbol(t, HIP_SYMBOL(g_pick_ticks), sizeof(t)) == hipSuccess) {
+            if (read_pick_ticks(t)) {
                 std::fprintf(stderr, "pick ticks (10 ns, summed):");
                 for (unsigned long long v : t) std::fprintf(stderr, " %llu", v);
                 std::fprintf(stderr, "\n");
@@ -452,7 +490,9 @@ struct Session {
                         static_cast<void*>(logit_log), static_cast<void*>(cells), static_cast<void*>(xcells),
                         static_cast<void*>(ctl), static_cast<void*>(pp_x), static_cast<void*>(pp_q),
                         static_cast<void*>(pp_attn), static_cast<void*>(pp_norm),
-                        static_cast<void*>(pp_hidden), static_cast<void*>(score_logits)})
+                        static_cast<void*>(pp_hidden), static_cast<void*>(pp_split),
+                        static_cast<void*>(pp_split_hidden), static_cast<void*>(nll_part),
+                        static_cast<void*>(nll_target)})
             if (p) (void)hipFree(p);
         if (host_logits) (void)hipHostFree(host_logits);
         if (host_ids) (void)hipHostFree(host_ids);
@@ -732,31 +772,6 @@ static int enqueue_step(Session& s, bool pick_first = false) {
 
 // ---- persistent engine
 
-using PersistKernel = void (*)(const PersistParams);
-
-// The shapes the persistent kernel is built for (head size 64, d_model and FFN
-// width multiples of 256); nullptr for anything else.
-// row_lds: the sampler's working row fits in LDS.
-template <bool ROW_LDS, bool FEED>
-static PersistKernel persist_kernel_of(const Shape& sh) {
-    if (sh.head_size() != 64) return nullptr;
-    const int d = sh.d_model, F = sh.d_ff();
-    if (sh.modern()) {
-        if (d == 768 && F == 2048) return persist_decode_kernel<3, 8, true, ROW_LDS, FEED>;
-        return nullptr;
-    }
-    if (d == 512) return persist_decode_kernel<2, 8, false, ROW_LDS, FEED>;
-    if (d == 768) return persist_decode_kernel<3, 12, false, ROW_LDS, FEED>;
-    if (d == 1024) return persist_decode_kernel<4, 16, false, ROW_LDS, FEED>;
-    return nullptr;
-}
-// feed: the variant that reports its picks to the host and can be told to stop.
-static PersistKernel persist_kernel_for(const Shape& sh, bool row_lds, bool feed = false) {
-    if (feed) return row_lds ? persist_kernel_of<true, true>(sh) : persist_kernel_of<false, true>(sh);
-    return row_lds ? persist_kernel_of<true, false>(sh) : persist_kernel_of<false, false>(sh);
-}
-
-
 // ---- the XCD-sharded form of the persistent kernel (kernels_xcd.h)
 
 // The XCD-sharded kernel runs only where GH_FLAG_XCD_PERSISTENT asks for it.  It used to
@@ -766,14 +781,6 @@ static PersistKernel persist_kernel_for(const Shape& sh, bool row_lds, bool feed
 // position.  Per token on one box, Llama block d768 L8 V16000, greedy, XCD-sharded /
 // all-to-all: positions 256..512 168 / 132, 512..768 178 / 144, 1024..1280 196 / 149,
 // 2048..2304 228 / 156, 3072..3328 259 / 160, 3800..4056 277 / 162.
-
-using XcdKernel = void (*)(const XcdParams);
-
-static XcdKernel xcd_kernel_for(const Shape& sh, bool row_lds, bool feed) {
-    if (!sh.modern() || sh.head_size() != 64 || sh.d_model != 768) return nullptr;
-    if (feed) return row_lds ? xcd_decode_kernel<3, true, true> : xcd_decode_kernel<3, false, true>;
-    return row_lds ? xcd_decode_kernel<3, true, false> : xcd_decode_kernel<3, false, false>;
-}
 
 // Splits the model over eight XCDs: heads g and g + 8, and a run of hidden units
 // sized so that every XCD streams about the same number of bytes per layer.
@@ -1416,33 +1423,21 @@ constexpr size_t kPromptPassRows = 32768; // rows per pass; longer prompts run i
 
 static bool prompt_pass_ok(const Session& s, int len) {
     const Shape& sh = s.m->shape;
-    return len >= kPromptPassMin && sh.head_size() == 64 && sh.d_model % 128 == 0 && sh.d_ff() % 128 == 0;
+    return len >= kPromptPassMin && rows_shape_ok(sh);
 }
+
+// Passes of this many rows and more take the split projections (kernels_split.h); below,
+// the small fp32 tiles of the decode step, whose norms ride inside the projections (one
+// sequence of the 69M Llama block: 96 tokens 588 us against 619, 128: 627 against 654, 244:
+// 820 against 664).
+constexpr int kSplitMinRows = 160;
 
 // One projection over M rows (norm folded in for RMSNorm, a norm kernel for LayerNorm).
-// Long row blocks take the compute-bound 128 x 128 tiling, short ones the
-// latency-bound small tiles.
-template <int EPI, bool RMS>
-static void launch_rows_gemm(const GemvParams& g, int M, hipStream_t st) {
-    if (gemm128_ok(g, M)) {
-        // per instantiation, once: the tile needs more than the default 64 KB of LDS
-        static std::once_flag lds_raised;
-        std::call_once(lds_raised, [] {
-            HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm128_kernel<EPI, RMS>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          static_cast<int>(kBigLdsBytes)));
-        });
-        launch_gemm128<EPI, RMS>(g, M, st);
-    } else {
-        launch_gemm16<EPI, RMS>(g, M, st);
-    }
-}
-
 template <int PRO, int EPI>
 static void project_rows(Session& s, GemvParams g, int M) {
     hipStream_t st = s.stream;
     if (PRO == PRO_RMSNORM) {
-        launch_rows_gemm<EPI, true>(g, M, st);
+        launch_gemm16<EPI, true>(g, M, st);
     } else {
         if (PRO == PRO_LAYERNORM) {
             hipLaunchKernelGGL(norm_rows_kernel, dim3((M + 3) / 4), dim3(256), 0, st, g.in, g.gamma, g.beta,
@@ -1451,7 +1446,7 @@ static void project_rows(Session& s, GemvParams g, int M) {
             g.in = s.pp_norm;
             g.in_stride = g.K;
         }
-        launch_rows_gemm<EPI, false>(g, M, st);
+        launch_gemm16<EPI, false>(g, M, st);
     }
     HIP_CHECK(hipGetLastError());
 }
@@ -1463,39 +1458,210 @@ struct ScoreSink {
     float* nll;
 };
 
+static SplitGemmParams split_params(const char* A, const char* W, int M, int N, int K) {
+    SplitGemmParams g{};
+    g.A = A;
+    g.W = W;
+    g.M = M;
+    g.N = N;
+    g.K = K;
+    return g;
+}
+
 // Final norm, logits and the target's negative log-likelihood for rows
-// pp_x[0 .. M) of a slice (row m = seq * n + t, position t0 + t), a block of rows
-// at a time so that the logits of a block stay a modest buffer.
+// pp_x[0 .. M) of a slice (row m = seq * n + t, position t0 + t).  The logits are not
+// stored: every run of outputs leaves its maximum and its sum of exponentials.
 static void score_rows(Session& s, const ScoreSink& sink, int M, int n, int t0, int len) {
     const Model& m = *s.m;
     const Shape& sh = m.shape;
-    const size_t V = sh.vocab;
-    const size_t want = std::min<size_t>(static_cast<size_t>(M),
-                                         std::max<size_t>(128, ((size_t{64} << 20) / V) / 128 * 128));
-    if (s.score_rows < want) {
-        if (s.score_logits) HIP_CHECK(hipFree(s.score_logits));
-        s.score_logits = nullptr;
-        dev_alloc(s.score_logits, want * V);
-        s.score_rows = want;
+    if (s.nll_rows < static_cast<size_t>(M)) {
+        if (s.nll_part) HIP_CHECK(hipFree(s.nll_part));
+        if (s.nll_target) HIP_CHECK(hipFree(s.nll_target));
+        s.nll_part = nullptr;
+        s.nll_target = nullptr;
+        s.nll_rows = 0;
+        dev_alloc(s.nll_part, static_cast<size_t>(M) * split_nll_stride(sh.vocab));
+        dev_alloc(s.nll_target, M);
+        s.nll_rows = M;
     }
-    for (int r0 = 0; r0 < M; r0 += static_cast<int>(s.score_rows)) {
-        const int rows = std::min<int>(static_cast<int>(s.score_rows), M - r0);
-        GemvParams g{};
-        g.W = m.E;
-        g.N = sh.vocab;
-        g.K = sh.d_model;
-        g.in = s.pp_x + static_cast<size_t>(r0) * sh.d_model;
-        g.in_stride = sh.d_model;
-        g.gamma = m.gf;
-        g.beta = m.bf;
-        g.out = s.score_logits;
-        g.out_stride = sh.vocab;
-        if (sh.modern()) project_rows<PRO_RMSNORM, EPI_STORE>(s, g, rows);
-        else project_rows<PRO_LAYERNORM, EPI_STORE>(s, g, rows);
-        hipLaunchKernelGGL(nll_rows_kernel, dim3(rows), dim3(256), 0, s.stream, s.score_logits, sh.vocab, r0, n, t0,
-                           len, sink.targets, sink.nll);
-        HIP_CHECK(hipGetLastError());
+    norm_split(sh.modern(), s.pp_x, m.gf, m.bf, s.pp_split, M, sh.d_model, s.stream);
+    SplitGemmParams g = split_params(s.pp_split, m.s_E, M, sh.vocab, sh.d_model);
+    g.rows_per_seq = n;
+    g.targets = sink.targets;
+    g.nll_t0 = t0;
+    g.nll_len = len;
+    g.nll_part = s.nll_part;
+    g.nll_target = s.nll_target;
+    split_gemm<EPI_STORE>(g, s.stream);
+    nll_parts(g, sink.nll, s.stream);
+}
+
+static PrefillAttnParams prompt_attn_params(const Session& s, int layer, int n, int pos_base) {
+    const Shape& sh = s.m->shape;
+    PrefillAttnParams a{};
+    a.q = s.pp_q;
+    a.kv = kv_layout(s);
+    a.layer = layer;
+    a.d_model = sh.d_model;
+    a.len = n;
+    a.pos_base = pos_base;
+    a.scale = 1.0f / std::sqrt(static_cast<float>(sh.head_size()));
+    return a;
+}
+
+static void launch_prompt_attn(const Session& s, const PrefillAttnParams& a) {
+    const int heads = s.m->shape.heads;
+    // from 512 tokens on, 128 queries per workgroup (16 sequences: 1000 tokens 512 against
+    // 585 us, 1536 tokens 860 against 977; at 300 tokens 76 against 60: too few workgroups)
+    if (a.len >= 512)
+        hipLaunchKernelGGL(attn_prefill128_kernel, dim3((a.len + 127) / 128, heads, s.B), dim3(256), 0, s.stream, a);
+    else
+        hipLaunchKernelGGL(attn_prefill64_kernel, dim3((a.len + 63) / 64, heads, s.B), dim3(256), 0, s.stream, a);
+    HIP_CHECK(hipGetLastError());
+}
+
+// One layer over M = n * B rows of pp_x through the split projections.
+static void prompt_layer_split(Session& s, int layer, int n, int pos_base) {
+    const Model& m = *s.m;
+    const Shape& sh = m.shape;
+    const LayerWeights& w = m.layers[layer];
+    const int d = sh.d_model, F = sh.d_ff(), M = n * s.B;
+    hipStream_t st = s.stream;
+
+    norm_split(sh.modern(), s.pp_x, w.g1, w.be1, s.pp_split, M, d, st);
+    SplitGemmParams g = split_params(s.pp_split, w.s_wqkv, M, 3 * d, d);
+    g.bias = w.bqkv;
+    g.out = s.pp_q;
+    g.out_stride = d;
+    g.kv = kv_layout(s);
+    g.layer = layer;
+    g.d_model = d;
+    g.rope = sh.modern();
+    g.rope_cos = m.rope_cos;
+    g.rope_sin = m.rope_sin;
+    g.rows_per_seq = n;
+    g.pos_base = pos_base;
+    split_gemm<EPI_QKV>(g, st);
+
+    PrefillAttnParams a = prompt_attn_params(s, layer, n, pos_base);
+    a.out_split = s.pp_split;
+    launch_prompt_attn(s, a);
+
+    g = split_params(s.pp_split, w.s_wo, M, d, d);
+    g.bias = w.bo;
+    g.out = s.pp_x;
+    g.out_stride = d;
+    split_gemm<EPI_RESID>(g, st);
+
+    norm_split(sh.modern(), s.pp_x, w.g2, w.be2, s.pp_split, M, d, st);
+    g = split_params(s.pp_split, w.s_w1, M, sh.modern() ? 2 * F : F, d);
+    g.bias = sh.modern() ? nullptr : w.b1;
+    g.out_split = s.pp_split_hidden;
+    g.out_kblocks = F / kSplitCols;
+    if (sh.modern()) split_gemm<EPI_SWIGLU>(g, st);
+    else split_gemm<EPI_GELU>(g, st);
+
+    g = split_params(s.pp_split_hidden, w.s_w2, M, d, F);
+    g.bias = sh.modern() ? nullptr : w.b2;
+    g.out = s.pp_x;
+    g.out_stride = d;
+    split_gemm<EPI_RESID>(g, st);
+}
+
+// The same layer through the decode step's small fp32 tiles (few rows).
+static void prompt_layer_small(Session& s, int layer, int n, int pos_base) {
+    const Model& m = *s.m;
+    const Shape& sh = m.shape;
+    const LayerWeights& w = m.layers[layer];
+    const int d = sh.d_model, F = sh.d_ff(), M = n * s.B;
+    const bool modern = sh.modern();
+    GemvParams g{};
+    g.kv = kv_layout(s);
+    g.layer = layer;
+    g.d_model = d;
+    g.st = s.st;
+    g.rows_per_seq = n;
+    g.pos_base = pos_base;
+    g.W = w.wqkv;
+    g.bias = w.bqkv;
+    g.N = 3 * d;
+    g.K = d;
+    g.in = s.pp_x;
+    g.in_stride = d;
+    g.gamma = w.g1;
+    g.beta = w.be1;
+    g.out = s.pp_q;
+    g.out_stride = d;
+    g.rope = modern;
+    g.rope_cos = m.rope_cos;
+    g.rope_sin = m.rope_sin;
+    if (modern) project_rows<PRO_RMSNORM, EPI_QKV>(s, g, M);
+    else project_rows<PRO_LAYERNORM, EPI_QKV>(s, g, M);
+
+    PrefillAttnParams a = prompt_attn_params(s, layer, n, pos_base);
+    a.out = s.pp_attn;
+    launch_prompt_attn(s, a);
+
+    g.W = w.wo;
+    g.bias = w.bo;
+    g.N = d;
+    g.K = d;
+    g.in = s.pp_attn;
+    g.in_stride = d;
+    g.out = s.pp_x;
+    g.out_stride = d;
+    project_rows<PRO_PLAIN, EPI_RESID>(s, g, M);
+
+    g.in = s.pp_x;
+    g.in_stride = d;
+    g.gamma = w.g2;
+    g.beta = w.be2;
+    g.out = s.pp_hidden;
+    g.out_stride = F;
+    g.W = w.w1;
+    g.K = d;
+    if (modern) {
+        g.bias = nullptr;
+        g.N = 2 * F;
+        project_rows<PRO_RMSNORM, EPI_SWIGLU>(s, g, M);
+    } else {
+        g.bias = w.b1;
+        g.N = F;
+        project_rows<PRO_LAYERNORM, EPI_GELU>(s, g, M);
     }
+    g.W = w.w2;
+    g.bias = modern ? nullptr : w.b2;
+    g.N = d;
+    g.K = F;
+    g.in = s.pp_hidden;
+    g.in_stride = F;
+    g.out = s.pp_x;
+    g.out_stride = d;
+    project_rows<PRO_PLAIN, EPI_RESID>(s, g, M);
+}
+
+// Activations of a prompt pass of up to `rows` rows (grown on demand).
+static void reserve_prompt_rows(Session& s, size_t rows) {
+    const size_t d = s.m->shape.d_model, F = s.m->shape.d_ff();
+    if (s.pp_rows >= rows) return;
+    for (float** b : {&s.pp_x, &s.pp_q, &s.pp_attn, &s.pp_norm, &s.pp_hidden}) {
+        if (*b) HIP_CHECK(hipFree(*b));
+        *b = nullptr;
+    }
+    for (char** b : {&s.pp_split, &s.pp_split_hidden}) {
+        if (*b) HIP_CHECK(hipFree(*b));
+        *b = nullptr;
+    }
+    s.pp_rows = 0;
+    dev_alloc(s.pp_x, rows * d);
+    dev_alloc(s.pp_q, rows * d);
+    const size_t few = std::min<size_t>(rows, kSplitMinRows);  // what the small tiles still take
+    dev_alloc(s.pp_attn, few * d);
+    dev_alloc(s.pp_norm, few * d);
+    dev_alloc(s.pp_hidden, few * F);
+    dev_alloc(s.pp_split, split_bytes(rows, d));
+    dev_alloc(s.pp_split_hidden, split_bytes(rows, F));
+    s.pp_rows = rows;
 }
 
 // Tokens hist[n_hist .. n_hist + len) of every sequence, positions pos .. pos + len.
@@ -1504,23 +1670,10 @@ static void score_rows(Session& s, const ScoreSink& sink, int M, int n, int t0, 
 static void prompt_pass(Session& s, int len, const ScoreSink* sink = nullptr) {
     const Model& m = *s.m;
     const Shape& sh = m.shape;
-    const int d = sh.d_model, F = sh.d_ff(), B = s.B;
-    const bool modern = sh.modern();
+    const int d = sh.d_model, B = s.B;
     hipStream_t st = s.stream;
     const int slice = static_cast<int>(std::max<size_t>(1, std::min<size_t>(len, kPromptPassRows / B)));
-    const size_t rows_cap = static_cast<size_t>(slice) * B;
-    if (s.pp_rows < rows_cap) {
-        for (float** b : {&s.pp_x, &s.pp_q, &s.pp_attn, &s.pp_norm, &s.pp_hidden}) {
-            if (*b) HIP_CHECK(hipFree(*b));
-            *b = nullptr;
-        }
-        dev_alloc(s.pp_x, rows_cap * d);
-        dev_alloc(s.pp_q, rows_cap * d);
-        dev_alloc(s.pp_attn, rows_cap * d);
-        dev_alloc(s.pp_norm, rows_cap * d);
-        dev_alloc(s.pp_hidden, rows_cap * F);
-        s.pp_rows = rows_cap;
-    }
+    reserve_prompt_rows(s, static_cast<size_t>(slice) * B);
     for (int t0 = 0; t0 < len; t0 += slice) {
         const int n = std::min(slice, len - t0);
         const int M = n * B;
@@ -1529,83 +1682,8 @@ static void prompt_pass(Session& s, int len, const ScoreSink* sink = nullptr) {
                            s.hist_stride, s.n_hist + t0, n, pos_base, s.pp_x, d);
         HIP_CHECK(hipGetLastError());
         for (int l = 0; l < sh.layers; l++) {
-            const LayerWeights& w = m.layers[l];
-            GemvParams g{};
-            g.kv = kv_layout(s);
-            g.layer = l;
-            g.d_model = d;
-            g.st = s.st;
-            g.rows_per_seq = n;
-            g.pos_base = pos_base;
-            g.W = w.wqkv;
-            g.bias = w.bqkv;
-            g.N = 3 * d;
-            g.K = d;
-            g.in = s.pp_x;
-            g.in_stride = d;
-            g.gamma = w.g1;
-            g.beta = w.be1;
-            g.out = s.pp_q;
-            g.out_stride = d;
-            g.rope = modern;
-            g.rope_cos = m.rope_cos;
-            g.rope_sin = m.rope_sin;
-            if (modern) project_rows<PRO_RMSNORM, EPI_QKV>(s, g, M);
-            else project_rows<PRO_LAYERNORM, EPI_QKV>(s, g, M);
-
-            PrefillAttnParams a{};
-            a.q = s.pp_q;
-            a.out = s.pp_attn;
-            a.kv = g.kv;
-            a.layer = l;
-            a.d_model = d;
-            a.len = n;
-            a.pos_base = pos_base;
-            a.scale = 1.0f / std::sqrt(static_cast<float>(sh.head_size()));
-            // from 512 tokens on, 128 queries per workgroup (16 sequences: 1000 tokens 512 against
-            // 585 us, 1536 tokens 860 against 977; at 300 tokens 76 against 60: too few workgroups)
-            if (n >= 512)
-                hipLaunchKernelGGL(attn_prefill128_kernel, dim3((n + 127) / 128, sh.heads, B), dim3(256), 0, st, a);
-            else
-                hipLaunchKernelGGL(attn_prefill64_kernel, dim3((n + 63) / 64, sh.heads, B), dim3(256), 0, st, a);
-            HIP_CHECK(hipGetLastError());
-
-            g.W = w.wo;
-            g.bias = w.bo;
-            g.N = d;
-            g.K = d;
-            g.in = s.pp_attn;
-            g.in_stride = d;
-            g.out = s.pp_x;
-            g.out_stride = d;
-            project_rows<PRO_PLAIN, EPI_RESID>(s, g, M);
-
-            g.in = s.pp_x;
-            g.in_stride = d;
-            g.gamma = w.g2;
-            g.beta = w.be2;
-            g.out = s.pp_hidden;
-            g.out_stride = F;
-            g.W = w.w1;
-            g.K = d;
-            if (modern) {
-                g.bias = nullptr;
-                g.N = 2 * F;
-                project_rows<PRO_RMSNORM, EPI_SWIGLU>(s, g, M);
-            } else {
-                g.bias = w.b1;
-                g.N = F;
-                project_rows<PRO_LAYERNORM, EPI_GELU>(s, g, M);
-            }
-            g.W = w.w2;
-            g.bias = modern ? nullptr : w.b2;
-            g.N = d;
-            g.K = F;
-            g.in = s.pp_hidden;
-            g.in_stride = F;
-            g.out = s.pp_x;
-            g.out_stride = d;
-            project_rows<PRO_PLAIN, EPI_RESID>(s, g, M);
+            if (M >= kSplitMinRows) prompt_layer_split(s, l, n, pos_base);
+            else prompt_layer_small(s, l, n, pos_base);
         }
         if (sink) score_rows(s, *sink, M, n, t0, len);
         if (t0 + n == len) {

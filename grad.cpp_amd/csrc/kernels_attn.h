@@ -7,7 +7,7 @@
 // softmax_row (:60-67).
 #pragma once
 
-#include "kernels_common.h"
+#include "kernels_split.h"
 
 namespace gh {
 
@@ -429,6 +429,7 @@ __global__ __launch_bounds__(256) void attn_decode64_kernel(const AttnParams p) 
 struct PrefillAttnParams {
     const float* q;  // [batch * len][d_model], rotated
     float* out;      // [batch * len][d_model]
+    char* out_split;  // when set: the output rows in split form instead (split_offset)
     KvLayout kv;
     int layer, d_model, len, pos_base;
     float scale;
@@ -446,7 +447,7 @@ struct PrefillAttnParams {
 // inference.cpp:211-225 computes the same numbers one query at a time.
 typedef float attn_v4f __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(256) void attn_prefill64_kernel(const PrefillAttnParams p) {
+static __global__ __launch_bounds__(256) void attn_prefill64_kernel(const PrefillAttnParams p) {
     constexpr int HS = 64, TILE = 64, LDK = HS + 4, LDV = TILE + 4;  // padded rows: float4 reads of 16 rows hit 64 banks
     __shared__ float Ks[TILE * LDK];  // [key][dim]
     __shared__ float Vt[HS * LDV];    // [dim][key]
@@ -556,6 +557,13 @@ __global__ __launch_bounds__(256) void attn_prefill64_kernel(const PrefillAttnPa
     }
     if (live) {
         const float inv = 1.0f / l;
+        if (p.out_split) {
+#pragma unroll
+            for (int db = 0; db < 4; db++)
+                store_split4(p.out_split, b * p.len + t, h * HS + db * 16 + g * 4, p.d_model / kSplitCols, o[db][0] * inv,
+                             o[db][1] * inv, o[db][2] * inv, o[db][3] * inv);
+            return;
+        }
         float* orow = p.out + (static_cast<size_t>(b) * p.len + t) * p.d_model + h * HS;
 #pragma unroll
         for (int db = 0; db < 4; db++)
@@ -584,7 +592,7 @@ __global__ __launch_bounds__(256) void attn_prefill64_kernel(const PrefillAttnPa
 // are 0.39; with scores in units of ln 2 and the hardware's 2^x it is 0.78 ms.
 typedef float attn_v16f __attribute__((ext_vector_type(16)));
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill128_kernel(const PrefillAttnParams p) {
+static __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill128_kernel(const PrefillAttnParams p) {
     constexpr int HS = 64, TILE = 64, QB = 128, LDK = HS + 4, LDV = TILE + 4;
     __shared__ float Ks[TILE * LDK];  // [key][dim]
     __shared__ float Vt[HS * LDV];    // [dim][key]
@@ -748,6 +756,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     if (live) {
         const float inv = 1.0f / l;
+        if (p.out_split) {
+#pragma unroll
+            for (int db = 0; db < 2; db++)
+#pragma unroll
+                for (int q4 = 0; q4 < 4; q4++)
+                    store_split4(p.out_split, b * p.len + t, h * HS + db * 32 + q4 * 8 + h32 * 4, p.d_model / kSplitCols,
+                                 o[db][4 * q4 + 0] * inv, o[db][4 * q4 + 1] * inv, o[db][4 * q4 + 2] * inv,
+                                 o[db][4 * q4 + 3] * inv);
+            return;
+        }
         float* orow = p.out + (static_cast<size_t>(b) * p.len + t) * p.d_model + h * HS;
 #pragma unroll
         for (int db = 0; db < 2; db++)

@@ -14,7 +14,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 // h[m] = norm(x[m]) for every row (layer_norm_row, inference.cpp:30-58).
 // One wavefront per row; kind is PRO_LAYERNORM or PRO_RMSNORM.
-__global__ __launch_bounds__(256) void norm_rows_kernel(const float* __restrict__ x,
+static __global__ __launch_bounds__(256) void norm_rows_kernel(const float* __restrict__ x,
                                                         const float* __restrict__ gamma,
                                                         const float* __restrict__ beta, float* h,
                                                         int M, int d, int kind) {

@@ -331,7 +331,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvParams p) {
 
 // x[b] = E[token[b]] * 1.0 (+ P[pos]) — inference.cpp:159-182 (the embedding
 // scale is 1.0, token_embedding.h:12).
-__global__ void embed_kernel(const float* __restrict__ E, const float* __restrict__ P,
+static __global__ void embed_kernel(const float* __restrict__ E, const float* __restrict__ P,
                              const int* __restrict__ tok, const DevState* st, float* x, int d) {
     const int b = blockIdx.y;
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
@@ -343,7 +343,7 @@ __global__ void embed_kernel(const float* __restrict__ E, const float* __restric
 
 // The same for every token of a prompt pass: row m = seq * len + t holds token
 // t of sequence seq, at position pos_base + t.
-__global__ void embed_rows_kernel(const float* __restrict__ E, const float* __restrict__ P,
+static __global__ void embed_rows_kernel(const float* __restrict__ E, const float* __restrict__ P,
                                   const int* __restrict__ hist, int hist_stride, int hist_base, int len,
                                   int pos_base, float* x, int d) {
     const int m = blockIdx.y;
@@ -357,7 +357,7 @@ __global__ void embed_rows_kernel(const float* __restrict__ E, const float* __re
 }
 
 // rows[b] = x[b * len + len - 1]: the last position of every sequence.
-__global__ void take_last_rows_kernel(const float* __restrict__ x, int len, float* rows, int d) {
+static __global__ void take_last_rows_kernel(const float* __restrict__ x, int len, float* rows, int d) {
     const int b = blockIdx.y;
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j < d) rows[static_cast<size_t>(b) * d + j] = x[(static_cast<size_t>(b) * len + len - 1) * d + j];
@@ -369,7 +369,7 @@ __global__ void take_last_rows_kernel(const float* __restrict__ x, int len, floa
 // workgroup per row; row r of this launch is row `row0 + r` of a prompt pass
 // whose row m = seq * slice_len + t holds position t0 + t of sequence seq.
 // nll[seq * len + t0 + t] = log(sum_j exp(x_j - max)) + max - x_target.
-__global__ __launch_bounds__(256) void nll_rows_kernel(const float* __restrict__ logits, int V, int row0,
+static __global__ __launch_bounds__(256) void nll_rows_kernel(const float* __restrict__ logits, int V, int row0,
                                                        int slice_len, int t0, int len,
                                                        const int* __restrict__ targets, float* __restrict__ nll) {
     __shared__ float scratch[4];

@@ -995,7 +995,7 @@ __global__ __launch_bounds__(kPickThreads) void pick_kernel(const PickParams p) 
 // the token in the history and writes the step's input row.
 constexpr int kArgmaxThreads = 256;
 
-__global__ __launch_bounds__(kArgmaxThreads) void argmax_embed_kernel(const float2* __restrict__ best, int n16,
+static __global__ __launch_bounds__(kArgmaxThreads) void argmax_embed_kernel(const float2* __restrict__ best, int n16,
                                                                       const DevState* st, int* hist, int hist_stride,
                                                                       int* tok, const float* __restrict__ E,
                                                                       const float* __restrict__ P, float* x, int d) {

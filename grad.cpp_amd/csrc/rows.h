@@ -1,0 +1,30 @@
+// Host side of the many-row projections (kernels_split.h).
+#pragma once
+
+#include "kernels_split.h"
+
+namespace gh {
+
+constexpr int kSplitPad = 128;  // rows of a split matrix are allocated in whole tiles of this many
+
+inline size_t split_bytes(size_t rows, size_t cols) {
+    return (rows + kSplitPad - 1) / kSplitPad * kSplitPad * cols * 6;
+}
+
+// Writes the split form of src (N x K); gate_up: src rows are (gate, up) pairs.
+void split_weights(const float* src, int N, int K, bool gate_up, char* dst, hipStream_t st);
+
+// norm(x) of M rows in split form.
+void norm_split(bool rms, const float* x, const float* gamma, const float* beta, char* out, int M, int d, hipStream_t st);
+
+// One projection; p.n_tiles, p.tiles (and p.nll_stride) are filled in.  EPI_STORE: scoring.
+template <int EPI>
+void split_gemm(SplitGemmParams& p, hipStream_t st);
+
+// Widest run of partial results per row that split_gemm<EPI_STORE> leaves.
+inline int split_nll_stride(int N) { return (N + kSplitPad - 1) / kSplitPad * 4; }
+
+// nll of M scored rows from those partial results.
+void nll_parts(const SplitGemmParams& p, float* nll, hipStream_t st);
+
+}  // namespace gh

@@ -4,6 +4,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 PKG = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(PKG, "csrc")
@@ -14,11 +15,12 @@ LIB = os.path.join(LIB_DIR, "libgradhip.so")
 # wrong results on this hardware pool.  No fast-math: GELU/SiLU/softmax/RoPE use
 # the precise expf/tanhf.
 HIPCC_FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
+    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-fno-fast-math", "-Wall", "-Wno-unused-function", *os.environ.get("GRADHIP_EXTRA_FLAGS", "").split(),
 ]
-SOURCES = ["engine.hip", "checkpoint.cpp", "tokenizer.cpp"]
+SOURCES = ["engine.hip", "persist.hip", "xcd.hip", "checkpoint.cpp", "tokenizer.cpp"]
+OBJ_DIR = os.path.join(PKG, "build")
 
 
 BIN_DIR = os.path.join(PKG, "bin")
@@ -29,10 +31,20 @@ INCLUDE = os.path.join(os.path.dirname(PKG), "include")
 def build(verbose: bool = True) -> str:
     os.makedirs(LIB_DIR, exist_ok=True)
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    cmd = [hipcc, *HIPCC_FLAGS, "-o", LIB, *[os.path.join(CSRC, s) for s in SOURCES]]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    subprocess.check_call(cmd)
+    os.makedirs(OBJ_DIR, exist_ok=True)
+
+    def compile_one(src: str) -> str:
+        obj = os.path.join(OBJ_DIR, src + ".o")
+        cmd = [hipcc, *HIPCC_FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        subprocess.check_call(cmd)
+        return obj
+
+    # the translation units do not share device code: compile them side by side
+    with ThreadPoolExecutor(len(SOURCES)) as pool:
+        objs = list(pool.map(compile_one, SOURCES))
+    subprocess.check_call([hipcc, "--offload-arch=gfx950", "-shared", "-o", LIB, *objs])
     # the command-line caller: plain C++ over the header-only adapter
     os.makedirs(BIN_DIR, exist_ok=True)
     for src, exe in (("generate.cpp", CLI), ("chat.cpp", os.path.join(BIN_DIR, "gradhip-chat")),

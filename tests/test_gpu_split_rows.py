@@ -1,0 +1,38 @@
+"""Passes over many rows (prompts and scoring) on the split bf16 products: every tiling the rows
+can take, at row counts that leave ragged tiles, against the float64 forward.  The bound is
+what fp32 sums give, an order below the engine's common 1e-4."""
+import numpy as np
+import pytest
+
+import gradhip as G
+import ref_forward
+from gradhip import synth
+from helpers import lively_std
+
+pytestmark = pytest.mark.gpu
+
+CASES = {
+    # name: (config, batch, tokens per sequence)
+    "one-block-per-set": (synth.Config(synth.ARCH_MODERN, 37, 64, 2, 1, 200), 1, 161),       # K = 64, 32 x 32 tiles
+    "32-gpt2": (synth.Config(synth.ARCH_GPT2, 301, 128, 2, 2, 200), 1, 193),
+    "64-k4-modern": (synth.Config(synth.ARCH_MODERN, 1000, 256, 2, 4, 192), 4, 159),         # hidden width 704: 11 blocks per set
+    "64-gpt2": (synth.Config(synth.ARCH_GPT2, 1001, 256, 1, 4, 200), 12, 150),               # one set over all of K
+    "128-modern": (synth.Config(synth.ARCH_MODERN, 530, 192, 1, 3, 1100), 24, 1057),         # 24 k rows
+    "128-gpt2": (synth.Config(synth.ARCH_GPT2, 515, 128, 1, 2, 2100), 17, 2049),             # two slices of rows
+}
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_rows_match_the_float64_forward(name):
+    cfg, B, n = CASES[name]
+    W = synth.make_weights(cfg, 71, std=lively_std(cfg), norm_noise=0.1)
+    gm = G.Model.from_tensors(cfg, W)
+    tokens = synth.uniform_tokens(B * (n + 1), cfg.vocab, 72).reshape(B, n + 1)
+    nll = G.Session(gm, batch=B).score(tokens[:, :-1], tokens[:, 1:])
+    last = G.Session(gm, batch=B).prefill(tokens[:, :-1])
+    for b in sorted({0, B - 1}):
+        ref = ref_forward.forward(cfg, W, tokens[b, :-1])
+        top = ref.max(axis=1)
+        want = np.log(np.exp(ref - top[:, None]).sum(axis=1)) + top - ref[np.arange(n), tokens[b, 1:]]
+        assert np.abs(nll[b] - want).max() <= 2e-5 * max(1.0, np.abs(want).max()), (name, b)
+        assert np.abs(last[b] - ref[-1]).max() <= 1e-5 * np.abs(ref[-1]).max(), (name, b)
