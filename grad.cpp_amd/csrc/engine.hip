@@ -121,7 +121,11 @@ struct LayerWeights {
     float *w1, *b1;      // GPT-2: (F, d), F.  Modern: (2F, d) rows (gate_p, up_p) interleaved
     float *w2, *b2;      // (d, F), d (GPT-2 only)
     float *g1, *be1, *g2, *be2;
-    char *s_wqkv, *s_wo, *s_w1, *s_w2;  // split forms for passes over many rows (kernels_split.h)
+};
+
+// The split forms of a layer's matrices, for passes over many rows (kernels_split.h).
+struct SplitLayer {
+    char *wqkv, *wo, *w1, *w2;
 };
 
 // Where tensor i of the file lives on the device.
@@ -142,8 +146,13 @@ struct Model {
     float *gf = nullptr, *bf = nullptr;
     float *rope_cos = nullptr, *rope_sin = nullptr;  // (max_len, head_size/2)
     std::vector<Placement> place;                    // file order
-    char* split_blob = nullptr;  // split forms of the matrices; null for shapes without a prompt pass
-    char* s_E = nullptr;
+
+    // Split forms of the matrices: six bytes per weight beside the four above, written by the
+    // first pass over many rows (split_model) and kept.
+    mutable std::mutex split_mutex;
+    mutable char* split_blob = nullptr;
+    mutable char* split_E = nullptr;
+    mutable std::vector<SplitLayer> split_layers;
 
     // The XCD-sharded persistent kernel reads the weights from a second copy laid
     // out as one contiguous stream per workgroup (kernels_xcd.h); built by the
@@ -209,7 +218,7 @@ static void plan_model(Model& m) {
         LayerWeights& w = m.layers[l];
         w = {B + lo[l].wqkv, B + lo[l].bqkv, B + lo[l].wo, B + lo[l].bo, B + lo[l].w1,
              B + lo[l].b1,   B + lo[l].w2,   B + lo[l].b2, B + lo[l].g1, B + lo[l].be1,
-             B + lo[l].g2,   B + lo[l].be2,  nullptr,      nullptr,      nullptr,      nullptr};
+             B + lo[l].g2,   B + lo[l].be2};
         for (int q = 0; q < 3; q++) m.place.push_back({w.wqkv + q * d * d, true, 1, 0});
         m.place.push_back({w.wo, true, 1, 0});
         for (int q = 0; q < 3; q++) m.place.push_back({w.bqkv + q * d, false, 1, 0});
@@ -244,14 +253,14 @@ static bool rows_shape_ok(const Shape& sh) {
     return sh.head_size() == 64 && sh.d_model % 64 == 0 && sh.d_ff() % 64 == 0 && sh.d_model <= 4096;
 }
 
-// The second form of every matrix that passes over many rows read: six bytes per weight,
-// written once, here.
-static void split_model(Model& m) {
+// Writes the second form of every matrix, once per model.
+static void split_model(const Model& m) {
+    std::lock_guard<std::mutex> lock(m.split_mutex);
+    if (m.split_E) return;
     const Shape& sh = m.shape;
-    if (!rows_shape_ok(sh)) return;
     const int d = sh.d_model, F = sh.d_ff(), up = sh.modern() ? 2 : 1;
     const size_t per_layer = split_bytes(3 * d, d) + split_bytes(d, d) + split_bytes(up * F, d) + split_bytes(d, F);
-    HIP_CHECK(hipMalloc(&m.split_blob, sh.layers * per_layer + split_bytes(sh.vocab, d)));
+    if (!m.split_blob) HIP_CHECK(hipMalloc(&m.split_blob, sh.layers * per_layer + split_bytes(sh.vocab, d)));
     char* at = m.split_blob;
     const auto place = [&](const float* src, int N, int K, bool gate_up) {
         split_weights(src, N, K, gate_up, at, nullptr);
@@ -259,14 +268,18 @@ static void split_model(Model& m) {
         at += split_bytes(N, K);
         return here;
     };
-    for (LayerWeights& w : m.layers) {
-        w.s_wqkv = place(w.wqkv, 3 * d, d, false);
-        w.s_wo = place(w.wo, d, d, false);
-        w.s_w1 = place(w.w1, up * F, d, sh.modern());
-        w.s_w2 = place(w.w2, d, F, false);
+    m.split_layers.clear();
+    for (const LayerWeights& w : m.layers) {
+        SplitLayer l;
+        l.wqkv = place(w.wqkv, 3 * d, d, false);
+        l.wo = place(w.wo, d, d, false);
+        l.w1 = place(w.w1, up * F, d, sh.modern());
+        l.w2 = place(w.w2, d, F, false);
+        m.split_layers.push_back(l);
     }
-    m.s_E = place(m.E, sh.vocab, d, false);
+    char* const E = place(m.E, sh.vocab, d, false);
     HIP_CHECK(hipDeviceSynchronize());
+    m.split_E = E;
 }
 
 static std::unique_ptr<Model> upload_model(const Shape& shape, const std::vector<const float*>& t,
@@ -325,7 +338,6 @@ static std::unique_ptr<Model> upload_model(const Shape& shape, const std::vector
             HIP_CHECK(hipMemcpy(m->rope_sin, sn.data(), sn.size() * 4, hipMemcpyHostToDevice));
         }
     }
-    split_model(*m);
     return m;
 }
 
@@ -408,6 +420,10 @@ struct Session {
     float *pp_x = nullptr, *pp_q = nullptr, *pp_attn = nullptr, *pp_norm = nullptr, *pp_hidden = nullptr;
     char *pp_split = nullptr, *pp_split_hidden = nullptr;  // split rows of d_model and of d_ff columns
     size_t pp_rows = 0;
+    char* pp_kv = nullptr;  // split keys and values of the layer at hand
+    size_t pp_kv_bytes = 0;
+    float* pp_part = nullptr;  // partial attention results
+    size_t pp_part_floats = 0;
     float2* nll_part = nullptr;  // [pp_rows][split_nll_stride(vocab)] of rows being scored
     float* nll_target = nullptr;  // [pp_rows]
     size_t nll_rows = 0;
@@ -491,7 +507,7 @@ struct Session {
                         static_cast<void*>(ctl), static_cast<void*>(pp_x), static_cast<void*>(pp_q),
                         static_cast<void*>(pp_attn), static_cast<void*>(pp_norm),
                         static_cast<void*>(pp_hidden), static_cast<void*>(pp_split),
-                        static_cast<void*>(pp_split_hidden), static_cast<void*>(nll_part),
+                        static_cast<void*>(pp_split_hidden), static_cast<void*>(pp_kv), static_cast<void*>(pp_part), static_cast<void*>(nll_part),
                         static_cast<void*>(nll_target)})
             if (p) (void)hipFree(p);
         if (host_logits) (void)hipHostFree(host_logits);
@@ -1427,10 +1443,14 @@ static bool prompt_pass_ok(const Session& s, int len) {
 }
 
 // Passes of this many rows and more take the split projections (kernels_split.h); below,
-// the small fp32 tiles of the decode step, whose norms ride inside the projections (one
-// sequence of the 69M Llama block: 96 tokens 588 us against 619, 128: 627 against 654, 244:
-// 820 against 664).
-constexpr int kSplitMinRows = 160;
+// the small fp32 tiles of the decode step, whose norms ride inside the projections.  Speed
+// alone puts the line at 160 rows (one sequence of the 69M Llama block: 128 tokens 627 us
+// against 654, 244 tokens 820 against 664), and for scoring it lies there.  A prompt that is
+// continued stays on the fp32 sums up to 512 rows: an unfiltered draw over a flat distribution
+// of 16000 tokens falls within an fp32 rounding of the next token's boundary about once in a
+// hundred picks, so the order of a prompt's sums shows in the reply, and under 512 rows the
+// prompt is the small part of the request (397 tokens and 64 sampled ones: 1.4 of 12.5 ms).
+constexpr int kSplitMinRows = 512, kSplitMinScoreRows = 160;
 
 // One projection over M rows (norm folded in for RMSNorm, a norm kernel for LayerNorm).
 template <int PRO, int EPI>
@@ -1485,7 +1505,7 @@ static void score_rows(Session& s, const ScoreSink& sink, int M, int n, int t0, 
         s.nll_rows = M;
     }
     norm_split(sh.modern(), s.pp_x, m.gf, m.bf, s.pp_split, M, sh.d_model, s.stream);
-    SplitGemmParams g = split_params(s.pp_split, m.s_E, M, sh.vocab, sh.d_model);
+    SplitGemmParams g = split_params(s.pp_split, m.split_E, M, sh.vocab, sh.d_model);
     g.rows_per_seq = n;
     g.targets = sink.targets;
     g.nll_t0 = t0;
@@ -1509,14 +1529,13 @@ static PrefillAttnParams prompt_attn_params(const Session& s, int layer, int n, 
     return a;
 }
 
+// Up to this many new tokens per sequence the fp32 kernel does a split pass's attention as
+// well: splitting a context's keys and values costs as much as so few queries read of them
+// (64 sequences of 128 tokens 48 us against 56, 13 of 77 10 against 18; 8 of 256 36 against 27).
+constexpr int kSplitAttnMin = 128;
+
 static void launch_prompt_attn(const Session& s, const PrefillAttnParams& a) {
-    const int heads = s.m->shape.heads;
-    // from 512 tokens on, 128 queries per workgroup (16 sequences: 1000 tokens 512 against
-    // 585 us, 1536 tokens 860 against 977; at 300 tokens 76 against 60: too few workgroups)
-    if (a.len >= 512)
-        hipLaunchKernelGGL(attn_prefill128_kernel, dim3((a.len + 127) / 128, heads, s.B), dim3(256), 0, s.stream, a);
-    else
-        hipLaunchKernelGGL(attn_prefill64_kernel, dim3((a.len + 63) / 64, heads, s.B), dim3(256), 0, s.stream, a);
+    hipLaunchKernelGGL(attn_prefill64_kernel, dim3((a.len + 63) / 64, s.m->shape.heads, s.B), dim3(256), 0, s.stream, a);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -1525,11 +1544,12 @@ static void prompt_layer_split(Session& s, int layer, int n, int pos_base) {
     const Model& m = *s.m;
     const Shape& sh = m.shape;
     const LayerWeights& w = m.layers[layer];
+    const SplitLayer& sw = m.split_layers[layer];
     const int d = sh.d_model, F = sh.d_ff(), M = n * s.B;
     hipStream_t st = s.stream;
 
     norm_split(sh.modern(), s.pp_x, w.g1, w.be1, s.pp_split, M, d, st);
-    SplitGemmParams g = split_params(s.pp_split, w.s_wqkv, M, 3 * d, d);
+    SplitGemmParams g = split_params(s.pp_split, sw.wqkv, M, 3 * d, d);
     g.bias = w.bqkv;
     g.out = s.pp_q;
     g.out_stride = d;
@@ -1545,23 +1565,24 @@ static void prompt_layer_split(Session& s, int layer, int n, int pos_base) {
 
     PrefillAttnParams a = prompt_attn_params(s, layer, n, pos_base);
     a.out_split = s.pp_split;
-    launch_prompt_attn(s, a);
+    if (n > kSplitAttnMin) split_attention(a, s.B, s.pp_kv, s.pp_part, st);
+    else launch_prompt_attn(s, a);
 
-    g = split_params(s.pp_split, w.s_wo, M, d, d);
+    g = split_params(s.pp_split, sw.wo, M, d, d);
     g.bias = w.bo;
     g.out = s.pp_x;
     g.out_stride = d;
     split_gemm<EPI_RESID>(g, st);
 
     norm_split(sh.modern(), s.pp_x, w.g2, w.be2, s.pp_split, M, d, st);
-    g = split_params(s.pp_split, w.s_w1, M, sh.modern() ? 2 * F : F, d);
+    g = split_params(s.pp_split, sw.w1, M, sh.modern() ? 2 * F : F, d);
     g.bias = sh.modern() ? nullptr : w.b1;
     g.out_split = s.pp_split_hidden;
     g.out_kblocks = F / kSplitCols;
     if (sh.modern()) split_gemm<EPI_SWIGLU>(g, st);
     else split_gemm<EPI_GELU>(g, st);
 
-    g = split_params(s.pp_split_hidden, w.s_w2, M, d, F);
+    g = split_params(s.pp_split_hidden, sw.w2, M, d, F);
     g.bias = sh.modern() ? nullptr : w.b2;
     g.out = s.pp_x;
     g.out_stride = d;
@@ -1664,6 +1685,26 @@ static void reserve_prompt_rows(Session& s, size_t rows) {
     s.pp_rows = rows;
 }
 
+// Scratch of a split pass's attention over n new positions behind pos_base (grown on demand).
+static void reserve_split_attention(Session& s, int n, int pos_base) {
+    if (n <= kSplitAttnMin) return;
+    const SplitAttnSpace need = split_attention_space(s.B, s.m->shape.heads, n, pos_base);
+    if (s.pp_kv_bytes < need.kv_bytes) {
+        if (s.pp_kv) HIP_CHECK(hipFree(s.pp_kv));
+        s.pp_kv = nullptr;
+        s.pp_kv_bytes = 0;
+        dev_alloc(s.pp_kv, need.kv_bytes);
+        s.pp_kv_bytes = need.kv_bytes;
+    }
+    if (s.pp_part_floats < need.part_floats) {
+        if (s.pp_part) HIP_CHECK(hipFree(s.pp_part));
+        s.pp_part = nullptr;
+        s.pp_part_floats = 0;
+        dev_alloc(s.pp_part, need.part_floats);
+        s.pp_part_floats = need.part_floats;
+    }
+}
+
 // Tokens hist[n_hist .. n_hist + len) of every sequence, positions pos .. pos + len.
 // Equivalent to len step() calls (text_gen.cpp:44-46); only the last logits are
 // formed unless a sink asks for the likelihood of a target at every position.
@@ -1678,11 +1719,14 @@ static void prompt_pass(Session& s, int len, const ScoreSink* sink = nullptr) {
         const int n = std::min(slice, len - t0);
         const int M = n * B;
         const int pos_base = s.pos + t0;
+        const bool split = M >= (sink ? kSplitMinScoreRows : kSplitMinRows);
+        if (split || sink) split_model(m);
+        if (split) reserve_split_attention(s, n, pos_base);
         hipLaunchKernelGGL(embed_rows_kernel, dim3((d + 255) / 256, M), dim3(256), 0, st, m.E, m.P, s.hist,
                            s.hist_stride, s.n_hist + t0, n, pos_base, s.pp_x, d);
         HIP_CHECK(hipGetLastError());
         for (int l = 0; l < sh.layers; l++) {
-            if (M >= kSplitMinRows) prompt_layer_split(s, l, n, pos_base);
+            if (split) prompt_layer_split(s, l, n, pos_base);
             else prompt_layer_small(s, l, n, pos_base);
         }
         if (sink) score_rows(s, *sink, M, n, t0, len);

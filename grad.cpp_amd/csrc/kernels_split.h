@@ -276,34 +276,25 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
         const unsigned g = at / kSplitBlockBytes;
         src[i] = g * (row_blocks * kSplitBlockBytes) + (at - g * kSplitBlockBytes);
     }
-    const auto issue = [&](int step, int stage) {
-        const char* a_at = a_base + static_cast<size_t>(step) * kSplitBlockBytes;
-        const char* w_at = w_base + static_cast<size_t>(step) * kSplitBlockBytes;
-#pragma unroll
-        for (int i = 0; i < kLoads; i++) {
-            const int u = min(wave + i * kWaves, kUnits - 1);
-            load_to_lds(u < kUnitsA ? a_at : w_at, src[i], lds0 + stage * kStage + u * 1024);
-        }
+    const auto issue_one = [&](int i, int step, int stage) {
+        const int u = min(wave + i * kWaves, kUnits - 1);
+        const char* at = (u < kUnitsA ? a_base : w_base) + static_cast<size_t>(step) * kSplitBlockBytes;
+        load_to_lds(at, src[i], lds0 + stage * kStage + u * 1024);
     };
     // operand reads: row lane % 32 of a 32-row block, columns 8 (lane / 32) .. + 7
     const int r32 = lane & 31, h32 = lane >> 5;
     const int chunk_at = r32 * kSplitRowBytes + ((h32 ^ ((r32 >> 3) & 1)) << 4);
-    struct Fragments {
-        v8bf w[NB][3], a[MB][3];
+    // the parts of the rows of A and W of a step
+    v8bf a0[MB], a1[MB], a2[MB], w0[NB], w1[NB], w2[NB];
+    const auto read_a = [&](int stage, int q, v8bf (&f)[MB]) {
+        const char* at = lds_split + (kg * STAGES + stage) * kStage + chunk_at + q * kSplitPartBytes;
+#pragma unroll
+        for (int x = 0; x < MB; x++) f[x] = *reinterpret_cast<const v8bf*>(at + (wm * MB + x) * 2 * kSplitBlockBytes);
     };
-    const auto read = [&](int stage, Fragments& f) {
-        const char* at = lds_split + (kg * STAGES + stage) * kStage + chunk_at;
+    const auto read_w = [&](int stage, int q, v8bf (&f)[NB]) {
+        const char* at = lds_split + (kg * STAGES + stage) * kStage + chunk_at + q * kSplitPartBytes + TM / kSplitRows * kSplitBlockBytes;
 #pragma unroll
-        for (int b = 0; b < MB; b++)
-#pragma unroll
-            for (int q = 0; q < 3; q++)
-                f.a[b][q] = *reinterpret_cast<const v8bf*>(at + (wm * MB + b) * 2 * kSplitBlockBytes + q * kSplitPartBytes);
-        at += TM / kSplitRows * kSplitBlockBytes;
-#pragma unroll
-        for (int a = 0; a < NB; a++)
-#pragma unroll
-            for (int q = 0; q < 3; q++)
-                f.w[a][q] = *reinterpret_cast<const v8bf*>(at + (wn * NB + a) * 2 * kSplitBlockBytes + q * kSplitPartBytes);
+        for (int x = 0; x < NB; x++) f[x] = *reinterpret_cast<const v8bf*>(at + (wn * NB + x) * 2 * kSplitBlockBytes);
     };
     // The products of the first parts and the other five in accumulators of their own: what
     // rounds in a sum of K products is the large running value, and the small products, added to
@@ -315,43 +306,67 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
         for (int b = 0; b < MB; b++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[a][b][r] = low[a][b][r] = 0.0f;
-    const auto multiply = [&](const Fragments& f) {
-        constexpr int kW[6] = {0, 0, 1, 1, 0, 2}, kA[6] = {0, 1, 0, 1, 2, 0};
+    const auto multiply = [&](const v8bf (&w)[NB], const v8bf (&x)[MB], v16f (&sum)[NB][MB]) {
 #pragma unroll
-        for (int t = 0; t < 6; t++)
+        for (int a = 0; a < NB; a++)
 #pragma unroll
-            for (int a = 0; a < NB; a++)
-#pragma unroll
-                for (int b = 0; b < MB; b++) {
-                    v16f& sum = t == 0 ? acc[a][b] : low[a][b];
-                    sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[a][kW[t]], f.a[b][kA[t]], sum, 0, 0, 0);
-                }
+            for (int b = 0; b < MB; b++) sum[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[a], x[b], sum[a][b], 0, 0, 0);
     };
 
 #pragma unroll
     for (int s = 0; s < STAGES; s++)
-        if (s < kblocks) issue(s, s);
+        if (s < kblocks) {
+#pragma unroll
+            for (int i = 0; i < kLoads; i++) issue_one(i, s, s);
+        }
     if (kblocks >= STAGES) wait_loads<(STAGES - 1) * kLoads>();
     else wait_loads<0>();
     meet();
-    Fragments f[2];
-    read(0, f[0]);
+    read_w(0, 0, w0);
+    read_a(0, 2, a2);
+    read_a(0, 1, a1);
+    read_w(0, 1, w1);
+    // A step's six rounds of products, in an order that uses up one part after the other, so
+    // that a part of the next step is read into the registers of this step's a round or two
+    // before it is needed (with every part in two places the 64 x 64 wavefronts run out of
+    // registers).  Reads and loads go out between the rounds: all at once behind the meeting
+    // they held up the first product of every wavefront.  One path through the loop: a second
+    // copy of the products would hold the accumulators in other registers.
     int stage = 0;
-    // one step: `now` is in registers, `then` is read for the step after it
-    const auto step = [&](int s, const Fragments& now, Fragments& then) {
-        if (s + 1 < kblocks) {
-            if (s + STAGES <= kblocks) wait_loads<(STAGES - 2) * kLoads>();
-            else wait_loads<0>();
-            meet();
-            if (s + STAGES < kblocks) issue(s + STAGES, stage);  // everyone has read this step's place
-            stage = stage == STAGES - 1 ? 0 : stage + 1;
-            read(stage, then);
-        }
-        multiply(now);
-    };
-    for (int s = 0; s < kblocks; s += 2) {  // (an odd number of blocks: one step less at the end)
-        step(s, f[0], f[1]);
-        if (s + 1 < kblocks) step(s + 1, f[1], f[0]);
+    for (int s = 0; s < kblocks; s++) {
+        const int next = stage == STAGES - 1 ? 0 : stage + 1;
+        const bool more = s + STAGES < kblocks;
+        const auto send = [&](int t) {  // a quarter of the loads of step s + STAGES, into this step's place
+            constexpr int kPer = (kLoads + 3) / 4;
+            if (more) {
+#pragma unroll
+                for (int i = t * kPer; i < (t + 1) * kPer; i++)
+                    if (i < kLoads) issue_one(i, s + STAGES, stage);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        multiply(w0, a2, low);
+        read_w(stage, 2, w2);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(w0, a1, low);
+        read_a(stage, 0, a0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (STAGES > 2 && s + STAGES <= kblocks) wait_loads<(STAGES - 2) * kLoads>();  // step s + 1 is here
+        else wait_loads<0>();
+        meet();  // ... for everyone, and everyone has read this step's place
+        multiply(w0, a0, acc);
+        read_a(next, 2, a2);
+        send(0);
+        multiply(w1, a1, low);
+        read_w(next, 0, w0);
+        send(1);
+        multiply(w1, a0, low);
+        read_a(next, 1, a1);
+        send(2);
+        multiply(w2, a0, low);
+        read_w(next, 1, w1);
+        send(3);
+        stage = next;
     }
 #pragma unroll
     for (int a = 0; a < NB; a++)

@@ -1,6 +1,7 @@
 // Host side of the many-row projections (kernels_split.h).
 #pragma once
 
+#include "kernels_attn.h"
 #include "kernels_split.h"
 
 namespace gh {
@@ -20,6 +21,14 @@ void norm_split(bool rms, const float* x, const float* gamma, const float* beta,
 // One projection; p.n_tiles, p.tiles (and p.nll_stride) are filled in.  EPI_STORE: scoring.
 template <int EPI>
 void split_gemm(SplitGemmParams& p, hipStream_t st);
+
+// Causal attention of p.len new positions of every sequence over the cache, output rows in split form.
+// kv and part: scratch of the sizes split_attention_space names, for the length of the call.
+struct SplitAttnSpace {
+    size_t kv_bytes, part_floats;
+};
+SplitAttnSpace split_attention_space(int batch, int heads, int len, int pos_base);
+void split_attention(const PrefillAttnParams& p, int batch, char* kv, float* part, hipStream_t st);
 
 // Widest run of partial results per row that split_gemm<EPI_STORE> leaves.
 inline int split_nll_stride(int N) { return (N + kSplitPad - 1) / kSplitPad * 4; }

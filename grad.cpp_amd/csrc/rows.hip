@@ -2,6 +2,8 @@
 // their own.
 #include "rows.h"
 
+#include "kernels_split_attn.h"
+
 #include <stdexcept>
 #include <string>
 
@@ -32,26 +34,26 @@ void norm_split(bool rms, const float* x, const float* gamma, const float* beta,
     else norm_split_as<false>(x, gamma, beta, out, M, d, st);
 }
 
-// Which tiling.  Measured over 16 row counts from 128 to 8192 against six matrices (768 and
-// 512 columns: 768, 2304, 4096, 512 outputs; 2048 columns: 768, 512 outputs), the rule takes the
-// fastest of the four or one within 7 % of it:
-// - While 32 x 32 tiles leave no compute unit with two, they win, and after them 64 x 64 tiles
-//   with K over four sets of wavefronts: such a launch is a chain of K steps of about 280 ns
-//   each (load, LDS, registers, product), so the shorter chain is what counts (1001 x 768 x
-//   2048: 26 us against 39 with K in one set; 100 x 768 x 2048: 13 against 22).
-// - With more tiles than compute units the chains hide behind each other.  A compute unit's
-//   time per step is 190 ns for a 64 x 64 tile and 624 ns for a 128 x 128 one, which moves half as
-//   many operands per product; the cheaper one once tiles are dealt to 256 compute units in
-//   whole rounds (4096 x 2304 x 768: 87 us against 95; 8192 x 4096 x 768: 263, i.e. 196 TFLOP/s of
-//   fp32 products or 1.18 PFLOP/s of bf16, against 292).
+// Which tiling.  Measured over 14 row counts from 160 to 8192 against five matrices (768
+// columns: 768, 2304, 4096 outputs; 2048 columns: 768, 512 outputs), the rule takes the fastest
+// of the four or one within 6 % of it:
+// - With two 32 x 32 tiles per compute unit at most they win, K shared by four sets of
+//   wavefronts, and after them 64 x 64 tiles with K shared the same way: such a launch is a chain
+//   of K steps of about 250 ns each (load, LDS, registers, product), so the shorter chain is what
+//   counts (1001 x 768 x 2048: 25 us against 35 with K in one set; 160 x 768 x 2048: 11 against 21).
+// - With more tiles than compute units the chains hide behind each other.  Tiles are dealt to 256
+//   compute units in whole rounds, and a round of 128 x 128 tiles costs 2.8 times one of 64 x 64
+//   (four times the products, half the operand bytes per product): the cheaper one
+//   (6000 x 768 x 2048: 120 us against 126; 8192 x 4096 x 768: 247, i.e. 208 TFLOP/s of fp32 products
+//   or 1.25 PFLOP/s of bf16, against 303).
 enum Tiling { TILE_32_K4, TILE_64_K4, TILE_64, TILE_128 };
 
 static Tiling pick_tiling(int M, int N) {
     const auto tiles = [&](int t) { return static_cast<long>((M + t - 1) / t) * ((N + t - 1) / t); };
     const auto rounds = [&](int t) { return (tiles(t) + 255) / 256; };
-    if (rounds(32) == 1) return TILE_32_K4;
+    if (rounds(32) <= 2) return TILE_32_K4;
     if (rounds(64) == 1) return TILE_64_K4;
-    return rounds(128) > 1 && rounds(128) * 624 < rounds(64) * 190 ? TILE_128 : TILE_64;
+    return rounds(128) * 28 < rounds(64) * 10 ? TILE_128 : TILE_64;
 }
 
 template <int EPI, int MB, int NB, int WM, int WN, int KG, int STAGES, int PER_CU>
@@ -76,7 +78,72 @@ void split_gemm(SplitGemmParams& p, hipStream_t st) {
         case TILE_32_K4: launch<EPI, 1, 1, 1, 1, 4, 3, 4>(p, st); break;
         case TILE_64_K4: launch<EPI, 1, 1, 2, 2, 4, 3, 1>(p, st); break;
         case TILE_64: launch<EPI, 1, 1, 2, 2, 1, 3, 4>(p, st); break;
-        case TILE_128: launch<EPI, 2, 2, 2, 2, 1, 2, 2>(p, st); break;
+        case TILE_128: launch<EPI, 2, 2, 2, 2, 1, 3, 2>(p, st); break;
+    }
+}
+
+// Key tiles per workgroup, as a shift.  Query blocks are whole workgroups (128 queries against
+// all their keys) while there are enough of them or the longest has six tiles at most (8
+// sequences of 256 tokens: 18 us, shared 18 and 8 for the merge); below 640 workgroups the keys of the
+// long blocks are shared, as coarsely as reaches 640 (12 heads of 1999 tokens: 89 us unshared, 76 in runs of
+// 1024 keys, 47 of 512, 46 of 256, 48 of 128; the merge costs 1, 6, 8, 12, 18 us more).
+static int attn_chunk_shift(int pairs, int len, int pos_base) {
+    const int blocks = (len + kAttnQueries - 1) / kAttnQueries;
+    int shift = 20;
+    const auto workgroups = [&](int sh) {
+        int n = 0;
+        for (int i = 0; i < blocks; i++) n += attn_parts(i, len, pos_base, sh);
+        return static_cast<long>(n) * pairs;
+    };
+    if (workgroups(20) >= 640 || attn_key_tiles(blocks - 1, len, pos_base) <= 6) return 20;
+    for (shift = 5; shift > 1 && workgroups(shift) < 640; shift--) {
+    }
+    return shift;
+}
+
+static int attn_items(int len, int pos_base, int shift) {
+    int n = 0;
+    for (int i = 0; i * kAttnQueries < len; i++) n += attn_parts(i, len, pos_base, shift);
+    return n;
+}
+
+SplitAttnSpace split_attention_space(int batch, int heads, int len, int pos_base) {
+    const size_t pairs = static_cast<size_t>(batch) * heads;
+    const int shift = attn_chunk_shift(batch * heads, len, pos_base);
+    SplitAttnSpace need;
+    need.kv_bytes = pairs * ((pos_base + len + 63) / 64) * kAttnTile;
+    need.part_floats = shift == 20 ? 0 : pairs * attn_items(len, pos_base, shift) * kAttnPart;
+    return need;
+}
+
+void split_attention(const PrefillAttnParams& a, int batch, char* kv, float* part, hipStream_t st) {
+    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_split_kernel),
+                                                         hipFuncAttributeMaxDynamicSharedMemorySize, kAttnLds);
+    check(raised, "hipFuncSetAttribute");
+    const int heads = a.kv.heads, pairs = batch * heads;
+    const SplitKvParams k{a.kv, a.layer, a.pos_base + a.len, kv};
+    SplitAttnParams p{};
+    p.q = a.q;
+    p.kv = kv;
+    p.tiles = (k.positions + 63) / 64;
+    p.out = a.out_split;
+    p.part = part;
+    p.d_model = a.d_model;
+    p.heads = heads;
+    p.len = a.len;
+    p.pos_base = a.pos_base;
+    p.chunk_shift = attn_chunk_shift(pairs, a.len, a.pos_base);
+    p.items = attn_items(a.len, a.pos_base, p.chunk_shift);
+    p.batch = batch;
+    p.scale = a.scale;
+    hipLaunchKernelGGL(split_kv_kernel, dim3(p.tiles, heads, batch), dim3(256), 0, st, k);
+    check(hipGetLastError(), "split_kv");
+    hipLaunchKernelGGL(attn_split_kernel, dim3((pairs + 7) / 8 * 8 * p.items), dim3(256), kAttnLds, st, p);
+    check(hipGetLastError(), "attn_split");
+    const int blocks = (a.len + kAttnQueries - 1) / kAttnQueries;
+    if (p.items > blocks) {
+        hipLaunchKernelGGL(attn_split_merge_kernel, dim3(blocks, heads, batch), dim3(256), 0, st, p);
+        check(hipGetLastError(), "attn_split_merge");
     }
 }
 

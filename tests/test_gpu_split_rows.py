@@ -18,8 +18,23 @@ CASES = {
     "64-k4-modern": (synth.Config(synth.ARCH_MODERN, 1000, 256, 2, 4, 192), 4, 159),         # hidden width 704: 11 blocks per set
     "64-gpt2": (synth.Config(synth.ARCH_GPT2, 1001, 256, 1, 4, 200), 12, 150),               # one set over all of K
     "128-modern": (synth.Config(synth.ARCH_MODERN, 530, 192, 1, 3, 1100), 24, 1057),         # 24 k rows
+    "shared-keys": (synth.Config(synth.ARCH_MODERN, 130, 128, 1, 2, 1400), 1, 1301),        # key runs of 128, merged
     "128-gpt2": (synth.Config(synth.ARCH_GPT2, 515, 128, 1, 2, 2100), 17, 2049),             # two slices of rows
 }
+
+
+def test_a_continued_pass_sees_the_cache_of_the_passes_before():
+    """600 tokens behind 333 cached ones: key tiles that begin before the pass, pages of 16."""
+    cfg = synth.Config(synth.ARCH_MODERN, 130, 128, 2, 2, 1000)
+    W = synth.make_weights(cfg, 73, std=lively_std(cfg), norm_noise=0.1)
+    gm = G.Model.from_tensors(cfg, W)
+    tokens = synth.uniform_tokens(2 * 933, cfg.vocab, 74).reshape(2, 933)
+    s = G.Session(gm, batch=2, page_tokens=16, shuffle_pages=True)
+    s.prefill(tokens[:, :333])
+    last = s.prefill(tokens[:, 333:])
+    for b in range(2):
+        ref = ref_forward.forward(cfg, W, tokens[b])
+        assert np.abs(last[b] - ref[-1]).max() <= 1e-5 * np.abs(ref[-1]).max(), b
 
 
 @pytest.mark.parametrize("name", sorted(CASES))
