@@ -662,27 +662,15 @@ static int enqueue_logits(Session& s, bool advance) {
                   : project<PRO_LAYERNORM, EPI_STORE>(s, g, s.stream);
 }
 
-// One InferenceSession::step for every sequence (inference.cpp:150-258),
-// enqueued on the session stream.  Returns the number of launches.
-// pick_first: the step opens with the greedy pick from what the last logits launch
-// left in s.best (text_gen.cpp:52-60), which also writes the input rows.
-static int enqueue_step(Session& s, bool pick_first = false) {
+// One layer of a step for every sequence, on the rows in s.x at the position in s.st.
+// query_only: the position's key and value are in the cache already.
+static int enqueue_layer(Session& s, int l, bool query_only) {
     const Model& m = *s.m;
     const Shape& sh = m.shape;
     const int d = sh.d_model, F = sh.d_ff(), B = s.B;
     const bool modern = sh.modern();
     hipStream_t st = s.stream;
     int launches = 0;
-
-    if (pick_first) {
-        hipLaunchKernelGGL(argmax_embed_kernel, dim3(B), dim3(kArgmaxThreads), 0, st, s.best, s.best_stride, s.st,
-                           s.hist, s.hist_stride, s.tok, m.E, m.P, s.x, d);
-    } else {
-        hipLaunchKernelGGL(embed_kernel, dim3((d + 255) / 256, B), dim3(256), 0, st, m.E, m.P, s.tok,
-                           s.st, s.x, d);
-    }
-    HIP_CHECK(hipGetLastError());
-    launches++;
 
     // What a projection launch touches into the L2s for the projection after it (NextWeights):
     // the whole matrix, in the 16-row tiles that launch reads it in; up to 48 sequences.
@@ -698,90 +686,112 @@ static int enqueue_step(Session& s, bool pick_first = false) {
         return f;
     };
 
-    for (int l = 0; l < sh.layers; l++) {
-        const LayerWeights& w = m.layers[l];
-        GemvParams g{};
-        g.kv = kv_layout(s);
-        g.layer = l;
-        g.d_model = d;
-        g.st = s.st;
+    const LayerWeights& w = m.layers[l];
+    GemvParams g{};
+    g.kv = kv_layout(s);
+    g.layer = l;
+    g.d_model = d;
+    g.st = s.st;
 
-        // norm1 -> fused Q,K,V projection (+bias, RoPE) -> q buffer / cache row
-        g.W = w.wqkv;
-        g.bias = w.bqkv;
-        g.N = 3 * d;
-        g.K = d;
-        g.in = s.x;
-        g.in_stride = d;
-        g.gamma = w.g1;
-        g.beta = w.be1;
-        g.out = s.q;
-        g.out_stride = d;
-        g.rope = modern;
-        g.rope_cos = m.rope_cos;
-        g.rope_sin = m.rope_sin;
-        g.next = NextWeights{};  // attention follows
-        launches += modern ? project<PRO_RMSNORM, EPI_QKV>(s, g, st)
-                           : project<PRO_LAYERNORM, EPI_QKV>(s, g, st);
+    // norm1 -> fused Q,K,V projection (+bias, RoPE) -> q buffer / cache row
+    g.W = w.wqkv;
+    g.bias = w.bqkv;
+    g.N = query_only ? d : 3 * d;
+    g.K = d;
+    g.in = s.x;
+    g.in_stride = d;
+    g.gamma = w.g1;
+    g.beta = w.be1;
+    g.out = s.q;
+    g.out_stride = d;
+    g.rope = modern;
+    g.rope_cos = m.rope_cos;
+    g.rope_sin = m.rope_sin;
+    g.next = NextWeights{};  // attention follows
+    launches += modern ? project<PRO_RMSNORM, EPI_QKV>(s, g, st)
+                       : project<PRO_LAYERNORM, EPI_QKV>(s, g, st);
 
-        AttnParams a{};
-        a.q = s.q;
-        a.out = s.attn;
-        a.kv = g.kv;
-        a.layer = l;
-        a.d_model = d;
-        a.st = s.st;
-        a.chunk = s.attn_chunk;
-        a.max_chunks = s.attn_max_chunks;
-        a.scale = 1.0f / std::sqrt(static_cast<float>(sh.head_size()));
-        a.part = s.attn_part;
-        a.tickets = s.attn_tickets;
-        launch_attn(a, B, st);
-        launches++;
+    AttnParams a{};
+    a.q = s.q;
+    a.out = s.attn;
+    a.kv = g.kv;
+    a.layer = l;
+    a.d_model = d;
+    a.st = s.st;
+    a.chunk = s.attn_chunk;
+    a.max_chunks = s.attn_max_chunks;
+    a.scale = 1.0f / std::sqrt(static_cast<float>(sh.head_size()));
+    a.part = s.attn_part;
+    a.tickets = s.attn_tickets;
+    launch_attn(a, B, st);
+    launches++;
 
-        // x += b_o + attn @ W_o
-        g.W = w.wo;
-        g.bias = w.bo;
-        g.N = d;
-        g.K = d;
-        g.in = s.attn;
-        g.in_stride = d;
-        g.out = s.x;
-        g.out_stride = d;
-        g.next = next_matrix(w.w1, modern ? 2 * F : F, d);
-        launches += project<PRO_PLAIN, EPI_RESID>(s, g, st);
+    // x += b_o + attn @ W_o
+    g.W = w.wo;
+    g.bias = w.bo;
+    g.N = d;
+    g.K = d;
+    g.in = s.attn;
+    g.in_stride = d;
+    g.out = s.x;
+    g.out_stride = d;
+    g.next = next_matrix(w.w1, modern ? 2 * F : F, d);
+    launches += project<PRO_PLAIN, EPI_RESID>(s, g, st);
 
-        // norm2 -> FFN
-        g.in = s.x;
-        g.in_stride = d;
-        g.gamma = w.g2;
-        g.beta = w.be2;
-        g.out = s.hidden;
-        g.out_stride = F;
-        g.W = w.w1;
-        g.K = d;
-        g.next = next_matrix(w.w2, d, F);
-        if (modern) {
-            g.bias = nullptr;
-            g.N = 2 * F;
-            launches += project<PRO_RMSNORM, EPI_SWIGLU>(s, g, st);
-        } else {
-            g.bias = w.b1;
-            g.N = F;
-            launches += project<PRO_LAYERNORM, EPI_GELU>(s, g, st);
-        }
-        g.W = w.w2;
-        g.bias = modern ? nullptr : w.b2;
-        g.N = d;
-        g.K = F;
-        g.in = s.hidden;
-        g.in_stride = F;
-        g.out = s.x;
-        g.out_stride = d;
-        g.next = l + 1 < sh.layers ? next_matrix(m.layers[l + 1].wqkv, 3 * d, d) : NextWeights{};
-        launches += project<PRO_PLAIN, EPI_RESID>(s, g, st);
+    // norm2 -> FFN
+    g.in = s.x;
+    g.in_stride = d;
+    g.gamma = w.g2;
+    g.beta = w.be2;
+    g.out = s.hidden;
+    g.out_stride = F;
+    g.W = w.w1;
+    g.K = d;
+    g.next = next_matrix(w.w2, d, F);
+    if (modern) {
+        g.bias = nullptr;
+        g.N = 2 * F;
+        launches += project<PRO_RMSNORM, EPI_SWIGLU>(s, g, st);
+    } else {
+        g.bias = w.b1;
+        g.N = F;
+        launches += project<PRO_LAYERNORM, EPI_GELU>(s, g, st);
     }
+    g.W = w.w2;
+    g.bias = modern ? nullptr : w.b2;
+    g.N = d;
+    g.K = F;
+    g.in = s.hidden;
+    g.in_stride = F;
+    g.out = s.x;
+    g.out_stride = d;
+    g.next = l + 1 < sh.layers ? next_matrix(m.layers[l + 1].wqkv, 3 * d, d) : NextWeights{};
+    launches += project<PRO_PLAIN, EPI_RESID>(s, g, st);
+    return launches;
+}
 
+// One InferenceSession::step for every sequence (inference.cpp:150-258),
+// enqueued on the session stream.  Returns the number of launches.
+// pick_first: the step opens with the greedy pick from what the last logits launch
+// left in s.best (text_gen.cpp:52-60), which also writes the input rows.
+static int enqueue_step(Session& s, bool pick_first = false) {
+    const Model& m = *s.m;
+    const Shape& sh = m.shape;
+    const int d = sh.d_model, B = s.B;
+    hipStream_t st = s.stream;
+    int launches = 0;
+
+    if (pick_first) {
+        hipLaunchKernelGGL(argmax_embed_kernel, dim3(B), dim3(kArgmaxThreads), 0, st, s.best, s.best_stride, s.st,
+                           s.hist, s.hist_stride, s.tok, m.E, m.P, s.x, d);
+    } else {
+        hipLaunchKernelGGL(embed_kernel, dim3((d + 255) / 256, B), dim3(256), 0, st, m.E, m.P, s.tok,
+                           s.st, s.x, d);
+    }
+    HIP_CHECK(hipGetLastError());
+    launches++;
+
+    for (int l = 0; l < sh.layers; l++) launches += enqueue_layer(s, l, /*query_only=*/false);
     launches += enqueue_logits(s, /*advance=*/true);
     return launches;
 }
@@ -1539,8 +1549,9 @@ static void launch_prompt_attn(const Session& s, const PrefillAttnParams& a) {
     HIP_CHECK(hipGetLastError());
 }
 
-// One layer over M = n * B rows of pp_x through the split projections.
-static void prompt_layer_split(Session& s, int layer, int n, int pos_base) {
+// One layer over M = n * B rows of pp_x through the split projections.  keys_only: nothing but
+// the keys and values.
+static void prompt_layer_split(Session& s, int layer, int n, int pos_base, bool keys_only) {
     const Model& m = *s.m;
     const Shape& sh = m.shape;
     const LayerWeights& w = m.layers[layer];
@@ -1550,6 +1561,11 @@ static void prompt_layer_split(Session& s, int layer, int n, int pos_base) {
 
     norm_split(sh.modern(), s.pp_x, w.g1, w.be1, s.pp_split, M, d, st);
     SplitGemmParams g = split_params(s.pp_split, sw.wqkv, M, 3 * d, d);
+    if (keys_only) {
+        g.W += static_cast<size_t>(d / kSplitRows) * (d / kSplitCols) * kSplitBlockBytes;
+        g.N = 2 * d;
+        g.first = d;
+    }
     g.bias = w.bqkv;
     g.out = s.pp_q;
     g.out_stride = d;
@@ -1562,6 +1578,7 @@ static void prompt_layer_split(Session& s, int layer, int n, int pos_base) {
     g.rows_per_seq = n;
     g.pos_base = pos_base;
     split_gemm<EPI_QKV>(g, st);
+    if (keys_only) return;
 
     PrefillAttnParams a = prompt_attn_params(s, layer, n, pos_base);
     a.out_split = s.pp_split;
@@ -1725,8 +1742,11 @@ static void prompt_pass(Session& s, int len, const ScoreSink* sink = nullptr) {
         hipLaunchKernelGGL(embed_rows_kernel, dim3((d + 255) / 256, M), dim3(256), 0, st, m.E, m.P, s.hist,
                            s.hist_stride, s.n_hist + t0, n, pos_base, s.pp_x, d);
         HIP_CHECK(hipGetLastError());
+        // Of the last layer a pass that is not scored needs the keys and values, and everything
+        // else at the last position alone, where the decode step's launches are as good.
+        const bool trim = split && !sink;
         for (int l = 0; l < sh.layers; l++) {
-            if (split) prompt_layer_split(s, l, n, pos_base);
+            if (split) prompt_layer_split(s, l, n, pos_base, trim && l == sh.layers - 1);
             else prompt_layer_small(s, l, n, pos_base);
         }
         if (sink) score_rows(s, *sink, M, n, t0, len);
@@ -1734,6 +1754,11 @@ static void prompt_pass(Session& s, int len, const ScoreSink* sink = nullptr) {
             hipLaunchKernelGGL(take_last_rows_kernel, dim3((d + 255) / 256, B), dim3(256), 0, st, s.pp_x, n,
                                s.x, d);
             HIP_CHECK(hipGetLastError());
+            if (trim) {
+                hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, st, s.st, pos_base + n - 1, s.n_hist, s.picks);
+                HIP_CHECK(hipGetLastError());
+                enqueue_layer(s, sh.layers - 1, /*query_only=*/true);
+            }
         }
     }
     s.pos += len;

@@ -188,7 +188,8 @@ struct SplitGemmParams {
     int out_stride;
     char* out_split;  // EPI_GELU, EPI_SWIGLU: split rows of out_cols columns
     int out_kblocks;
-    // EPI_QKV (rows of a prompt pass, as in GemvParams)
+    // EPI_QKV (rows of a prompt pass, as in GemvParams); outputs first .. first + N of the fused product
+    int first;
     KvLayout kv;
     int layer, d_model, rope;
     const float *rope_cos, *rope_sin;
@@ -471,10 +472,10 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
                     for (int r = 0; r < 8; r++) o[r] = v[8 + r] * silu(v[r]);
                     store_split8(p.out_split, m, n >> 1, p.out_kblocks, o);
                 } else if constexpr (EPI == EPI_QKV) {
-                    const int sec = n / p.d_model, c = n - sec * p.d_model, head = c >> 6, j = c & 63;
+                    const int sec = (p.first + n) / p.d_model, c = p.first + n - sec * p.d_model, head = c >> 6, j = c & 63;
 #pragma unroll
                     for (int q = 0; q < 4; q++) {
-                        const float4 bb = *reinterpret_cast<const float4*>(p.bias + n + 4 * q);
+                        const float4 bb = *reinterpret_cast<const float4*>(p.bias + p.first + n + 4 * q);
                         v[4 * q] += bb.x, v[4 * q + 1] += bb.y, v[4 * q + 2] += bb.z, v[4 * q + 3] += bb.w;
                     }
                     if (p.rope && sec < 2) {
