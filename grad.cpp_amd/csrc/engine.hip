@@ -1875,7 +1875,7 @@ static __device__ __align__(256) float scratch[kNoAllocScratchFloats];
 __global__ __launch_bounds__(kPickThreads) void pick_noalloc_kernel(const PickParams p, int* out_ids) {
     extern __shared__ __attribute__((aligned(128))) float lds[];
     const int b = blockIdx.x;
-    const int chosen = pick_body<false, kPickThreads>(p, b, p.work + static_cast<size_t>(b) * p.work_stride, lds);
+    const int chosen = pick_body<false, kPickThreads, false>(p, b, p.work + static_cast<size_t>(b) * p.work_stride, lds);
     if (threadIdx.x == 0) out_ids[b] = chosen;
 }
 

@@ -267,8 +267,8 @@ __device__ __forceinline__ bool persist_pick(const PersistParams& p, float* lds,
     }
     unsigned long long* pp = (p.prof && i_pick < 1024) ? p.prof + p.prof_cap / 2 + 4 * i_pick : nullptr;
     if (pp && tid == 0) pp[0] = __builtin_amdgcn_s_memrealtime();
-    const int chosen = ROW_LDS ? pick_body<true, NT>(pk, 0, lds, lds + pk.V, u)
-                               : pick_body<true, NT>(pk, 0, pk.work, lds, u);
+    const int chosen = ROW_LDS ? pick_body<true, NT, true>(pk, 0, lds, lds + pk.V, u)
+                               : pick_body<true, NT, false>(pk, 0, pk.work, lds, u);
     if (chosen_out) *chosen_out = chosen;
     if (tid == 0) {
         __hip_atomic_store(&p.hist[pk.n_hist], chosen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -414,7 +414,7 @@ constexpr int kFastLdsFloats = 3 * kFastCandCap + 3 * 64 + 128;
 // the row's (-1 otherwise); last_id: the row's last token id (the walk's answer when
 // rounding keeps the running sum below the draw, text_gen.cpp:202-208).
 template <int NT, int ROUNDS>
-__device__ inline int sample_topk_fast(const float* val, int V, float inv_t, int k, float top_p, float u,
+__device__ __forceinline__ int sample_topk_fast(const float* val, int V, float inv_t, int k, float top_p, float u,
                                        float* work, float* red, int* ishare, const int* ids = nullptr,
                                        float outside = -INFINITY, int last_id = 0) {
     constexpr int nt = NT, nw = NT / 64;
@@ -425,6 +425,7 @@ __device__ inline int sample_topk_fast(const float* val, int V, float inv_t, int
     // per-round masks alone are 2 * ROUNDS scalar registers, which end up spilled to
     // scratch memory and reloaded one trip per round.  Opaque copies keep them here.
     int tid = threadIdx.x;
+    V = __builtin_amdgcn_readfirstlane(V);
     asm volatile("" : "+v"(tid), "+s"(V));
     const int lane = tid & 63, wave = tid >> 6;
     if (V > ROUNDS * NT) return -1;
@@ -674,55 +675,55 @@ __device__ inline int block_first_reach(Get get, int n, float thr, float* parts,
 }
 
 
+// Sum of what mine() gives every thread: wavefront totals, then those left to right.  One
+// barrier per call: successive calls alternate between two sets of slots.
+struct BlockMass {
+    float (*slots)[kPickThreads / 64];  // [2]
+    int calls = 0;
+    template <int NT>
+    __device__ __forceinline__ float add(float mass) {
+        const float w = wave_sum(mass);
+        float* slot = slots[calls & 1];
+        calls++;
+        if ((threadIdx.x & 63) == 0) slot[threadIdx.x >> 6] = w;
+        __syncthreads();
+        float total = 0.0f;
+        const int nw = (NT > 0 ? NT : static_cast<int>(blockDim.x)) >> 6;
+        for (int q = 0; q < nw; q++) total += slot[q];
+        return total;
+    }
+};
+
+// The largest key in [lo, hi] whose upper mass reaches top_p; that of lo does.
+template <class Mass>
+__device__ __forceinline__ unsigned top_p_bisect(unsigned lo, unsigned hi, float top_p, Mass upper_mass) {
+    while (lo < hi) {
+        const unsigned mid = lo + (hi - lo + 1u) / 2u;
+        if (upper_mass(mid) >= top_p) lo = mid;
+        else hi = mid - 1u;
+    }
+    return lo;
+}
+
 // The top-p cut without sorting (text_gen.cpp:160-177).  The reference sorts the
 // probabilities, adds them in descending order until the sum reaches top_p and
 // cuts below the value found there.  That value is the largest probability c
 // whose upper mass (the sum of everything >= c) reaches top_p, which a bisection
 // over the bit patterns of the (positive) probabilities finds in 31 passes of
 // compare-and-add.  If even the whole mass stays below top_p the reference keeps
-// only the maximum.  NT > 0: the workgroup has NT threads and V <= ROUNDS * NT,
-// so a thread's elements stay in registers across the passes; NT == 0 reads the
-// row on every pass.
-template <int NT, int ROUNDS>
-__device__ inline float top_p_cutoff(const float* val, int V, float top_p, float* red) {
-    const int tid = threadIdx.x, nt = NT > 0 ? NT : static_cast<int>(blockDim.x);
-    float x[ROUNDS];
+// only the maximum.  This form reads the row on every pass.
+__device__ inline float top_p_cutoff_row(const float* val, int V, float top_p, float* red) {
+    const int nt = static_cast<int>(blockDim.x);
     float pmax = 0.0f;
-    if constexpr (NT > 0) {
-#pragma unroll
-        for (int r = 0; r < ROUNDS; r++) {
-            x[r] = 0.0f;
-            if (r * NT < V) {  // uniform; the last round may read (and discard) floats just past V
-                const float raw = val[r * NT + tid];
-                x[r] = (tid < V - r * NT) ? raw : 0.0f;
-            }
-            pmax = fmaxf(pmax, x[r]);
-        }
-    } else {
-        row_pass(val, V, [&](int, float v) { pmax = fmaxf(pmax, v); }, nt);
-    }
+    row_pass(val, V, [&](int, float v) { pmax = fmaxf(pmax, v); }, nt);
     pmax = block_max(pmax, red, nt);
     __shared__ float sums[2][kPickThreads / 64];
-    int calls = 0;
-    auto upper_mass = [&](unsigned key) {
+    BlockMass sum{sums};
+    const auto upper_mass = [&](unsigned key) {
         const float t = __uint_as_float(key);
         float mass = 0.0f;
-        if constexpr (NT > 0) {
-#pragma unroll
-            for (int r = 0; r < ROUNDS; r++) mass += (x[r] >= t) ? x[r] : 0.0f;
-        } else {
-            row_pass(val, V, [&](int, float v) { mass += (v >= t) ? v : 0.0f; }, nt);
-        }
-        // block sum with one barrier per call: successive calls alternate between two
-        // sets of per-wavefront slots
-        const float w = wave_sum(mass);
-        float* slot = sums[calls & 1];
-        calls++;
-        if ((tid & 63) == 0) slot[tid >> 6] = w;
-        __syncthreads();
-        float total = 0.0f;
-        for (int q = 0; q < (nt >> 6); q++) total += slot[q];
-        return total;
+        row_pass(val, V, [&](int, float v) { mass += (v >= t) ? v : 0.0f; }, nt);
+        return sum.add<0>(mass);
     };
     const unsigned top = __float_as_uint(pmax);  // bit patterns of positive floats order like the floats
     if (top < 1u || upper_mass(1u) < top_p) {
@@ -730,15 +731,281 @@ __device__ inline float top_p_cutoff(const float* val, int V, float top_p, float
         return pmax;
     }
     // the cut is rarely more than 2^-20 below the maximum: try that as the lower end
-    unsigned lo = 1u, hi = top;
+    unsigned lo = 1u;
     if (top > (20u << 23) && upper_mass(top - (20u << 23)) >= top_p) lo = top - (20u << 23);
-    while (lo < hi) {
-        const unsigned mid = lo + (hi - lo + 1u) / 2u;
-        if (upper_mass(mid) >= top_p) lo = mid;
-        else hi = mid - 1u;
-    }
+    lo = top_p_bisect(lo, top, top_p, upper_mass);
     __syncthreads();
     return __uint_as_float(lo);
+}
+
+// The same cut over a row in registers, element r * NT + tid in x[r], and in val.  A pass costs
+// 0.56 us at 512 threads and 16000 entries (half of it the barrier and the sum over wavefronts),
+// and a bisection takes 28.  Which key comes out does not depend on the keys tried, only on
+// their exact upper masses, so most of the way goes by estimates: a histogram of the mass over
+// 64 bins per octave (whole numbers: float atomics in LDS took 20 us, these take 1.1) names the
+// bin where the mass reaches top_p, exact passes at its two ends confirm it, its few dozen
+// values are ranked, their running sum names one of them, and exact passes at that value and
+// its neighbour confirm again.  What is not confirmed, and a bin of more than kCutList values,
+// is bisected.  15.6 -> 9 us.
+constexpr float kCutUnit = 1073741824.0f;  // the histogram counts mass in units of 2^-30
+constexpr int kCutBins = 1280, kCutList = 128, kCutShift = 17;  // 20 octaves below the maximum
+constexpr int kCutFloats = kCutBins + 64 + 2 * kCutList;
+
+template <int NT, int ROUNDS>
+__device__ __forceinline__ float top_p_cutoff(const float (&x)[ROUNDS], const float* val, int V, float top_p,
+                                              float* red, float* work, int* ishare) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    __shared__ float sums[2][kPickThreads / 64];
+    float pmax = 0.0f;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) pmax = fmaxf(pmax, x[r]);
+    unsigned* bins = reinterpret_cast<unsigned*>(work);
+    for (int i = tid; i < kCutBins; i += NT) bins[i] = 0u;
+    if (tid == 0) ishare[1] = 0;
+    pmax = block_max(pmax, red, NT);  // (its barriers order the zeros before the sums)
+    const unsigned top = __float_as_uint(pmax);  // bit patterns of positive floats order like the floats
+    if (top < 1u) return pmax;
+    BlockMass sum{sums};
+    const auto upper_mass = [&](unsigned key) {
+        const float t = __uint_as_float(key);
+        float mass = 0.0f;
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++) mass += (x[r] >= t) ? x[r] : 0.0f;
+        return sum.template add<NT>(mass);
+    };
+    const unsigned low = top > (20u << 23) ? top - (20u << 23) + 1u : 1u;  // lowest key of the last bin
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        // (what lies below the bins goes to slots behind them, one per lane: no branch)
+        const unsigned key = __float_as_uint(x[r]);
+        atomicAdd(&bins[key >= low ? (top - key) >> kCutShift : kCutBins + lane], static_cast<unsigned>(x[r] * kCutUnit));
+    }
+    __syncthreads();
+    if (tid < 64) {
+        constexpr int kPer = kCutBins / 64;
+        unsigned mine = 0u;
+#pragma unroll
+        for (int q = 0; q < kPer; q++) mine += bins[lane * kPer + q];
+        const unsigned run = static_cast<unsigned>(wave_inclusive_scan(static_cast<int>(mine)));
+        const unsigned want = static_cast<unsigned>(top_p * kCutUnit);
+        const unsigned long long reach = __ballot(run >= want);
+        const int at = reach ? __ffsll(static_cast<long long>(reach)) - 1 : 63;
+        if (lane == at) {
+            unsigned m = run - mine;
+            int bin = lane * kPer;
+            for (int q = 0; q < kPer - 1; q++) {
+                m += bins[lane * kPer + q];
+                if (m >= want) break;
+                bin++;
+            }
+            ishare[0] = bin;
+        }
+    }
+    __syncthreads();
+    const unsigned bin = min(static_cast<unsigned>(ishare[0]), (top - low) >> kCutShift);
+    unsigned hi = top - (bin << kCutShift);
+    unsigned lo = hi - low < (1u << kCutShift) ? low : hi - (1u << kCutShift) + 1u;
+    // ends of the bin: the mass above it stays short of top_p, with it it does not
+    const float above = hi < top ? upper_mass(hi + 1u) : 0.0f;
+    if (hi < top && above >= top_p) {
+        lo = top_p_bisect(hi + 1u, top, top_p, upper_mass);
+        __syncthreads();
+        return __uint_as_float(lo);
+    }
+    if (upper_mass(lo) < top_p) {
+        hi = lo - 1u;
+        const bool any = hi >= 1u && upper_mass(1u) >= top_p;
+        if (any) lo = top_p_bisect(1u, hi, top_p, upper_mass);
+        __syncthreads();
+        return any ? __uint_as_float(lo) : pmax;
+    }
+    float* list = work + kCutBins + 64;
+    float* sorted = list + kCutList;
+    {
+        // A thread's hits as a mask, slots with one atomic per wavefront, then the hits one by one.
+        // (From the row in val and in a loop: this runs once per pick, and unrolled over the
+        // registers fetching its code took longer than running it.)
+        unsigned long long mine = 0ull;
+#pragma unroll 1
+        for (int r0 = 0; r0 * NT < V; r0 += 4) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = val[min((r0 + e) * NT + tid, V - 1)];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const unsigned key = __float_as_uint(v[e]);
+                const bool in = key >= lo && key <= hi && (r0 + e) * NT + tid < V;
+                mine |= static_cast<unsigned long long>(in) << (r0 + e);
+            }
+        }
+        const int mine_n = __popcll(mine), upto = wave_inclusive_scan(mine_n);
+        const int wave_n = __builtin_amdgcn_readlane(upto, 63);
+        int base = 0;
+        if (wave_n) {  // uniform
+            if (lane == 63) base = atomicAdd(&ishare[1], wave_n);
+            base = __builtin_amdgcn_readlane(base, 63);
+        }
+        for (int slot = base + upto - mine_n; mine; slot++) {
+            const int r = __ffsll(static_cast<long long>(mine)) - 1;
+            mine &= mine - 1ull;
+            if (slot < kCutList) list[slot] = val[r * NT + tid];
+        }
+    }
+    __syncthreads();
+    const int n = ishare[1];
+    if (n > kCutList) {
+        lo = top_p_bisect(lo, hi, top_p, upper_mass);
+        __syncthreads();
+        return __uint_as_float(lo);
+    }
+    {
+        // rank of every value: NT / kCutList threads share the comparisons of one
+        constexpr int kShare = NT / kCutList < 4 ? NT / kCutList : 4;  // neighbouring lanes
+        const int j = tid / kShare, part = tid % kShare;
+        const float me = list[min(j, kCutList - 1)];
+        int rank = 0;
+        for (int q0 = part; q0 < n; q0 += 8 * kShare) {  // eight reads in flight
+            float o[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) o[e] = list[min(q0 + e * kShare, kCutList - 1)];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const int q = q0 + e * kShare;
+                rank += (q < n && (o[e] > me || (o[e] == me && q < j))) ? 1 : 0;
+            }
+        }
+#pragma unroll
+        for (int o = 1; o < kShare; o <<= 1) rank += __shfl_xor(rank, o, kWave);
+        if (j < n && part == 0) sorted[rank] = me;
+    }
+    __syncthreads();
+    if (tid < 64) {
+        const int v0 = 2 * lane < n ? static_cast<int>(sorted[2 * lane] * kCutUnit) : 0;
+        const int v1 = 2 * lane + 1 < n ? static_cast<int>(sorted[2 * lane + 1] * kCutUnit) : 0;
+        const int run = wave_inclusive_scan(v0 + v1), want = static_cast<int>((top_p - above) * kCutUnit);
+        const unsigned long long reach = __ballot(run >= want);
+        const int at = reach ? __ffsll(static_cast<long long>(reach)) - 1 : 63;
+        if (lane == at) ishare[0] = run - v1 >= want ? 2 * lane : 2 * lane + 1;
+    }
+    __syncthreads();
+    // sorted[ok] reaches top_p (the last one does: its upper mass is that of lo), sorted[bad] does not
+    int ok = n - 1, bad = -1, probe = ishare[0];
+    for (int tries = 0; ok - bad > 1; tries++) {
+        if (tries > 1 || probe <= bad || probe >= ok) probe = tries == 0 ? ok - 1 : (bad + ok) >> 1;
+        if (upper_mass(__float_as_uint(sorted[probe])) >= top_p) ok = probe--;
+        else bad = probe++;
+    }
+    const float cut = sorted[ok];
+    __syncthreads();
+    return cut;
+}
+
+// Softmax, top-p and the draw (text_gen.cpp:156-208) over the row val[0..V) of scaled logits, or
+// of logits still to be multiplied by scale, with a thread's elements in registers: r * NT + tid
+// for everything that goes by element, then, through val, a contiguous run for the ordered sums.
+// The sums are those of the forms that read the row on every pass (block_ordered_total,
+// block_first_reach), in the same order.  At 512 threads and 16000 entries: 29.7 us for the
+// passes it replaces, of which the cut 15.6 and the walk 7.2 (every quotient formed twice,
+// every thread walking); 17 us here.
+template <int NT, int ROUNDS>
+__device__ __forceinline__ int sample_row(float* val, int V, float scale, float top_p, float u, float* work, float* red, int* ishare) {
+    int tid = threadIdx.x;
+    V = __builtin_amdgcn_readfirstlane(V);
+    asm volatile("" : "+v"(tid));  // as in sample_topk_fast
+    const int lane = tid & 63, wave = tid >> 6;
+    float x[ROUNDS];
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) x[r] = val[min(r * NT + tid, V - 1)];
+    float m = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        x[r] *= scale;
+        m = fmaxf(m, x[r]);
+    }
+    m = block_max(m, red, NT);
+    float sum = 0.0f;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        const float e = expf(x[r] - m);
+        x[r] = tid < V - r * NT ? e : 0.0f;
+        sum += x[r];
+    }
+    sum = block_sum(sum, red, NT);
+    const float inv_sum = 1.0f / sum;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) x[r] *= inv_sum;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++)
+        if (tid < V - r * NT) val[r * NT + tid] = x[r];
+    const bool renorm = top_p < 1.0f;
+    const float cutoff = renorm ? top_p_cutoff<NT, ROUNDS>(x, val, V, top_p, red, work, ishare) : 0.0f;
+    if (tid == 0) ishare[0] = V;
+    __syncthreads();
+    // this thread's run; its length is odd: lane l starts at l * run, and an even stride would
+    // put many lanes of a wavefront on the same LDS bank
+    const int run = ((V + NT - 1) / NT) | 1;
+    const int lo = min(V, tid * run), n = min(V, lo + run) - lo;
+    float y[ROUNDS + 1];
+    const auto in_order = [&](float (&parts)[2]) {  // sum of the run; running sum of the wavefront's runs and its total
+        float part = 0.0f;
+#pragma unroll
+        for (int i = 0; i < ROUNDS + 1; i++) part += y[i];
+        const float incl = wave_serial_prefix(part, 64);
+        if (lane == 63) red[wave] = incl;
+        parts[0] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(incl), 0x138 /* wave_shr:1 */, 0xF, 0xF, true));
+        parts[1] = part;
+        __syncthreads();
+    };
+#pragma unroll
+    for (int i = 0; i < ROUNDS + 1; i++) y[i] = val[min(lo + i, V - 1)];
+#pragma unroll
+    for (int i = 0; i < ROUNDS + 1; i++) y[i] = i < n && y[i] >= cutoff ? y[i] : 0.0f;
+    float parts[2];
+    in_order(parts);
+    if (renorm) {
+        // renormalise by the index-order total of what is left (text_gen.cpp:178-192)
+        float total = 0.0f;
+        for (int w = 0; w < NT / 64; w++) total += red[w];
+        __syncthreads();
+        if (total > 0.0f) {
+#pragma unroll
+            for (int i = 0; i < ROUNDS + 1; i++) y[i] = y[i] / total;
+        }
+        in_order(parts);
+    }
+    // the first element whose running sum reaches u, in index order (text_gen.cpp:202-208)
+    float cumulative = 0.0f;
+    for (int w = 0; w < wave; w++) cumulative += red[w];
+    cumulative += parts[0];
+    // a run whose end stays short of u by far more than the roundings of its at most 33
+    // additions cannot reach it on the way
+    if (cumulative < u && cumulative + parts[1] >= u * 0.9999f) {
+        int at = V;
+#pragma unroll
+        for (int i = 0; i < ROUNDS + 1; i++) {
+            cumulative += y[i];
+            if (at == V && i < n && cumulative >= u) at = lo + i;
+        }
+        if (at < V) atomicMin(&ishare[0], at);
+    }
+    __syncthreads();
+    const int at = ishare[0];
+    __syncthreads();
+    return u <= 0.0f ? 0 : at < V ? at : V - 1;
+}
+
+// The same as a call, for the one-launch engine: inlined there, its registers cost the loop over
+// layers some of theirs (1.3 us per token at 12 layers).  The row is in LDS.
+using LdsFloat = __attribute__((address_space(3))) float;
+using LdsInt = __attribute__((address_space(3))) int;
+__device__ __forceinline__ float uniform(float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+template <int NT, int ROUNDS>
+__device__ __attribute__((noinline)) int sample_row_call(LdsFloat* val, int V, float scale, float top_p, float u,
+                                                         LdsFloat* work, LdsFloat* red, LdsInt* ishare) {
+    return sample_row<NT, ROUNDS>((float*)val, V, uniform(scale), uniform(top_p), uniform(u), (float*)work, (float*)red,
+                                  (int*)ishare);
 }
 
 // The pick for sequence b.  val: the working row ([V] floats, LDS or global,
@@ -746,7 +1013,7 @@ __device__ inline float top_p_cutoff(const float* val, int V, float top_p, float
 // Every thread of the workgroup must call it; all get the chosen id.
 // coherent: read the logits with device-scope loads (they were written by other
 // workgroups of the same running kernel).
-// NT: threads of the workgroup.
+// NT: threads of the workgroup.  ROW_LDS: val is in LDS.
 // Always inlined: each call site knows whether val is LDS or global memory, and
 // the row's loads and stores are compiled for that address space.
 // The uniform draw of pick p.pick_idx of sequence b: the caller's, or word
@@ -760,7 +1027,7 @@ __device__ __forceinline__ float pick_draw(const PickParams& p, int b) {
 
 // u_ready: the draw when the caller has already formed it (it does not depend on
 // the logits, so it can be had while they are still on their way); negative: form it here.
-template <bool coherent, int NT>
+template <bool coherent, int NT, bool ROW_LDS>
 __device__ __forceinline__ int pick_body(const PickParams& p, int b, float* val, float* srt,
                                          float u_ready = -1.0f) {
     __shared__ float red[kPickThreads / 64];
@@ -774,6 +1041,7 @@ __device__ __forceinline__ int pick_body(const PickParams& p, int b, float* val,
     // ahead of a caller's loop and kept in registers through it.
     int tid = threadIdx.x;
     int V = p.V;
+    V = __builtin_amdgcn_readfirstlane(V);
     asm volatile("" : "+v"(tid), "+s"(V));
     const float* logits = p.logits + static_cast<size_t>(b) * V;
     const int* hist = p.hist + static_cast<size_t>(b) * p.hist_stride;
@@ -893,9 +1161,14 @@ __device__ __forceinline__ int pick_body(const PickParams& p, int b, float* val,
             __syncthreads();
             if (c >= 0) return c;
         }
-        row_pass(val, V, [&](int i, float v) { val[i] = v * inv_t; }, nt);
-        __syncthreads();
-        if (p.top_k > 0 && p.top_k < V) {
+        // (64 elements, held as drawn and in index order, would go through scratch memory)
+        const bool in_registers = (ROW_LDS || !coherent) && per_thread <= 32 && p.sort_cap >= kCutFloats;
+        const bool cut_k = p.top_k > 0 && p.top_k < V;
+        if (cut_k || !in_registers) {
+            row_pass(val, V, [&](int i, float v) { val[i] = v * inv_t; }, nt);
+            __syncthreads();
+        }
+        if (cut_k) {
             const float thr = kth_largest_block(val, V, p.top_k, srt, p.sort_cap, hist256, bcast, ishare, nt);
             // Survivors of the cut (ties at the threshold included).  When they fit
             // one wavefront the rest of the sampler runs there.
@@ -925,6 +1198,17 @@ __device__ __forceinline__ int pick_body(const PickParams& p, int b, float* val,
             }, nt);
             __syncthreads();
         }
+        if (in_registers) {
+            const float scale = cut_k ? 1.0f : inv_t;
+            if constexpr (coherent) {
+                const auto row = [&](auto* call) {
+                    return call((LdsFloat*)val, V, scale, p.top_p, u, (LdsFloat*)srt, (LdsFloat*)red, (LdsInt*)ishare);
+                };
+                return per_thread <= 16 ? row(sample_row_call<NT, 16>) : row(sample_row_call<NT, 32>);
+            }
+            if (per_thread <= 16) return sample_row<NT, 16>(val, V, scale, p.top_p, u, srt, red, ishare);
+            return sample_row<NT, 32>(val, V, scale, p.top_p, u, srt, red, ishare);
+        }
         float m = -INFINITY;
         row_pass(val, V, [&](int, float v) { m = fmaxf(m, v); }, nt);
         m = block_max(m, red, nt);
@@ -939,10 +1223,7 @@ __device__ __forceinline__ int pick_body(const PickParams& p, int b, float* val,
         row_pass(val, V, [&](int i, float v) { val[i] = v * inv_sum; }, nt);
 
         if (p.top_p < 1.0f) {
-            float cutoff;
-            if (per_thread <= 32) cutoff = top_p_cutoff<NT, 32>(val, V, p.top_p, red);
-            else if (per_thread <= 64) cutoff = top_p_cutoff<NT, 64>(val, V, p.top_p, red);
-            else cutoff = top_p_cutoff<0, 1>(val, V, p.top_p, red);
+            const float cutoff = top_p_cutoff_row(val, V, p.top_p, red);
             row_pass(val, V, [&](int i, float v) {
                 if (v < cutoff) val[i] = 0.0f;
             }, nt);
@@ -980,8 +1261,8 @@ __global__ __launch_bounds__(kPickThreads) void pick_kernel(const PickParams p) 
     extern __shared__ __attribute__((aligned(128))) float lds[];
     const int b = blockIdx.x;
     const int chosen =
-        ROW_LDS ? pick_body<false, kPickThreads>(p, b, lds, lds + p.V)
-                : pick_body<false, kPickThreads>(p, b, p.work + static_cast<size_t>(b) * p.work_stride, lds);
+        ROW_LDS ? pick_body<false, kPickThreads, true>(p, b, lds, lds + p.V)
+                : pick_body<false, kPickThreads, false>(p, b, p.work + static_cast<size_t>(b) * p.work_stride, lds);
     if (threadIdx.x == 0) {
         p.hist[static_cast<size_t>(b) * p.hist_stride + p.n_hist] = chosen;  // tokens.push_back(next)
         p.tok[b] = chosen;
