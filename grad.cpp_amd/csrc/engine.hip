@@ -400,8 +400,9 @@ struct Session {
     hipGraphExec_t exec_fused = nullptr;
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
 
-    float* kv_pool = nullptr;
-    int* page_table = nullptr;
+    void* block = nullptr;       // the one device allocation of what a session has from the start:
+    float* kv_pool = nullptr;    // everything from here to st, best, and the one-launch engine's
+    int* page_table = nullptr;   // cells, xcells and ctl
     float *x = nullptr, *h = nullptr, *q = nullptr, *attn = nullptr, *hidden = nullptr,
           *logits = nullptr;
     float* work = nullptr;
@@ -424,6 +425,9 @@ struct Session {
     size_t pp_kv_bytes = 0;
     float* pp_part = nullptr;  // partial attention results
     size_t pp_part_floats = 0;
+    int* score_targets = nullptr;  // [B][length] of the scored tokens, and
+    float* score_nll = nullptr;    // what they cost
+    size_t score_cap = 0;
     float2* nll_part = nullptr;  // [pp_rows][split_nll_stride(vocab)] of rows being scored
     float* nll_target = nullptr;  // [pp_rows]
     size_t nll_rows = 0;
@@ -449,10 +453,11 @@ struct Session {
     size_t xcd_lds = 0;
     bool xcd_all_slices = false;  // every workgroup of an XCD takes a slice of the attention at any context
 
-    float* host_logits = nullptr;  // pinned, B * V
-    int* host_ids = nullptr;       // pinned staging for ids
-    int* host_err = nullptr;       // pinned landing spot for the device error flag
-    // streaming from the persistent kernel: pinned words the kernel writes / reads directly
+    void* host_block = nullptr;    // one pinned allocation, which kernels read and write directly:
+    float* host_logits = nullptr;  // B * V
+    int* host_ids = nullptr;       // [2][B * hist_stride] ids on their way to or from the device
+    int* host_err = nullptr;       // landing spot for the device error flag
+    // streaming from the persistent kernel
     unsigned long long* feed = nullptr;  // [hist_stride] {token, tag} per pick of a launch
     unsigned* stop_word = nullptr;       // set by the host to end a run at the next pick
     unsigned feed_base = 0;              // tags of a launch are feed_base + 1 ...; never reused
@@ -493,28 +498,16 @@ struct Session {
         if (graph) (void)hipGraphDestroy(graph);
         if (exec_fused) (void)hipGraphExecDestroy(exec_fused);
         if (graph_fused) (void)hipGraphDestroy(graph_fused);
-        if (best) (void)hipFree(best);
         for (hipEvent_t e : ev)
             if (e) (void)hipEventDestroy(e);
-        for (void* p : {static_cast<void*>(kv_pool), static_cast<void*>(page_table),
-                        static_cast<void*>(x), static_cast<void*>(h), static_cast<void*>(q),
-                        static_cast<void*>(attn), static_cast<void*>(hidden),
-                        static_cast<void*>(logits), static_cast<void*>(work),
-                        static_cast<void*>(attn_part), static_cast<void*>(attn_tickets),
-                        static_cast<void*>(tok), static_cast<void*>(hist), static_cast<void*>(st),
-                        static_cast<void*>(uniforms),
-                        static_cast<void*>(logit_log), static_cast<void*>(cells), static_cast<void*>(xcells),
-                        static_cast<void*>(ctl), static_cast<void*>(pp_x), static_cast<void*>(pp_q),
-                        static_cast<void*>(pp_attn), static_cast<void*>(pp_norm),
-                        static_cast<void*>(pp_hidden), static_cast<void*>(pp_split),
-                        static_cast<void*>(pp_split_hidden), static_cast<void*>(pp_kv), static_cast<void*>(pp_part), static_cast<void*>(nll_part),
-                        static_cast<void*>(nll_target)})
+        for (void* p : {block, static_cast<void*>(uniforms), static_cast<void*>(logit_log),
+                        static_cast<void*>(pp_x), static_cast<void*>(pp_q), static_cast<void*>(pp_attn),
+                        static_cast<void*>(pp_norm), static_cast<void*>(pp_hidden), static_cast<void*>(pp_split),
+                        static_cast<void*>(pp_split_hidden), static_cast<void*>(pp_kv), static_cast<void*>(pp_part),
+                        static_cast<void*>(score_targets), static_cast<void*>(score_nll),
+                        static_cast<void*>(nll_part), static_cast<void*>(nll_target)})
             if (p) (void)hipFree(p);
-        if (host_logits) (void)hipHostFree(host_logits);
-        if (host_ids) (void)hipHostFree(host_ids);
-        if (host_err) (void)hipHostFree(host_err);
-        if (feed) (void)hipHostFree(feed);
-        if (stop_word) (void)hipHostFree(stop_word);
+        if (host_block) (void)hipHostFree(host_block);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -559,6 +552,29 @@ static void dev_alloc(T*& p, size_t n) {
     HIP_CHECK(hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(T)));
     HIP_CHECK(hipMemset(p, 0, std::max<size_t>(n, 1) * sizeof(T)));
 }
+
+// Several arrays in one allocation, each on a boundary of 256 bytes: a session has some twenty,
+// and allocating, clearing and freeing them one by one was most of the 375 us that creating and
+// destroying it took.
+struct Block {
+    struct Part {
+        void* at;  // T**
+        size_t offset;
+    };
+    std::vector<Part> parts;
+    size_t bytes = 0;
+    template <typename T>
+    void add(T*& p, size_t n) {
+        parts.push_back({static_cast<void*>(&p), bytes});
+        bytes += (std::max<size_t>(n, 1) * sizeof(T) + 255) / 256 * 256;
+    }
+    void place(void* base) const {
+        for (const Part& part : parts) {
+            void* p = static_cast<char*>(base) + part.offset;
+            std::memcpy(part.at, &p, sizeof(p));
+        }
+    }
+};
 
 // ---- kernel dispatch
 
@@ -1086,10 +1102,9 @@ static void persist_run(Session& s, int n_prompt, int n_steps, int n_picks, bool
     s.picks += n_picks;
 }
 
-// After a synchronisation: did the kernel give up waiting somewhere?
+// After a synchronisation of what deliver() enqueued: did the kernel give up waiting somewhere?
 static void check_persist_abort(Session& s) {
     if (s.engine != GH_ENGINE_PERSISTENT) return;
-    HIP_CHECK(hipMemcpy(s.host_err, &s.ctl->abort, sizeof(int), hipMemcpyDeviceToHost));
     if (*s.host_err) {
         unsigned where = 0;
         HIP_CHECK(hipMemcpy(s.host_err, &s.ctl->where, sizeof(int), hipMemcpyDeviceToHost));
@@ -1134,16 +1149,60 @@ __global__ void load_tok_kernel(const int* hist, int stride, int t, int* tok, in
     if (b < B) tok[b] = hist[static_cast<size_t>(b) * stride + t];
 }
 
-// hist[b][t] = tok[b]
-__global__ void store_hist_kernel(int* hist, int stride, int t, const int* tok, int B) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < B) hist[static_cast<size_t>(b) * stride + t] = tok[b];
+// Ids the host left in pinned memory, [B][n] on end, to rows of a device array and, of n == 1, to
+// tok.  (One launch: a copy per sequence took 5 us each.)
+__global__ void stage_ids_kernel(const int* __restrict__ host, size_t total, int n, int* rows, int stride, int at,
+                                 int* tok) {
+    const size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
+    if (i >= total) return;
+    const size_t b = i / n;
+    rows[b * stride + at + (i - b * n)] = host[i];
+    if (tok) tok[b] = host[i];
+}
+
+static void stage_ids(Session& s, const int* host, int n, int* rows, int stride, int at, int* tok = nullptr) {
+    const size_t total = static_cast<size_t>(s.B) * n;
+    hipLaunchKernelGGL(stage_ids_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, s.stream, host,
+                       total, n, rows, stride, at, tok);
+    HIP_CHECK(hipGetLastError());
+}
+
+// What a call hands back, from device memory to pinned host memory, and with it the one-launch
+// engine's error word: total 4-byte words in rows of n, which are src_stride apart there and
+// follow each other here.  (One launch behind the last: each copy enqueued on its own costs 5 us
+// more, a word read back by a blocking copy another 10.)
+__global__ void deliver_kernel(const unsigned* __restrict__ src, size_t total, size_t n, size_t src_stride,
+                               unsigned* __restrict__ dst, const unsigned* abort, int* err) {
+    const size_t first = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
+    for (size_t i = first; i < total; i += gridDim.x * static_cast<size_t>(blockDim.x)) {
+        const size_t b = i / n;
+        dst[i] = src[b * src_stride + (i - b * n)];
+    }
+    if (abort && first == 0) *err = static_cast<int>(*abort);
+}
+
+// ... after which check_persist_abort needs no copy of its own.
+static void deliver(Session& s, const void* src, size_t src_stride, size_t rows, size_t n, void* dst) {
+    const unsigned* abort = s.engine == GH_ENGINE_PERSISTENT ? &s.ctl->abort : nullptr;
+    const size_t groups = std::min<size_t>(256, std::max<size_t>(1, (rows * n + 255) / 256));
+    hipLaunchKernelGGL(deliver_kernel, dim3(static_cast<unsigned>(groups)), dim3(256), 0, s.stream,
+                       static_cast<const unsigned*>(src), rows * n, n, src_stride, static_cast<unsigned*>(dst), abort,
+                       s.host_err);
+    HIP_CHECK(hipGetLastError());
+}
+
+static void deliver_logits(Session& s) {
+    const size_t V = s.m->shape.vocab;
+    deliver(s, s.logits, 0, 1, s.B * V, s.host_logits);
 }
 
 static void reset_session(Session& s) {
     s.pos = 0;
     s.n_hist = 0;
     s.picks = 0;
+    // (the one-launch engine gets its position with the launch, and a prompt pass sets what it
+    // needs of the device's copy itself)
+    if (s.engine == GH_ENGINE_PERSISTENT) return;
     hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, s.stream, s.st, 0, 0, 0);
     HIP_CHECK(hipGetLastError());
 }
@@ -1183,32 +1242,23 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
             std::swap(table[i - 1], table[x % i]);
         }
     }
-    dev_alloc(s.page_table, table.size());
-    HIP_CHECK(hipMemcpy(s.page_table, table.data(), table.size() * sizeof(int),
-                        hipMemcpyHostToDevice));
+    Block parts;
+    parts.add(s.page_table, table.size());
     const size_t page_floats = 2ull * sh.heads * page_tokens * sh.head_size();
-    dev_alloc(s.kv_pool, static_cast<size_t>(sh.layers) * s.n_pages * page_floats);
+    parts.add(s.kv_pool, static_cast<size_t>(sh.layers) * s.n_pages * page_floats);
 
-    dev_alloc(s.x, B * d);
-    dev_alloc(s.h, B * std::max(d, F));
-    dev_alloc(s.q, B * d);
-    dev_alloc(s.attn, B * d);
-    dev_alloc(s.hidden, B * F);
-    dev_alloc(s.logits, B * V);
+    parts.add(s.x, B * d);
+    parts.add(s.h, B * std::max(d, F));
+    parts.add(s.q, B * d);
+    parts.add(s.attn, B * d);
+    parts.add(s.hidden, B * F);
+    parts.add(s.logits, B * V);
     s.work_stride = static_cast<int>((V + kPickThreads + 3) / 4 * 4);
-    dev_alloc(s.work, B * static_cast<size_t>(s.work_stride));
-    dev_alloc(s.tok, B);
+    parts.add(s.work, B * static_cast<size_t>(s.work_stride));
+    parts.add(s.tok, B);
     s.hist_stride = sh.max_len + 2;
-    dev_alloc(s.hist, B * s.hist_stride);
-    dev_alloc(s.st, 1);
-    HIP_CHECK(hipHostMalloc(&s.host_logits, B * V * sizeof(float)));
-    HIP_CHECK(hipHostMalloc(&s.host_ids, B * s.hist_stride * sizeof(int)));
-    HIP_CHECK(hipHostMalloc(&s.host_err, sizeof(int)));
-    HIP_CHECK(hipHostMalloc(&s.feed, s.hist_stride * sizeof(unsigned long long), hipHostMallocCoherent));
-    HIP_CHECK(hipHostMalloc(&s.stop_word, sizeof(unsigned), hipHostMallocCoherent));
-    std::memset(s.feed, 0, s.hist_stride * sizeof(unsigned long long));
-    *s.stop_word = 0;
-
+    parts.add(s.hist, B * s.hist_stride);
+    parts.add(s.st, 1);
     // Attention chunking: a (sequence, head) is split over several workgroups in
     // runs of 512 cache positions, or 256 when that leaves fewer than ~192
     // workgroups at a full context.  Longer runs win even when they leave compute
@@ -1220,8 +1270,8 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
     if (o.flags & GH_FLAG_SMALL_ATTENTION_CHUNKS) chunk = 16;
     s.attn_chunk = chunk;
     s.attn_max_chunks = (sh.max_len + chunk - 1) / chunk;
-    dev_alloc(s.attn_part, B * sh.heads * s.attn_max_chunks * (sh.head_size() + 2));
-    dev_alloc(s.attn_tickets, B * sh.heads);
+    parts.add(s.attn_part, B * sh.heads * s.attn_max_chunks * (sh.head_size() + 2));
+    parts.add(s.attn_tickets, B * sh.heads);
 
     // The pick keeps its working row in LDS when vocab floats fit there beside the
     // work area and the kernel's static arrays; otherwise the row stays in global
@@ -1242,9 +1292,9 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
     }
 
     {
-        hipDeviceProp_t prop;
-        HIP_CHECK(hipGetDeviceProperties(&prop, dev));
-        const char* why = persist_unavailable(s, lds_bytes, prop.multiProcessorCount);
+        int cus = 0;
+        HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        const char* why = persist_unavailable(s, lds_bytes, cus);
         if (s.engine == GH_ENGINE_PERSISTENT && why) throw ApiError{GH_ERR_INVALID_ARGUMENT, why};
         if (s.engine == GH_ENGINE_AUTO) s.engine = why ? GH_ENGINE_GRAPH : GH_ENGINE_PERSISTENT;
         if (s.engine == GH_ENGINE_PERSISTENT) {
@@ -1259,7 +1309,7 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
             // is slower.
             const int ffn1_items = static_cast<int>(sh.modern() ? F : F / 2);
             const int want = ((ffn1_items + kPersistWaves - 1) / kPersistWaves + 15) / 16 * 16;
-            s.persist_grid = std::min(std::min(prop.multiProcessorCount, 256), std::max(32, want));
+            s.persist_grid = std::min(std::min(cus, 256), std::max(32, want));
             // the exchange cells, the token cell (and one of padding), then what the workgroups
             // leave for a pick each of them makes itself: nine planes of one cell per
             // workgroup and a stop word
@@ -1267,29 +1317,8 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
             // and, from an even index, what the workgroups that share a head's long context
             // leave for the head's own: up to fifteen shares of 66 cells for each of up to 16 heads
             s.cells_count = ((s.cells_count + 1) & ~static_cast<size_t>(1)) + 16 * 15 * 66;
-            dev_alloc(s.cells, s.cells_count);
-            // Rows of the cache written earlier in a launch by other workgroups are read
-            // with ordinary loads.  That is sound only because a row is never read before
-            // it is written and shares no 128-byte cache line with another row: rows are
-            // head_size floats from a base that hipMalloc aligns.
-            if ((sh.head_size() * sizeof(float)) % 128 != 0 || reinterpret_cast<uintptr_t>(s.kv_pool) % 256 != 0)
-                throw ApiError{GH_ERR_DEVICE, "persistent engine: cache rows are not whole 128-byte lines"};
-            dev_alloc(s.ctl, 1);
-            if (const char* near = std::getenv("GRADHIP_TEST_NEAR_WRAP")) {
-                // Test aid: start the session's two running counts `near` steps before the
-                // points where the arrival counters wrap around 2^32 and where the cell tags
-                // are re-based, so that a short run crosses both.
-                // (a test hook: values outside 1..4096 are ignored, so a stray variable cannot
-                // leave the counters inconsistent)
-                const long asked = std::strtol(near, nullptr, 10);
-                const unsigned n = asked >= 1 && asked <= 4096 ? static_cast<unsigned>(asked) : 0u;
-                if (n != 0u) {
-                    s.arrive_total = (0u - n * static_cast<unsigned>(s.persist_grid)) / static_cast<unsigned>(s.persist_grid);
-                    const unsigned sum = s.arrive_total * static_cast<unsigned>(s.persist_grid);
-                    HIP_CHECK(hipMemcpy(&s.ctl->arrive[0], &sum, sizeof(sum), hipMemcpyHostToDevice));
-                    s.epoch = static_cast<unsigned>(0xF0000000ull / (static_cast<unsigned long long>(sh.layers + 1) * 8ull)) - n;
-                }
-            }
+            parts.add(s.cells, s.cells_count);
+            parts.add(s.ctl, 1);
             if (std::getenv("GRADHIP_PROF_DUMP")) {
                 s.prof_cap = 1 << 16;
                 dev_alloc(s.prof, s.prof_cap);
@@ -1307,7 +1336,7 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
             const bool xcd_wanted = (o.flags & GH_FLAG_XCD_PERSISTENT) != 0;
             if ((o.flags & GH_FLAG_XCD_PERSISTENT) != 0 && (o.flags & GH_FLAG_CLASSIC_PERSISTENT) != 0)
                 throw ApiError{GH_ERR_INVALID_ARGUMENT, "GH_FLAG_CLASSIC_PERSISTENT and GH_FLAG_XCD_PERSISTENT exclude each other"};
-            if (xcd_wanted && prop.multiProcessorCount == kXcds * kWgPerXcd && xcd_geometry(sh, gm)
+            if (xcd_wanted && cus == kXcds * kWgPerXcd && xcd_geometry(sh, gm)
                 && s.pages_per_seq <= 1024) {
                 const size_t statics = 4096;  // the kernel's static LDS (control words, the pick's scratch), rounded up
                 const size_t work = (2 * d + kWgPerXcd * kApCells + 512 + kXcdRowWaves * (128 + 32) + 192 + s.pages_per_seq)
@@ -1335,7 +1364,7 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
                     s.xcd_lds = std::max(ring + work, ring0 + std::max(work, s.xcd_row_lds ? pick_row : pick_small));
                     const XcdCells cl = xcd_cells(m.xcd_geom);
                     s.xcd_cells_count = cl.total;
-                    dev_alloc(s.xcells, cl.total);
+                    parts.add(s.xcells, cl.total);
                     for (const bool feed : {false, true})
                         HIP_CHECK(hipFuncSetAttribute(
                             reinterpret_cast<const void*>(xcd_kernel_for(sh, s.xcd_row_lds, feed)),
@@ -1345,15 +1374,53 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
         }
     }
 
-    reset_session(s);
-    HIP_CHECK(hipStreamSynchronize(s.stream));
-
     // The matrix-core logits launch can leave what a greedy pick needs (a batch of at
     // least two sequences takes it; the wide form and the tiled form both can).
     if (s.engine != GH_ENGINE_PERSISTENT && s.B >= kMinGemmBatch && gemm_shape_ok(sh.d_model, sh.d_model)) {
         s.best_stride = (sh.vocab + 15) / 16;
-        dev_alloc(s.best, static_cast<size_t>(s.B) * s.best_stride);
+        parts.add(s.best, static_cast<size_t>(s.B) * s.best_stride);
     }
+
+    HIP_CHECK(hipMalloc(&s.block, parts.bytes));
+    parts.place(s.block);
+    HIP_CHECK(hipMemsetAsync(s.block, 0, parts.bytes, s.stream));
+    Block pinned;
+    pinned.add(s.host_logits, B * V);
+    pinned.add(s.host_ids, 2 * B * s.hist_stride);
+    pinned.add(s.host_err, 1);
+    pinned.add(s.feed, s.hist_stride);
+    pinned.add(s.stop_word, 1);
+    HIP_CHECK(hipHostMalloc(&s.host_block, pinned.bytes, hipHostMallocCoherent));
+    pinned.place(s.host_block);
+    std::memset(s.feed, 0, s.hist_stride * sizeof(unsigned long long));
+    *s.stop_word = 0;
+    *s.host_err = 0;
+    HIP_CHECK(hipMemcpyAsync(s.page_table, table.data(), table.size() * sizeof(int), hipMemcpyHostToDevice, s.stream));
+    if (s.engine == GH_ENGINE_PERSISTENT) {
+        // Rows of the cache written earlier in a launch by other workgroups are read
+        // with ordinary loads.  That is sound only because a row is never read before
+        // it is written and shares no 128-byte cache line with another row: rows are
+        // head_size floats from a base that hipMalloc aligns.
+        if ((sh.head_size() * sizeof(float)) % 128 != 0 || reinterpret_cast<uintptr_t>(s.kv_pool) % 256 != 0)
+            throw ApiError{GH_ERR_DEVICE, "persistent engine: cache rows are not whole 128-byte lines"};
+        if (const char* near = std::getenv("GRADHIP_TEST_NEAR_WRAP")) {
+            // Test aid: start the session's two running counts `near` steps before the
+            // points where the arrival counters wrap around 2^32 and where the cell tags
+            // are re-based, so that a short run crosses both.
+            // (a test hook: values outside 1..4096 are ignored, so a stray variable cannot
+            // leave the counters inconsistent)
+            const long asked = std::strtol(near, nullptr, 10);
+            const unsigned n = asked >= 1 && asked <= 4096 ? static_cast<unsigned>(asked) : 0u;
+            if (n != 0u) {
+                s.arrive_total = (0u - n * static_cast<unsigned>(s.persist_grid)) / static_cast<unsigned>(s.persist_grid);
+                const unsigned sum = s.arrive_total * static_cast<unsigned>(s.persist_grid);
+                HIP_CHECK(hipMemcpy(&s.ctl->arrive[0], &sum, sizeof(sum), hipMemcpyHostToDevice));
+                s.epoch = static_cast<unsigned>(0xF0000000ull / (static_cast<unsigned long long>(sh.layers + 1) * 8ull)) - n;
+            }
+        }
+    }
+    reset_session(s);
+    HIP_CHECK(hipStreamSynchronize(s.stream));
 
     if (s.engine == GH_ENGINE_PERSISTENT) {
         // nothing to record: one launch runs any number of steps
@@ -2292,7 +2359,7 @@ gh_status gh_session_reset(gh_session* s) {
     return guard([&] {
         if (!s) throw ApiError{GH_ERR_INVALID_ARGUMENT, "null session"};
         reset_session(*s->impl);
-        HIP_CHECK(hipStreamSynchronize(s->impl->stream));
+        if (s->impl->engine != GH_ENGINE_PERSISTENT) HIP_CHECK(hipStreamSynchronize(s->impl->stream));
     });
 }
 
@@ -2306,19 +2373,13 @@ gh_status gh_session_step(gh_session* sess, const int32_t* ids, float* logits_ho
         const size_t V = s.m->shape.vocab;
         const bool one_launch = s.engine == GH_ENGINE_PERSISTENT && s.n_hist == s.pos;
         if (one_launch) {
-            // One launch, one copy back and one wait per call: the token travels in the
-            // kernel's arguments (the kernel records it in the history, whose index is the
-            // position), and the kernel's "gave up" word comes back with the logits.
+            // The token travels in the kernel's arguments (the kernel records it in the history,
+            // whose index is the position).
             persist_run(s, 1, 1, 0, false, nullptr, nullptr, 0, 0, nullptr, false, -1, ids[0]);
-            HIP_CHECK(hipMemcpyAsync(s.host_err, &s.ctl->abort, sizeof(int), hipMemcpyDeviceToHost, s.stream));
         } else {
             std::memcpy(s.host_ids, ids, s.B * sizeof(int));
-            HIP_CHECK(hipMemcpyAsync(s.tok, s.host_ids, s.B * sizeof(int), hipMemcpyHostToDevice,
-                                     s.stream));
             // The history (index == position) feeds the repetition penalty of later picks.
-            hipLaunchKernelGGL(store_hist_kernel, dim3((s.B + 63) / 64), dim3(64), 0, s.stream, s.hist,
-                               s.hist_stride, s.n_hist, s.tok, s.B);
-            HIP_CHECK(hipGetLastError());
+            stage_ids(s, s.host_ids, 1, s.hist, s.hist_stride, s.n_hist, s.tok);
             if (s.engine == GH_ENGINE_PERSISTENT) {
                 persist_run(s, 1, 1, 0, false, nullptr, nullptr, 0, 0, nullptr);
             } else {
@@ -2326,11 +2387,9 @@ gh_status gh_session_step(gh_session* sess, const int32_t* ids, float* logits_ho
                 run_step(s);
             }
         }
-        HIP_CHECK(hipMemcpyAsync(s.host_logits, s.logits, s.B * V * sizeof(float),
-                                 hipMemcpyDeviceToHost, s.stream));
+        deliver_logits(s);
         HIP_CHECK(hipStreamSynchronize(s.stream));
-        // (the word read back with the logits says whether the kernel finished its waits)
-        if (!one_launch || *s.host_err != 0) check_persist_abort(s);
+        check_persist_abort(s);
         if (logits_host) std::memcpy(logits_host, s.host_logits, s.B * V * sizeof(float));
     });
 }
@@ -2355,17 +2414,10 @@ gh_status gh_session_prefill(gh_session* sess, const int32_t* ids, int32_t len,
         check_ids(s, ids, static_cast<size_t>(s.B) * len);
         const size_t V = s.m->shape.vocab;
         // Stage the ids into the history, then step through them.
-        const int base = s.n_hist;
-        for (int b = 0; b < s.B; b++) {
-            std::memcpy(s.host_ids + static_cast<size_t>(b) * s.hist_stride,
-                        ids + static_cast<size_t>(b) * len, len * sizeof(int));
-            HIP_CHECK(hipMemcpyAsync(s.hist + static_cast<size_t>(b) * s.hist_stride + base,
-                                     s.host_ids + static_cast<size_t>(b) * s.hist_stride,
-                                     len * sizeof(int), hipMemcpyHostToDevice, s.stream));
-        }
+        std::memcpy(s.host_ids, ids, static_cast<size_t>(s.B) * len * sizeof(int));
+        stage_ids(s, s.host_ids, len, s.hist, s.hist_stride, s.n_hist);
         run_prompt(s, len, nullptr, nullptr);
-        HIP_CHECK(hipMemcpyAsync(s.host_logits, s.logits, s.B * V * sizeof(float),
-                                 hipMemcpyDeviceToHost, s.stream));
+        deliver_logits(s);
         HIP_CHECK(hipStreamSynchronize(s.stream));
         check_persist_abort(s);
         if (last_logits_host) std::memcpy(last_logits_host, s.host_logits, s.B * V * sizeof(float));
@@ -2386,26 +2438,22 @@ gh_status gh_session_score(gh_session* sess, const int32_t* ids, const int32_t* 
         check_ids(s, ids, n);
         check_ids(s, targets, n);
         const int base = s.n_hist;
-        for (int b = 0; b < s.B; b++) {
-            std::memcpy(s.host_ids + static_cast<size_t>(b) * s.hist_stride,
-                        ids + static_cast<size_t>(b) * len, len * sizeof(int));
-            HIP_CHECK(hipMemcpyAsync(s.hist + static_cast<size_t>(b) * s.hist_stride + base,
-                                     s.host_ids + static_cast<size_t>(b) * s.hist_stride,
-                                     len * sizeof(int), hipMemcpyHostToDevice, s.stream));
+        int* host_targets = s.host_ids + static_cast<size_t>(s.B) * s.hist_stride;
+        std::memcpy(s.host_ids, ids, n * sizeof(int));
+        std::memcpy(host_targets, targets, n * sizeof(int));
+        stage_ids(s, s.host_ids, len, s.hist, s.hist_stride, base);
+        if (s.score_cap < n) {
+            if (s.score_targets) HIP_CHECK(hipFree(s.score_targets));
+            if (s.score_nll) HIP_CHECK(hipFree(s.score_nll));
+            s.score_targets = nullptr;
+            s.score_nll = nullptr;
+            s.score_cap = 0;
+            dev_alloc(s.score_targets, n);
+            dev_alloc(s.score_nll, n);
+            s.score_cap = n;
         }
-        // targets and results live for this call only
-        struct Scratch {
-            int* targets = nullptr;
-            float* nll = nullptr;
-            ~Scratch() {
-                if (targets) (void)hipFree(targets);
-                if (nll) (void)hipFree(nll);
-            }
-        } tmp;
-        dev_alloc(tmp.targets, n);
-        dev_alloc(tmp.nll, n);
-        HIP_CHECK(hipMemcpyAsync(tmp.targets, targets, n * sizeof(int), hipMemcpyHostToDevice, s.stream));
-        const ScoreSink sink{tmp.targets, tmp.nll};
+        stage_ids(s, host_targets, len, s.score_targets, len, 0);
+        const ScoreSink sink{s.score_targets, s.score_nll};
         if (s.use_prompt_pass && prompt_pass_ok(s, len)) {
             prompt_pass(s, len, &sink);
         } else {
@@ -2426,9 +2474,10 @@ gh_status gh_session_score(gh_session* sess, const int32_t* ids, const int32_t* 
             }
             if (s.engine != GH_ENGINE_PERSISTENT) s.n_hist += len;
         }
-        HIP_CHECK(hipMemcpyAsync(nll_host, tmp.nll, n * sizeof(float), hipMemcpyDeviceToHost, s.stream));
+        deliver(s, s.score_nll, 0, 1, n, s.host_ids);  // (the ids have long been read)
         HIP_CHECK(hipStreamSynchronize(s.stream));
         check_persist_abort(s);
+        std::memcpy(nll_host, s.host_ids, n * sizeof(float));
     });
 }
 
@@ -2488,8 +2537,7 @@ gh_status gh_session_pick(gh_session* sess, const gh_sampling* opt, const float*
         if (du) s.picks = 0;
         launch_pick(s, *opt, du, 1, seed, false);  // the stand-alone pick kernel serves every engine
         if (du) s.picks = saved + 1;
-        HIP_CHECK(hipMemcpyAsync(s.host_ids, s.tok, s.B * sizeof(int), hipMemcpyDeviceToHost,
-                                 s.stream));
+        deliver(s, s.tok, 0, 1, s.B, s.host_ids);
         HIP_CHECK(hipStreamSynchronize(s.stream));
         if (out_ids) std::memcpy(out_ids, s.host_ids, s.B * sizeof(int));
     });
@@ -2517,16 +2565,12 @@ gh_status gh_session_decode(gh_session* sess, int32_t max_tokens, const gh_sampl
         const auto [made, stepped] = run_decode(s, max_tokens, *opt, du, max_tokens, seed, nullptr, nullptr);
         HIP_CHECK(hipEventRecord(s.ev[2], s.stream));
         if (du) s.picks = saved_picks + made;
-        for (size_t b = 0; b < B; b++)
-            HIP_CHECK(hipMemcpyAsync(s.host_ids + b * s.hist_stride,
-                                     s.hist + b * s.hist_stride + first, made * sizeof(int),
-                                     hipMemcpyDeviceToHost, s.stream));
+        deliver(s, s.hist + first, s.hist_stride, s.B, made, s.host_ids);
         HIP_CHECK(hipStreamSynchronize(s.stream));
         check_persist_abort(s);
         if (out_ids)
             for (size_t b = 0; b < B; b++)
-                std::memcpy(out_ids + b * max_tokens, s.host_ids + b * s.hist_stride,
-                            made * sizeof(int));
+                std::memcpy(out_ids + b * max_tokens, s.host_ids + b * made, made * sizeof(int));
         *out_count = made;
         HIP_CHECK(hipEventElapsedTime(&s.timing.decode_ms, s.ev[1], s.ev[2]));
         s.timing.decode_steps = stepped;
@@ -2620,6 +2664,7 @@ gh_status gh_session_decode_stream(gh_session* sess, int32_t max_tokens, const g
                 *out_count = made;
                 throw;
             }
+            deliver(s, nullptr, 0, 1, 0, nullptr);
             HIP_CHECK(hipStreamSynchronize(s.stream));
             check_persist_abort(s);
             // persist_run advanced the host's view by the planned run: take back what was not run
@@ -2630,7 +2675,7 @@ gh_status gh_session_decode_stream(gh_session* sess, int32_t max_tokens, const g
             for (int i = 0; i < max_tokens; i++) {
                 if (s.n_hist >= s.hist_stride) break;
                 launch_pick(s, *opt, du, max_tokens, seed, true);
-                HIP_CHECK(hipMemcpyAsync(s.host_ids, s.tok, B * sizeof(int), hipMemcpyDeviceToHost, s.stream));
+                deliver(s, s.tok, 0, 1, B, s.host_ids);
                 HIP_CHECK(hipStreamSynchronize(s.stream));
                 if (out_ids)
                     for (int b = 0; b < B; b++) out_ids[static_cast<size_t>(b) * max_tokens + i] = s.host_ids[b];
@@ -2680,11 +2725,8 @@ gh_status gh_session_generate(gh_session* sess, const int32_t* prompts, int32_t 
         const size_t B = s.B, V = sh.vocab;
 
         reset_session(s);
-        for (size_t b = 0; b < B; b++)
-            std::memcpy(s.host_ids + b * s.hist_stride, prompts + b * prompt_len,
-                        prompt_len * sizeof(int));
-        HIP_CHECK(hipMemcpyAsync(s.hist, s.host_ids, B * s.hist_stride * sizeof(int),
-                                 hipMemcpyHostToDevice, s.stream));
+        std::memcpy(s.host_ids, prompts, B * prompt_len * sizeof(int));
+        stage_ids(s, s.host_ids, prompt_len, s.hist, s.hist_stride, 0);
         const float* du =
             opt->greedy ? nullptr : stage_uniforms(s, uniforms, B * static_cast<size_t>(max_tokens));
         float* log = nullptr;
@@ -2707,14 +2749,12 @@ gh_status gh_session_generate(gh_session* sess, const int32_t* prompts, int32_t 
         HIP_CHECK(hipEventRecord(s.ev[2], s.stream));
 
         const int total = s.n_hist;
-        HIP_CHECK(hipMemcpyAsync(s.host_ids, s.hist, B * s.hist_stride * sizeof(int),
-                                 hipMemcpyDeviceToHost, s.stream));
+        deliver(s, s.hist, s.hist_stride, s.B, total, s.host_ids);
         HIP_CHECK(hipStreamSynchronize(s.stream));
         check_persist_abort(s);
         const size_t out_stride = static_cast<size_t>(prompt_len) + max_tokens;
         for (size_t b = 0; b < B; b++)
-            std::memcpy(out_tokens + b * out_stride, s.host_ids + b * s.hist_stride,
-                        total * sizeof(int));
+            std::memcpy(out_tokens + b * out_stride, s.host_ids + b * total, total * sizeof(int));
         *out_len = total;
         if (step_logits_host)
             HIP_CHECK(hipMemcpy(step_logits_host, s.logit_log, steps * B * V * sizeof(float),
