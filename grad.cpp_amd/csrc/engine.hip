@@ -375,6 +375,10 @@ static std::vector<std::vector<float>> download_model(const Model& m) {
 
 // ----------------------------------------------------------------- session
 
+// What a batched step opens with: the embedding of s.tok, the greedy pick from what the last logits
+// launch left and the embedding of what it picked, or nothing (the pick launch left the rows).
+enum StepForm { STEP_EMBED, STEP_ARGMAX, STEP_ROWS, kStepForms };
+
 struct Session {
     const Model* m = nullptr;
     int B = 1;
@@ -389,15 +393,13 @@ struct Session {
     int launches_per_step = 0;
 
     hipStream_t stream = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
+    hipGraph_t graph[kStepForms] = {};
+    hipGraphExec_t exec[kStepForms] = {};
     // Batched greedy decoding without a penalty: the logits launch leaves the largest
     // value of every run of 16 columns, and a second form of the step opens with the
     // launch that picks from those and embeds (no pick launch, no embedding launch).
     float2* best = nullptr;  // [B][best_stride]
     int best_stride = 0;
-    hipGraph_t graph_fused = nullptr;
-    hipGraphExec_t exec_fused = nullptr;
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
 
     void* block = nullptr;       // the one device allocation of what a session has from the start:
@@ -494,10 +496,10 @@ struct Session {
             }
             (void)hipFree(prof);
         }
-        if (exec) (void)hipGraphExecDestroy(exec);
-        if (graph) (void)hipGraphDestroy(graph);
-        if (exec_fused) (void)hipGraphExecDestroy(exec_fused);
-        if (graph_fused) (void)hipGraphDestroy(graph_fused);
+        for (hipGraphExec_t e : exec)
+            if (e) (void)hipGraphExecDestroy(e);
+        for (hipGraph_t g : graph)
+            if (g) (void)hipGraphDestroy(g);
         for (hipEvent_t e : ev)
             if (e) (void)hipEventDestroy(e);
         for (void* p : {block, static_cast<void*>(uniforms), static_cast<void*>(logit_log),
@@ -788,24 +790,23 @@ static int enqueue_layer(Session& s, int l, bool query_only) {
 
 // One InferenceSession::step for every sequence (inference.cpp:150-258),
 // enqueued on the session stream.  Returns the number of launches.
-// pick_first: the step opens with the greedy pick from what the last logits launch
-// left in s.best (text_gen.cpp:52-60), which also writes the input rows.
-static int enqueue_step(Session& s, bool pick_first = false) {
+static int enqueue_step(Session& s, StepForm form) {
     const Model& m = *s.m;
     const Shape& sh = m.shape;
     const int d = sh.d_model, B = s.B;
     hipStream_t st = s.stream;
     int launches = 0;
 
-    if (pick_first) {
+    if (form == STEP_ARGMAX) {
+        // text_gen.cpp:52-60
         hipLaunchKernelGGL(argmax_embed_kernel, dim3(B), dim3(kArgmaxThreads), 0, st, s.best, s.best_stride, s.st,
                            s.hist, s.hist_stride, s.tok, m.E, m.P, s.x, d);
-    } else {
+    } else if (form == STEP_EMBED) {
         hipLaunchKernelGGL(embed_kernel, dim3((d + 255) / 256, B), dim3(256), 0, st, m.E, m.P, s.tok,
                            s.st, s.x, d);
     }
     HIP_CHECK(hipGetLastError());
-    launches++;
+    launches += form != STEP_ROWS;
 
     for (int l = 0; l < sh.layers; l++) launches += enqueue_layer(s, l, /*query_only=*/false);
     launches += enqueue_logits(s, /*advance=*/true);
@@ -1114,11 +1115,31 @@ static void check_persist_abort(Session& s) {
     }
 }
 
-static void run_step(Session& s, bool pick_first = false) {
+// Records the launches of a step; returns their number.
+static int capture_step(Session& s, StepForm form, hipGraph_t* graph) {
+    int launches = 0;
+    HIP_CHECK(hipStreamBeginCapture(s.stream, hipStreamCaptureModeThreadLocal));
+    try {
+        launches = enqueue_step(s, form);
+    } catch (...) {
+        hipGraph_t g = nullptr;
+        (void)hipStreamEndCapture(s.stream, &g);
+        if (g) (void)hipGraphDestroy(g);
+        throw;
+    }
+    HIP_CHECK(hipStreamEndCapture(s.stream, graph));
+    return launches;
+}
+
+static void run_step(Session& s, StepForm form = STEP_EMBED) {
     if (s.engine == GH_ENGINE_GRAPH) {
-        HIP_CHECK(hipGraphLaunch(pick_first ? s.exec_fused : s.exec, s.stream));
+        if (!s.exec[form]) {  // (a form's graph is made when it is first wanted)
+            if (!s.graph[form]) capture_step(s, form, &s.graph[form]);
+            HIP_CHECK(hipGraphInstantiate(&s.exec[form], s.graph[form], nullptr, nullptr, 0));
+        }
+        HIP_CHECK(hipGraphLaunch(s.exec[form], s.stream));
     } else {
-        enqueue_step(s, pick_first);
+        enqueue_step(s, form);
     }
     s.pos++;
 }
@@ -1424,44 +1445,9 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
 
     if (s.engine == GH_ENGINE_PERSISTENT) {
         // nothing to record: one launch runs any number of steps
-    } else if (s.engine == GH_ENGINE_GRAPH) {
-        HIP_CHECK(hipStreamBeginCapture(s.stream, hipStreamCaptureModeThreadLocal));
-        try {
-            s.launches_per_step = enqueue_step(s);
-        } catch (...) {
-            hipGraph_t g = nullptr;
-            (void)hipStreamEndCapture(s.stream, &g);
-            if (g) (void)hipGraphDestroy(g);
-            throw;
-        }
-        HIP_CHECK(hipStreamEndCapture(s.stream, &s.graph));
-        HIP_CHECK(hipGraphInstantiate(&s.exec, s.graph, nullptr, nullptr, 0));
-        if (s.best) {
-            HIP_CHECK(hipStreamBeginCapture(s.stream, hipStreamCaptureModeThreadLocal));
-            try {
-                enqueue_step(s, true);
-            } catch (...) {
-                hipGraph_t g = nullptr;
-                (void)hipStreamEndCapture(s.stream, &g);
-                if (g) (void)hipGraphDestroy(g);
-                throw;
-            }
-            HIP_CHECK(hipStreamEndCapture(s.stream, &s.graph_fused));
-            HIP_CHECK(hipGraphInstantiate(&s.exec_fused, s.graph_fused, nullptr, nullptr, 0));
-        }
     } else {
-        // Count the launches of one step without running it twice: a dry capture.
-        HIP_CHECK(hipStreamBeginCapture(s.stream, hipStreamCaptureModeThreadLocal));
-        hipGraph_t g = nullptr;
-        try {
-            s.launches_per_step = enqueue_step(s);
-        } catch (...) {
-            (void)hipStreamEndCapture(s.stream, &g);
-            if (g) (void)hipGraphDestroy(g);
-            throw;
-        }
-        HIP_CHECK(hipStreamEndCapture(s.stream, &g));
-        if (g) (void)hipGraphDestroy(g);
+        // Counts the launches of a step without running one.
+        s.launches_per_step = capture_step(s, STEP_EMBED, &s.graph[STEP_EMBED]);
     }
     return sp;
 }
@@ -1469,7 +1455,9 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
 // commit: the pick becomes part of the token history right away (the generate
 // loop steps it next); otherwise the caller's following step() records it.
 static void launch_pick(Session& s, const gh_sampling& o, const float* dev_uniforms, int u_stride,
-                        uint64_t seed, bool commit) {
+                        uint64_t seed, bool commit, bool embed = false) {
+    const Model& m = *s.m;
+    const PickEmbed e{m.E, m.P, embed ? s.x : nullptr, m.shape.d_model, s.pos};
     PickParams p{};
     p.logits = s.logits;
     p.work = s.work;
@@ -1492,10 +1480,10 @@ static void launch_pick(Session& s, const gh_sampling& o, const float* dev_unifo
     p.sort_cap = kPickWorkFloats;
     if (s.pick_row_in_lds) {
         hipLaunchKernelGGL(pick_kernel<true>, dim3(s.B), dim3(kPickThreads),
-                           static_cast<size_t>(p.V + kPickWorkFloats) * sizeof(float), s.stream, p);
+                           static_cast<size_t>(p.V + kPickWorkFloats) * sizeof(float), s.stream, p, e);
     } else {
         hipLaunchKernelGGL(pick_kernel<false>, dim3(s.B), dim3(kPickThreads), kPickWorkFloats * sizeof(float),
-                           s.stream, p);
+                           s.stream, p, e);
     }
     HIP_CHECK(hipGetLastError());
     if (commit) s.n_hist++;
@@ -1903,11 +1891,11 @@ static std::pair<int, int> run_decode(Session& s, int max_tokens, const gh_sampl
             s.n_hist++;
             s.picks++;
         } else {
-            launch_pick(s, o, du, u_stride, seed, true);
+            launch_pick(s, o, du, u_stride, seed, true, /*embed=*/s.pos < C);
         }
         picks++;
         if (s.pos >= C) break;
-        run_step(s, riding);
+        run_step(s, riding ? STEP_ARGMAX : STEP_ROWS);
         steps++;
         if (log) {
             HIP_CHECK(hipMemcpyAsync(log + *steps_logged * BV, s.logits, BV * sizeof(float),
@@ -2674,7 +2662,7 @@ gh_status gh_session_decode_stream(gh_session* sess, int32_t max_tokens, const g
             int n_seen = 0;
             for (int i = 0; i < max_tokens; i++) {
                 if (s.n_hist >= s.hist_stride) break;
-                launch_pick(s, *opt, du, max_tokens, seed, true);
+                launch_pick(s, *opt, du, max_tokens, seed, true, /*embed=*/s.pos < C);
                 deliver(s, s.tok, 0, 1, B, s.host_ids);
                 HIP_CHECK(hipStreamSynchronize(s.stream));
                 if (out_ids)
@@ -2687,7 +2675,7 @@ gh_status gh_session_decode_stream(gh_session* sess, int32_t max_tokens, const g
                         n_seen++;
                     }
                 if (s.pos >= C) break;
-                run_step(s);
+                run_step(s, STEP_ROWS);
                 stepped++;
                 if (asked != 0 || n_seen == B) break;
             }

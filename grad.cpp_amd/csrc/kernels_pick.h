@@ -1254,10 +1254,18 @@ __device__ __forceinline__ int pick_body(const PickParams& p, int b, float* val,
     return chosen;
 }
 
+// Where the picked token's embedding goes, the input of the step that follows; x null: nowhere.
+struct PickEmbed {
+    const float *E, *P;
+    float* x;
+    int d, pos;
+};
+
 // ROW_LDS: the working row sits in LDS in front of the work area; otherwise in
-// p.work.
+// p.work.  The workgroup that made the pick embeds it (inference.cpp:159-182), which as a launch
+// of its own was 4.6 us of every step.
 template <bool ROW_LDS>
-__global__ __launch_bounds__(kPickThreads) void pick_kernel(const PickParams p) {
+__global__ __launch_bounds__(kPickThreads) void pick_kernel(const PickParams p, const PickEmbed e) {
     extern __shared__ __attribute__((aligned(128))) float lds[];
     const int b = blockIdx.x;
     const int chosen =
@@ -1266,6 +1274,13 @@ __global__ __launch_bounds__(kPickThreads) void pick_kernel(const PickParams p) 
     if (threadIdx.x == 0) {
         p.hist[static_cast<size_t>(b) * p.hist_stride + p.n_hist] = chosen;  // tokens.push_back(next)
         p.tok[b] = chosen;
+    }
+    if (e.x) {
+        for (int j = threadIdx.x; j < e.d; j += kPickThreads) {
+            float v = e.E[static_cast<size_t>(chosen) * e.d + j];
+            if (e.P) v += e.P[static_cast<size_t>(e.pos) * e.d + j];
+            e.x[static_cast<size_t>(b) * e.d + j] = v;
+        }
     }
 }
 
