@@ -422,13 +422,14 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
                 }
             }
             mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+            const float base = mx == -INFINITY ? 0.0f : mx;  // (nothing but -inf here: a mass of 0)
             float sum = 0.0f;
 #pragma unroll
             for (int a = 0; a < NB; a++) {
                 const int n = n0 + 32 * a + 16 * h32;
 #pragma unroll
                 for (int r = 0; r < 16; r++)
-                    if (n + r < p.N) sum += expf(acc[a][b][r] - mx);
+                    if (n + r < p.N) sum += expf(acc[a][b][r] - base);
             }
             sum += __shfl_xor(sum, 32, kWave);
             if (m < p.M && h32 == 0)
@@ -526,7 +527,7 @@ static __global__ __launch_bounds__(256) void nll_parts_kernel(const float2* __r
     float sum = 0.0f;
     for (int i = lane; i < stride; i += 64) {
         const float2 v = row[i];
-        if (v.y > 0.0f) sum += v.y * expf(v.x - mx);
+        if (v.y != 0.0f) sum += v.y * expf(v.x - mx);  // (a run without mass has no maximum; NaN is mass)
     }
     sum = wave_sum(sum);
     if (lane == 0) {

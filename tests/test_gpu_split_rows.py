@@ -51,3 +51,16 @@ def test_rows_match_the_float64_forward(name):
         want = np.log(np.exp(ref - top[:, None]).sum(axis=1)) + top - ref[np.arange(n), tokens[b, 1:]]
         assert np.abs(nll[b] - want).max() <= 2e-5 * max(1.0, np.abs(want).max()), (name, b)
         assert np.abs(last[b] - ref[-1]).max() <= 1e-5 * np.abs(ref[-1]).max(), (name, b)
+
+
+@pytest.mark.parametrize("n", [60, 171])
+def test_a_logit_that_is_not_a_number_reaches_the_loss(n):
+    """One NaN in a row of the embedding that no input uses: every loss is NaN, as it is token by token."""
+    cfg = synth.Config(synth.ARCH_MODERN, 301, 128, 1, 2, 200)
+    W = synth.make_weights(cfg, 81, std=lively_std(cfg), norm_noise=0.1)
+    W[0][300, 5] = np.nan
+    tokens = synth.uniform_tokens(2 * (n + 1), 300, 82).reshape(2, n + 1)
+    gm = G.Model.from_tensors(cfg, W)
+    for flags in (0, G.FLAG_STEPWISE_PROMPT):
+        nll = G.Session(gm, batch=2, flags=flags).score(tokens[:, :-1], tokens[:, 1:])
+        assert np.isnan(nll).all(), (flags, nll)
