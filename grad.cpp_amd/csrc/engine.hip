@@ -128,6 +128,16 @@ struct SplitLayer {
     char *wqkv, *wo, *w1, *w2;
 };
 
+// One allocation of split matrices.
+struct SplitForm {
+    std::mutex mutex;
+    char* blob = nullptr;
+    bool ready = false;
+    ~SplitForm() {
+        if (blob) (void)hipFree(blob);
+    }
+};
+
 // Where tensor i of the file lives on the device.
 struct Placement {
     float* dst;
@@ -147,11 +157,10 @@ struct Model {
     float *rope_cos = nullptr, *rope_sin = nullptr;  // (max_len, head_size/2)
     std::vector<Placement> place;                    // file order
 
-    // Split forms of the matrices: six bytes per weight beside the four above, written by the
-    // first pass over many rows (split_model) and kept.
-    mutable std::mutex split_mutex;
-    mutable char* split_blob = nullptr;
-    mutable char* split_E = nullptr;
+    // Split forms of the matrices, six bytes per weight beside the four above, each written by the
+    // first pass that multiplies by it and kept: the layers' (split_layers), and the logits matrix,
+    // which scoring alone needs and at any length (split_logits).
+    mutable SplitForm layers_split, logits_split;
     mutable std::vector<SplitLayer> split_layers;
 
     // The XCD-sharded persistent kernel reads the weights from a second copy laid
@@ -163,7 +172,6 @@ struct Model {
 
     ~Model() {
         if (blob) (void)hipFree(blob);
-        if (split_blob) (void)hipFree(split_blob);
         if (xcd_stream) (void)hipFree(xcd_stream);
     }
 };
@@ -253,33 +261,44 @@ static bool rows_shape_ok(const Shape& sh) {
     return sh.head_size() == 64 && sh.d_model % 64 == 0 && sh.d_ff() % 64 == 0 && sh.d_model <= 4096;
 }
 
-// Writes the second form of every matrix, once per model.
-static void split_model(const Model& m) {
-    std::lock_guard<std::mutex> lock(m.split_mutex);
-    if (m.split_E) return;
-    const Shape& sh = m.shape;
-    const int d = sh.d_model, F = sh.d_ff(), up = sh.modern() ? 2 : 1;
-    const size_t per_layer = split_bytes(3 * d, d) + split_bytes(d, d) + split_bytes(up * F, d) + split_bytes(d, F);
-    if (!m.split_blob) HIP_CHECK(hipMalloc(&m.split_blob, sh.layers * per_layer + split_bytes(sh.vocab, d)));
-    char* at = m.split_blob;
-    const auto place = [&](const float* src, int N, int K, bool gate_up) {
+// Writes a split form, once per model: fill calls place(src, N, K, gate_up) for every matrix and
+// is given the place of its split form.
+template <class Fill>
+static void make_split_form(SplitForm& f, size_t bytes, Fill fill) {
+    std::lock_guard<std::mutex> lock(f.mutex);
+    if (f.ready) return;
+    if (!f.blob) HIP_CHECK(hipMalloc(&f.blob, bytes));
+    char* at = f.blob;
+    fill([&](const float* src, int N, int K, bool gate_up) {
         split_weights(src, N, K, gate_up, at, nullptr);
         char* const here = at;
         at += split_bytes(N, K);
         return here;
-    };
-    m.split_layers.clear();
-    for (const LayerWeights& w : m.layers) {
-        SplitLayer l;
-        l.wqkv = place(w.wqkv, 3 * d, d, false);
-        l.wo = place(w.wo, d, d, false);
-        l.w1 = place(w.w1, up * F, d, sh.modern());
-        l.w2 = place(w.w2, d, F, false);
-        m.split_layers.push_back(l);
-    }
-    char* const E = place(m.E, sh.vocab, d, false);
+    });
     HIP_CHECK(hipDeviceSynchronize());
-    m.split_E = E;
+    f.ready = true;
+}
+
+static void split_layers(const Model& m) {
+    const Shape& sh = m.shape;
+    const int d = sh.d_model, F = sh.d_ff(), up = sh.modern() ? 2 : 1;
+    const size_t per_layer = split_bytes(3 * d, d) + split_bytes(d, d) + split_bytes(up * F, d) + split_bytes(d, F);
+    make_split_form(m.layers_split, sh.layers * per_layer, [&](auto place) {
+        m.split_layers.clear();
+        for (const LayerWeights& w : m.layers) {
+            SplitLayer l;
+            l.wqkv = place(w.wqkv, 3 * d, d, false);
+            l.wo = place(w.wo, d, d, false);
+            l.w1 = place(w.w1, up * F, d, sh.modern());
+            l.w2 = place(w.w2, d, F, false);
+            m.split_layers.push_back(l);
+        }
+    });
+}
+
+static void split_logits(const Model& m) {
+    make_split_form(m.logits_split, split_bytes(m.shape.vocab, m.shape.d_model),
+                    [&](auto place) { place(m.E, m.shape.vocab, m.shape.d_model, false); });
 }
 
 static std::unique_ptr<Model> upload_model(const Shape& shape, const std::vector<const float*>& t,
@@ -1570,7 +1589,7 @@ static void score_rows(Session& s, const ScoreSink& sink, int M, int n, int t0, 
         s.nll_rows = M;
     }
     norm_split(sh.modern(), s.pp_x, m.gf, m.bf, s.pp_split, M, sh.d_model, s.stream);
-    SplitGemmParams g = split_params(s.pp_split, m.split_E, M, sh.vocab, sh.d_model);
+    SplitGemmParams g = split_params(s.pp_split, m.logits_split.blob, M, sh.vocab, sh.d_model);
     g.rows_per_seq = n;
     g.targets = sink.targets;
     g.nll_t0 = t0;
@@ -1792,7 +1811,8 @@ static void prompt_pass(Session& s, int len, const ScoreSink* sink = nullptr) {
         const int M = n * B;
         const int pos_base = s.pos + t0;
         const bool split = M >= (sink ? kSplitMinScoreRows : kSplitMinRows);
-        if (split || sink) split_model(m);
+        if (split) split_layers(m);
+        if (sink) split_logits(m);
         if (split) reserve_split_attention(s, n, pos_base);
         hipLaunchKernelGGL(embed_rows_kernel, dim3((d + 255) / 256, M), dim3(256), 0, st, m.E, m.P, s.hist,
                            s.hist_stride, s.n_hist + t0, n, pos_base, s.pp_x, d);

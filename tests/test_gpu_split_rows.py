@@ -1,6 +1,8 @@
 """Passes over many rows (prompts and scoring) on the split bf16 products: every tiling the rows
 can take, at row counts that leave ragged tiles, against the float64 forward.  The bound is
 what fp32 sums give, an order below the engine's common 1e-4."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -64,3 +66,35 @@ def test_a_logit_that_is_not_a_number_reaches_the_loss(n):
     for flags in (0, G.FLAG_STEPWISE_PROMPT):
         nll = G.Session(gm, batch=2, flags=flags).score(tokens[:, :-1], tokens[:, 1:])
         assert np.isnan(nll).all(), (flags, nll)
+
+
+def _free_bytes():
+    # by soname: the HIP runtime the process already has
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipDeviceSynchronize() == 0
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_a_short_scoring_pass_does_not_copy_the_layers():
+    """Below 160 rows the layers run on the fp32 weights: only the logits matrix is split."""
+    cfg = synth.Config(synth.ARCH_GPT2, 301, 1024, 4, 16, 200)
+    rng = np.random.default_rng(87)
+    W = [rng.standard_normal((r, c), dtype=np.float32) * np.float32(0.02) for _, r, c, _ in synth.tensor_specs(cfg)]
+    layers = 6 * 4 * 12 * 1024 * 1024  # bytes of their split form
+    gm = G.Model.from_tensors(cfg, W)
+    tokens = synth.uniform_tokens(172, cfg.vocab, 88)
+    s = G.Session(gm)
+    s.score(tokens[:20], tokens[1:21])
+    before = _free_bytes()
+    gm2 = G.Model.from_tensors(cfg, W)
+    model = before - _free_bytes()
+    s2 = G.Session(gm2)
+    s2.score(tokens[:20], tokens[1:21])
+    assert before - model - _free_bytes() < layers // 4
+    s2.score(tokens[:151], tokens[1:152])
+    assert before - model - _free_bytes() < layers // 4
+    s2.reset()
+    s2.score(tokens[:171], tokens[1:172])
+    assert before - model - _free_bytes() >= layers  # from 160 rows on they are
