@@ -133,6 +133,7 @@ struct SplitForm {
     std::mutex mutex;
     char* blob = nullptr;
     bool ready = false;
+    bool unfit = false;  // a weight is outside the range of the parts (kSplitTop): fp32 products only
     ~SplitForm() {
         if (blob) (void)hipFree(blob);
     }
@@ -262,28 +263,37 @@ static bool rows_shape_ok(const Shape& sh) {
 }
 
 // Writes a split form, once per model: fill calls place(src, N, K, gate_up) for every matrix and
-// is given the place of its split form.
+// is given the place of its split form.  False: the weights have none.
 template <class Fill>
-static void make_split_form(SplitForm& f, size_t bytes, Fill fill) {
+static bool make_split_form(SplitForm& f, size_t bytes, Fill fill) {
     std::lock_guard<std::mutex> lock(f.mutex);
-    if (f.ready) return;
-    if (!f.blob) HIP_CHECK(hipMalloc(&f.blob, bytes));
+    if (f.ready || f.unfit) return f.ready;
+    if (!f.blob) HIP_CHECK(hipMalloc(&f.blob, bytes + sizeof(int)));
+    int* const beyond = reinterpret_cast<int*>(f.blob + bytes);  // set if any weight is out of range
+    HIP_CHECK(hipMemset(beyond, 0, sizeof(int)));
     char* at = f.blob;
     fill([&](const float* src, int N, int K, bool gate_up) {
-        split_weights(src, N, K, gate_up, at, nullptr);
+        split_weights(src, N, K, gate_up, at, beyond, nullptr);
         char* const here = at;
         at += split_bytes(N, K);
         return here;
     });
-    HIP_CHECK(hipDeviceSynchronize());
-    f.ready = true;
+    int found = 0;
+    HIP_CHECK(hipMemcpy(&found, beyond, sizeof(int), hipMemcpyDeviceToHost));
+    f.unfit = found != 0;
+    f.ready = !f.unfit;
+    if (f.unfit) {
+        HIP_CHECK(hipFree(f.blob));
+        f.blob = nullptr;
+    }
+    return f.ready;
 }
 
-static void split_layers(const Model& m) {
+static bool split_layers(const Model& m) {
     const Shape& sh = m.shape;
     const int d = sh.d_model, F = sh.d_ff(), up = sh.modern() ? 2 : 1;
     const size_t per_layer = split_bytes(3 * d, d) + split_bytes(d, d) + split_bytes(up * F, d) + split_bytes(d, F);
-    make_split_form(m.layers_split, sh.layers * per_layer, [&](auto place) {
+    return make_split_form(m.layers_split, sh.layers * per_layer, [&](auto place) {
         m.split_layers.clear();
         for (const LayerWeights& w : m.layers) {
             SplitLayer l;
@@ -296,9 +306,9 @@ static void split_layers(const Model& m) {
     });
 }
 
-static void split_logits(const Model& m) {
-    make_split_form(m.logits_split, split_bytes(m.shape.vocab, m.shape.d_model),
-                    [&](auto place) { place(m.E, m.shape.vocab, m.shape.d_model, false); });
+static bool split_logits(const Model& m) {
+    return make_split_form(m.logits_split, split_bytes(m.shape.vocab, m.shape.d_model),
+                           [&](auto place) { place(m.E, m.shape.vocab, m.shape.d_model, false); });
 }
 
 static std::unique_ptr<Model> upload_model(const Shape& shape, const std::vector<const float*>& t,
@@ -1523,7 +1533,7 @@ constexpr size_t kPromptPassRows = 32768; // rows per pass; longer prompts run i
 
 static bool prompt_pass_ok(const Session& s, int len) {
     const Shape& sh = s.m->shape;
-    return len >= kPromptPassMin && rows_shape_ok(sh);
+    return s.use_prompt_pass && len >= kPromptPassMin && rows_shape_ok(sh);
 }
 
 // Passes of this many rows and more take the split projections (kernels_split.h); below,
@@ -1535,6 +1545,24 @@ static bool prompt_pass_ok(const Session& s, int len) {
 // hundred picks, so the order of a prompt's sums shows in the reply, and under 512 rows the
 // prompt is the small part of the request (397 tokens and 64 sampled ones: 1.4 of 12.5 ms).
 constexpr int kSplitMinRows = 512, kSplitMinScoreRows = 160;
+
+// How a pass over len tokens of every sequence runs: in slices of `slice` tokens (0: token by
+// token), those of split_rows rows and more on the split weights.
+struct RowsPlan {
+    int slice;
+    int split_rows;
+};
+
+// Decided before anything is launched.  Weights without a split form leave the small fp32 tiles,
+// in slices below the rows from which the split projections take over (the tiles' buffers hold no
+// more), and for scoring, whose logits come from the split matrix alone, the token-by-token way.
+static RowsPlan plan_rows(const Session& s, int len, bool score) {
+    if (!prompt_pass_ok(s, len) || (score && !split_logits(*s.m))) return {0, 0};
+    const int most = static_cast<int>(std::max<size_t>(1, std::min<size_t>(len, kPromptPassRows / s.B)));
+    const int split_rows = score ? kSplitMinScoreRows : kSplitMinRows;
+    if (static_cast<long>(most) * s.B < split_rows || split_layers(*s.m)) return {most, split_rows};
+    return {std::min(len, (kSplitMinRows - 1) / s.B), kSplitMinRows};
+}
 
 // One projection over M rows (norm folded in for RMSNorm, a norm kernel for LayerNorm).
 template <int PRO, int EPI>
@@ -1799,20 +1827,18 @@ static void reserve_split_attention(Session& s, int n, int pos_base) {
 // Tokens hist[n_hist .. n_hist + len) of every sequence, positions pos .. pos + len.
 // Equivalent to len step() calls (text_gen.cpp:44-46); only the last logits are
 // formed unless a sink asks for the likelihood of a target at every position.
-static void prompt_pass(Session& s, int len, const ScoreSink* sink = nullptr) {
+static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSink* sink = nullptr) {
     const Model& m = *s.m;
     const Shape& sh = m.shape;
     const int d = sh.d_model, B = s.B;
     hipStream_t st = s.stream;
-    const int slice = static_cast<int>(std::max<size_t>(1, std::min<size_t>(len, kPromptPassRows / B)));
+    const int slice = plan.slice;
     reserve_prompt_rows(s, static_cast<size_t>(slice) * B);
     for (int t0 = 0; t0 < len; t0 += slice) {
         const int n = std::min(slice, len - t0);
         const int M = n * B;
         const int pos_base = s.pos + t0;
-        const bool split = M >= (sink ? kSplitMinScoreRows : kSplitMinRows);
-        if (split) split_layers(m);
-        if (sink) split_logits(m);
+        const bool split = M >= plan.split_rows;
         if (split) reserve_split_attention(s, n, pos_base);
         hipLaunchKernelGGL(embed_rows_kernel, dim3((d + 255) / 256, M), dim3(256), 0, st, m.E, m.P, s.hist,
                            s.hist_stride, s.n_hist + t0, n, pos_base, s.pp_x, d);
@@ -1848,8 +1874,9 @@ static void prompt_pass(Session& s, int len, const ScoreSink* sink = nullptr) {
 // prompt loop of text_gen.cpp:44-46).  log: per-step logits destination or null.
 static void run_prompt(Session& s, int len, float* log, size_t* steps_logged) {
     const size_t BV = static_cast<size_t>(s.B) * s.m->shape.vocab;
-    if (!log && s.use_prompt_pass && prompt_pass_ok(s, len)) {
-        prompt_pass(s, len);
+    const RowsPlan plan = log ? RowsPlan{0, 0} : plan_rows(s, len, /*score=*/false);
+    if (plan.slice > 0) {
+        prompt_pass(s, len, plan);
         if (steps_logged) *steps_logged += len;
         return;
     }
@@ -2462,8 +2489,9 @@ gh_status gh_session_score(gh_session* sess, const int32_t* ids, const int32_t* 
         }
         stage_ids(s, host_targets, len, s.score_targets, len, 0);
         const ScoreSink sink{s.score_targets, s.score_nll};
-        if (s.use_prompt_pass && prompt_pass_ok(s, len)) {
-            prompt_pass(s, len, &sink);
+        const RowsPlan plan = plan_rows(s, len, /*score=*/true);
+        if (plan.slice > 0) {
+            prompt_pass(s, len, plan, &sink);
         } else {
             // token by token: every step leaves the logits of its position
             const int V = s.m->shape.vocab;

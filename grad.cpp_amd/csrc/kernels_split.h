@@ -4,7 +4,7 @@
 //
 //   a = a1 + a2 + a3,  a1 = bf16(a), a2 = bf16(a - a1), a3 = bf16(a - a1 - a2)
 //
-// The split is exact: rounding to nearest leaves |a - a1| <= 2^-9 |a| (16 significant bits),
+// The split is exact in its range: rounding to nearest leaves |a - a1| <= 2^-9 |a| (16 significant bits),
 // |a - a1 - a2| <= 2^-18 |a| (8 bits), which a3 holds whole.  A product of two such numbers
 // needs the nine products of parts; the six kept here are those down to 2^-18 of a b
 // (a1 b1, a1 b2, a2 b1, a2 b2, a1 b3, a3 b1).  The three left out sum to less than
@@ -12,6 +12,13 @@
 // fp32 dot product formed this way is as good as one formed of fp32 products: both are
 // dominated by the roundings of the running sum, and there are fewer of those here (one per
 // 16 terms against one per 2).
+//
+// The range: from kSplitTop (3.396e38, the last 2^-9 below the largest float) a1 would be infinite
+// and a2 not a number, so weights are checked when they are split, and a form with one that large,
+// or an infinite one, is not used: its passes stay on fp32 products (a NaN is one either way).
+// Activations are not checked; one there lies within 2^-9 of its own overflow.  Below 2^-103 the
+// small parts are subnormal: at most 2^-125 times the other factor is lost, nothing in a sum that
+// any ordinary weight takes part in.
 //
 // Why: on this part an fp32 matrix product runs at the vector rate (157 TFLOP/s; nothing
 // vector issues beside it), a bf16 one at sixteen times that, so six of them are still 2.7
@@ -42,6 +49,8 @@ __device__ __forceinline__ void split_pair(float x, float y, unsigned& p1, unsig
     p2 = pack(x, y);
     p3 = pack(x - lo(p2), y - hi(p2));
 }
+
+constexpr unsigned kSplitTop = 0x7F7F8000u;  // bits of the smallest magnitude that rounds to an infinite bf16
 
 // Storage of a split matrix (rows x K, K a multiple of 16): blocks of 16 rows x 16 columns,
 // 1536 contiguous bytes each, row group by row group and inside one along K.  In a block a
@@ -101,10 +110,10 @@ __host__ __device__ __forceinline__ int split_output_of_row(int row) {
 }
 
 // Writes the split form of a weight matrix src (N x K, row per output).  Row `row` of the split matrix is
-// output split_output_of_row(row), zeros past N.  gate_up: src rows are (gate, up) pairs, and
+// output split_output_of_row(row), zeros past N; *beyond is set if a weight is out of range.  gate_up: src rows are (gate, up) pairs, and
 // every 16 outputs are the gates of eight hidden units and then their ups.
 static __global__ __launch_bounds__(256) void split_weights_kernel(const float* __restrict__ src, int N, int K,
-                                                                   int rows, int gate_up, char* dst) {
+                                                                   int rows, int gate_up, char* dst, int* beyond) {
     const int chunks = K >> 3;
     const size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
     if (i >= static_cast<size_t>(rows) * chunks) return;
@@ -117,6 +126,13 @@ static __global__ __launch_bounds__(256) void split_weights_kernel(const float* 
         const float4 b = *reinterpret_cast<const float4*>(src + static_cast<size_t>(n) * K + k + 4);
         v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
     }
+    bool out = false;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const unsigned size = __float_as_uint(v[e]) & 0x7FFFFFFFu;
+        out |= size >= kSplitTop && size <= 0x7F800000u;
+    }
+    if (out) *beyond = 1;
     store_split8(dst, row, k, K / kSplitCols, v);
 }
 

@@ -12,8 +12,9 @@ inline size_t split_bytes(size_t rows, size_t cols) {
     return (rows + kSplitPad - 1) / kSplitPad * kSplitPad * cols * 6;
 }
 
-// Writes the split form of src (N x K); gate_up: src rows are (gate, up) pairs.
-void split_weights(const float* src, int N, int K, bool gate_up, char* dst, hipStream_t st);
+// Writes the split form of src (N x K); gate_up: src rows are (gate, up) pairs.  *beyond is set if
+// a weight is outside the range of the parts.
+void split_weights(const float* src, int N, int K, bool gate_up, char* dst, int* beyond, hipStream_t st);
 
 // norm(x) of M rows in split form.
 void norm_split(bool rms, const float* x, const float* gamma, const float* beta, char* out, int M, int d, hipStream_t st);

@@ -13,11 +13,11 @@ static void check(hipError_t e, const char* what) {
     if (e != hipSuccess) throw std::runtime_error(std::string("HIP error in ") + what + ": " + hipGetErrorString(e));
 }
 
-void split_weights(const float* src, int N, int K, bool gate_up, char* dst, hipStream_t st) {
+void split_weights(const float* src, int N, int K, bool gate_up, char* dst, int* beyond, hipStream_t st) {
     const int rows = (N + kSplitPad - 1) / kSplitPad * kSplitPad;
     const size_t chunks = static_cast<size_t>(rows) * (K / 8);
     hipLaunchKernelGGL(split_weights_kernel, dim3(static_cast<unsigned>((chunks + 255) / 256)), dim3(256), 0, st, src, N,
-                       K, rows, gate_up ? 1 : 0, dst);
+                       K, rows, gate_up ? 1 : 0, dst, beyond);
     check(hipGetLastError(), "split_weights");
 }
 

@@ -98,3 +98,42 @@ def test_a_short_scoring_pass_does_not_copy_the_layers():
     s2.reset()
     s2.score(tokens[:171], tokens[1:172])
     assert before - model - _free_bytes() >= layers  # from 160 rows on they are
+
+
+def _loss(ref, targets):
+    top = ref.max(axis=1)
+    return np.log(np.exp(ref - top[:, None]).sum(axis=1)) + top - ref[np.arange(len(targets)), targets]
+
+
+@pytest.mark.parametrize("n", [60, 171])
+def test_an_infinitely_unlikely_token_adds_nothing_to_the_loss(n):
+    """A logit of -inf: an infinite weight against an activation that is positive at every position."""
+    cfg = synth.Config(synth.ARCH_GPT2, 301, 128, 1, 2, 200)
+    W = synth.make_weights(cfg, 83, std=lively_std(cfg), norm_noise=0.1)
+    W[0][300, 5] = -np.inf
+    W[-1][0, 5] = 30.0  # beta of the final norm
+    tokens = synth.uniform_tokens(2 * (n + 1), 300, 84).reshape(2, n + 1)
+    ref = ref_forward.forward(cfg, W, tokens[1, :-1])
+    assert (ref[:, 300] == -np.inf).all()
+    want = _loss(ref, tokens[1, 1:])
+    nll = G.Session(G.Model.from_tensors(cfg, W), batch=2).score(tokens[:, :-1], tokens[:, 1:])
+    assert np.abs(nll[1] - want).max() <= 2e-5 * max(1.0, np.abs(want).max())
+
+
+def test_weights_beyond_the_range_of_the_split():
+    """A weight that rounds to an infinite bf16: the gate of a hidden unit whose output is not used."""
+    cfg = synth.Config(synth.ARCH_MODERN, 301, 128, 1, 2, 640)
+    W = synth.make_weights(cfg, 85, std=lively_std(cfg), norm_noise=0.1)
+    names = [what[0] for what in synth.tensor_specs(cfg)]
+    W[names.index("layer 0 FFN gate")][5, 0] = 3.4e38
+    W[names.index("layer 0 norm2 gamma")][0, 5] = 1e-3
+    W[names.index("layer 0 FFN down")][0, :] = 0.0
+    tokens = synth.uniform_tokens(601, cfg.vocab, 86)
+    with np.errstate(over="ignore"):
+        ref = ref_forward.forward(cfg, W, tokens[:-1])
+    gm = G.Model.from_tensors(cfg, W)
+    last = G.Session(gm).prefill(tokens[:-1])[0]
+    assert np.abs(last - ref[-1]).max() <= 1e-5 * np.abs(ref[-1]).max()
+    nll = G.Session(gm).score(tokens[:-1], tokens[1:])[0]
+    want = _loss(ref, tokens[1:])
+    assert np.abs(nll - want).max() <= 2e-5 * max(1.0, np.abs(want).max())
