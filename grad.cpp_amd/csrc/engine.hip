@@ -78,6 +78,25 @@ static void require_gpu() {
     }
 }
 
+// Device memory that a call is faster with and can do without, uncleared: false, and nothing
+// allocated, if there is not enough.
+template <typename T>
+static bool try_alloc(T*& p, size_t n) {
+    p = nullptr;
+    const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
+    // Test aid: no allocation of this kind above so many bytes.
+    if (const char* most = std::getenv("GRADHIP_TEST_SPARE_BYTES"))
+        if (bytes > std::strtoull(most, nullptr, 10)) return false;
+    const hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();  // (a later launch's check would find it)
+        p = nullptr;
+        return false;
+    }
+    HIP_CHECK(e);
+    return true;
+}
+
 // ------------------------------------------------------------ device model
 
 // Layout kernels.  Matrices arrive (in, out) row-major as grad.cpp stores them
@@ -263,12 +282,13 @@ static bool rows_shape_ok(const Shape& sh) {
 }
 
 // Writes a split form, once per model: fill calls place(src, N, K, gate_up) for every matrix and
-// is given the place of its split form.  False: the weights have none.
+// is given the place of its split form.  False: the weights have none, or there is no memory for it
+// now (the next pass asks again).
 template <class Fill>
 static bool make_split_form(SplitForm& f, size_t bytes, Fill fill) {
     std::lock_guard<std::mutex> lock(f.mutex);
     if (f.ready || f.unfit) return f.ready;
-    if (!f.blob) HIP_CHECK(hipMalloc(&f.blob, bytes + sizeof(int)));
+    if (!f.blob && !try_alloc(f.blob, bytes + sizeof(int))) return false;
     int* const beyond = reinterpret_cast<int*>(f.blob + bytes);  // set if any weight is out of range
     HIP_CHECK(hipMemset(beyond, 0, sizeof(int)));
     char* at = f.blob;
@@ -1553,7 +1573,7 @@ struct RowsPlan {
     int split_rows;
 };
 
-// Decided before anything is launched.  Weights without a split form leave the small fp32 tiles,
+// Decided before anything is launched.  Weights without a split form, or no memory for it, leave the small fp32 tiles,
 // in slices below the rows from which the split projections take over (the tiles' buffers hold no
 // more), and for scoring, whose logits come from the split matrix alone, the token-by-token way.
 static RowsPlan plan_rows(const Session& s, int len, bool score) {
@@ -1606,16 +1626,6 @@ static SplitGemmParams split_params(const char* A, const char* W, int M, int N, 
 static void score_rows(Session& s, const ScoreSink& sink, int M, int n, int t0, int len) {
     const Model& m = *s.m;
     const Shape& sh = m.shape;
-    if (s.nll_rows < static_cast<size_t>(M)) {
-        if (s.nll_part) HIP_CHECK(hipFree(s.nll_part));
-        if (s.nll_target) HIP_CHECK(hipFree(s.nll_target));
-        s.nll_part = nullptr;
-        s.nll_target = nullptr;
-        s.nll_rows = 0;
-        dev_alloc(s.nll_part, static_cast<size_t>(M) * split_nll_stride(sh.vocab));
-        dev_alloc(s.nll_target, M);
-        s.nll_rows = M;
-    }
     norm_split(sh.modern(), s.pp_x, m.gf, m.bf, s.pp_split, M, sh.d_model, s.stream);
     SplitGemmParams g = split_params(s.pp_split, m.logits_split.blob, M, sh.vocab, sh.d_model);
     g.rows_per_seq = n;
@@ -1651,9 +1661,9 @@ static void launch_prompt_attn(const Session& s, const PrefillAttnParams& a) {
     HIP_CHECK(hipGetLastError());
 }
 
-// One layer over M = n * B rows of pp_x through the split projections.  keys_only: nothing but
-// the keys and values.
-static void prompt_layer_split(Session& s, int layer, int n, int pos_base, bool keys_only) {
+// One layer over M = n * B rows of pp_x through the split projections, and with split_attn through the
+// split attention.  keys_only: nothing but the keys and values.
+static void prompt_layer_split(Session& s, int layer, int n, int pos_base, bool split_attn, bool keys_only) {
     const Model& m = *s.m;
     const Shape& sh = m.shape;
     const LayerWeights& w = m.layers[layer];
@@ -1684,7 +1694,7 @@ static void prompt_layer_split(Session& s, int layer, int n, int pos_base, bool 
 
     PrefillAttnParams a = prompt_attn_params(s, layer, n, pos_base);
     a.out_split = s.pp_split;
-    if (n > kSplitAttnMin) split_attention(a, s.B, s.pp_kv, s.pp_part, st);
+    if (split_attn) split_attention(a, s.B, s.pp_kv, s.pp_part, st);
     else launch_prompt_attn(s, a);
 
     g = split_params(s.pp_split, sw.wo, M, d, d);
@@ -1780,48 +1790,55 @@ static void prompt_layer_small(Session& s, int layer, int n, int pos_base) {
     project_rows<PRO_PLAIN, EPI_RESID>(s, g, M);
 }
 
-// Activations of a prompt pass of up to `rows` rows (grown on demand).
-static void reserve_prompt_rows(Session& s, size_t rows) {
-    const size_t d = s.m->shape.d_model, F = s.m->shape.d_ff();
-    if (s.pp_rows >= rows) return;
-    for (float** b : {&s.pp_x, &s.pp_q, &s.pp_attn, &s.pp_norm, &s.pp_hidden}) {
-        if (*b) HIP_CHECK(hipFree(*b));
-        *b = nullptr;
-    }
-    for (char** b : {&s.pp_split, &s.pp_split_hidden}) {
-        if (*b) HIP_CHECK(hipFree(*b));
-        *b = nullptr;
-    }
-    s.pp_rows = 0;
-    dev_alloc(s.pp_x, rows * d);
-    dev_alloc(s.pp_q, rows * d);
-    const size_t few = std::min<size_t>(rows, kSplitMinRows);  // what the small tiles still take
-    dev_alloc(s.pp_attn, few * d);
-    dev_alloc(s.pp_norm, few * d);
-    dev_alloc(s.pp_hidden, few * F);
-    dev_alloc(s.pp_split, split_bytes(rows, d));
-    dev_alloc(s.pp_split_hidden, split_bytes(rows, F));
-    s.pp_rows = rows;
+// The session's buffer p of n elements, cleared, in place of the one it had.
+template <typename T>
+static bool replace_buffer(Session& s, T*& p, size_t n) {
+    if (p) HIP_CHECK(hipFree(p));
+    if (!try_alloc(p, n)) return false;
+    HIP_CHECK(hipMemsetAsync(p, 0, std::max<size_t>(n, 1) * sizeof(T), s.stream));
+    return true;
 }
 
-// Scratch of a split pass's attention over n new positions behind pos_base (grown on demand).
-static void reserve_split_attention(Session& s, int n, int pos_base) {
-    if (n <= kSplitAttnMin) return;
+// Activations of a prompt pass of up to `rows` rows (grown on demand).  False: not enough memory.
+static bool reserve_prompt_rows(Session& s, size_t rows) {
+    const size_t d = s.m->shape.d_model, F = s.m->shape.d_ff();
+    if (s.pp_rows >= rows) return true;
+    s.pp_rows = 0;
+    const size_t few = std::min<size_t>(rows, kSplitMinRows);  // what the small tiles still take
+    const bool all = replace_buffer(s, s.pp_x, rows * d) && replace_buffer(s, s.pp_q, rows * d)
+                     && replace_buffer(s, s.pp_attn, few * d) && replace_buffer(s, s.pp_norm, few * d)
+                     && replace_buffer(s, s.pp_hidden, few * F) && replace_buffer(s, s.pp_split, split_bytes(rows, d))
+                     && replace_buffer(s, s.pp_split_hidden, split_bytes(rows, F));
+    if (all) s.pp_rows = rows;
+    return all;
+}
+
+// What scoring leaves of that many rows' logits.
+static bool reserve_score_rows(Session& s, size_t rows) {
+    if (s.nll_rows >= rows) return true;
+    s.nll_rows = 0;
+    const bool all = replace_buffer(s, s.nll_part, rows * split_nll_stride(s.m->shape.vocab))
+                     && replace_buffer(s, s.nll_target, rows);
+    if (all) s.nll_rows = rows;
+    return all;
+}
+
+// Scratch of a split pass's attention over n new positions behind pos_base (grown on demand).  False:
+// the fp32 kernel, which needs none, does it.
+static bool reserve_split_attention(Session& s, int n, int pos_base) {
+    if (n <= kSplitAttnMin) return false;
     const SplitAttnSpace need = split_attention_space(s.B, s.m->shape.heads, n, pos_base);
     if (s.pp_kv_bytes < need.kv_bytes) {
-        if (s.pp_kv) HIP_CHECK(hipFree(s.pp_kv));
-        s.pp_kv = nullptr;
         s.pp_kv_bytes = 0;
-        dev_alloc(s.pp_kv, need.kv_bytes);
+        if (!replace_buffer(s, s.pp_kv, need.kv_bytes)) return false;
         s.pp_kv_bytes = need.kv_bytes;
     }
     if (s.pp_part_floats < need.part_floats) {
-        if (s.pp_part) HIP_CHECK(hipFree(s.pp_part));
-        s.pp_part = nullptr;
         s.pp_part_floats = 0;
-        dev_alloc(s.pp_part, need.part_floats);
+        if (!replace_buffer(s, s.pp_part, need.part_floats)) return false;
         s.pp_part_floats = need.part_floats;
     }
+    return true;
 }
 
 // Tokens hist[n_hist .. n_hist + len) of every sequence, positions pos .. pos + len.
@@ -1832,14 +1849,22 @@ static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSi
     const Shape& sh = m.shape;
     const int d = sh.d_model, B = s.B;
     hipStream_t st = s.stream;
-    const int slice = plan.slice;
-    reserve_prompt_rows(s, static_cast<size_t>(slice) * B);
+    // (too little memory for the slices: shorter ones, down to the rows that the small tiles take)
+    int slice = plan.slice;
+    const auto reserved = [&] {
+        const size_t rows = static_cast<size_t>(slice) * B;
+        return reserve_prompt_rows(s, rows) && (!sink || reserve_score_rows(s, rows));
+    };
+    while (!reserved()) {
+        if (slice == 1 || slice * B < kSplitMinRows) throw ApiError{GH_ERR_DEVICE, "out of device memory for a prompt pass"};
+        slice = (slice + 1) / 2;
+    }
     for (int t0 = 0; t0 < len; t0 += slice) {
         const int n = std::min(slice, len - t0);
         const int M = n * B;
         const int pos_base = s.pos + t0;
         const bool split = M >= plan.split_rows;
-        if (split) reserve_split_attention(s, n, pos_base);
+        const bool split_attn = split && reserve_split_attention(s, n, pos_base);
         hipLaunchKernelGGL(embed_rows_kernel, dim3((d + 255) / 256, M), dim3(256), 0, st, m.E, m.P, s.hist,
                            s.hist_stride, s.n_hist + t0, n, pos_base, s.pp_x, d);
         HIP_CHECK(hipGetLastError());
@@ -1847,7 +1872,7 @@ static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSi
         // else at the last position alone, where the decode step's launches are as good.
         const bool trim = split && !sink;
         for (int l = 0; l < sh.layers; l++) {
-            if (split) prompt_layer_split(s, l, n, pos_base, trim && l == sh.layers - 1);
+            if (split) prompt_layer_split(s, l, n, pos_base, split_attn, trim && l == sh.layers - 1);
             else prompt_layer_small(s, l, n, pos_base);
         }
         if (sink) score_rows(s, *sink, M, n, t0, len);

@@ -137,3 +137,23 @@ def test_weights_beyond_the_range_of_the_split():
     nll = G.Session(gm).score(tokens[:-1], tokens[1:])[0]
     want = _loss(ref, tokens[1:])
     assert np.abs(nll - want).max() <= 2e-5 * max(1.0, np.abs(want).max())
+
+
+@pytest.mark.parametrize("spare", [7 << 18, 3 << 20, 11 << 20])
+def test_passes_that_find_little_memory_left(spare, monkeypatch):
+    """8 x 1000 rows with no allocation above 1.75 MiB (nothing is split, slices of 504 rows), 3 MiB (the
+    logits matrix is) and 11 MiB (the layers are; slices of 2000 rows, the last with the fp32 attention).
+    (No rotation: at position 1000 its fp32 angles are 2e-5 of eight layers' logits.)"""
+    cfg = synth.Config(synth.ARCH_GPT2, 3000, 128, 8, 2, 1001)
+    W = synth.make_weights(cfg, 89, std=lively_std(cfg), norm_noise=0.1)
+    tokens = synth.uniform_tokens(8 * 1001, cfg.vocab, 90).reshape(8, 1001)
+    ref = ref_forward.forward(cfg, W, tokens[7, :-1])
+    monkeypatch.setenv("GRADHIP_TEST_SPARE_BYTES", str(spare))
+    gm = G.Model.from_tensors(cfg, W)
+    last = G.Session(gm, batch=8).prefill(tokens[:, :-1])
+    assert np.abs(last[7] - ref[-1]).max() <= 1e-5 * np.abs(ref[-1]).max()
+    nll = G.Session(gm, batch=8).score(tokens[:, :-1], tokens[:, 1:])
+    want = _loss(ref, tokens[7, 1:])
+    assert np.abs(nll[7] - want).max() <= 2e-5 * max(1.0, np.abs(want).max())
+    monkeypatch.delenv("GRADHIP_TEST_SPARE_BYTES")
+    assert np.abs(G.Session(gm, batch=8).score(tokens[:, :-1], tokens[:, 1:]) - nll).max() <= 2e-5 * np.abs(want).max()
