@@ -1694,7 +1694,7 @@ static void prompt_layer_split(Session& s, int layer, int n, int pos_base, bool 
 
     PrefillAttnParams a = prompt_attn_params(s, layer, n, pos_base);
     a.out_split = s.pp_split;
-    if (split_attn) split_attention(a, s.B, s.pp_kv, s.pp_part, st);
+    if (split_attn) split_attention(a, s.B, s.pp_kv, s.pp_kv_bytes, s.pp_part, st);
     else launch_prompt_attn(s, a);
 
     g = split_params(s.pp_split, sw.wo, M, d, d);
@@ -1823,20 +1823,25 @@ static bool reserve_score_rows(Session& s, size_t rows) {
     return all;
 }
 
-// Scratch of a split pass's attention over n new positions behind pos_base (grown on demand).  False:
-// the fp32 kernel, which needs none, does it.
+// Scratch of a split pass's attention over n new positions behind pos_base: for keys and values what
+// the session's whole context can use, so that it is allocated once (nothing in it is read that the
+// pass has not written, so it is not cleared); partial results grow in steps of 8 MB, up to some 45.
+// False: there is no memory, or too little work; the fp32 kernel, which needs none, does it.
 static bool reserve_split_attention(Session& s, int n, int pos_base) {
     if (n <= kSplitAttnMin) return false;
-    const SplitAttnSpace need = split_attention_space(s.B, s.m->shape.heads, n, pos_base);
-    if (s.pp_kv_bytes < need.kv_bytes) {
-        s.pp_kv_bytes = 0;
-        if (!replace_buffer(s, s.pp_kv, need.kv_bytes)) return false;
-        s.pp_kv_bytes = need.kv_bytes;
+    const int heads = s.m->shape.heads;
+    if (!s.pp_kv) {
+        const size_t bytes = split_attention_kv_bytes(s.B, heads, s.m->shape.max_len);
+        if (!try_alloc(s.pp_kv, bytes)) return false;
+        s.pp_kv_bytes = bytes;
     }
-    if (s.pp_part_floats < need.part_floats) {
+    const size_t need = split_attention_part_floats(s.B, heads, n, pos_base, s.pp_kv_bytes);
+    if (s.pp_part_floats < need) {
+        if (s.pp_part) HIP_CHECK(hipFree(s.pp_part));
         s.pp_part_floats = 0;
-        if (!replace_buffer(s, s.pp_part, need.part_floats)) return false;
-        s.pp_part_floats = need.part_floats;
+        const size_t floats = align_up(need, size_t{2} << 20);
+        if (!try_alloc(s.pp_part, floats)) return false;
+        s.pp_part_floats = floats;
     }
     return true;
 }

@@ -14,19 +14,22 @@ namespace gh {
 constexpr int kAttnOperand = 64 * 4 * kSplitRowBytes;  // 24 KB
 constexpr int kAttnTile = 2 * kAttnOperand;
 
+// A launch covers a run of the (sequence, head) pairs, sequence by sequence.
 struct SplitKvParams {
     KvLayout kv;
     int layer;
+    int first;      // pair of workgroups y = 0
     int positions;  // filled positions of every sequence
-    char* out;      // [batch][heads][ceil(positions / 64)][kAttnTile]
+    char* out;      // [pairs of the launch][ceil(positions / 64)][kAttnTile]
 };
 
 // One workgroup per tile; rows past the last position become zeros (their scores are masked,
 // and a weight of zero times what an earlier pass left must stay zero).
 static __global__ __launch_bounds__(256) void split_kv_kernel(const SplitKvParams p) {
     __shared__ float vs[64][65];
-    const int tile = blockIdx.x, h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x;
-    char* out = p.out + ((static_cast<size_t>(b) * p.kv.heads + h) * gridDim.x + tile) * kAttnTile;
+    const int tile = blockIdx.x, tid = threadIdx.x;
+    const int pair = p.first + blockIdx.y, b = pair / p.kv.heads, h = pair - b * p.kv.heads;
+    char* out = p.out + (static_cast<size_t>(blockIdx.y) * gridDim.x + tile) * kAttnTile;
 #pragma unroll
     for (int i = 0; i < 2; i++) {
         const int row = (tid >> 3) + 32 * i, k = (tid & 7) * 8, pos = tile * 64 + row;
@@ -58,25 +61,24 @@ static __global__ __launch_bounds__(256) void split_kv_kernel(const SplitKvParam
 struct SplitAttnParams {
     const float* q;  // [batch * len][d_model], rotated
     const char* kv;  // split_kv_kernel's tiles
-    int tiles;       // ... per (sequence, head)
+    int tiles;       // ... per pair
     char* out;       // split rows [batch * len] x d_model
     float* part;     // partial results of query blocks whose keys are shared among workgroups
     int d_model, heads, len, pos_base;
     int chunk_shift;  // a workgroup takes up to 1 << chunk_shift tiles of keys
-    int items;        // workgroups per (sequence, head)
-    int batch;
+    int items;        // workgroups per pair
+    int first, pairs;  // the pairs of this launch
     float scale;
 };
 
 // Workgroup ids go round-robin over the eight XCDs.  With many (sequence, head) pairs all
 // workgroups of one sit on one XCD, whose L2 then serves its keys and values to every query
 // block after the first (192 pairs: 1024 tokens 247 -> 198 us, 1536 tokens 411 -> 388); with few the pairs would
-// not spread evenly (12 pairs, 1999 tokens: 47 -> 57 us) and ids are dealt as they come.  False
-// for an id past the last pair.
-__device__ __forceinline__ bool attn_place(const SplitAttnParams& p, int& b, int& h, int& item) {
-    const int id = static_cast<int>(blockIdx.x), pairs = p.batch * p.heads;
-    int pair;
-    if (pairs >= 64 || (pairs & 7) == 0) {
+// not spread evenly (12 pairs, 1999 tokens: 47 -> 57 us) and ids are dealt as they come.  pair:
+// counted from the launch's first.  False for an id past the last pair.
+__device__ __forceinline__ bool attn_place(const SplitAttnParams& p, int& pair, int& b, int& h, int& item) {
+    const int id = static_cast<int>(blockIdx.x);
+    if (p.pairs >= 64 || (p.pairs & 7) == 0) {
         const int slot = id >> 3, g = slot / p.items;
         pair = (id & 7) + 8 * g;
         item = slot - g * p.items;
@@ -84,9 +86,9 @@ __device__ __forceinline__ bool attn_place(const SplitAttnParams& p, int& b, int
         pair = id / p.items;
         item = id - pair * p.items;
     }
-    b = pair / p.heads;
-    h = pair - b * p.heads;
-    return pair < pairs;
+    b = (p.first + pair) / p.heads;
+    h = p.first + pair - b * p.heads;
+    return pair < p.pairs;
 }
 
 constexpr int kAttnQueries = 128;
@@ -119,8 +121,8 @@ __host__ __device__ __forceinline__ int attn_parts(int i, int len, int pos_base,
 // split of the probabilities) runs beside the other's 96 products.
 static __global__ __launch_bounds__(256, 2) void attn_split_kernel(const SplitAttnParams p) {
     extern __shared__ __attribute__((aligned(1024))) char lds_attn[];
-    int b, h, item;
-    if (!attn_place(p, b, h, item)) return;
+    int pair, b, h, item;
+    if (!attn_place(p, pair, b, h, item)) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n32 = lane & 31, h32 = lane >> 5;
     // longest query blocks first
@@ -136,7 +138,7 @@ static __global__ __launch_bounds__(256, 2) void attn_split_kernel(const SplitAt
     const int wave_last = p.pos_base + min(p.len, qb * kAttnQueries + wave * 32 + 32) - 1;  // last key of this wavefront
     const int wave_first = p.pos_base + min(p.len - 1, qb * kAttnQueries + wave * 32);      // position of its first query
 
-    const char* const src = p.kv + (static_cast<size_t>(b) * p.heads + h) * p.tiles * kAttnTile;
+    const char* const src = p.kv + static_cast<size_t>(pair) * p.tiles * kAttnTile;
     const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) char*)lds_attn));
     constexpr int kLoads = kAttnOperand / 1024 / 4;  // per wavefront and operand: two in front of each of three steps
     const int operands = 2 * (tile1 - tile0);
@@ -297,7 +299,7 @@ static __global__ __launch_bounds__(256, 2) void attn_split_kernel(const SplitAt
         slot = slot == kAttnRing - 1 ? 0 : slot + 1;
     }
     if (parts > 1) {
-        float* part = p.part + ((static_cast<size_t>(b) * p.heads + h) * p.items + item) * kAttnPart + wave * (34 * 64) + lane;
+        float* part = p.part + (static_cast<size_t>(pair) * p.items + item) * kAttnPart + wave * (34 * 64) + lane;
         part[0] = m;
         part[64] = l;
 #pragma unroll
@@ -316,14 +318,14 @@ static __global__ __launch_bounds__(256, 2) void attn_split_kernel(const SplitAt
 
 // Folds the partial results of a query block, in the order of the keys.
 static __global__ __launch_bounds__(256) void attn_split_merge_kernel(const SplitAttnParams p) {
-    const int h = blockIdx.y, b = blockIdx.z;
+    const int pair = p.first + blockIdx.y, b = pair / p.heads, h = pair - b * p.heads;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h32 = lane >> 5;
     const int qb = (p.len + kAttnQueries - 1) / kAttnQueries - 1 - static_cast<int>(blockIdx.x);
     int first = 0;
     for (int i = qb + 1; i * kAttnQueries < p.len; i++) first += attn_parts(i, p.len, p.pos_base, p.chunk_shift);
     const int parts = attn_parts(qb, p.len, p.pos_base, p.chunk_shift), t = qb * kAttnQueries + wave * 32 + (lane & 31);
     if (parts == 1 || t >= p.len) return;
-    const float* part = p.part + ((static_cast<size_t>(b) * p.heads + h) * p.items + first) * kAttnPart + wave * (34 * 64) + lane;
+    const float* part = p.part + (static_cast<size_t>(blockIdx.y) * p.items + first) * kAttnPart + wave * (34 * 64) + lane;
     float m = -INFINITY, l = 0.0f, o[32];
     for (int c = 0; c < parts; c++) m = fmaxf(m, part[static_cast<size_t>(c) * kAttnPart]);
 #pragma unroll

@@ -24,12 +24,12 @@ template <int EPI>
 void split_gemm(SplitGemmParams& p, hipStream_t st);
 
 // Causal attention of p.len new positions of every sequence over the cache, output rows in split form.
-// kv and part: scratch of the sizes split_attention_space names, for the length of the call.
-struct SplitAttnSpace {
-    size_t kv_bytes, part_floats;
-};
-SplitAttnSpace split_attention_space(int batch, int heads, int len, int pos_base);
-void split_attention(const PrefillAttnParams& p, int batch, char* kv, float* part, hipStream_t st);
+// kv: scratch of kv_bytes, at least one (sequence, head) pair's keys and values; the pairs go in groups
+// that fit.  split_attention_kv_bytes: what is worth giving for so many filled positions.
+// part: scratch of the size split_attention_part_floats names for the call.
+size_t split_attention_kv_bytes(int batch, int heads, int positions);
+size_t split_attention_part_floats(int batch, int heads, int len, int pos_base, size_t kv_bytes);
+void split_attention(const PrefillAttnParams& p, int batch, char* kv, size_t kv_bytes, float* part, hipStream_t st);
 
 // Widest run of partial results per row that split_gemm<EPI_STORE> leaves.
 inline int split_nll_stride(int N) { return (N + kSplitPad - 1) / kSplitPad * 4; }

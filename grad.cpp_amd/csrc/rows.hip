@@ -4,6 +4,7 @@
 
 #include "kernels_split_attn.h"
 
+#include <algorithm>
 #include <stdexcept>
 #include <string>
 
@@ -85,7 +86,7 @@ void split_gemm(SplitGemmParams& p, hipStream_t st) {
 // Key tiles per workgroup, as a shift.  Query blocks are whole workgroups (128 queries against
 // all their keys) while there are enough of them or the longest has six tiles at most (8
 // sequences of 256 tokens: 18 us, shared 18 and 8 for the merge); below 640 workgroups the keys of the
-// long blocks are shared, as coarsely as reaches 640 (12 heads of 1999 tokens: 89 us unshared, 76 in runs of
+// long blocks are shared, as coarsely as reaches 640 and so among 1300 or so at most (12 heads of 1999 tokens: 89 us unshared, 76 in runs of
 // 1024 keys, 47 of 512, 46 of 256, 48 of 128; the merge costs 1, 6, 8, 12, 18 us more).
 static int attn_chunk_shift(int pairs, int len, int pos_base) {
     const int blocks = (len + kAttnQueries - 1) / kAttnQueries;
@@ -96,7 +97,7 @@ static int attn_chunk_shift(int pairs, int len, int pos_base) {
         return static_cast<long>(n) * pairs;
     };
     if (workgroups(20) >= 640 || attn_key_tiles(blocks - 1, len, pos_base) <= 6) return 20;
-    for (shift = 5; shift > 1 && workgroups(shift) < 640; shift--) {
+    for (shift = 14; shift > 1 && workgroups(shift) < 640; shift--) {
     }
     return shift;
 }
@@ -107,43 +108,60 @@ static int attn_items(int len, int pos_base, int shift) {
     return n;
 }
 
-SplitAttnSpace split_attention_space(int batch, int heads, int len, int pos_base) {
-    const size_t pairs = static_cast<size_t>(batch) * heads;
-    const int shift = attn_chunk_shift(batch * heads, len, pos_base);
-    SplitAttnSpace need;
-    need.kv_bytes = pairs * ((pos_base + len + 63) / 64) * kAttnTile;
-    need.part_floats = shift == 20 ? 0 : pairs * attn_items(len, pos_base, shift) * kAttnPart;
+// Pairs whose keys and values are split at a time.
+static int attn_group(int pairs, int positions, size_t kv_bytes) {
+    const size_t fit = kv_bytes / (static_cast<size_t>((positions + 63) / 64) * kAttnTile);
+    return static_cast<int>(std::min<size_t>(std::max<size_t>(fit, 1), pairs));
+}
+
+// Splitting goes pair by pair anyway and a quarter of a gigabyte is thousands of workgroups' worth,
+// so more would only be more memory.
+size_t split_attention_kv_bytes(int batch, int heads, int positions) {
+    const size_t pair = static_cast<size_t>((positions + 63) / 64) * kAttnTile;
+    return std::max(pair, std::min(pair * batch * heads, size_t{256} << 20));
+}
+
+size_t split_attention_part_floats(int batch, int heads, int len, int pos_base, size_t kv_bytes) {
+    size_t need = 0;
+    const int pairs = batch * heads, group = attn_group(pairs, pos_base + len, kv_bytes);
+    for (const int n : {group, pairs % group}) {
+        const int shift = n ? attn_chunk_shift(n, len, pos_base) : 20;
+        if (shift != 20) need = std::max(need, static_cast<size_t>(n) * attn_items(len, pos_base, shift) * kAttnPart);
+    }
     return need;
 }
 
-void split_attention(const PrefillAttnParams& a, int batch, char* kv, float* part, hipStream_t st) {
+void split_attention(const PrefillAttnParams& a, int batch, char* kv, size_t kv_bytes, float* part, hipStream_t st) {
     static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_split_kernel),
                                                          hipFuncAttributeMaxDynamicSharedMemorySize, kAttnLds);
     check(raised, "hipFuncSetAttribute");
-    const int heads = a.kv.heads, pairs = batch * heads;
-    const SplitKvParams k{a.kv, a.layer, a.pos_base + a.len, kv};
+    const int heads = a.kv.heads, pairs = batch * heads, positions = a.pos_base + a.len;
+    const int group = attn_group(pairs, positions, kv_bytes);
+    const int blocks = (a.len + kAttnQueries - 1) / kAttnQueries;
     SplitAttnParams p{};
     p.q = a.q;
     p.kv = kv;
-    p.tiles = (k.positions + 63) / 64;
+    p.tiles = (positions + 63) / 64;
     p.out = a.out_split;
     p.part = part;
     p.d_model = a.d_model;
     p.heads = heads;
     p.len = a.len;
     p.pos_base = a.pos_base;
-    p.chunk_shift = attn_chunk_shift(pairs, a.len, a.pos_base);
-    p.items = attn_items(a.len, a.pos_base, p.chunk_shift);
-    p.batch = batch;
     p.scale = a.scale;
-    hipLaunchKernelGGL(split_kv_kernel, dim3(p.tiles, heads, batch), dim3(256), 0, st, k);
-    check(hipGetLastError(), "split_kv");
-    hipLaunchKernelGGL(attn_split_kernel, dim3((pairs + 7) / 8 * 8 * p.items), dim3(256), kAttnLds, st, p);
-    check(hipGetLastError(), "attn_split");
-    const int blocks = (a.len + kAttnQueries - 1) / kAttnQueries;
-    if (p.items > blocks) {
-        hipLaunchKernelGGL(attn_split_merge_kernel, dim3(blocks, heads, batch), dim3(256), 0, st, p);
-        check(hipGetLastError(), "attn_split_merge");
+    for (p.first = 0; p.first < pairs; p.first += group) {
+        p.pairs = std::min(group, pairs - p.first);
+        p.chunk_shift = attn_chunk_shift(p.pairs, a.len, a.pos_base);
+        p.items = attn_items(a.len, a.pos_base, p.chunk_shift);
+        const SplitKvParams k{a.kv, a.layer, p.first, positions, kv};
+        hipLaunchKernelGGL(split_kv_kernel, dim3(p.tiles, p.pairs), dim3(256), 0, st, k);
+        check(hipGetLastError(), "split_kv");
+        hipLaunchKernelGGL(attn_split_kernel, dim3((p.pairs + 7) / 8 * 8 * p.items), dim3(256), kAttnLds, st, p);
+        check(hipGetLastError(), "attn_split");
+        if (p.items > blocks) {
+            hipLaunchKernelGGL(attn_split_merge_kernel, dim3(blocks, p.pairs), dim3(256), 0, st, p);
+            check(hipGetLastError(), "attn_split_merge");
+        }
     }
 }
 

@@ -157,3 +157,22 @@ def test_passes_that_find_little_memory_left(spare, monkeypatch):
     assert np.abs(nll[7] - want).max() <= 2e-5 * max(1.0, np.abs(want).max())
     monkeypatch.delenv("GRADHIP_TEST_SPARE_BYTES")
     assert np.abs(G.Session(gm, batch=8).score(tokens[:, :-1], tokens[:, 1:]) - nll).max() <= 2e-5 * np.abs(want).max()
+
+
+def test_attention_scratch_stays_bounded():
+    """64 sequences of 4500 tokens, whose split keys and values would be 670 MB: they go in groups of
+    (sequence, head) pairs, some of which begin in the middle of a sequence's heads.  MiB: 231 of
+    activations (a slice of 32768 rows x 7296 bytes and 512 rows of the fp32 tiles' buffers), 256 of
+    keys and values, at most 1300 partial results (43, in steps of 8)."""
+    cfg = synth.Config(synth.ARCH_GPT2, 130, 192, 1, 3, 4500)
+    W = synth.make_weights(cfg, 91, std=lively_std(cfg), norm_noise=0.1)
+    tokens = synth.uniform_tokens(64 * 4500, cfg.vocab, 92).reshape(64, 4500)
+    gm = G.Model.from_tensors(cfg, W)
+    G.Session(gm, batch=1).prefill(tokens[:1, :600])  # the weights' split form
+    s = G.Session(gm, batch=64)
+    before = _free_bytes()
+    last = s.prefill(tokens)
+    assert before - _free_bytes() <= (231 + 256 + 48) << 20
+    for b in (0, 25, 63):
+        ref = ref_forward.forward(cfg, W, tokens[b])
+        assert np.abs(last[b] - ref[-1]).max() <= 1e-5 * np.abs(ref[-1]).max(), b
