@@ -194,6 +194,45 @@ static __global__ __launch_bounds__(1024) void norm_split_kernel(const float* __
     }
 }
 
+// The same for rows that do not fit the registers: one pass over the row per sum and one to write,
+// the later ones from the L2.
+template <bool RMS>
+static __global__ __launch_bounds__(1024) void norm_split_long_kernel(const float* __restrict__ x,
+                                                                      const float* __restrict__ gamma,
+                                                                      const float* __restrict__ beta, char* out, int M,
+                                                                      int d) {
+    const int lane = threadIdx.x & 63;
+    const int m = blockIdx.x * 16 + (threadIdx.x >> 6);
+    if (m >= M) return;
+    const float* xr = x + static_cast<size_t>(m) * d;
+    float s = 0.0f;
+    for (int k = lane * 4; k < d; k += 256) {
+        const float4 a = *reinterpret_cast<const float4*>(xr + k);
+        s += RMS ? dot4(a, a) : (a.x + a.y) + (a.z + a.w);
+    }
+    s = wave_sum(s) / static_cast<float>(d);
+    const float mean = RMS ? 0.0f : s;
+    if (!RMS) {
+        s = 0.0f;
+        for (int k = lane * 4; k < d; k += 256) {
+            float4 a = *reinterpret_cast<const float4*>(xr + k);
+            a = make_float4(a.x - mean, a.y - mean, a.z - mean, a.w - mean);
+            s += dot4(a, a);
+        }
+        s = wave_sum(s) / static_cast<float>(d);
+    }
+    const float scale = 1.0f / sqrtf(s + kNormEps);
+    for (int k = lane * 8; k < d; k += 512) {
+        float o[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            o[e] = gamma[k + e] * (xr[k + e] - mean) * scale;
+            if (!RMS) o[e] += beta[k + e];
+        }
+        store_split8(out, m, k, d / kSplitCols, o);
+    }
+}
+
 struct SplitGemmParams {
     const char* A;  // split activations, M rows (storage for whole tiles)
     const char* W;  // split weights (storage for whole tiles, outputs in split_output_of_row order)

@@ -26,7 +26,8 @@ template <bool RMS>
 static void norm_split_as(const float* x, const float* gamma, const float* beta, char* out, int M, int d, hipStream_t st) {
     const dim3 grid((M + 15) / 16), block(1024);
     if (d <= 1024) hipLaunchKernelGGL((norm_split_kernel<RMS, 2>), grid, block, 0, st, x, gamma, beta, out, M, d);
-    else hipLaunchKernelGGL((norm_split_kernel<RMS, 8>), grid, block, 0, st, x, gamma, beta, out, M, d);
+    else if (d <= 4096) hipLaunchKernelGGL((norm_split_kernel<RMS, 8>), grid, block, 0, st, x, gamma, beta, out, M, d);
+    else hipLaunchKernelGGL((norm_split_long_kernel<RMS>), grid, block, 0, st, x, gamma, beta, out, M, d);
     check(hipGetLastError(), "norm_split");
 }
 

@@ -2,6 +2,7 @@
 can take, at row counts that leave ragged tiles, against the float64 forward.  The bound is
 what fp32 sums give, an order below the engine's common 1e-4."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -176,3 +177,32 @@ def test_attention_scratch_stays_bounded():
     for b in (0, 25, 63):
         ref = ref_forward.forward(cfg, W, tokens[b])
         assert np.abs(last[b] - ref[-1]).max() <= 1e-5 * np.abs(ref[-1]).max(), b
+
+
+@pytest.mark.parametrize("arch", [synth.ARCH_GPT2, synth.ARCH_MODERN])
+@pytest.mark.parametrize("d", [1088, 4160])
+def test_wide_models_take_the_pass_too(arch, d):
+    """Rows of more than 1024 columns, and of more than the 4096 that a wavefront's registers hold."""
+    cfg = synth.Config(arch, 67, d, 1, d // 64, 180)
+    rng = np.random.default_rng(93)
+    W = [rng.standard_normal((r, c), dtype=np.float32) * np.float32(lively_std(cfg) if what in ("matrix", "bias") else 0.1)
+         + np.float32(what == "gamma") for _, r, c, what in synth.tensor_specs(cfg)]
+    tokens = synth.uniform_tokens(3 * 172, cfg.vocab, 94).reshape(3, 172)
+    gm = G.Model.from_tensors(cfg, W)
+    nll = G.Session(gm, batch=3).score(tokens[:, :-1], tokens[:, 1:])
+    s, stepwise = G.Session(gm, batch=3), G.Session(gm, batch=3, flags=G.FLAG_STEPWISE_PROMPT)
+    last = s.prefill(tokens[:, :-1])
+    ref = ref_forward.forward(cfg, W, tokens[2, :-1])
+    want = _loss(ref, tokens[2, 1:])
+    assert np.abs(nll[2] - want).max() <= 2e-5 * max(1.0, np.abs(want).max())
+    assert np.abs(last[2] - ref[-1]).max() <= 1e-5 * np.abs(ref[-1]).max()
+
+    def seconds(session):
+        session.reset()
+        begin = time.perf_counter()
+        session.prefill(tokens[:, :-1])
+        return time.perf_counter() - begin
+
+    stepwise.prefill(tokens[:, :-1])
+    # 171 steps read every weight 171 times; the pass measured 84 to 105 times as fast
+    assert min(seconds(s) for _ in range(3)) < 0.25 * min(seconds(stepwise) for _ in range(3))
