@@ -636,7 +636,7 @@ static void launch_gemv(const GemvParams& p, int batch, hipStream_t st) {
     auto go = [&](auto kernel, int rows_per_wave) {
         const int waves = (p.N + rows_per_wave - 1) / rows_per_wave;
         const dim3 grid((waves + 3) / 4, batch);
-        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, p);
+        enqueue(kernel, grid, dim3(256), 0, st, p);
     };
     switch (kv) {
         case 1: go(gemv_kernel<1, 2, PRO, EPI>, 4); break;
@@ -655,20 +655,20 @@ static void launch_attn(const AttnParams& p, int batch, hipStream_t st) {
     const dim3 grid(p.max_chunks, p.kv.heads, batch);
     if (hs == 64) {
         if (p.kv.page_shift >= 5 && p.chunk % 128 == 0)
-            hipLaunchKernelGGL(attn_decode64_kernel<true>, grid, dim3(256), 0, st, p);
+            enqueue(attn_decode64_kernel<true>, grid, dim3(256), 0, st, p);
         else
-            hipLaunchKernelGGL(attn_decode64_kernel<false>, grid, dim3(256), 0, st, p);
+            enqueue(attn_decode64_kernel<false>, grid, dim3(256), 0, st, p);
         HIP_CHECK(hipGetLastError());
         return;
     }
     const size_t lds = (static_cast<size_t>(p.chunk) + 4 * hs + 8) * sizeof(float);
     switch (hs) {
-        case 8: hipLaunchKernelGGL(attn_decode_kernel<8>, grid, dim3(256), lds, st, p); break;
-        case 16: hipLaunchKernelGGL(attn_decode_kernel<16>, grid, dim3(256), lds, st, p); break;
-        case 32: hipLaunchKernelGGL(attn_decode_kernel<32>, grid, dim3(256), lds, st, p); break;
-        case 64: hipLaunchKernelGGL(attn_decode_kernel<64>, grid, dim3(256), lds, st, p); break;
-        case 128: hipLaunchKernelGGL(attn_decode_kernel<128>, grid, dim3(256), lds, st, p); break;
-        default: hipLaunchKernelGGL(attn_decode_kernel<0>, grid, dim3(256), lds, st, p); break;
+        case 8: enqueue(attn_decode_kernel<8>, grid, dim3(256), lds, st, p); break;
+        case 16: enqueue(attn_decode_kernel<16>, grid, dim3(256), lds, st, p); break;
+        case 32: enqueue(attn_decode_kernel<32>, grid, dim3(256), lds, st, p); break;
+        case 64: enqueue(attn_decode_kernel<64>, grid, dim3(256), lds, st, p); break;
+        case 128: enqueue(attn_decode_kernel<128>, grid, dim3(256), lds, st, p); break;
+        default: enqueue(attn_decode_kernel<0>, grid, dim3(256), lds, st, p); break;
     }
     HIP_CHECK(hipGetLastError());
 }
@@ -689,8 +689,8 @@ static int project(Session& s, GemvParams g, hipStream_t st) {
         }
         int launches = 1;
         if (PRO != PRO_PLAIN) {
-            hipLaunchKernelGGL(norm_rows_kernel, dim3((B + 3) / 4), dim3(256), 0, st, g.in, g.gamma,
-                               g.beta, s.h, B, g.K, static_cast<int>(PRO));
+            enqueue(norm_rows_kernel, dim3((B + 3) / 4), dim3(256), 0, st, g.in, g.gamma, g.beta, s.h, B, g.K,
+                    static_cast<int>(PRO));
             HIP_CHECK(hipGetLastError());
             g.in = s.h;
             g.in_stride = g.K;
@@ -847,11 +847,10 @@ static int enqueue_step(Session& s, StepForm form) {
 
     if (form == STEP_ARGMAX) {
         // text_gen.cpp:52-60
-        hipLaunchKernelGGL(argmax_embed_kernel, dim3(B), dim3(kArgmaxThreads), 0, st, s.best, s.best_stride, s.st,
-                           s.hist, s.hist_stride, s.tok, m.E, m.P, s.x, d);
+        enqueue(argmax_embed_kernel, dim3(B), dim3(kArgmaxThreads), 0, st, s.best, s.best_stride, s.st, s.hist,
+                s.hist_stride, s.tok, m.E, m.P, s.x, d);
     } else if (form == STEP_EMBED) {
-        hipLaunchKernelGGL(embed_kernel, dim3((d + 255) / 256, B), dim3(256), 0, st, m.E, m.P, s.tok,
-                           s.st, s.x, d);
+        enqueue(embed_kernel, dim3((d + 255) / 256, B), dim3(256), 0, st, m.E, m.P, s.tok, s.st, s.x, d);
     }
     HIP_CHECK(hipGetLastError());
     launches += form != STEP_ROWS;
@@ -1163,26 +1162,30 @@ static void check_persist_abort(Session& s) {
     }
 }
 
-// Records the launches of a step; returns their number.
-static int capture_step(Session& s, StepForm form, hipGraph_t* graph) {
-    int launches = 0;
-    HIP_CHECK(hipStreamBeginCapture(s.stream, hipStreamCaptureModeThreadLocal));
-    try {
-        launches = enqueue_step(s, form);
-    } catch (...) {
-        hipGraph_t g = nullptr;
-        (void)hipStreamEndCapture(s.stream, &g);
-        if (g) (void)hipGraphDestroy(g);
-        throw;
-    }
-    HIP_CHECK(hipStreamEndCapture(s.stream, graph));
+// Makes the graph of a step's launches; returns their number.
+static int record_step(Session& s, StepForm form, hipGraph_t* graph) {
+    struct Scope {  // launches go to their streams again, and an unfinished graph goes, on every path out
+        StepRecording recording;
+        Scope() {
+            HIP_CHECK(hipGraphCreate(&recording.graph, 0));
+            t_recording = &recording;
+        }
+        ~Scope() {
+            t_recording = nullptr;
+            if (recording.graph) (void)hipGraphDestroy(recording.graph);
+        }
+    } scope;
+    const int launches = enqueue_step(s, form);
+    HIP_CHECK(scope.recording.error);
+    *graph = scope.recording.graph;
+    scope.recording.graph = nullptr;
     return launches;
 }
 
 static void run_step(Session& s, StepForm form = STEP_EMBED) {
     if (s.engine == GH_ENGINE_GRAPH) {
         if (!s.exec[form]) {  // (a form's graph is made when it is first wanted)
-            if (!s.graph[form]) capture_step(s, form, &s.graph[form]);
+            if (!s.graph[form]) record_step(s, form, &s.graph[form]);
             HIP_CHECK(hipGraphInstantiate(&s.exec[form], s.graph[form], nullptr, nullptr, 0));
         }
         HIP_CHECK(hipGraphLaunch(s.exec[form], s.stream));
@@ -1495,7 +1498,7 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
         // nothing to record: one launch runs any number of steps
     } else {
         // Counts the launches of a step without running one.
-        s.launches_per_step = capture_step(s, STEP_EMBED, &s.graph[STEP_EMBED]);
+        s.launches_per_step = record_step(s, STEP_EMBED, &s.graph[STEP_EMBED]);
     }
     return sp;
 }

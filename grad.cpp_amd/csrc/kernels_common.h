@@ -5,8 +5,46 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <tuple>
 
 namespace gh {
+
+// A step on its way into a graph: launches become kernel nodes, each behind the one before.
+// Built node by node and not captured from a stream: while a stream is being captured, the
+// runtime refuses another thread's plain copy ("operation would make the legacy stream depend on a
+// capturing blocking stream", also with a non-blocking stream in thread-local mode) and the
+// capture fails with it, and a form is recorded inside the call that first wants it.
+struct StepRecording {
+    hipGraph_t graph = nullptr;
+    hipGraphNode_t last = nullptr;
+    hipError_t error = hipSuccess;  // of the first node that failed
+};
+inline thread_local StepRecording* t_recording = nullptr;  // this thread's, null: launches go to their stream
+
+// Every launch that a step consists of.
+template <class... P, class... A>
+inline void enqueue(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t st, const A&... args) {
+    if (!t_recording) {
+        hipLaunchKernelGGL(kernel, grid, block, lds, st, args...);
+        return;
+    }
+    std::tuple<P...> held(args...);  // the node takes copies
+    std::apply(
+        [&](auto&... arg) {
+            void* at[] = {const_cast<void*>(static_cast<const void*>(&arg))...};
+            hipKernelNodeParams node{};
+            node.func = reinterpret_cast<void*>(kernel);
+            node.gridDim = grid;
+            node.blockDim = block;
+            node.sharedMemBytes = static_cast<unsigned>(lds);
+            node.kernelParams = at;
+            StepRecording& r = *t_recording;
+            const hipGraphNode_t before = r.last;
+            const hipError_t e = hipGraphAddKernelNode(&r.last, r.graph, before ? &before : nullptr, before ? 1 : 0, &node);
+            if (r.error == hipSuccess) r.error = e;
+        },
+        held);
+}
 
 constexpr int kWave = 64;
 constexpr float kNormEps = 1e-5f;  // include/grad/transformer/layer_norm.h:18

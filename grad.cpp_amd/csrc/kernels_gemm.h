@@ -310,8 +310,8 @@ inline void launch_gemm16_as(const GemvParams& p, int M, hipStream_t st) {
     const int m_groups = (M + 16 * MT - 1) / (16 * MT);
     const int n_groups = (p.N + 16 * NT - 1) / (16 * NT);
     const int n_groups8 = (n_groups + 7) / 8 * 8;  // whole rounds of the 8 XCDs
-    hipLaunchKernelGGL((gemm16_kernel<EPI, RMS, MT, NT, KW>), dim3(n_groups8 * m_groups + p.next.blocks),
-                       dim3(64 * KW), 0, st, p, M, m_groups);
+    enqueue(gemm16_kernel<EPI, RMS, MT, NT, KW>, dim3(n_groups8 * m_groups + p.next.blocks),
+            dim3(64 * KW), 0, st, p, M, m_groups);
 }
 
 // Weight tiles per workgroup of the wide kernel: 16000 rows = 250 workgroups.
@@ -506,8 +506,7 @@ inline bool gemm_wide_ok(const GemvParams& p, int M) {
 template <bool RMS, int MT, int KS>
 inline void launch_gemm_wide_as(const GemvParams& p, int M, hipStream_t st) {
     const int n_tiles = (p.N + 15) / 16;
-    hipLaunchKernelGGL((gemm_wide_kernel<RMS, MT, KS>), dim3((n_tiles + kWideTiles - 1) / kWideTiles), dim3(512),
-                       0, st, p, M);
+    enqueue(gemm_wide_kernel<RMS, MT, KS>, dim3((n_tiles + kWideTiles - 1) / kWideTiles), dim3(512), 0, st, p, M);
 }
 
 template <bool RMS, int MT>

@@ -71,6 +71,63 @@ def test_two_host_threads_each_decode_on_a_persistent_session(llama768):
         check_greedy_stream(got[i][0], refs[i][0], refs[i][1], 9, f"thread {i}")
 
 
+def test_steps_are_recorded_while_another_thread_uses_the_null_stream(llama768):
+    """One thread opens batched sessions, whose step graphs are recorded when the session is made and
+    inside its first calls; the other loads models and scores and prompts on fresh sessions, which
+    clear, copy and launch on the null stream.  Neither may disturb the other."""
+    import threading
+    cfg, W, om, gm = llama768
+    small = synth.Config(synth.ARCH_MODERN, 301, 128, 2, 2, 640)
+    W2 = synth.make_weights(small, 32, std=lively_std(small), norm_noise=0.1)
+    toks = synth.uniform_tokens(601, small.vocab, 33)
+    prompts = np.stack([synth.uniform_tokens(9, cfg.vocab, 70 + i) for i in range(3)])
+    greedy, drawn = G.sampling(greedy=True, repetition_penalty=1.0), G.sampling(0.8, 40, 0.9, 1.1)
+    other = threading.Event()
+
+    def decode():
+        s = G.Session(gm, batch=3)
+        out = [s.generate(prompts, 6, greedy), s.generate(prompts, 6, drawn, seed=5)]
+        s.reset()
+        out.append(s.step(prompts[:, 0]))
+        s.close()
+        return out
+
+    def load_and_score():
+        m = G.Model.from_tensors(small, W2)
+        a = G.Session(m).score(toks[:-1], toks[1:])
+        b = G.Session(m).prefill(toks[:-1])
+        m.close()
+        return [a, b]
+
+    want = [decode(), load_and_score()]
+    got, errs = [[], []], []
+
+    def work(i, once):
+        try:
+            while len(got[i]) < 12 or not other.is_set():
+                got[i].append(once())
+                if len(got[i]) == 12 and i == 1:
+                    other.set()
+                    break
+                if len(got[i]) > 2000:
+                    break
+        except Exception as e:  # noqa: BLE001
+            errs.append((i, repr(e)))
+            other.set()
+
+    threads = [threading.Thread(target=work, args=a) for a in ((0, decode), (1, load_and_score))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errs, errs
+    for i in range(2):
+        assert len(got[i]) >= 12
+        for once in got[i]:
+            for x, y in zip(once, want[i]):
+                assert np.array_equal(x, y), i
+
+
 @pytest.mark.parametrize("batch", [7, 19, 33, 130])
 def test_batches_that_do_not_fill_a_tile(batch):
     cfg = synth.Config(synth.ARCH_MODERN, 301, 128, 2, 2, 24)
