@@ -629,6 +629,10 @@ __device__ inline float block_ordered_total(Get get, int n, float* parts, int nt
 
 // First i in [0, n) whose running sum x(0) + ... + x(i) reaches thr, n when none
 // does.  slot: one int of LDS.
+// A thread walks its run element by element from the sum in front of it; the sum in front of the
+// next run adds the run's total at once and can round higher.  Where thr lies between the two, no
+// element of the walk reaches it and the next run starts beyond it: it is the last element of the
+// run that adds anything.
 template <class Get>
 __device__ inline int block_first_reach(Get get, int n, float thr, float* parts, int* slot,
                                         int nt = blockDim.x) {
@@ -649,24 +653,27 @@ __device__ inline int block_first_reach(Get get, int n, float thr, float* parts,
         const float pj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(part), j));
         before += (j < lane) ? pj : 0.0f;
     }
-    const float wtotal = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(before + part), 63));
+    const float upto = before + part;
+    const float wtotal = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(upto), 63));
     __syncthreads();
     if (lane == 0) parts[wave] = wtotal;
     if (tid == 0) *slot = n;
     __syncthreads();
     float base = 0.0f;
     for (int w = 0; w < wave; w++) base += parts[w];
+    const float next = base + upto;  // (what the next thread computes: the same additions)
     base += before;
     if (base < thr) {
         float cumulative = base;
+        int last = n, at = n;
         run_pass(get, lo, hi, [&](int i, float x) {
             cumulative += x;
-            if (cumulative >= thr) {
-                atomicMin(slot, i);
-                return false;
-            }
-            return true;
+            if (x > 0.0f) last = i;
+            if (cumulative >= thr) at = i;
+            return at == n;
         });
+        if (at == n && next >= thr) at = last;
+        if (at < n) atomicMin(slot, at);
     }
     __syncthreads();
     const int at = *slot;
@@ -946,7 +953,7 @@ __device__ __forceinline__ int sample_row(float* val, int V, float scale, float 
     const int run = ((V + NT - 1) / NT) | 1;
     const int lo = min(V, tid * run), n = min(V, lo + run) - lo;
     float y[ROUNDS + 1];
-    const auto in_order = [&](float (&parts)[2]) {  // sum of the run; running sum of the wavefront's runs and its total
+    const auto in_order = [&](float (&parts)[3]) {  // running sum of the wavefront's runs in front of this one, its sum, both
         float part = 0.0f;
 #pragma unroll
         for (int i = 0; i < ROUNDS + 1; i++) part += y[i];
@@ -954,13 +961,14 @@ __device__ __forceinline__ int sample_row(float* val, int V, float scale, float 
         if (lane == 63) red[wave] = incl;
         parts[0] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(incl), 0x138 /* wave_shr:1 */, 0xF, 0xF, true));
         parts[1] = part;
+        parts[2] = incl;
         __syncthreads();
     };
 #pragma unroll
     for (int i = 0; i < ROUNDS + 1; i++) y[i] = val[min(lo + i, V - 1)];
 #pragma unroll
     for (int i = 0; i < ROUNDS + 1; i++) y[i] = i < n && y[i] >= cutoff ? y[i] : 0.0f;
-    float parts[2];
+    float parts[3];
     in_order(parts);
     if (renorm) {
         // renormalise by the index-order total of what is left (text_gen.cpp:178-192)
@@ -976,15 +984,22 @@ __device__ __forceinline__ int sample_row(float* val, int V, float scale, float 
     // the first element whose running sum reaches u, in index order (text_gen.cpp:202-208)
     float cumulative = 0.0f;
     for (int w = 0; w < wave; w++) cumulative += red[w];
+    const float next = cumulative + parts[2];  // the sum in front of the next run
     cumulative += parts[0];
     // a run whose end stays short of u by far more than the roundings of its at most 33
     // additions cannot reach it on the way
     if (cumulative < u && cumulative + parts[1] >= u * 0.9999f) {
+        // (between the end of the walk and the next run's start: block_first_reach.  The walk's own
+        // end is found where the last element that adds anything is.)
+        float end = cumulative;
+#pragma unroll
+        for (int i = 0; i < ROUNDS + 1; i++) end += y[i];
+        const float reach = next >= u ? fminf(u, end) : u;
         int at = V;
 #pragma unroll
         for (int i = 0; i < ROUNDS + 1; i++) {
             cumulative += y[i];
-            if (at == V && i < n && cumulative >= u) at = lo + i;
+            if (at == V && i < n && cumulative >= reach) at = lo + i;
         }
         if (at < V) atomicMin(&ishare[0], at);
     }
