@@ -2536,8 +2536,8 @@ gh_status gh_session_score(gh_session* sess, const int32_t* ids, const int32_t* 
                     HIP_CHECK(hipGetLastError());
                     run_step(s);
                 }
-                hipLaunchKernelGGL(nll_rows_kernel, dim3(s.B), dim3(256), 0, s.stream, s.logits, V, 0, 1, t, len,
-                                   sink.targets, sink.nll);
+                hipLaunchKernelGGL(nll_rows_kernel, dim3(s.B), dim3(256), 0, s.stream, s.logits, V, t, len, sink.targets,
+                                   sink.nll);
                 HIP_CHECK(hipGetLastError());
             }
             if (s.engine != GH_ENGINE_PERSISTENT) s.n_hist += len;

@@ -251,10 +251,9 @@ struct SplitGemmParams {
     int rows_per_seq, pos_base;
     // EPI_STORE: logits that are scored, not stored.  Every 64 outputs of a row leave
     // (largest, sum of exp(v - largest)), and the target's logit is kept.
-    // Row m is row nll_row0 + m of the pass, whose row seq * rows_per_seq + t is position
-    // nll_t0 + t of sequence seq.
+    // Row m = seq * rows_per_seq + t is position nll_t0 + t of sequence seq.
     const int* targets;  // [batch][nll_len]
-    int nll_row0, nll_t0, nll_len;
+    int nll_t0, nll_len;
     float2* nll_part;  // [M][nll_stride]
     int nll_stride;    // n_tiles * WN
     float* nll_target;  // [M]
@@ -464,7 +463,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
             float mx = -INFINITY;
             int target = -1;
             if (m < p.M) {
-                const int g = p.nll_row0 + m, seq = g / p.rows_per_seq, t = g - seq * p.rows_per_seq;
+                const int seq = m / p.rows_per_seq, t = m - seq * p.rows_per_seq;
                 target = p.targets[static_cast<size_t>(seq) * p.nll_len + p.nll_t0 + t];
             }
 #pragma unroll
@@ -568,11 +567,10 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
 
 // nll of a scored row from what the logits launch left of it: log of the sum of all
 // exponentials, less the target's logit (Variable::cross_entropy, variable.cpp:589-592).  One
-// wavefront per row; row m of the launch is row row0 + m of a prompt pass whose row
-// seq * slice_len + t holds position t0 + t of sequence seq.
+// wavefront per row; row seq * slice_len + t holds position t0 + t of sequence seq.
 static __global__ __launch_bounds__(256) void nll_parts_kernel(const float2* __restrict__ part, int stride,
-                                                               const float* __restrict__ target, int M, int row0,
-                                                               int slice_len, int t0, int len, float* nll) {
+                                                               const float* __restrict__ target, int M, int slice_len,
+                                                               int t0, int len, float* nll) {
     const int lane = threadIdx.x & 63, m = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (m >= M) return;
     const float2* row = part + static_cast<size_t>(m) * stride;
@@ -586,7 +584,7 @@ static __global__ __launch_bounds__(256) void nll_parts_kernel(const float2* __r
     }
     sum = wave_sum(sum);
     if (lane == 0) {
-        const int g = row0 + m, seq = g / slice_len, t = g - seq * slice_len;
+        const int seq = m / slice_len, t = m - seq * slice_len;
         nll[static_cast<size_t>(seq) * len + t0 + t] = (logf(sum) + mx) - target[m];
     }
 }

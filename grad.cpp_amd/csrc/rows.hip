@@ -77,7 +77,7 @@ static void launch(SplitGemmParams& p, hipStream_t st) {
 template <int EPI>
 void split_gemm(SplitGemmParams& p, hipStream_t st) {
     switch (pick_tiling(p.M, p.N)) {
-        case TILE_32_K4: launch<EPI, 1, 1, 1, 1, 4, 3, 4>(p, st); break;
+        case TILE_32_K4: launch<EPI, 1, 1, 1, 1, 4, 3, 2>(p, st); break;
         case TILE_64_K4: launch<EPI, 1, 1, 2, 2, 4, 3, 1>(p, st); break;
         case TILE_64: launch<EPI, 1, 1, 2, 2, 1, 3, 4>(p, st); break;
         case TILE_128: launch<EPI, 2, 2, 2, 2, 1, 3, 2>(p, st); break;
@@ -168,7 +168,7 @@ void split_attention(const PrefillAttnParams& a, int batch, char* kv, size_t kv_
 
 void nll_parts(const SplitGemmParams& p, float* nll, hipStream_t st) {
     hipLaunchKernelGGL(nll_parts_kernel, dim3((p.M + 3) / 4), dim3(256), 0, st, p.nll_part, p.nll_stride, p.nll_target,
-                       p.M, p.nll_row0, p.rows_per_seq, p.nll_t0, p.nll_len, nll);
+                       p.M, p.rows_per_seq, p.nll_t0, p.nll_len, nll);
     check(hipGetLastError(), "nll_parts");
 }
 
