@@ -1566,6 +1566,7 @@ static bool prompt_pass_ok(const Session& s, int len) {
 // of 16000 tokens falls within an fp32 rounding of the next token's boundary about once in a
 // hundred picks, so the order of a prompt's sums shows in the reply, and under 512 rows the
 // prompt is the small part of the request (397 tokens and 64 sampled ones: 1.4 of 12.5 ms).
+// What that keeps is the replies, not precision: the split sums are the closer ones to float64.
 constexpr int kSplitMinRows = 512, kSplitMinScoreRows = 160;
 
 // How a pass over len tokens of every sequence runs: in slices of `slice` tokens (0: token by
@@ -1656,6 +1657,15 @@ static PrefillAttnParams prompt_attn_params(const Session& s, int layer, int n, 
 // Up to this many new tokens per sequence the fp32 kernel does a split pass's attention as
 // well: splitting a context's keys and values costs as much as so few queries read of them
 // (64 sequences of 128 tokens 48 us against 56, 13 of 77 10 against 18; 8 of 256 36 against 27).
+// The line was drawn at position 0, where splitting weighs most: behind a cache both forms read
+// what is cached, and what the split one saves grows with it.  Per layer of 12 heads, fp32 less
+// split (us), 129 to 384 tokens of 1 to 32 sequences: -9..19 at position 0, 2..43 behind 256
+// tokens, 50..147 behind 1024, 177..342 behind 3000.  Below the line 1 to 8 sequences would gain too
+// behind a long cache (39..60 behind 1024, 160..216 behind 3000); 32 sequences would lose (5..66,
+// 10..133).
+// Precision, split form (2^x of scores in units of ln 2) against the fp32 one (expf), 130 to 511
+// tokens at width 256, error of the losses over their size against float64: 6.7e-8..7.1e-8
+// against 7.3e-8..7.9e-8 without rotation, 2.3e-7..6.5e-7 against 2.3e-7..6.6e-7 with.
 constexpr int kSplitAttnMin = 128;
 
 static void launch_prompt_attn(const Session& s, const PrefillAttnParams& a) {

@@ -162,7 +162,9 @@ gh_status gh_session_logits(gh_session* s, const float** logits);
  * equivalent to `len` step() calls (text_gen.cpp:44-46) whose logits are
  * dropped except the last.  Prompts of 8 tokens and more go through each layer
  * in one pass (matrix-core projections over all tokens, causal attention over
- * the cache they fill).  last_logits_host may be NULL. */
+ * the cache they fill).  A model's first pass of 512 rows (tokens of all sequences; 160 where they
+ * are scored) leaves it a second copy of its matrices, 1.5 times the size of the first, for as long
+ * as it lives; without memory for it such passes are slower.  last_logits_host may be NULL. */
 gh_status gh_session_prefill(gh_session* s, const int32_t* ids, int32_t len,
                              float* last_logits_host);
 

@@ -16,8 +16,8 @@ CASES = {
     "tiny-gpt2-stepwise": (synth.Config(synth.ARCH_GPT2, 97, 64, 2, 4, 40), 2, 24),     # head size 16: token by token
     "hs64-modern": (synth.Config(synth.ARCH_MODERN, 301, 128, 2, 2, 64), 3, 40),         # one pass, small tiles
     "hs64-gpt2": (synth.Config(synth.ARCH_GPT2, 301, 128, 2, 2, 64), 3, 40),
-    "big-tiles": (synth.Config(synth.ARCH_MODERN, 1000, 256, 2, 4, 192), 4, 160),        # 640 rows: 128 x 128 tiles
-    "blocks-of-rows": (synth.Config(synth.ARCH_MODERN, 70001, 128, 1, 2, 96), 12, 90),   # logits in several blocks
+    "big-tiles": (synth.Config(synth.ARCH_MODERN, 1000, 256, 2, 4, 192), 4, 160),        # 640 rows: split products
+    "blocks-of-rows": (synth.Config(synth.ARCH_MODERN, 70001, 128, 1, 2, 96), 12, 90),   # 1080 rows, 70 k logits a row
     "persistent-short": (synth.Config(synth.ARCH_GPT2, 500, 512, 1, 8, 32), 1, 5),       # shorter than one pass takes
     "persistent-pass": (synth.Config(synth.ARCH_GPT2, 500, 512, 1, 8, 32), 1, 20),
 }

@@ -40,6 +40,20 @@ def test_a_continued_pass_sees_the_cache_of_the_passes_before():
         assert np.abs(last[b] - ref[-1]).max() <= 1e-5 * np.abs(ref[-1]).max(), b
 
 
+@pytest.mark.parametrize("n", [127, 128, 129])
+def test_either_attention_behind_a_cache(n):
+    """Up to 128 new tokens take the fp32 attention, more the split one: both sides behind 333."""
+    cfg = synth.Config(synth.ARCH_GPT2, 130, 128, 2, 2, 500)
+    W = synth.make_weights(cfg, 75, std=lively_std(cfg), norm_noise=0.1)
+    tokens = synth.uniform_tokens(2 * 334 + 2 * n, cfg.vocab, 76).reshape(2, 334 + n)
+    s = G.Session(G.Model.from_tensors(cfg, W), batch=2)
+    s.prefill(tokens[:, :333])
+    nll = s.score(tokens[:, 333:-1], tokens[:, 334:])
+    for b in range(2):
+        want = _loss(ref_forward.forward(cfg, W, tokens[b, :-1])[333:], tokens[b, 334:])
+        assert np.abs(nll[b] - want).max() <= 2e-5 * max(1.0, np.abs(want).max()), b
+
+
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_rows_match_the_float64_forward(name):
     cfg, B, n = CASES[name]
