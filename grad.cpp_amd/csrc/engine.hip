@@ -689,8 +689,7 @@ static int project(Session& s, GemvParams g, hipStream_t st) {
         }
         int launches = 1;
         if (PRO != PRO_PLAIN) {
-            enqueue(norm_rows_kernel, dim3((B + 3) / 4), dim3(256), 0, st, g.in, g.gamma, g.beta, s.h, B, g.K,
-                    static_cast<int>(PRO));
+            launch_layernorm_rows(g.in, g.gamma, g.beta, s.h, B, g.K, st);
             HIP_CHECK(hipGetLastError());
             g.in = s.h;
             g.in_stride = g.K;
@@ -1595,8 +1594,7 @@ static void project_rows(Session& s, GemvParams g, int M) {
         launch_gemm16<EPI, true>(g, M, st);
     } else {
         if (PRO == PRO_LAYERNORM) {
-            hipLaunchKernelGGL(norm_rows_kernel, dim3((M + 3) / 4), dim3(256), 0, st, g.in, g.gamma, g.beta,
-                               s.pp_norm, M, g.K, static_cast<int>(PRO));
+            launch_layernorm_rows(g.in, g.gamma, g.beta, s.pp_norm, M, g.K, st);
             HIP_CHECK(hipGetLastError());
             g.in = s.pp_norm;
             g.in_stride = g.K;

@@ -13,7 +13,8 @@ namespace gh {
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 // h[m] = norm(x[m]) for every row (layer_norm_row, inference.cpp:30-58).
-// One wavefront per row; kind is PRO_LAYERNORM or PRO_RMSNORM.
+// One wavefront per row; kind is PRO_LAYERNORM or PRO_RMSNORM.  Any width: three passes
+// over the row, each a chain of loads and additions.
 static __global__ __launch_bounds__(256) void norm_rows_kernel(const float* __restrict__ x,
                                                         const float* __restrict__ gamma,
                                                         const float* __restrict__ beta, float* h,
@@ -36,6 +37,54 @@ static __global__ __launch_bounds__(256) void norm_rows_kernel(const float* __re
         for (int k = lane; k < d; k += 64) var += (xr[k] - mean) * (xr[k] - mean);
         const float inv_std = 1.0f / sqrtf(wave_sum(var) / static_cast<float>(d) + kNormEps);
         for (int k = lane; k < d; k += 64) hr[k] = gamma[k] * (xr[k] - mean) * inv_std + beta[k];
+    }
+}
+
+// The LayerNorm of rows of 64 N elements with the row in registers, the same sums in the same
+// order.  The launch is one trip to memory long: row, gain and shift are requested
+// together, a wavefront is a workgroup of its own so that few rows still spread over the chip.
+// Per launch: 2 rows of 512 5.7 us -> 1.8, 100 rows of 768 9.6 -> 2.9.
+template <int N>
+static __global__ __launch_bounds__(64) void layernorm_rows_kernel(const float* __restrict__ x,
+                                                                   const float* __restrict__ gamma,
+                                                                   const float* __restrict__ beta, float* h) {
+    const int lane = threadIdx.x;
+    const size_t at = static_cast<size_t>(blockIdx.x) * (64 * N) + lane;
+    float v[N], g[N], b[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = x[at + 64 * i];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        g[i] = gamma[64 * i + lane];
+        b[i] = beta[64 * i + lane];
+    }
+    // (spelled out where norm_rows_kernel's loops leave the compiler no choice: a width it knows to be
+    // a power of two would become a factor and join the next addition, and of the first two
+    // squares it would round the other one)
+    float width = 64 * N;
+    asm volatile("" : "+v"(width));
+    float s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < N; i++) s += v[i];
+    const float mean = wave_sum(s) / width;
+    float var = 0.0f;
+#pragma unroll
+    for (int i = 0; i < N; i++) var = fmaf(v[i] - mean, v[i] - mean, var);
+    const float inv_std = 1.0f / sqrtf(wave_sum(var) / width + kNormEps);
+#pragma unroll
+    for (int i = 0; i < N; i++) h[at + 64 * i] = fmaf(inv_std, g[i] * (v[i] - mean), b[i]);
+}
+
+inline void launch_layernorm_rows(const float* x, const float* gamma, const float* beta, float* h, int M, int d,
+                                  hipStream_t st) {
+    switch (d) {
+        case 256: enqueue(layernorm_rows_kernel<4>, dim3(M), dim3(64), 0, st, x, gamma, beta, h); break;
+        case 512: enqueue(layernorm_rows_kernel<8>, dim3(M), dim3(64), 0, st, x, gamma, beta, h); break;
+        case 768: enqueue(layernorm_rows_kernel<12>, dim3(M), dim3(64), 0, st, x, gamma, beta, h); break;
+        case 1024: enqueue(layernorm_rows_kernel<16>, dim3(M), dim3(64), 0, st, x, gamma, beta, h); break;
+        default:
+            enqueue(norm_rows_kernel, dim3((M + 3) / 4), dim3(256), 0, st, x, gamma, beta, h, M, d,
+                    static_cast<int>(PRO_LAYERNORM));
     }
 }
 

@@ -1,0 +1,26 @@
+"""Passes over up to a few hundred rows (batched steps, prompts below the split products): the same
+rows give the same bits whatever the tiles, the blocks of queries and the company they are in, and
+agree with the float64 forward."""
+import numpy as np
+import pytest
+
+import gradhip as G
+import ref_forward
+from gradhip import synth
+from helpers import assert_logits_close, lively_std
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d", [256, 320, 512, 768, 1024])
+def test_layernorm_of_batched_steps(d):
+    """The widths whose rows stay in registers, and one that takes the general norm."""
+    cfg = synth.Config(synth.ARCH_GPT2, 201, d, 2, d // 64, 16)
+    W = synth.make_weights(cfg, 91, std=lively_std(cfg), norm_noise=0.3)
+    s = G.Session(G.Model.from_tensors(cfg, W), batch=3)
+    tokens = synth.uniform_tokens(15, cfg.vocab, 92).reshape(3, 5)
+    got = [s.step(tokens[:, t]) for t in range(5)]
+    for b in range(3):
+        ref = ref_forward.forward(cfg, W, tokens[b])
+        for t in range(5):
+            assert_logits_close(got[t][b], ref[t], what=f"layernorm {d} step {t}")
