@@ -8,6 +8,8 @@
 
 #include "kernels_gemv.h"
 
+#include <algorithm>
+
 namespace gh {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -572,6 +574,32 @@ inline void launch_gemm_wide(const GemvParams& p, int M, hipStream_t st) {
     else launch_gemm_wide_ks<RMS, 2>(p, M, st);
 }
 
+// More than 64 rows on eight wavefronts a workgroup: the tiles per workgroup that finish first.  All
+// of them give the same sums.  A launch costs a start and then, for every workgroup that a
+// compute unit is dealt, a time that grows more slowly than the tiles in it, since more tiles
+// share the rows they read (what is being paid for is operand traffic from the L2s and operand
+// permutes, 2 x 2 tiles having half of both per product).  Measured over 65 to 511 rows against eight
+// matrices (512 to 4096 outputs, 512 to 3072 columns): 1 x 1 tiles 1.7 us per workgroup and 768 columns,
+// two tiles 2.4, 2 x 2 4.0; the rule's pick is the fastest of them or within 15 % of it.
+// 1 x 1 for narrow matrices and 4 x 1 for the others, as it was: 100 x 4096 x 768 17.1 us -> 14.3,
+// 244 x 2304 x 768 24.4 -> 17.1, 397 x 4096 x 768 52.5 -> 35.8, 244 x 768 x 2048 12.8 -> 12.2.
+// (Both operands through an LDS ring, 32 x 32 to 64 x 64 outputs per workgroup: 35-36 us at 397 x 4096 x
+// 768, slower than this at every narrower shape.)
+template <int EPI, bool RMS>
+inline void launch_gemm16_many(const GemvParams& p, int M, hipStream_t st) {
+    const auto cost = [&](int mt, int nt, int each) {
+        const long groups = static_cast<long>((M + 16 * mt - 1) / (16 * mt)) * ((p.N + 16 * nt - 1) / (16 * nt));
+        return (groups + 255) / 256 * each;
+    };
+    const bool wide = p.N > 1024;
+    const long c11 = cost(1, 1, 17), c12 = cost(1, 2, wide ? 24 : 25), c21 = cost(2, 1, wide ? 25 : 24), c22 = cost(2, 2, 40);
+    const long least = std::min(std::min(c11, c12), std::min(c21, c22));
+    if (c22 == least) launch_gemm16_as<EPI, RMS, 2, 2, 8>(p, M, st);
+    else if (c12 == least) launch_gemm16_as<EPI, RMS, 1, 2, 8>(p, M, st);
+    else if (c21 == least) launch_gemm16_as<EPI, RMS, 2, 1, 8>(p, M, st);
+    else launch_gemm16_as<EPI, RMS, 1, 1, 8>(p, M, st);
+}
+
 // At 64 rows (0.4575 ms per step with 2 x 1 tiles on 8 wavefronts for the wide projections and
 // 2 x 2 on 4 for the logits): wide 2 x 1 on 4 wavefronts 0.4384 (2 x 2 on 8: 0.4432, 1 x 4: 0.4504,
 // 2 x 4: 0.4742, 4 x 2: 0.4990, 2 x 1 on 2: 0.5125, 4 x 1 on 4: 0.5128); narrow 1 x 1 on 8 stays
@@ -588,6 +616,7 @@ inline void launch_gemm16(const GemvParams& p, int M, hipStream_t st) {
         if (gemm_wide_ok(p, M)) return launch_gemm_wide<RMS>(p, M, st);
     }
     const bool k8 = p.K % 128 == 0;
+    if (k8 && M > 64 && p.N <= 8192) return launch_gemm16_many<EPI, RMS>(p, M, st);
     if (p.N <= 1024 || M <= 16) {
         if (k8) launch_gemm16_as<EPI, RMS, 1, 1, 8>(p, M, st);
         else launch_gemm16_as<EPI, RMS, 1, 1, 4>(p, M, st);
@@ -600,8 +629,7 @@ inline void launch_gemm16(const GemvParams& p, int M, hipStream_t st) {
         if (k8 && M <= 32) launch_gemm16_as<EPI, RMS, 2, 1, 8>(p, M, st);
         else launch_gemm16_as<EPI, RMS, 2, 1, 4>(p, M, st);
     } else {
-        if (k8) launch_gemm16_as<EPI, RMS, 4, 1, 8>(p, M, st);
-        else launch_gemm16_as<EPI, RMS, 4, 1, 4>(p, M, st);
+        launch_gemm16_as<EPI, RMS, 4, 1, 4>(p, M, st);
     }
 }
 

@@ -24,3 +24,21 @@ def test_layernorm_of_batched_steps(d):
         ref = ref_forward.forward(cfg, W, tokens[b])
         for t in range(5):
             assert_logits_close(got[t][b], ref[t], what=f"layernorm {d} step {t}")
+
+
+@pytest.mark.parametrize("arch, d", [(synth.ARCH_GPT2, 512), (synth.ARCH_MODERN, 768)])
+def test_tiles_do_not_change_a_pass(arch, d):
+    """Row counts from 65 to 511 take different tiles; a sequence's logits are the same in all of them."""
+    cfg = synth.Config(arch, 201, d, 2, d // 64, 80)
+    W = synth.make_weights(cfg, 93, std=lively_std(cfg), norm_noise=0.1)
+    gm = G.Model.from_tensors(cfg, W)
+    tokens = synth.uniform_tokens(73, cfg.vocab, 94)
+    ref = ref_forward.forward(cfg, W, tokens)[-1]
+    last = None
+    for batch in (1, 2, 3, 4, 5, 6, 7):
+        got = G.Session(gm, batch=batch).prefill(np.tile(tokens, (batch, 1)))
+        assert_logits_close(got[0], ref, what=f"tiles batch {batch}")
+        if batch > 1:  # (one sequence's logits are formed by another kernel)
+            last = got[0] if last is None else last
+            for b in range(batch):
+                assert got[b].tobytes() == last.tobytes(), (batch, b)
