@@ -1666,8 +1666,19 @@ static PrefillAttnParams prompt_attn_params(const Session& s, int layer, int n, 
 // against 7.3e-8..7.9e-8 without rotation, 2.3e-7..6.5e-7 against 2.3e-7..6.6e-7 with.
 constexpr int kSplitAttnMin = 128;
 
+// The fp32 attention in blocks of 16 or of 64 queries, the same sums in either.  While the 16-query blocks
+// do not fill the chip three times over what counts is the chain through a block's keys, four times as
+// long with 64 queries on four wavefronts (12 heads; us per layer, 64 / 16 queries: 1 x 61 tokens 6.9 /
+// 3.9, 1 x 397 31.5 / 17.6, 13 x 77 15.2 / 9.6, 3 x 333 31.5 / 19.4, 8 x 61 behind 500 48 / 27); beyond, keys read
+// once for 64 queries (64 x 64 17.2 / 22.1, 64 x 128 46.8 / 65.3), unless most of a 64-query block would be
+// empty (64 x 31 13.3 / 11.2, 64 x 8 behind 900 180 / 67).
 static void launch_prompt_attn(const Session& s, const PrefillAttnParams& a) {
-    hipLaunchKernelGGL(attn_prefill64_kernel, dim3((a.len + 63) / 64, s.m->shape.heads, s.B), dim3(256), 0, s.stream, a);
+    const long pairs = static_cast<long>(s.m->shape.heads) * s.B;
+    const long wide = (a.len + 63) / 64 * pairs, narrow = (a.len + 15) / 16 * pairs;
+    if (s.page_shift >= 6 && (narrow <= 800 || narrow <= 2 * wide))
+        hipLaunchKernelGGL(attn_prefill16_kernel, dim3((a.len + 15) / 16, s.m->shape.heads, s.B), dim3(256), 0, s.stream, a);
+    else
+        hipLaunchKernelGGL(attn_prefill64_kernel, dim3((a.len + 63) / 64, s.m->shape.heads, s.B), dim3(256), 0, s.stream, a);
     HIP_CHECK(hipGetLastError());
 }
 

@@ -572,4 +572,124 @@ static __global__ __launch_bounds__(256) void attn_prefill64_kernel(const Prefil
     }
 }
 
+// The same attention, the same sums bit for bit, by more and shorter chains: one workgroup = 16 queries of
+// one (sequence, head).  Of a tile of 64 keys, wavefront w forms the scores of keys 16 w .. + 15 and
+// the outputs of dims 16 w .. + 15; the maxima and the probabilities meet in LDS.  Keys and
+// values go from memory to the operand registers of the one wavefront that uses them, a tile
+// ahead.  For pages of 64 positions and more (a tile sits in one page).
+static __global__ __launch_bounds__(256) void attn_prefill16_kernel(const PrefillAttnParams p) {
+    constexpr int HS = 64, TILE = 64;
+    __shared__ float peak[2][4][16];         // [tile parity][wavefront][query]
+    __shared__ float4 prob[2][4][64];        // [tile parity][block of keys][lane]
+    const int qb = gridDim.x - 1 - blockIdx.x, h = blockIdx.y, b = blockIdx.z;  // longest first
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int j = lane & 15, g = lane >> 4;
+    const int t = qb * 16 + j;  // this lane's query (token index in the pass)
+    const bool live = t < p.len;
+    const int qpos = p.pos_base + min(t, p.len - 1);
+    const int last_pos = p.pos_base + min(p.len, qb * 16 + 16) - 1;  // last key the workgroup needs
+    float4 qf[4];
+    {
+        const float* qr = p.q + (static_cast<size_t>(b) * p.len + min(t, p.len - 1)) * p.d_model + h * HS;
+#pragma unroll
+        for (int db = 0; db < 4; db++) {
+            const float4 v = *reinterpret_cast<const float4*>(qr + db * 16 + g * 4);
+            qf[db] = make_float4(v.x * p.scale, v.y * p.scale, v.z * p.scale, v.w * p.scale);
+        }
+    }
+    const int* table = p.kv.page_table + b * p.kv.pages_per_seq;
+    const int shift = p.kv.page_shift;
+    const size_t head_stride = static_cast<size_t>(HS) << shift, kv_stride = head_stride * p.kv.heads;
+    const float* pool = p.kv.pool + static_cast<size_t>(p.layer) * p.kv.n_pages * 2 * kv_stride + h * head_stride;
+    const int slot_mask = (1 << shift) - 1;
+    // keys 16 wave + j, dims 16 db + 4 g .. + 3; values of keys 16 kb + 4 g + r, dim 16 wave + j
+    // (keys behind the last one needed are not read: zeros)
+    const auto fetch = [&](int k0, int page, float4 (&k4)[4], float (&v)[16]) {
+        const float* base = pool + static_cast<size_t>(page) * 2 * kv_stride + static_cast<size_t>(k0 & slot_mask) * HS;
+        const float* kr = base + (wave * 16 + j) * HS + g * 4;
+        const float* vr = base + kv_stride + 4 * g * HS + wave * 16 + j;
+        const bool in = k0 + wave * 16 + j <= last_pos;
+#pragma unroll
+        for (int db = 0; db < 4; db++) k4[db] = in ? *reinterpret_cast<const float4*>(kr + db * 16) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            const int key = (e >> 2) * 16 + (e & 3);
+            v[e] = k0 + key + 4 * g <= last_pos ? vr[key * HS] : 0.0f;
+        }
+    };
+    attn_v4f o = attn_v4f{0.f, 0.f, 0.f, 0.f};  // O^T: lane holds query j, dims 16 * wave + 4g + r
+    float m = -INFINITY, l = 0.0f;
+    float4 k4[4], nk4[4];
+    float v[16], nv[16];
+    int page = table[0], next_page = TILE <= last_pos ? table[TILE >> shift] : 0;
+    fetch(0, page, nk4, nv);
+    int parity = 0;
+    for (int k0 = 0; k0 <= last_pos; k0 += TILE, parity ^= 1) {
+#pragma unroll
+        for (int db = 0; db < 4; db++) k4[db] = nk4[db];
+#pragma unroll
+        for (int e = 0; e < 16; e++) v[e] = nv[e];
+        page = next_page;
+        if (k0 + TILE <= last_pos) fetch(k0 + TILE, page, nk4, nv);
+        if (k0 + 2 * TILE <= last_pos) next_page = table[(k0 + 2 * TILE) >> shift];
+        attn_v4f s = attn_v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int db = 0; db < 4; db++) {
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[db].x, qf[db].x, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[db].y, qf[db].y, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[db].z, qf[db].z, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[db].w, qf[db].w, s, 0, 0, 0);
+        }
+        float mb = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            s[r] = (k0 + wave * 16 + 4 * g + r <= qpos) ? s[r] : -INFINITY;
+            mb = fmaxf(mb, s[r]);
+        }
+        mb = fmaxf(mb, __shfl_xor(mb, 16, kWave));
+        mb = fmaxf(mb, __shfl_xor(mb, 32, kWave));
+        if (lane < 16) peak[parity][wave][lane] = mb;
+        __syncthreads();
+        const float mn = fmaxf(fmaxf(fmaxf(m, peak[parity][0][j]), fmaxf(peak[parity][1][j], peak[parity][2][j])), peak[parity][3][j]);
+        const float f = expf(m - mn);  // 0 on the first tile
+        prob[parity][wave][lane] = make_float4(expf(s[0] - mn), expf(s[1] - mn), expf(s[2] - mn), expf(s[3] - mn));
+        __syncthreads();
+        float psum = 0.0f;
+        float4 e[4];
+#pragma unroll
+        for (int kb = 0; kb < 4; kb++) {
+            e[kb] = prob[parity][kb][lane];
+            psum += e[kb].x;
+            psum += e[kb].y;
+            psum += e[kb].z;
+            psum += e[kb].w;
+        }
+        psum += __shfl_xor(psum, 16, kWave);
+        psum += __shfl_xor(psum, 32, kWave);
+        l = l * f + psum;
+        o[0] *= f;
+        o[1] *= f;
+        o[2] *= f;
+        o[3] *= f;
+#pragma unroll
+        for (int kb = 0; kb < 4; kb++) {
+            o = __builtin_amdgcn_mfma_f32_16x16x4f32(v[4 * kb + 0], e[kb].x, o, 0, 0, 0);
+            o = __builtin_amdgcn_mfma_f32_16x16x4f32(v[4 * kb + 1], e[kb].y, o, 0, 0, 0);
+            o = __builtin_amdgcn_mfma_f32_16x16x4f32(v[4 * kb + 2], e[kb].z, o, 0, 0, 0);
+            o = __builtin_amdgcn_mfma_f32_16x16x4f32(v[4 * kb + 3], e[kb].w, o, 0, 0, 0);
+        }
+        m = mn;
+    }
+    if (live) {
+        const float inv = 1.0f / l;
+        const int at = h * HS + wave * 16 + g * 4;
+        if (p.out_split) {
+            store_split4(p.out_split, b * p.len + t, at, p.d_model / kSplitCols, o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv);
+        } else {
+            *reinterpret_cast<float4*>(p.out + (static_cast<size_t>(b) * p.len + t) * p.d_model + at) =
+                make_float4(o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv);
+        }
+    }
+}
+
 }  // namespace gh

@@ -42,3 +42,22 @@ def test_tiles_do_not_change_a_pass(arch, d):
             last = got[0] if last is None else last
             for b in range(batch):
                 assert got[b].tobytes() == last.tobytes(), (batch, b)
+
+
+@pytest.mark.parametrize("batch, n, before", [(1, 8, 0), (1, 16, 0), (1, 17, 3), (1, 64, 0), (1, 65, 0), (2, 129, 0), (1, 33, 70),
+                                              (3, 50, 127), (40, 9, 60)])
+def test_query_blocks_do_not_change_a_pass(batch, n, before):
+    """Blocks of 16 queries (pages of 64 positions and more) against blocks of 64 (smaller pages)."""
+    cfg = synth.Config(synth.ARCH_MODERN, 130, 128, 2, 2, 300)
+    W = synth.make_weights(cfg, 95, std=lively_std(cfg), norm_noise=0.1)
+    gm = G.Model.from_tensors(cfg, W)
+    tokens = synth.uniform_tokens(batch * (n + before), cfg.vocab, 96).reshape(batch, -1)
+    got = []
+    for page in (32, 64, 128):
+        s = G.Session(gm, batch=batch, page_tokens=page, shuffle_pages=True)
+        if before:
+            s.prefill(tokens[:, :before])
+        got.append(s.prefill(tokens[:, before:]))
+    assert got[1].tobytes() == got[0].tobytes() and got[2].tobytes() == got[0].tobytes()
+    ref = ref_forward.forward(cfg, W, tokens[batch - 1])[-1]
+    assert_logits_close(got[1][batch - 1], ref, what=f"queries {batch} x {n}")
