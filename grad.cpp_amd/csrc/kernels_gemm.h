@@ -625,8 +625,13 @@ inline void launch_gemm16(const GemvParams& p, int M, hipStream_t st) {
         else if (M <= 64) launch_gemm16_as<EPI, RMS, 2, 2, 4>(p, M, st);
         else launch_gemm16_as<EPI, RMS, 4, 2, 4>(p, M, st);
     } else if (M <= 64) {
-        // more than 32 rows: K over four wavefronts, twice as many (smaller) workgroups per compute unit
+        // More than 32 rows: K over four wavefronts, twice as many (smaller) workgroups per compute unit.
+        // One tile per workgroup while that makes at most three of them per compute unit
+        // (stand-alone, one tile / two: 64 x 2304 x 768 7.4 us / 8.2, 48 x 4096 x 768 7.9 / 8.5, 64 x 3072 x
+        // 768 7.0 / 7.5; with four per compute unit, 64 x 4096 x 768, 9.4 / 8.7).  Per decode step of the 69M
+        // Llama block: 33 sequences 355 us -> 334, 48 376 -> 357, 64 403 -> 398.
         if (k8 && M <= 32) launch_gemm16_as<EPI, RMS, 2, 1, 8>(p, M, st);
+        else if ((M + 15) / 16 * ((p.N + 15) / 16) <= 768) launch_gemm16_as<EPI, RMS, 1, 1, 4>(p, M, st);
         else launch_gemm16_as<EPI, RMS, 2, 1, 4>(p, M, st);
     } else {
         launch_gemm16_as<EPI, RMS, 4, 1, 4>(p, M, st);

@@ -44,6 +44,24 @@ def test_tiles_do_not_change_a_pass(arch, d):
                 assert got[b].tobytes() == last.tobytes(), (batch, b)
 
 
+def test_tiles_do_not_change_a_batched_step():
+    """33 to 64 sequences: up to 48 the FFN's first matrix goes tile by tile, beyond in pairs of tiles."""
+    cfg = synth.Config(synth.ARCH_MODERN, 201, 768, 1, 12, 16)
+    W = synth.make_weights(cfg, 97, std=lively_std(cfg), norm_noise=0.1)
+    gm = G.Model.from_tensors(cfg, W)
+    tokens = synth.uniform_tokens(3, cfg.vocab, 98)
+    ref = ref_forward.forward(cfg, W, tokens)[-1]
+    last = None
+    for batch in (33, 48, 49, 64):
+        s = G.Session(gm, batch=batch)
+        for t in tokens:
+            got = s.step(np.full(batch, t, np.int32))
+        assert_logits_close(got[0], ref, what=f"step tiles batch {batch}")
+        last = got[0].copy() if last is None else last
+        for b in range(batch):
+            assert got[b].tobytes() == last.tobytes(), (batch, b)
+
+
 @pytest.mark.parametrize("batch, n, before", [(1, 8, 0), (1, 16, 0), (1, 17, 3), (1, 64, 0), (1, 65, 0), (2, 129, 0), (1, 33, 70),
                                               (3, 50, 127), (40, 9, 60)])
 def test_query_blocks_do_not_change_a_pass(batch, n, before):
