@@ -17,10 +17,12 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <mutex>
 #include <numeric>
 #include <string>
+#include <tuple>
 #include <vector>
 
 namespace gh {
@@ -503,6 +505,16 @@ struct Session {
     size_t xcd_lds = 0;
     bool xcd_all_slices = false;  // every workgroup of an XCD takes a slice of the attention at any context
 
+    // steps of a few sequences as one launch for all layers (kernels_resident.h)
+    bool resident = false;  // ... is built for this session and has not failed
+    Cell* rcells = nullptr;
+    size_t rcells_count = 0;
+    ResidentCtl* rctl = nullptr;
+    unsigned repoch = 1;    // tag base; grows with every launch, re-based by clearing the cells
+    unsigned rspin_limit = 1u << 18;
+    std::unique_lock<std::mutex> resident_lock;  // this call's hold on g_persist_gate
+    float* start_logits = nullptr;  // a copy of the logits that a run of steps began with
+
     void* host_block = nullptr;    // one pinned allocation, which kernels read and write directly:
     float* host_logits = nullptr;  // B * V
     int* host_ids = nullptr;       // [2][B * hist_stride] ids on their way to or from the device
@@ -555,7 +567,7 @@ struct Session {
                         static_cast<void*>(pp_norm), static_cast<void*>(pp_hidden), static_cast<void*>(pp_split),
                         static_cast<void*>(pp_split_hidden), static_cast<void*>(pp_kv), static_cast<void*>(pp_part),
                         static_cast<void*>(score_targets), static_cast<void*>(score_nll),
-                        static_cast<void*>(nll_part), static_cast<void*>(nll_target)})
+                        static_cast<void*>(nll_part), static_cast<void*>(nll_target), static_cast<void*>(start_logits)})
             if (p) (void)hipFree(p);
         if (host_block) (void)hipHostFree(host_block);
         if (stream) (void)hipStreamDestroy(stream);
@@ -835,9 +847,81 @@ static int enqueue_layer(Session& s, int l, bool query_only) {
     return launches;
 }
 
+// ---- all layers of a step in one launch (kernels_resident.h)
+
+// What this call launches may take the whole GPU from here on: the gate that resident launches share is this
+// session's until resident_end. False, and the step runs as a launch per operation, when another
+// session has it or this thread is inside a callback of one that does: both forms give the same bits.
+static bool resident_begin(Session& s) {
+    if (s.resident_lock.owns_lock()) return true;
+    if (g_gate_depth > 0) return false;
+    std::unique_lock<std::mutex> lock(g_persist_gate, std::try_to_lock);
+    if (!lock.owns_lock()) return false;
+    s.resident_lock = std::move(lock);
+    g_gate_depth++;
+    return true;
+}
+
+// The stream has been synchronised (or nothing resident is on it).
+static void resident_end(Session& s) {
+    if (!s.resident_lock.owns_lock()) return;
+    g_gate_depth--;
+    s.resident_lock.unlock();
+    s.resident_lock = {};
+}
+
+// Ends the call's hold however the call ends; what it launched has left the GPU by then.
+struct ResidentScope {
+    Session& s;
+    const int exceptions = std::uncaught_exceptions();
+    explicit ResidentScope(Session& session) : s(session) {}
+    ~ResidentScope() {
+        if (std::uncaught_exceptions() > exceptions && s.resident_lock.owns_lock()) (void)hipStreamSynchronize(s.stream);
+        resident_end(s);
+    }
+    ResidentScope(const ResidentScope&) = delete;
+    ResidentScope& operator=(const ResidentScope&) = delete;
+};
+
+// For the next step of this session: can and may it run that way?
+static bool resident_now(Session& s) {
+    if (!s.resident) return false;
+    const long runs = s.pos / s.attn_chunk + 1;  // of every (sequence, head)
+    return s.B * s.m->shape.heads * runs <= kResidentItems && resident_begin(s);
+}
+
+static void launch_resident(Session& s) {
+    const Model& m = *s.m;
+    const Shape& sh = m.shape;
+    // Tags are matched by equality and must not come round to one a stale cell holds.
+    if ((static_cast<unsigned long long>(s.repoch) + 2ull * sh.layers + 2ull) * 8ull >= 0xF0000000ull) {
+        HIP_CHECK(hipMemsetAsync(s.rcells, 0, s.rcells_count * sizeof(Cell), s.stream));
+        s.repoch = 1;
+    }
+    ResidentParams p{};
+    p.layer0 = m.layers[0].wqkv;
+    p.rope_cos = m.rope_cos;
+    p.rope_sin = m.rope_sin;
+    p.x = s.x;
+    p.kv = kv_layout(s);
+    p.cells = s.rcells;
+    p.ctl = s.rctl;
+    p.B = s.B;
+    p.L = sh.layers;
+    p.pos = s.pos;
+    p.chunk = s.attn_chunk;
+    p.epoch = s.repoch;
+    p.spin_limit = s.rspin_limit;
+    s.repoch += static_cast<unsigned>(sh.layers);
+    hipLaunchKernelGGL(resident_kernel_for(sh, s.B), dim3(kResidentGrid), dim3(kResidentThreads),
+                       static_cast<size_t>(s.B) * s.pages_per_seq * sizeof(int), s.stream, p);
+    HIP_CHECK(hipGetLastError());
+}
+
 // One InferenceSession::step for every sequence (inference.cpp:150-258),
 // enqueued on the session stream.  Returns the number of launches.
-static int enqueue_step(Session& s, StepForm form) {
+// resident: all layers in one launch.
+static int enqueue_step(Session& s, StepForm form, bool resident = false) {
     const Model& m = *s.m;
     const Shape& sh = m.shape;
     const int d = sh.d_model, B = s.B;
@@ -854,7 +938,12 @@ static int enqueue_step(Session& s, StepForm form) {
     HIP_CHECK(hipGetLastError());
     launches += form != STEP_ROWS;
 
-    for (int l = 0; l < sh.layers; l++) launches += enqueue_layer(s, l, /*query_only=*/false);
+    if (resident) {
+        launch_resident(s);
+        launches++;
+    } else {
+        for (int l = 0; l < sh.layers; l++) launches += enqueue_layer(s, l, /*query_only=*/false);
+    }
     launches += enqueue_logits(s, /*advance=*/true);
     return launches;
 }
@@ -1003,6 +1092,29 @@ static void xcd_build_stream(const Model& m) {
     m.xcd_stream = stream;
 }
 
+// The one-launch kernels find a layer's tensors by address arithmetic (layer_at): they must
+// follow each other without gaps, layer after layer.
+static bool layers_back_to_back(const Model& m) {
+    const Shape& sh = m.shape;
+    const size_t d = sh.d_model, F = sh.d_ff();
+    const size_t per_layer = layer_floats(d, F, sh.modern());
+    const float* base = m.layers[0].wqkv;
+    for (size_t l = 0; l < m.layers.size(); l++) {
+        const LayerWeights& w = m.layers[l];
+        const float* b = base + l * per_layer;
+        const float* want[12];
+        size_t i = 0;
+        for (const size_t n : {3 * d * d, 3 * d, d * d, d, (sh.modern() ? 2 : 1) * F * d, F, d * F, d, d, d, d, d}) {
+            want[i++] = b;
+            b += n;
+        }
+        const float* have[12] = {w.wqkv, w.bqkv, w.wo, w.bo, w.w1, w.b1, w.w2, w.b2, w.g1, w.be1, w.g2, w.be2};
+        for (i = 0; i < 12; i++)
+            if (have[i] != want[i]) return false;
+    }
+    return true;
+}
+
 static const char* persist_unavailable(const Session& s, int lds_bytes, int cus) {
     const Shape& sh = s.m->shape;
     if (s.B != 1) return "the persistent engine decodes one sequence";
@@ -1010,26 +1122,7 @@ static const char* persist_unavailable(const Session& s, int lds_bytes, int cus)
     if (sh.max_len > 4096) return "the persistent engine handles contexts up to 4096";
     if (cus < sh.heads) return "the GPU has fewer compute units than the model has heads";
     (void)lds_bytes;
-    // The kernel finds a layer's tensors by address arithmetic (layer_at): they must
-    // follow each other without gaps, layer after layer.
-    {
-        const size_t d = sh.d_model, F = sh.d_ff();
-        const size_t per_layer = layer_floats(d, F, sh.modern());
-        const float* base = s.m->layers[0].wqkv;
-        for (size_t l = 0; l < s.m->layers.size(); l++) {
-            const LayerWeights& w = s.m->layers[l];
-            const float* b = base + l * per_layer;
-            const float* want[12];
-            size_t i = 0;
-            for (const size_t n : {3 * d * d, 3 * d, d * d, d, (sh.modern() ? 2 : 1) * F * d, F, d * F, d, d, d, d, d}) {
-                want[i++] = b;
-                b += n;
-            }
-            const float* have[12] = {w.wqkv, w.bqkv, w.wo, w.bo, w.w1, w.b1, w.w2, w.b2, w.g1, w.be1, w.g2, w.be2};
-            for (i = 0; i < 12; i++)
-                if (have[i] != want[i]) return "the persistent engine needs the layers' tensors back to back";
-        }
-    }
+    if (!layers_back_to_back(*s.m)) return "the persistent engine needs the layers' tensors back to back";
     return nullptr;
 }
 
@@ -1182,9 +1275,14 @@ static int record_step(Session& s, StepForm form, hipGraph_t* graph) {
 }
 
 static void run_step(Session& s, StepForm form = STEP_EMBED) {
-    if (s.engine == GH_ENGINE_GRAPH) {
+    if (resident_now(s)) {
+        enqueue_step(s, form, /*resident=*/true);
+    } else if (s.engine == GH_ENGINE_GRAPH) {
         if (!s.exec[form]) {  // (a form's graph is made when it is first wanted)
-            if (!s.graph[form]) record_step(s, form, &s.graph[form]);
+            if (!s.graph[form]) {
+                const int launches = record_step(s, form, &s.graph[form]);
+                if (!s.resident) s.launches_per_step = launches;
+            }
             HIP_CHECK(hipGraphInstantiate(&s.exec[form], s.graph[form], nullptr, nullptr, 0));
         }
         HIP_CHECK(hipGraphLaunch(s.exec[form], s.stream));
@@ -1254,7 +1352,7 @@ __global__ void deliver_kernel(const unsigned* __restrict__ src, size_t total, s
 
 // ... after which check_persist_abort needs no copy of its own.
 static void deliver(Session& s, const void* src, size_t src_stride, size_t rows, size_t n, void* dst) {
-    const unsigned* abort = s.engine == GH_ENGINE_PERSISTENT ? &s.ctl->abort : nullptr;
+    const unsigned* abort = s.engine == GH_ENGINE_PERSISTENT ? &s.ctl->abort : s.resident ? &s.rctl->abort : nullptr;
     const size_t groups = std::min<size_t>(256, std::max<size_t>(1, (rows * n + 255) / 256));
     hipLaunchKernelGGL(deliver_kernel, dim3(static_cast<unsigned>(groups)), dim3(256), 0, s.stream,
                        static_cast<const unsigned*>(src), rows * n, n, src_stride, static_cast<unsigned*>(dst), abort,
@@ -1265,6 +1363,25 @@ static void deliver(Session& s, const void* src, size_t src_stride, size_t rows,
 static void deliver_logits(Session& s) {
     const size_t V = s.m->shape.vocab;
     deliver(s, s.logits, 0, 1, s.B * V, s.host_logits);
+}
+
+// Launches of a session whose steps may be resident, up to and with a deliver() and the synchronisation behind it. If a
+// resident step gave up its wait (something else held a part of the GPU for long), the session does
+// without from here on, and the call runs once more from where the session stood: the cache rows below that
+// position, the history and the call's ids are as they were, and what comes after is written again.
+template <class Work>
+static void run_resident(Session& s, Work work) {
+    const int pos = s.pos, n_hist = s.n_hist, picks = s.picks;
+    work();
+    if (!s.resident || *s.host_err == 0) return;
+    s.resident = false;
+    *s.host_err = 0;
+    s.pos = pos;
+    s.n_hist = n_hist;
+    s.picks = picks;
+    hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, s.stream, s.st, pos, n_hist, picks);
+    HIP_CHECK(hipGetLastError());
+    work();
 }
 
 static void reset_session(Session& s) {
@@ -1445,6 +1562,35 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
         }
     }
 
+    // Steps of 2 to 16 sequences: all layers in one launch, where the shape has such a kernel, it can be resident
+    // (a workgroup per compute unit) and the page table fits its LDS.
+    {
+        int cus = 0;
+        HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        const ResidentKernel kernel = resident_kernel_for(sh, s.B);
+        const size_t table_bytes = table.size() * sizeof(int);
+        if (o.engine == GH_ENGINE_AUTO && s.engine == GH_ENGINE_GRAPH && kernel && cus >= kResidentGrid
+            && table_bytes <= kResidentTableBytes && s.page_shift >= 5 && s.attn_chunk % 128 == 0 && layers_back_to_back(m)) {
+            s.resident = true;
+            s.rcells_count = resident_cells(d, F, B);
+            parts.add(s.rcells, s.rcells_count);
+            parts.add(s.rctl, 1);
+            HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          kResidentTableBytes));
+            // (embedding, layers, logits; a LayerNorm in front of the logits is a launch of its own)
+            s.launches_per_step = sh.modern() ? 3 : 4;
+            // Test aid: looks at a cell that a wait may take (0: the first look has to succeed).
+            if (const char* spins = std::getenv("GRADHIP_TEST_RESIDENT_SPINS"))
+                s.rspin_limit = static_cast<unsigned>(std::min(std::max(std::strtol(spins, nullptr, 10), 0l), 1l << 18));
+            // ... and steps until the tags start over (as for the one-launch engine, below).
+            if (const char* near = std::getenv("GRADHIP_TEST_NEAR_WRAP")) {
+                const long asked = std::strtol(near, nullptr, 10);
+                if (asked >= 1 && asked <= 4096)
+                    s.repoch = static_cast<unsigned>(0xF0000000ull / 8ull) - static_cast<unsigned>((asked + 2) * sh.layers);
+            }
+        }
+    }
+
     // The matrix-core logits launch can leave what a greedy pick needs (a batch of at
     // least two sequences takes it; the wide form and the tiled form both can).
     if (s.engine != GH_ENGINE_PERSISTENT && s.B >= kMinGemmBatch && gemm_shape_ok(sh.d_model, sh.d_model)) {
@@ -1495,7 +1641,7 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
 
     if (s.engine == GH_ENGINE_PERSISTENT) {
         // nothing to record: one launch runs any number of steps
-    } else {
+    } else if (!s.resident) {
         // Counts the launches of a step without running one.
         s.launches_per_step = record_step(s, STEP_EMBED, &s.graph[STEP_EMBED]);
     }
@@ -2004,6 +2150,41 @@ static std::pair<int, int> run_decode(Session& s, int max_tokens, const gh_sampl
     return {picks, steps};
 }
 
+// The logits that a run of steps begins with, kept while its steps may be resident: the first pick is
+// made from them and the steps overwrite them.  (Without memory for the copy the launches do.)
+static void keep_logits(Session& s, bool restore) {
+    const size_t n = static_cast<size_t>(s.B) * s.m->shape.vocab;
+    if (restore) {
+        HIP_CHECK(hipMemcpyAsync(s.logits, s.start_logits, n * sizeof(float), hipMemcpyDeviceToDevice, s.stream));
+        return;
+    }
+    if (!s.resident) return;
+    if (!s.start_logits && !try_alloc(s.start_logits, n)) {
+        s.resident = false;
+        return;
+    }
+    HIP_CHECK(hipMemcpyAsync(s.start_logits, s.logits, n * sizeof(float), hipMemcpyDeviceToDevice, s.stream));
+}
+
+// In a streamed run, after a synchronisation: if the last step was resident and gave up, it runs again as launches.
+// picked: a pick made from its logits is to be forgotten.  True if it had to.
+static bool repeat_step(Session& s, bool picked) {
+    if (!s.resident || *s.host_err == 0) return false;
+    s.resident = false;
+    *s.host_err = 0;
+    s.pos--;
+    if (picked) {
+        s.n_hist--;
+        s.picks--;
+    }
+    hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, s.stream, s.st, s.pos, s.n_hist, s.picks);
+    hipLaunchKernelGGL(load_tok_kernel, dim3((s.B + 63) / 64), dim3(64), 0, s.stream, s.hist, s.hist_stride, s.n_hist - 1, s.tok,
+                       s.B);
+    HIP_CHECK(hipGetLastError());
+    run_step(s);
+    return true;
+}
+
 // Copies the caller's uniforms to the device (grown on demand); null for none.
 static const float* stage_uniforms(Session& s, const float* uniforms, size_t n) {
     if (!uniforms || n == 0) return nullptr;
@@ -2454,6 +2635,7 @@ gh_status gh_session_step(gh_session* sess, const int32_t* ids, float* logits_ho
         if (!sess || !ids) throw ApiError{GH_ERR_INVALID_ARGUMENT, "null argument"};
         Session& s = *sess->impl;
         const PersistGate gate(s);  // held until this call has synchronised its launches
+        const ResidentScope scope(s);
         check_capacity(s);
         check_ids(s, ids, s.B);
         const size_t V = s.m->shape.vocab;
@@ -2466,15 +2648,16 @@ gh_status gh_session_step(gh_session* sess, const int32_t* ids, float* logits_ho
             std::memcpy(s.host_ids, ids, s.B * sizeof(int));
             // The history (index == position) feeds the repetition penalty of later picks.
             stage_ids(s, s.host_ids, 1, s.hist, s.hist_stride, s.n_hist, s.tok);
-            if (s.engine == GH_ENGINE_PERSISTENT) {
-                persist_run(s, 1, 1, 0, false, nullptr, nullptr, 0, 0, nullptr);
-            } else {
+            if (s.engine == GH_ENGINE_PERSISTENT) persist_run(s, 1, 1, 0, false, nullptr, nullptr, 0, 0, nullptr);
+        }
+        run_resident(s, [&] {
+            if (s.engine != GH_ENGINE_PERSISTENT) {
                 s.n_hist++;
                 run_step(s);
             }
-        }
-        deliver_logits(s);
-        HIP_CHECK(hipStreamSynchronize(s.stream));
+            deliver_logits(s);
+            HIP_CHECK(hipStreamSynchronize(s.stream));
+        });
         check_persist_abort(s);
         if (logits_host) std::memcpy(logits_host, s.host_logits, s.B * V * sizeof(float));
     });
@@ -2493,6 +2676,7 @@ gh_status gh_session_prefill(gh_session* sess, const int32_t* ids, int32_t len,
         if (!sess || !ids) throw ApiError{GH_ERR_INVALID_ARGUMENT, "null argument"};
         Session& s = *sess->impl;
         const PersistGate gate(s);  // held until this call has synchronised its launches
+        const ResidentScope scope(s);
         if (len < 0) throw ApiError{GH_ERR_INVALID_ARGUMENT, "negative length"};
         if (len == 0) return;
         if (s.pos + len > s.m->shape.max_len)
@@ -2502,9 +2686,11 @@ gh_status gh_session_prefill(gh_session* sess, const int32_t* ids, int32_t len,
         // Stage the ids into the history, then step through them.
         std::memcpy(s.host_ids, ids, static_cast<size_t>(s.B) * len * sizeof(int));
         stage_ids(s, s.host_ids, len, s.hist, s.hist_stride, s.n_hist);
-        run_prompt(s, len, nullptr, nullptr);
-        deliver_logits(s);
-        HIP_CHECK(hipStreamSynchronize(s.stream));
+        run_resident(s, [&] {
+            run_prompt(s, len, nullptr, nullptr);
+            deliver_logits(s);
+            HIP_CHECK(hipStreamSynchronize(s.stream));
+        });
         check_persist_abort(s);
         if (last_logits_host) std::memcpy(last_logits_host, s.host_logits, s.B * V * sizeof(float));
     });
@@ -2516,6 +2702,7 @@ gh_status gh_session_score(gh_session* sess, const int32_t* ids, const int32_t* 
         if (!sess || !ids || !targets || !nll_host) throw ApiError{GH_ERR_INVALID_ARGUMENT, "null argument"};
         Session& s = *sess->impl;
         const PersistGate gate(s);  // held until this call has synchronised its launches
+        const ResidentScope scope(s);
         if (len < 0) throw ApiError{GH_ERR_INVALID_ARGUMENT, "negative length"};
         if (len == 0) return;
         if (s.pos + len > s.m->shape.max_len)
@@ -2541,28 +2728,30 @@ gh_status gh_session_score(gh_session* sess, const int32_t* ids, const int32_t* 
         stage_ids(s, host_targets, len, s.score_targets, len, 0);
         const ScoreSink sink{s.score_targets, s.score_nll};
         const RowsPlan plan = plan_rows(s, len, /*score=*/true);
-        if (plan.slice > 0) {
-            prompt_pass(s, len, plan, &sink);
-        } else {
-            // token by token: every step leaves the logits of its position
-            const int V = s.m->shape.vocab;
-            for (int t = 0; t < len; t++) {
-                if (s.engine == GH_ENGINE_PERSISTENT) {
-                    persist_run(s, 1, 1, 0, false, nullptr, nullptr, 0, 0, nullptr);  // token from the history
-                } else {
-                    hipLaunchKernelGGL(load_tok_kernel, dim3((s.B + 63) / 64), dim3(64), 0, s.stream, s.hist,
-                                       s.hist_stride, base + t, s.tok, s.B);
+        run_resident(s, [&] {
+            if (plan.slice > 0) {
+                prompt_pass(s, len, plan, &sink);
+            } else {
+                // token by token: every step leaves the logits of its position
+                const int V = s.m->shape.vocab;
+                for (int t = 0; t < len; t++) {
+                    if (s.engine == GH_ENGINE_PERSISTENT) {
+                        persist_run(s, 1, 1, 0, false, nullptr, nullptr, 0, 0, nullptr);  // token from the history
+                    } else {
+                        hipLaunchKernelGGL(load_tok_kernel, dim3((s.B + 63) / 64), dim3(64), 0, s.stream, s.hist,
+                                           s.hist_stride, base + t, s.tok, s.B);
+                        HIP_CHECK(hipGetLastError());
+                        run_step(s);
+                    }
+                    hipLaunchKernelGGL(nll_rows_kernel, dim3(s.B), dim3(256), 0, s.stream, s.logits, V, t, len, sink.targets,
+                                       sink.nll);
                     HIP_CHECK(hipGetLastError());
-                    run_step(s);
                 }
-                hipLaunchKernelGGL(nll_rows_kernel, dim3(s.B), dim3(256), 0, s.stream, s.logits, V, t, len, sink.targets,
-                                   sink.nll);
-                HIP_CHECK(hipGetLastError());
+                if (s.engine != GH_ENGINE_PERSISTENT) s.n_hist += len;
             }
-            if (s.engine != GH_ENGINE_PERSISTENT) s.n_hist += len;
-        }
-        deliver(s, s.score_nll, 0, 1, n, s.host_ids);  // (the ids have long been read)
-        HIP_CHECK(hipStreamSynchronize(s.stream));
+            deliver(s, s.score_nll, 0, 1, n, s.host_ids);  // (the ids have long been read)
+            HIP_CHECK(hipStreamSynchronize(s.stream));
+        });
         check_persist_abort(s);
         std::memcpy(nll_host, s.host_ids, n * sizeof(float));
     });
@@ -2637,6 +2826,7 @@ gh_status gh_session_decode(gh_session* sess, int32_t max_tokens, const gh_sampl
         if (!sess || !opt || !out_count) throw ApiError{GH_ERR_INVALID_ARGUMENT, "null argument"};
         Session& s = *sess->impl;
         const PersistGate gate(s);  // held until this call has synchronised its launches
+        const ResidentScope scope(s);
         check_sampling(*opt);
         *out_count = 0;
         s.timing = gh_timing{};
@@ -2648,12 +2838,19 @@ gh_status gh_session_decode(gh_session* sess, int32_t max_tokens, const gh_sampl
         const int first = s.n_hist;
         const int saved_picks = s.picks;
         if (du) s.picks = 0;  // uniforms are indexed from this call's first pick
-        HIP_CHECK(hipEventRecord(s.ev[1], s.stream));
-        const auto [made, stepped] = run_decode(s, max_tokens, *opt, du, max_tokens, seed, nullptr, nullptr);
-        HIP_CHECK(hipEventRecord(s.ev[2], s.stream));
+        int made = 0, stepped = 0;
+        bool again = false;
+        keep_logits(s, /*restore=*/false);
+        run_resident(s, [&] {
+            if (again) keep_logits(s, /*restore=*/true);
+            again = true;
+            HIP_CHECK(hipEventRecord(s.ev[1], s.stream));
+            std::tie(made, stepped) = run_decode(s, max_tokens, *opt, du, max_tokens, seed, nullptr, nullptr);
+            HIP_CHECK(hipEventRecord(s.ev[2], s.stream));
+            deliver(s, s.hist + first, s.hist_stride, s.B, made, s.host_ids);
+            HIP_CHECK(hipStreamSynchronize(s.stream));
+        });
         if (du) s.picks = saved_picks + made;
-        deliver(s, s.hist + first, s.hist_stride, s.B, made, s.host_ids);
-        HIP_CHECK(hipStreamSynchronize(s.stream));
         check_persist_abort(s);
         if (out_ids)
             for (size_t b = 0; b < B; b++)
@@ -2672,6 +2869,7 @@ gh_status gh_session_decode_stream(gh_session* sess, int32_t max_tokens, const g
         if (!sess || !opt || !out_count || !on_tokens) throw ApiError{GH_ERR_INVALID_ARGUMENT, "null argument"};
         Session& s = *sess->impl;
         const PersistGate gate(s);  // held until this call has synchronised its launches
+        const ResidentScope scope(s);
         check_sampling(*opt);
         *out_count = 0;
         s.timing = gh_timing{};
@@ -2764,6 +2962,11 @@ gh_status gh_session_decode_stream(gh_session* sess, int32_t max_tokens, const g
                 launch_pick(s, *opt, du, max_tokens, seed, true, /*embed=*/s.pos < C);
                 deliver(s, s.tok, 0, 1, B, s.host_ids);
                 HIP_CHECK(hipStreamSynchronize(s.stream));
+                resident_end(s);  // the callback may use any session
+                if (repeat_step(s, /*picked=*/true)) {
+                    i--;  // its pick was made from nothing
+                    continue;
+                }
                 if (out_ids)
                     for (int b = 0; b < B; b++) out_ids[static_cast<size_t>(b) * max_tokens + i] = s.host_ids[b];
                 const int32_t asked = on_tokens(user, s.host_ids, i);
@@ -2779,7 +2982,9 @@ gh_status gh_session_decode_stream(gh_session* sess, int32_t max_tokens, const g
                 if (asked != 0 || n_seen == B) break;
             }
             HIP_CHECK(hipEventRecord(s.ev[2], s.stream));
+            if (s.resident) deliver(s, nullptr, 0, 1, 0, nullptr);
             HIP_CHECK(hipStreamSynchronize(s.stream));
+            if (repeat_step(s, /*picked=*/false)) HIP_CHECK(hipStreamSynchronize(s.stream));
         }
         if (du) s.picks = saved_picks + made;
         *out_count = made;
@@ -2797,6 +3002,7 @@ gh_status gh_session_generate(gh_session* sess, const int32_t* prompts, int32_t 
             throw ApiError{GH_ERR_INVALID_ARGUMENT, "null argument"};
         Session& s = *sess->impl;
         const PersistGate gate(s);  // held until this call has synchronised its launches
+        const ResidentScope scope(s);
         const Shape& sh = s.m->shape;
         check_sampling(*opt);
         *out_len = 0;
@@ -2828,16 +3034,19 @@ gh_status gh_session_generate(gh_session* sess, const int32_t* prompts, int32_t 
             log = s.logit_log;
         }
         size_t steps = 0;
-        HIP_CHECK(hipEventRecord(s.ev[0], s.stream));
-        run_prompt(s, prompt_len, log, &steps);
-        HIP_CHECK(hipEventRecord(s.ev[1], s.stream));
-        const auto [made, stepped] = run_decode(s, max_tokens, *opt, du, max_tokens, seed, log, &steps);
-        (void)made;
-        HIP_CHECK(hipEventRecord(s.ev[2], s.stream));
+        int made = 0, stepped = 0, total = 0;
+        run_resident(s, [&] {
+            steps = 0;
+            HIP_CHECK(hipEventRecord(s.ev[0], s.stream));
+            run_prompt(s, prompt_len, log, &steps);
+            HIP_CHECK(hipEventRecord(s.ev[1], s.stream));
+            std::tie(made, stepped) = run_decode(s, max_tokens, *opt, du, max_tokens, seed, log, &steps);
+            HIP_CHECK(hipEventRecord(s.ev[2], s.stream));
 
-        const int total = s.n_hist;
-        deliver(s, s.hist, s.hist_stride, s.B, total, s.host_ids);
-        HIP_CHECK(hipStreamSynchronize(s.stream));
+            total = s.n_hist;
+            deliver(s, s.hist, s.hist_stride, s.B, total, s.host_ids);
+            HIP_CHECK(hipStreamSynchronize(s.stream));
+        });
         check_persist_abort(s);
         const size_t out_stride = static_cast<size_t>(prompt_len) + max_tokens;
         for (size_t b = 0; b < B; b++)

@@ -4,12 +4,14 @@
 
 #include "checkpoint.h"
 #include "kernels_persist.h"
+#include "kernels_resident.h"
 #include "kernels_xcd.h"
 
 namespace gh {
 
 using PersistKernel = void (*)(const PersistParams);
 using XcdKernel = void (*)(const XcdParams);
+using ResidentKernel = void (*)(const ResidentParams);
 
 // The shapes the persistent kernel is built for (head size 64, d_model and FFN
 // width multiples of 256); nullptr for anything else.
@@ -19,6 +21,9 @@ PersistKernel persist_kernel_for(const Shape& sh, bool row_lds, bool feed = fals
 
 // The Llama block at d_model 768; nullptr for anything else.
 XcdKernel xcd_kernel_for(const Shape& sh, bool row_lds, bool feed);
+
+// All layers of a step of 2 to kResidentRows sequences; nullptr for shapes it is not built for.
+ResidentKernel resident_kernel_for(const Shape& sh, int batch);
 
 #ifdef GH_PICK_TICKS
 bool read_pick_ticks(unsigned long long (&t)[32]);

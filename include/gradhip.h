@@ -12,6 +12,9 @@
  * (batch 1, the shapes it is built for) take turns inside the library: its
  * kernel needs the whole GPU, so a call that launches it holds a process-wide
  * lock until the launch has finished; results do not depend on the order.
+ * Sessions of 2 to 16 sequences run a step's layers as one such launch (AUTO, the
+ * same shapes except d_model 1024) when the lock is free, and as a launch per
+ * operation when it is not: the results are the same to the bit.
  *
  * There is no CPU fallback: every compute entry point fails with
  * GH_ERR_DEVICE when no gfx950 device is usable.
@@ -92,7 +95,7 @@ gh_status gh_model_get_config(const gh_model* m, gh_config* out);
 /* ---------------------------------------------------------------- session */
 
 typedef enum gh_engine {
-    GH_ENGINE_AUTO = 0,
+    GH_ENGINE_AUTO = 0,      /* what is fastest for the shape and the batch */
     GH_ENGINE_GRAPH = 1,     /* one kernel per fused op, whole step replayed as a hipGraph */
     GH_ENGINE_EAGER = 2,     /* same kernels launched one by one (debugging, profiling) */
     GH_ENGINE_PERSISTENT = 3 /* one cooperative kernel per step; batch 1 only */
