@@ -883,11 +883,12 @@ struct ResidentScope {
     ResidentScope& operator=(const ResidentScope&) = delete;
 };
 
+// (sequence, head, run of positions): what the attention of the next step consists of.
+static int resident_items(const Session& s) { return s.B * s.m->shape.heads * (s.pos / s.attn_chunk + 1); }
+
 // For the next step of this session: can and may it run that way?
 static bool resident_now(Session& s) {
-    if (!s.resident) return false;
-    const long runs = s.pos / s.attn_chunk + 1;  // of every (sequence, head)
-    return s.B * s.m->shape.heads * runs <= kResidentItems && resident_begin(s);
+    return s.resident && resident_kernel_for(s.m->shape, s.B, resident_items(s)) && resident_begin(s);
 }
 
 static void launch_resident(Session& s) {
@@ -913,7 +914,7 @@ static void launch_resident(Session& s) {
     p.epoch = s.repoch;
     p.spin_limit = s.rspin_limit;
     s.repoch += static_cast<unsigned>(sh.layers);
-    hipLaunchKernelGGL(resident_kernel_for(sh, s.B), dim3(kResidentGrid), dim3(kResidentThreads),
+    hipLaunchKernelGGL(resident_kernel_for(sh, s.B, resident_items(s)), dim3(kResidentGrid), dim3(kResidentThreads),
                        static_cast<size_t>(s.B) * s.pages_per_seq * sizeof(int), s.stream, p);
     HIP_CHECK(hipGetLastError());
 }
@@ -1567,16 +1568,20 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
     {
         int cus = 0;
         HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        const ResidentKernel kernel = resident_kernel_for(sh, s.B);
+        const int pairs = s.B * sh.heads, runs = (sh.max_len + s.attn_chunk - 1) / s.attn_chunk;
         const size_t table_bytes = table.size() * sizeof(int);
-        if (o.engine == GH_ENGINE_AUTO && s.engine == GH_ENGINE_GRAPH && kernel && cus >= kResidentGrid
+        if (o.engine == GH_ENGINE_AUTO && s.engine == GH_ENGINE_GRAPH && resident_kernel_for(sh, s.B, pairs) && cus >= kResidentGrid
             && table_bytes <= kResidentTableBytes && s.page_shift >= 5 && s.attn_chunk % 128 == 0 && layers_back_to_back(m)) {
             s.resident = true;
             s.rcells_count = resident_cells(d, F, B);
             parts.add(s.rcells, s.rcells_count);
             parts.add(s.rctl, 1);
-            HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          kResidentTableBytes));
+            for (int n = 1; n <= runs; n++) {  // (with the context the variant changes once)
+                const ResidentKernel kernel = resident_kernel_for(sh, s.B, pairs * n);
+                if (kernel && (n == 1 || kernel != resident_kernel_for(sh, s.B, pairs * (n - 1))))
+                    HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, kResidentTableBytes));
+            }
             // (embedding, layers, logits; a LayerNorm in front of the logits is a launch of its own)
             s.launches_per_step = sh.modern() ? 3 : 4;
             // Test aid: looks at a cell that a wait may take (0: the first look has to succeed).

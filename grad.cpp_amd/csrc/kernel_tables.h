@@ -22,8 +22,9 @@ PersistKernel persist_kernel_for(const Shape& sh, bool row_lds, bool feed = fals
 // The Llama block at d_model 768; nullptr for anything else.
 XcdKernel xcd_kernel_for(const Shape& sh, bool row_lds, bool feed);
 
-// All layers of a step of 2 to kResidentRows sequences; nullptr for shapes it is not built for.
-ResidentKernel resident_kernel_for(const Shape& sh, int batch);
+// All layers of a step of 2 to kResidentRows sequences whose attention is cut into `items` runs of
+// positions; nullptr for what it is not built for.
+ResidentKernel resident_kernel_for(const Shape& sh, int batch, int items);
 
 #ifdef GH_PICK_TICKS
 bool read_pick_ticks(unsigned long long (&t)[32]);

@@ -19,7 +19,8 @@
 // of it until the rows are there), attention 2.4, W_o 2.5, FFN1 4.1, FFN2 4.7 (1.7 of it products, 16-row tiles for
 // 4 rows; 128 KB of weights through one compute unit).  Per step, launches -> this, context 200: Llama
 // block 2 sequences 246 us -> 152, 4 254 -> 167, 8 258 -> 193, 16 279 -> 204; GPT-2 block d768 2 sequences
-// 286 -> 175, 16 323 -> 241.
+// 286 -> 175, 16 323 -> 241; Llama block, 16 sequences behind 1900 positions 524 -> 460, 190 MB of cache per
+// layer in some 39 us of its 54.
 //
 // The order things are sent in is most of the design.  A wavefront's loads return in the order they
 // went out, and a workgroup's stores leave behind what its other wavefronts have asked for: weights are
@@ -35,7 +36,8 @@ namespace gh {
 
 constexpr int kResidentThreads = 512, kResidentGrid = 256, kResidentRows = 16;
 constexpr int kResidentTableBytes = 16384;                // page tables of all sequences, in LDS
-constexpr int kResidentItems = 2 * kResidentGrid;  // (sequence, head, run of positions) of the attention, two per workgroup
+constexpr int kResidentRounds = 4;
+constexpr int kResidentItems = 2 * kResidentGrid * kResidentRounds;  // (sequence, head, run of positions) of the attention: two per workgroup and round
 
 struct ResidentCtl {
     unsigned abort;  // set by any workgroup that gave up waiting
@@ -77,7 +79,10 @@ __device__ __forceinline__ void cell_put2(__amdgpu_buffer_rsrc_t rs, int cell, f
 // RP: rows a load of operands is dealt for (B <= RP, of 4, 8 and 16).  A product takes row lane % 16, so with few
 // rows most lanes would have nothing to load: 16 / RP units of two columns share a load instead, and
 // move to their lanes inside the registers.
-template <int KD, int KF, bool MODERN, int RP>
+// ROUNDS: more items of the attention than halves of workgroups.  A variant of its own: the loop over
+// rounds costs a step that has only one 1 to 3 %.  (A wavefront's next 32 positions requested before the
+// present ones are worked on: spills at d768, 2 to 6 % slower at every context but one.)
+template <int KD, int KF, bool MODERN, int RP, bool ROUNDS>
 __global__ __launch_bounds__(kResidentThreads) void resident_layers_kernel(const ResidentParams p) {
     constexpr int D = KD * 256, F = KF * 256, HS = 64, H = D / HS, KW = 8;
     constexpr int ND = D / KW / 16, NF = F / KW / 16;  // 16-column blocks of a wavefront's share of K
@@ -87,7 +92,8 @@ __global__ __launch_bounds__(kResidentThreads) void resident_layers_kernel(const
     static_assert(TO + TQ <= G && T1 <= 2 * NO, "every phase in one round");
     __shared__ float red[2][2][KW][256];  // [phase parity][tile][wavefront][row * 16 + column]
     __shared__ float ssq[2][KW][16];
-    __shared__ float part[2][2][4][68];  // [layer parity][item]: as in attn_decode64_kernel
+    __shared__ float part[2][2][4][68];  // [parity of the round][half]: as in attn_decode64_kernel
+    __shared__ float held[ROUNDS ? kResidentRounds : 1][2][66];  // the first run of a context in several
     __shared__ float rows[MODERN ? 1 : kResidentRows * LDX];
     __shared__ float mean[16], scale[16];
     extern __shared__ int ptab[];  // [B][pages_per_seq]
@@ -107,6 +113,7 @@ __global__ __launch_bounds__(kResidentThreads) void resident_layers_kernel(const
     const int order = wg >= TO + TQ ? wg - (TO + TQ) : wg >= TO ? wg - TO + (G - TO - TQ) : wg + (G - TO);
     const int ctx = pos + 1, nchunk = (ctx + p.chunk - 1) / p.chunk;
     const int items = B * H * nchunk;
+    const int rounds = ROUNDS ? (items + 2 * G - 1) / (2 * G) : 1;
     const bool has_items = order < items;
 
     const __amdgpu_buffer_rsrc_t rs = make_buffer(p.cells, static_cast<unsigned>(resident_cells(D, F, B) * sizeof(Cell)));
@@ -355,182 +362,209 @@ __global__ __launch_bounds__(kResidentThreads) void resident_layers_kernel(const
             __syncthreads();  // nobody's loads go out in front of these stores
         }
 
-        // ===== attention: attn_decode64_kernel's workgroup is half of this one
+        // ===== attention: attn_decode64_kernel's workgroup is half of this one.  With more items than halves of
+        // workgroups they go in rounds, and the runs of a longer context are folded when every round's are out (a run in
+        // a later round may be what another workgroup's fold waits for).
         if (has_items) {
             const int half = wave >> 2, wv = wave & 3;
-            const int item = order + half * G;
-            const bool live = item < items;
-            const int pair = live ? item / nchunk : 0, ck = live ? item - pair * nchunk : 0;
-            const int seq = pair / H, h = pair - seq * H;
             const int sub = lane >> 4, dl = lane & 15;
-            const int p0 = ck * p.chunk, p1 = min(ctx, p0 + p.chunk);
-            const int run = ((((p1 - p0) + 3) / 4) + 31) & ~31;
-            const int t0 = p0 + wv * run, t1 = min(p1, t0 + run);
             const int shift = p.kv.page_shift;
-            const int* table = ptab + seq * p.kv.pages_per_seq;
             const size_t head_stride = static_cast<size_t>(HS) << shift, kv_stride = head_stride * H;
-            const float* base = p.kv.pool + static_cast<size_t>(l) * p.kv.n_pages * 2 * kv_stride + h * head_stride;
-            const auto fetch = [&](int tb, float4 (&k4)[8], float4 (&v4)[8]) {
-                const float* at = base + static_cast<size_t>(table[min(tb, pos) >> shift]) * 2 * kv_stride;
-#pragma unroll
-                for (int it = 0; it < 8; it++) {
-                    const int tt = tb + it * 4 + sub;
-                    k4[it] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    v4[it] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (tt < t1 && tt < pos) {
-                        const float* row = at + static_cast<size_t>(tt & ((1 << shift) - 1)) * HS + dl * 4;
-                        k4[it] = *reinterpret_cast<const float4*>(row);
-                        v4[it] = *reinterpret_cast<const float4*>(row + kv_stride);
-                    }
-                }
+            const float* pool = p.kv.pool + static_cast<size_t>(l) * p.kv.n_pages * 2 * kv_stride;
+            const auto publish = [&](int seq, int h, float v) {  // two columns per store
+                const float next = dpp_move<0xB1, 0xF>(v, 0.0f);
+                if (!(lane & 1)) cell_put2(rs, c_at + operand_cell(h * HS + lane, seq, B), v, next, sb + 2u);
             };
-            float m = -INFINITY, lsum = 0.0f;
-            float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (live && t0 < t1) {
-                float4 k4[8], v4[8];
-                fetch(t0, k4, v4);  // in flight while q is on its way
-                const bool newest = t1 == ctx;
-                float4 q4, kn, vn;
-                {
-                    const unsigned at = static_cast<unsigned>(seq * D + h * HS + dl * 4) * 8u;
-                    const unsigned tag = sb + 1u;
+            // the other runs of a context whose first gave M, L and o, folded in order (attn_merge)
+            const auto fold = [&](int item, float M, float L, float o) {
+                const int pair = item / nchunk, seq = pair / H, h = pair - seq * H;
+                float all = M;
+                float cm = 0.0f, cl = 0.0f, co = 0.0f;
+                const auto look = [&](int c) {
+                    const Cell* theirs = p.cells + c_part + (item + c) * 66;
                     unsigned spins = 0;
                     for (;;) {
-                        v4i u[6];
-#pragma unroll
-                        for (int i = 0; i < 6; i++)
-                            u[i] = coherent_load16(rs, (i < 2 || newest) ? static_cast<unsigned>((c_q + (i >> 1) * D * B) * 8) + at + (i & 1) * 16 : kPastEnd);
-                        bool ok = true;
-#pragma unroll
-                        for (int i = 0; i < 6; i++)
-                            ok = ok && ((i >= 2 && !newest) || (u[i].y == static_cast<int>(tag) && u[i].w == static_cast<int>(tag)));
-                        q4 = make_float4(__int_as_float(u[0].x), __int_as_float(u[0].z), __int_as_float(u[1].x), __int_as_float(u[1].z));
-                        kn = make_float4(__int_as_float(u[2].x), __int_as_float(u[2].z), __int_as_float(u[3].x), __int_as_float(u[3].z));
-                        vn = make_float4(__int_as_float(u[4].x), __int_as_float(u[4].z), __int_as_float(u[5].x), __int_as_float(u[5].z));
-                        if (__all(ok)) break;
+                        const bool got_m = cell_get(theirs, sb + 6u, cm);
+                        const bool got_l = cell_get(theirs + 1, sb + 6u, cl);
+                        const bool got_o = cell_get(theirs + 2 + lane, sb + 6u, co);
+                        if (__all(got_m && got_l && got_o)) break;
                         if (hopeless(spins)) {
-                            give_up(tag);
+                            give_up(sb + 6u);
                             break;
                         }
                     }
-                }
-                for (int tb = t0; tb < t1; tb += 32) {
-                    if (tb > t0) fetch(tb, k4, v4);
-                    float sc[8];
-#pragma unroll
-                    for (int it = 0; it < 8; it++) {
-                        const int tt = tb + it * 4 + sub;
-                        if (tt == pos) {
-                            k4[it] = kn;
-                            v4[it] = vn;
-                        }
-                        const float sdot = row16_sum(dot4(q4, k4[it]));
-                        sc[it] = tt < t1 ? sdot * 0.125f : -INFINITY;  // 1/sqrt(64)
-                    }
-                    float mb = sc[0];
-#pragma unroll
-                    for (int it = 1; it < 8; it++) mb = fmaxf(mb, sc[it]);
-                    mb = fmaxf(mb, dpp_move<0x142, 0xA>(mb, mb));
-                    mb = fmaxf(mb, dpp_move<0x143, 0xC>(mb, mb));
-                    mb = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mb), 63));
-                    const float mn = fmaxf(m, mb);
-                    float arg = sc[0];
-#pragma unroll
-                    for (int it = 1; it < 8; it++) arg = (dl == it) ? sc[it] : arg;
-                    arg = (dl == 8) ? m : arg;
-                    const float em = expf(arg - mn);
-                    const float f = row_lane<8>(em);
-                    lsum *= f;
-                    acc.x *= f;
-                    acc.y *= f;
-                    acc.z *= f;
-                    acc.w *= f;
-                    const float e[8] = {row_lane<0>(em), row_lane<1>(em), row_lane<2>(em), row_lane<3>(em),
-                                        row_lane<4>(em), row_lane<5>(em), row_lane<6>(em), row_lane<7>(em)};
-#pragma unroll
-                    for (int it = 0; it < 8; it++) {
-                        lsum += e[it];
-                        acc.x += e[it] * v4[it].x;
-                        acc.y += e[it] * v4[it].y;
-                        acc.z += e[it] * v4[it].z;
-                        acc.w += e[it] * v4[it].w;
-                    }
-                    m = mn;
-                }
-            }
-            lsum += __shfl_xor(lsum, 16, kWave);
-            lsum += __shfl_xor(lsum, 32, kWave);
-#pragma unroll
-            for (int o = 16; o < 64; o <<= 1) {
-                acc.x += __shfl_xor(acc.x, o, kWave);
-                acc.y += __shfl_xor(acc.y, o, kWave);
-                acc.z += __shfl_xor(acc.z, o, kWave);
-                acc.w += __shfl_xor(acc.w, o, kWave);
-            }
-            if (lane < 16) reinterpret_cast<float4*>(&part[l & 1][half][wv][4])[lane] = acc;
-            if (lane == 0) {
-                part[l & 1][half][wv][0] = m;
-                part[l & 1][half][wv][1] = lsum;
-            }
-            __syncthreads();
-            if (g_wait_abandoned) return;
-            if (live && wv == 0) {
-                float M = -INFINITY, L = 0.0f, o = 0.0f;
-                for (int q = 0; q < 4; q++) M = fmaxf(M, part[l & 1][half][q][0]);
-                for (int q = 0; q < 4; q++) {
-                    const float f = expf(part[l & 1][half][q][0] - M);
-                    L += part[l & 1][half][q][1] * f;
-                    o += part[l & 1][half][q][4 + lane] * f;
-                }
-                const auto publish = [&](float v) {  // two columns per store
-                    const float next = dpp_move<0xB1, 0xF>(v, 0.0f);
-                    if (!(lane & 1)) cell_put2(rs, c_at + operand_cell(h * HS + lane, seq, B), v, next, sb + 2u);
                 };
-                if (nchunk == 1) {
-                    publish(o * (1.0f / L));
-                } else if (ck > 0) {
-                    Cell* mine = p.cells + c_part + item * 66;
-                    cell_put(mine + 2 + lane, o, sb + 6u);
-                    if (lane == 0) {
-                        cell_put(mine, M, sb + 6u);
-                        cell_put(mine + 1, L, sb + 6u);
-                    }
-                } else {
-                    // the other runs of this context, folded in order (attn_merge)
-                    float all = M;
-                    float cm = 0.0f, cl = 0.0f, co = 0.0f;
-                    const auto look = [&](int c) {
-                        const Cell* theirs = p.cells + c_part + (item + c) * 66;
-                        unsigned spins = 0;
-                        for (;;) {
-                            const bool got_m = cell_get(theirs, sb + 6u, cm);
-                            const bool got_l = cell_get(theirs + 1, sb + 6u, cl);
-                            const bool got_o = cell_get(theirs + 2 + lane, sb + 6u, co);
-                            if (__all(got_m && got_l && got_o)) break;
-                            if (hopeless(spins)) {
-                                give_up(sb + 6u);
-                                break;
+                for (int c = 1; c < nchunk; c++) {
+                    look(c);
+                    all = fmaxf(all, cm);
+                }
+                float f = expf(M - all);
+                float Ls = 0.0f, os = 0.0f;
+                Ls += L * f;
+                os += o * f;
+                for (int c = 1; c < nchunk; c++) {
+                    look(c);
+                    f = expf(cm - all);
+                    Ls += cl * f;
+                    os += co * f;
+                }
+                publish(seq, h, os * (1.0f / Ls));
+            };
+            for (int round = 0; round < rounds; round++) {
+                const int item = order + (2 * round + half) * G;
+                const bool live = item < items;
+                const int pair = live ? item / nchunk : 0, ck = live ? item - pair * nchunk : 0;
+                const int seq = pair / H, h = pair - seq * H;
+                const int p0 = ck * p.chunk, p1 = min(ctx, p0 + p.chunk);
+                const int run = ((((p1 - p0) + 3) / 4) + 31) & ~31;
+                const int t0 = p0 + wv * run, t1 = min(p1, t0 + run);
+                const int* table = ptab + seq * p.kv.pages_per_seq;
+                const float* base = pool + h * head_stride;
+                float m = -INFINITY, lsum = 0.0f;
+                float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (live && t0 < t1) {
+                    float4 k4[8], v4[8];
+                    const auto fetch = [&](int tb) {
+                        const float* at = base + static_cast<size_t>(table[tb >> shift]) * 2 * kv_stride;
+#pragma unroll
+                        for (int it = 0; it < 8; it++) {
+                            const int tt = tb + it * 4 + sub;
+                            k4[it] = make_float4(0.f, 0.f, 0.f, 0.f);
+                            v4[it] = make_float4(0.f, 0.f, 0.f, 0.f);
+                            if (tt < t1 && tt < pos) {
+                                const float* row = at + static_cast<size_t>(tt & ((1 << shift) - 1)) * HS + dl * 4;
+                                k4[it] = *reinterpret_cast<const float4*>(row);
+                                v4[it] = *reinterpret_cast<const float4*>(row + kv_stride);
                             }
                         }
                     };
-                    for (int c = 1; c < nchunk; c++) {
-                        look(c);
-                        all = fmaxf(all, cm);
+                    const bool newest = t1 == ctx;
+                    float4 q4, kn, vn;
+                    const auto work = [&](int tb) {
+                        float sc[8];
+#pragma unroll
+                        for (int it = 0; it < 8; it++) {
+                            const int tt = tb + it * 4 + sub;
+                            if (tt == pos) {
+                                k4[it] = kn;
+                                v4[it] = vn;
+                            }
+                            const float sdot = row16_sum(dot4(q4, k4[it]));
+                            sc[it] = tt < t1 ? sdot * 0.125f : -INFINITY;  // 1/sqrt(64)
+                        }
+                        float mb = sc[0];
+#pragma unroll
+                        for (int it = 1; it < 8; it++) mb = fmaxf(mb, sc[it]);
+                        mb = fmaxf(mb, dpp_move<0x142, 0xA>(mb, mb));
+                        mb = fmaxf(mb, dpp_move<0x143, 0xC>(mb, mb));
+                        mb = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mb), 63));
+                        const float mn = fmaxf(m, mb);
+                        float arg = sc[0];
+#pragma unroll
+                        for (int it = 1; it < 8; it++) arg = (dl == it) ? sc[it] : arg;
+                        arg = (dl == 8) ? m : arg;
+                        const float em = expf(arg - mn);
+                        const float f = row_lane<8>(em);
+                        lsum *= f;
+                        acc.x *= f;
+                        acc.y *= f;
+                        acc.z *= f;
+                        acc.w *= f;
+                        const float e[8] = {row_lane<0>(em), row_lane<1>(em), row_lane<2>(em), row_lane<3>(em),
+                                            row_lane<4>(em), row_lane<5>(em), row_lane<6>(em), row_lane<7>(em)};
+#pragma unroll
+                        for (int it = 0; it < 8; it++) {
+                            lsum += e[it];
+                            acc.x += e[it] * v4[it].x;
+                            acc.y += e[it] * v4[it].y;
+                            acc.z += e[it] * v4[it].z;
+                            acc.w += e[it] * v4[it].w;
+                        }
+                        m = mn;
+                    };
+                    fetch(t0);  // in flight while q is on its way
+                    {
+                        const unsigned at = static_cast<unsigned>(seq * D + h * HS + dl * 4) * 8u;
+                        const unsigned tag = sb + 1u;
+                        unsigned spins = 0;
+                        for (;;) {
+                            v4i u[6];
+#pragma unroll
+                            for (int i = 0; i < 6; i++)
+                                u[i] = coherent_load16(rs, (i < 2 || newest) ? static_cast<unsigned>((c_q + (i >> 1) * D * B) * 8) + at + (i & 1) * 16 : kPastEnd);
+                            bool ok = true;
+#pragma unroll
+                            for (int i = 0; i < 6; i++)
+                                ok = ok && ((i >= 2 && !newest) || (u[i].y == static_cast<int>(tag) && u[i].w == static_cast<int>(tag)));
+                            q4 = make_float4(__int_as_float(u[0].x), __int_as_float(u[0].z), __int_as_float(u[1].x), __int_as_float(u[1].z));
+                            kn = make_float4(__int_as_float(u[2].x), __int_as_float(u[2].z), __int_as_float(u[3].x), __int_as_float(u[3].z));
+                            vn = make_float4(__int_as_float(u[4].x), __int_as_float(u[4].z), __int_as_float(u[5].x), __int_as_float(u[5].z));
+                            if (__all(ok)) break;
+                            if (hopeless(spins)) {
+                                give_up(tag);
+                                break;
+                            }
+                        }
                     }
-                    float f = expf(M - all);
-                    float Ls = 0.0f, os = 0.0f;
-                    Ls += L * f;
-                    os += o * f;
-                    for (int c = 1; c < nchunk; c++) {
-                        look(c);
-                        f = expf(cm - all);
-                        Ls += cl * f;
-                        os += co * f;
+                    for (int tb = t0; tb < t1; tb += 32) {
+                        if (tb > t0) fetch(tb);
+                        work(tb);
                     }
-                    publish(os * (1.0f / Ls));
                 }
+                lsum += __shfl_xor(lsum, 16, kWave);
+                lsum += __shfl_xor(lsum, 32, kWave);
+#pragma unroll
+                for (int o = 16; o < 64; o <<= 1) {
+                    acc.x += __shfl_xor(acc.x, o, kWave);
+                    acc.y += __shfl_xor(acc.y, o, kWave);
+                    acc.z += __shfl_xor(acc.z, o, kWave);
+                    acc.w += __shfl_xor(acc.w, o, kWave);
+                }
+                float(*mine)[68] = part[(l * rounds + round) & 1][half];
+                if (lane < 16) reinterpret_cast<float4*>(&mine[wv][4])[lane] = acc;
+                if (lane == 0) {
+                    mine[wv][0] = m;
+                    mine[wv][1] = lsum;
+                }
+                __syncthreads();
+                if (g_wait_abandoned) return;
+                if (live && wv == 0) {
+                    float M = -INFINITY, L = 0.0f, o = 0.0f;
+                    for (int q = 0; q < 4; q++) M = fmaxf(M, mine[q][0]);
+                    for (int q = 0; q < 4; q++) {
+                        const float f = expf(mine[q][0] - M);
+                        L += mine[q][1] * f;
+                        o += mine[q][4 + lane] * f;
+                    }
+                    if (nchunk == 1) {
+                        publish(seq, h, o * (1.0f / L));
+                    } else if (ck > 0) {
+                        Cell* out = p.cells + c_part + item * 66;
+                        cell_put(out + 2 + lane, o, sb + 6u);
+                        if (lane == 0) {
+                            cell_put(out, M, sb + 6u);
+                            cell_put(out + 1, L, sb + 6u);
+                        }
+                    } else if (ROUNDS) {
+                        held[round][half][2 + lane] = o;
+                        held[round][half][0] = M;
+                        held[round][half][1] = L;
+                    } else {
+                        fold(item, M, L, o);
+                    }
+                }
+                __syncthreads();  // nobody's loads go out in front of these stores
             }
-            __syncthreads();
+            if (ROUNDS && nchunk > 1) {
+                if (wv == 0) {
+                    for (int round = 0; round < rounds; round++) {
+                        const int item = order + (2 * round + half) * G;
+                        if (item < items && item % nchunk == 0)
+                            fold(item, held[round][half][0], held[round][half][1], held[round][half][2 + lane]);
+                    }
+                }
+                __syncthreads();
+            }
         }
 
         if (owner) {

@@ -4,17 +4,19 @@
 namespace gh {
 
 template <int KD, int KF, bool MODERN>
-static ResidentKernel of_rows(int batch) {
-    if (batch <= 4) return resident_layers_kernel<KD, KF, MODERN, 4>;
-    if (batch <= 8) return resident_layers_kernel<KD, KF, MODERN, 8>;
-    return batch <= kResidentRows ? resident_layers_kernel<KD, KF, MODERN, 16> : nullptr;
+static ResidentKernel of_rows(int batch, bool rounds) {
+    if (batch <= 4) return rounds ? nullptr : resident_layers_kernel<KD, KF, MODERN, 4, false>;
+    if (batch <= 8) return rounds ? resident_layers_kernel<KD, KF, MODERN, 8, true> : resident_layers_kernel<KD, KF, MODERN, 8, false>;
+    if (batch > kResidentRows) return nullptr;
+    return rounds ? resident_layers_kernel<KD, KF, MODERN, 16, true> : resident_layers_kernel<KD, KF, MODERN, 16, false>;
 }
 
-ResidentKernel resident_kernel_for(const Shape& sh, int batch) {
-    if (sh.head_size() != 64 || batch < 2) return nullptr;
-    if (sh.modern()) return sh.d_model == 768 && sh.d_ff() == 2048 ? of_rows<3, 8, true>(batch) : nullptr;
-    if (sh.d_model == 512) return of_rows<2, 8, false>(batch);
-    if (sh.d_model == 768) return of_rows<3, 12, false>(batch);
+ResidentKernel resident_kernel_for(const Shape& sh, int batch, int items) {
+    if (sh.head_size() != 64 || batch < 2 || items > kResidentItems) return nullptr;
+    const bool rounds = items > 2 * kResidentGrid;
+    if (sh.modern()) return sh.d_model == 768 && sh.d_ff() == 2048 ? of_rows<3, 8, true>(batch, rounds) : nullptr;
+    if (sh.d_model == 512) return of_rows<2, 8, false>(batch, rounds);
+    if (sh.d_model == 768) return of_rows<3, 12, false>(batch, rounds);
     return nullptr;
 }
 

@@ -59,6 +59,19 @@ def test_bits_of_a_launch_per_operation(models, name, batch):
     assert one.last_timing()["launches_per_step"] == RESIDENT[name]
 
 
+def test_more_runs_of_positions_than_halves_of_workgroups():
+    """8 x 12 heads in 6 runs each behind 2560 positions: the attention goes in two rounds, and the step
+    before it in one."""
+    cfg = synth.Config(synth.ARCH_MODERN, 90, 768, 1, 12, 2600)
+    W = synth.make_weights(cfg, 103, std=lively_std(cfg), norm_noise=0.1)
+    one, many = _both(G.Model.from_tensors(cfg, W), 8, shuffle_pages=True)
+    tokens = synth.uniform_tokens(8 * 2563, cfg.vocab, 104).reshape(8, -1)
+    for s in (one, many):
+        s.prefill(tokens[:, :2558])
+    for t in range(2558, 2563):
+        assert one.step(tokens[:, t]).tobytes() == many.step(tokens[:, t]).tobytes(), t
+
+
 @pytest.mark.parametrize("name", sorted(SHAPES))
 def test_steps_match_the_checker(models, name):
     cfg, W, gm = models[name]
