@@ -980,8 +980,9 @@ __global__ __launch_bounds__(kPersistThreads) void persist_decode_kernel(const P
 
             // ===== phase D: norm2 + FFN1 (SwiGLU or GELU) -> hidden cells
             {
-                if (!early_ffn1) load_ffn1();
+                if (KD != 2 && !early_ffn1) load_ffn1();
                 __syncthreads();  // every wave is done reading xs (phase C)
+                if (KD == 2 && !early_ffn1) load_ffn1();  // (see phase E)
                 if (!gather_cells((p.cells + D), D, tag_of(l, 2), xs, p)) return;
                 for (int item = first; item < NIT; ) {
                     float4 h[KD];
@@ -1008,6 +1009,12 @@ __global__ __launch_bounds__(kPersistThreads) void persist_decode_kernel(const P
                     }
                 }
             }
+            // A workgroup's outputs leave behind whatever its other wavefronts have asked for: nobody requests
+            // rows of the next phase before all have stored theirs.  Where that pays was found by trying it behind
+            // every phase (greedy tokens at positions 60..124, us): here, d768 GPT-2 117.5 -> 115.9, Llama block
+            // 108.3 -> 107.2, d512 67.9 -> 68.0; in front of the FFN1 rows, d512 67.9 -> 67.4, d768
+            // 117.0 -> 126.8, Llama block 108.5 -> 114.8; behind QKV 118.0, 112.0, 68.4.
+            if constexpr (KD == 3) __syncthreads();
             stamp();
 
             // ===== phase E: x += (b2 +) hidden @ W2 -> next layer's input cells
@@ -1021,6 +1028,9 @@ __global__ __launch_bounds__(kPersistThreads) void persist_decode_kernel(const P
 #pragma unroll
                     for (int i = 0; i < KF; i++) w0[i] = make_float4(0.f, 0.f, 0.f, 0.f);
                 }
+                // A first look that comes a little too early costs a whole round (none / 0.1 / 0.3 us of
+                // patience: Llama block 107.1 / 106.5 / 106.4, the others 115.9 / 115.9 / 116.9 and 67.8 / 67.9 / 68.8).
+                if constexpr (MODERN) __builtin_amdgcn_s_sleep(4);
                 if (!gather_cells((p.cells + 6 * D), F, tag_of(l, 3), vin, p)) return;
                 for (int row = first; row < D; ) {
                     const float a = dot_row_lds<KF>(w0, vin, lane);
