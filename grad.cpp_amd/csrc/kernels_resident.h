@@ -334,7 +334,6 @@ __global__ __launch_bounds__(kResidentThreads) void resident_layers_kernel(const
             multiply(a, b, acc);
             leave(0, 0, acc);
             __syncthreads();
-            if (g_wait_abandoned) return;
             if (e_live) {
                 float v0, v1;
                 sum_pair(0, 0, v0, v1);
@@ -527,7 +526,6 @@ __global__ __launch_bounds__(kResidentThreads) void resident_layers_kernel(const
                     mine[wv][1] = lsum;
                 }
                 __syncthreads();
-                if (g_wait_abandoned) return;
                 if (live && wv == 0) {
                     float M = -INFINITY, L = 0.0f, o = 0.0f;
                     for (int q = 0; q < 4; q++) M = fmaxf(M, mine[q][0]);
@@ -587,7 +585,6 @@ __global__ __launch_bounds__(kResidentThreads) void resident_layers_kernel(const
             multiply(a, b, acc);
             leave(1, 0, acc);
             __syncthreads();
-            if (g_wait_abandoned) return;
             if (e_live) {
                 float v0, v1;
                 sum_pair(1, 0, v0, v1);
@@ -614,7 +611,6 @@ __global__ __launch_bounds__(kResidentThreads) void resident_layers_kernel(const
             }
             leave(0, 0, acc);
             __syncthreads();
-            if (g_wait_abandoned) return;
             if (e_live) {
                 float v0, v1;
                 sum_pair(0, 0, v0, v1);
@@ -656,7 +652,6 @@ __global__ __launch_bounds__(kResidentThreads) void resident_layers_kernel(const
                 leave(1, 1, acc2);
             }
             __syncthreads();
-            if (g_wait_abandoned) return;
             if (e_live) {
                 float r = 1.0f;
                 if (MODERN) r = rms(1);
@@ -677,6 +672,9 @@ __global__ __launch_bounds__(kResidentThreads) void resident_layers_kernel(const
             }
             __syncthreads();
         }
+        // (once per layer, and not in front of a phase's stores: behind an abandoned wait the layer goes on with
+        // values that nobody will use)
+        if (g_wait_abandoned) return;
     }
 }
 
