@@ -1407,9 +1407,12 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
     if (s.engine < GH_ENGINE_AUTO || s.engine > GH_ENGINE_PERSISTENT)
         throw ApiError{GH_ERR_INVALID_ARGUMENT, "unknown engine"};
     const Shape& sh = m.shape;
-    const int page_tokens = o.page_tokens > 0 ? o.page_tokens : 64;
+    int page_tokens = o.page_tokens > 0 ? o.page_tokens : 64;
     if (page_tokens & (page_tokens - 1))
         throw ApiError{GH_ERR_INVALID_ARGUMENT, "page_tokens must be a power of two"};
+    // The persistent engine's offsets inside a layer's pages are 32 bits: at most 64 Ki positions in a
+    // page (its contexts, 4096 at most, are one such page; longer ones of other engines take more of them).
+    page_tokens = std::min(page_tokens, 1 << 16);
     s.page_shift = 0;
     while ((1 << s.page_shift) < page_tokens) s.page_shift++;
     s.pages_per_seq = (sh.max_len + page_tokens - 1) / page_tokens;

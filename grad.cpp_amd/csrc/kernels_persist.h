@@ -648,6 +648,29 @@ __global__ __launch_bounds__(kPersistThreads) void persist_decode_kernel(const P
             lane = tid & 63;
             first = wg + G * wave;
 
+            // A head's cached rows come from beyond the L2 (a token streams the weights through it), and from 256
+            // positions on some are asked for only when q is there, among everybody's FFN1 rows.  The
+            // workgroups 16, 32, ... places further on are on the same XCD: their wavefronts
+            // without an item of phase A touch the rows' 128-byte lines now (greedy tokens behind 300 / 397 /
+            // 600: Llama block 117.5 / 122.3 / 138.9 us without, 112.3 / 113.4 / 135.7 with; GPT-2 d768 128.6 /
+            // 133.4 / 145.5, 121.0 / 123.2 / 140.0).  Fewer rows are there in time (Llama behind 33 and 190: 1.5
+            // slower), and so are those of the 512 block, whose weights are fewer (900: 80.4, 87.1).
+            if (KD >= 3 && pos >= 256 && wg >= 16 && (wg & 15) < H && first >= NQKV) {
+                const int busy = (NQKV - wg + G - 1) / G, idle = kPersistWaves - busy;
+                const int lanes = ((G >> 4) - 1) * idle * 64;
+                float touched = 0.0f;
+                const char* k_rows = reinterpret_cast<const char*>(
+                    p.kv.pool + ((static_cast<size_t>(l) * p.kv.n_pages * 2 * H + (wg & 15)) << p.kv.page_shift) * HS);
+                const char* v_rows = k_rows + (static_cast<size_t>(H) << p.kv.page_shift) * (HS * 4);
+                for (int u = (((wg >> 4) - 1) * idle + wave - busy) * 64 + lane; u < pos * 2; u += lanes) {
+                    const int tt = u >> 1, slot = tt & ((1 << p.kv.page_shift) - 1);
+                    const unsigned row = (static_cast<unsigned>(ptab[tt >> p.kv.page_shift] * 2 * H) << p.kv.page_shift) + slot;
+                    const unsigned at = row * (HS * 4u) + (u & 1) * 128u;
+                    touched += *reinterpret_cast<const float*>(k_rows + at) + *reinterpret_cast<const float*>(v_rows + at);
+                }
+                asm volatile("" ::"v"(touched));
+            }
+
             // ===== phase A: norm1 + QKV (+bias, RoPE) -> q / new k / new v cells and the cache
             for (int item = first; item < NQKV; ) {
                 const int row = 2 * item;
@@ -707,20 +730,35 @@ __global__ __launch_bounds__(kPersistThreads) void persist_decode_kernel(const P
                 Cell* share_cells = p.cells + ((6 * D + F + 2 + 9 * G + 2) & ~1);  // [H][15][66]
                 // Cached rows do not depend on this step's q: the first 32 positions of
                 // the run are fetched before waiting for q (all of it for contexts <= 256).
-                const float* pool = p.kv.pool;
+                // Without a branch: pages first, all eight reads of the table under one wait, and
+                // rows outside the run read zero from beyond the buffer's end.  Under a condition each, the
+                // eight pages were eight round trips of LDS, and the eight scores (below) eight
+                // chains one after the other: greedy tokens behind 397 positions took 126.8 us (Llama), 138.5
+                // (GPT-2 d768) and 79.6 (d512), without conditions 122.0, 132.7 and 73.8.
+                const float* k_rows = p.kv.pool + ((static_cast<size_t>(l) * p.kv.n_pages * 2 * H + hd) << p.kv.page_shift) * HS;
+                constexpr unsigned kNoRow = 0x80000000u;
+                const __amdgpu_buffer_rsrc_t rs_k = make_buffer(k_rows, kNoRow);
+                const unsigned v_at = (static_cast<unsigned>(H) << p.kv.page_shift) * (HS * 4u);
                 float4 k4[8], v4[8];
+                const auto fetch = [&](int batch) {
+                    int page[8];
+                    const int end = min(pos, hi);
 #pragma unroll
-                for (int it = 0; it < 8; it++) {
-                    const int tt = t0 + it * 4 + sub;
-                    k4[it] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    v4[it] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (it * 4 < chunk && tt < min(pos, hi)) {
-                        const unsigned ko = static_cast<unsigned>(kv_at(l, 0, hd, tt)) + dl * 4;
-                        const unsigned vo = static_cast<unsigned>(kv_at(l, 1, hd, tt)) + dl * 4;
-                        k4[it] = *reinterpret_cast<const float4*>(pool + ko);
-                        v4[it] = *reinterpret_cast<const float4*>(pool + vo);
+                    for (int it = 0; it < 8; it++)
+                        page[it] = ptab[min(t0 + batch * 32 + it * 4 + sub, pos) >> p.kv.page_shift];
+#pragma unroll
+                    for (int it = 0; it < 8; it++) {
+                        const int rel = batch * 32 + it * 4, tt = t0 + rel + sub;
+                        const int slot = tt & ((1 << p.kv.page_shift) - 1);
+                        const unsigned row = (static_cast<unsigned>(page[it] * 2 * H) << p.kv.page_shift) + slot;
+                        const unsigned at = (rel < chunk && tt < end) ? row * (HS * 4u) + dl * 16u : kNoRow;
+                        const v4i a = __builtin_amdgcn_raw_buffer_load_b128(rs_k, at, 0, 0);
+                        const v4i b = __builtin_amdgcn_raw_buffer_load_b128(rs_k, at, v_at, 0);
+                        k4[it] = make_float4(__int_as_float(a.x), __int_as_float(a.y), __int_as_float(a.z), __int_as_float(a.w));
+                        v4[it] = make_float4(__int_as_float(b.x), __int_as_float(b.y), __int_as_float(b.z), __int_as_float(b.w));
                     }
-                }
+                };
+                fetch(0);
                 // q, new key, new value of this head: one wait for all three (a workgroup with
                 // a share of older positions needs q alone)
                 {
@@ -751,32 +789,24 @@ __global__ __launch_bounds__(kPersistThreads) void persist_decode_kernel(const P
                 float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
                 // Batches of 8 iterations (32 positions); softmax state is merged online.
                 for (int batch = 0; batch * 32 < chunk; batch++) {
-                    if (batch >= 1) {
+                    if (batch >= 1) fetch(batch);
+                    // the new position, where this batch holds it
+                    const int at_pos = pos - t0 - batch * 32;
+                    if (pos < hi && at_pos >= 0 && at_pos < 32 && batch * 32 + at_pos < chunk) {
+                        const float4 kn = reinterpret_cast<const float4*>(qkv + 64)[dl], vn = reinterpret_cast<const float4*>(qkv + 128)[dl];
 #pragma unroll
-                        for (int it = 0; it < 8; it++) {
-                            const int tt = t0 + batch * 32 + it * 4 + sub;
-                            k4[it] = make_float4(0.f, 0.f, 0.f, 0.f);
-                            v4[it] = make_float4(0.f, 0.f, 0.f, 0.f);
-                            if (batch * 32 + it * 4 < chunk && tt < min(pos, hi)) {
-                                const unsigned ko = static_cast<unsigned>(kv_at(l, 0, hd, tt)) + dl * 4;
-                                const unsigned vo = static_cast<unsigned>(kv_at(l, 1, hd, tt)) + dl * 4;
-                                k4[it] = *reinterpret_cast<const float4*>(pool + ko);
-                                v4[it] = *reinterpret_cast<const float4*>(pool + vo);
+                        for (int it = 0; it < 8; it++)
+                            if (it * 4 + sub == at_pos) {
+                                k4[it] = kn;
+                                v4[it] = vn;
                             }
-                        }
                     }
                     float sc[8];
 #pragma unroll
                     for (int it = 0; it < 8; it++) {
                         const int rel = batch * 32 + it * 4 + sub;
-                        const int tt = t0 + rel;
-                        const bool in_run = rel < chunk;
-                        if (in_run && tt == pos) {
-                            k4[it] = reinterpret_cast<const float4*>(qkv + 64)[dl];
-                            v4[it] = reinterpret_cast<const float4*>(qkv + 128)[dl];
-                        }
                         const float sdot = row16_sum(dot4(q4, k4[it]));
-                        sc[it] = (in_run && tt < hi) ? sdot * 0.125f : -INFINITY;  // 1/sqrt(64)
+                        sc[it] = (rel < chunk && t0 + rel < hi) ? sdot * 0.125f : -INFINITY;  // 1/sqrt(64)
                     }
                     float mb = sc[0];
 #pragma unroll
@@ -866,7 +896,7 @@ __global__ __launch_bounds__(kPersistThreads) void persist_decode_kernel(const P
                 } else if (n_shares > 1) {
                     // the other shares, then the fold in share order with this one last
                     __syncthreads();  // part[] is read; it takes the shares now
-                    if (!gather_cells(share_cells + hd * (kAttnMaxShares - 1) * 66, (n_shares - 1) * 66, tag_of(l, 5), part, p)) return;
+                    gather_in_layer(share_cells + hd * (kAttnMaxShares - 1) * 66, (n_shares - 1) * 66, tag_of(l, 5), part, p);
                     if (tid < HS) {
                         float Mall = M;
                         for (int j = 0; j < n_shares - 1; j++) Mall = fmaxf(Mall, part[j * 66]);
