@@ -90,6 +90,7 @@ __global__ __launch_bounds__(kResidentThreads) void resident_layers_kernel(const
     constexpr int G = kResidentGrid, NO = G - TO;
     constexpr int LDX = D + 4;
     static_assert(TO + TQ <= G && T1 <= 2 * NO, "every phase in one round");
+    static_assert(TO % 8 == 0 && TQ % 8 == 0 && G % 8 == 0, "an item's XCD is its number modulo 8");
     __shared__ float red[2][2][KW][256];  // [phase parity][tile][wavefront][row * 16 + column]
     __shared__ float ssq[2][KW][16];
     __shared__ float part[2][2][4][68];  // [parity of the round][half]: as in attn_decode64_kernel
@@ -409,14 +410,51 @@ __global__ __launch_bounds__(kResidentThreads) void resident_layers_kernel(const
                 }
                 publish(seq, h, os * (1.0f / Ls));
             };
+            // this wavefront's positions [t0, t1) of an item, and where its rows are
+            const auto run_of = [&](int item, int& seq, int& h, int& ck, int& t0, int& t1) {
+                const int pair = item / nchunk;
+                ck = item - pair * nchunk;
+                seq = pair / H;
+                h = pair - seq * H;
+                const int p0 = ck * p.chunk, p1 = min(ctx, p0 + p.chunk);
+                const int run = ((((p1 - p0) + 3) / 4) + 31) & ~31;
+                t0 = p0 + wv * run;
+                t1 = min(p1, t0 + run);
+            };
+            // Brings rows [from, t1) of a run into this XCD's L2: lane i its 128-byte line of 64.
+            const auto touch = [&](int seq, int h, int from, int t1) {
+                float v = 0.0f;
+                for (int tb = from; tb < t1; tb += 32) {
+                    const float* at = pool + h * head_stride + static_cast<size_t>(ptab[seq * p.kv.pages_per_seq + (tb >> shift)]) * 2 * kv_stride
+                                      + static_cast<size_t>(tb & ((1 << shift) - 1)) * HS + lane * 32;
+                    if (tb + (lane >> 1) < min(t1, pos)) v += at[0] + at[kv_stride];
+                }
+                return v;
+            };
+            // Rows that come from beyond the L2 only when q is there are most of what a context costs.  The
+            // workgroups without a tile of QKV have that phase to spare: they touch the rows of their own
+            // runs beyond the first 32, and where their second half has no item, it touches those of the
+            // workgroups with a tile (an item's XCD is that of its number modulo 8, TO and TQ being multiples
+            // of 8).  That pays while all rows of an XCD fit its 4 MB of L2 beside the weights passing through,
+            // and from 64 positions on.  us per step, before and after, Llama block: 2 sequences behind 300 159 -> 152,
+            // 4 182 -> 170, 8 210 -> 184, 13 226 -> 213; 13 behind 130 198 -> 189; GPT-2 8 behind 300
+            // 232 -> 210.  Without the limits: 8 behind 600 238 -> 261, GPT-2 16 behind 30 202 -> 207.
+            const bool spare = wg >= TO + TQ;
+            constexpr int kTouchPositions = 53248;  // of all heads: 3.25 MB of rows per XCD
+            if (spare && half == 1 && order + G >= items && ctx > 64 && B * H * ctx <= kTouchPositions) {
+                float touched = 0.0f;
+                for (int item = order + (G - TO - TQ); item < min(items, G); item += G - TO - TQ) {
+                    int seq, h, ck, t0, t1;
+                    run_of(item, seq, h, ck, t0, t1);
+                    touched += touch(seq, h, t0, t1);
+                }
+                asm volatile("" ::"v"(touched));
+            }
             for (int round = 0; round < rounds; round++) {
                 const int item = order + (2 * round + half) * G;
                 const bool live = item < items;
-                const int pair = live ? item / nchunk : 0, ck = live ? item - pair * nchunk : 0;
-                const int seq = pair / H, h = pair - seq * H;
-                const int p0 = ck * p.chunk, p1 = min(ctx, p0 + p.chunk);
-                const int run = ((((p1 - p0) + 3) / 4) + 31) & ~31;
-                const int t0 = p0 + wv * run, t1 = min(p1, t0 + run);
+                int seq, h, ck, t0, t1;
+                run_of(live ? item : 0, seq, h, ck, t0, t1);
                 const int* table = ptab + seq * p.kv.pages_per_seq;
                 const float* base = pool + h * head_stride;
                 float m = -INFINITY, lsum = 0.0f;
@@ -489,6 +527,7 @@ __global__ __launch_bounds__(kResidentThreads) void resident_layers_kernel(const
                         m = mn;
                     };
                     fetch(t0);  // in flight while q is on its way
+                    const float touched = spare && round == 0 ? touch(seq, h, t0 + 32, t1) : 0.0f;
                     {
                         const unsigned at = static_cast<unsigned>(seq * D + h * HS + dl * 4) * 8u;
                         const unsigned tag = sb + 1u;
@@ -512,6 +551,7 @@ __global__ __launch_bounds__(kResidentThreads) void resident_layers_kernel(const
                             }
                         }
                     }
+                    asm volatile("" ::"v"(touched));
                     for (int tb = t0; tb < t1; tb += 32) {
                         if (tb > t0) fetch(tb);
                         work(tb);
