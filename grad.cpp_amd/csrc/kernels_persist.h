@@ -441,7 +441,8 @@ __global__ __launch_bounds__(kPersistThreads) void persist_decode_kernel(const P
     constexpr int RL = 8;  // logits rows per wavefront item
     // Beyond kAttnShareFrom positions a head's attention is shared by several workgroups,
     // kAttnShare positions each: what a workgroup's eight wavefronts take in one batch of 32.
-    // (One workgroup up to 512 positions: 256..512 ran at 132 us per token alone and 138 in two shares.)
+    // (One workgroup up to 512 positions: 256..512 ran at 132 us per token alone and 138 in two shares, before
+    // the attention lost its conditions; alone it is 113 now.)
     constexpr int kAttnShareFrom = 512, kAttnShare = 256, kAttnMaxShares = 16;
     float* xs = lds;                      // [D] residual stream of this step
     float* vin = lds + D;                 // [max(D, F)] attention output / FFN hidden

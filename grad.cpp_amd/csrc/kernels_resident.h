@@ -18,9 +18,9 @@
 // instructions on eight wavefronts.  One layer of the Llama block d768, 4 sequences behind 64 positions: QKV 3.1 us (1.1
 // of it until the rows are there), attention 2.4, W_o 2.5, FFN1 4.1, FFN2 4.7 (1.7 of it products, 16-row tiles for
 // 4 rows; 128 KB of weights through one compute unit).  Per step, launches -> this, context 200: Llama
-// block 2 sequences 246 us -> 152, 4 254 -> 167, 8 258 -> 193, 16 279 -> 204; GPT-2 block d768 2 sequences
-// 286 -> 175, 16 323 -> 241; Llama block, 16 sequences behind 1900 positions 524 -> 460, 190 MB of cache per
-// layer in some 39 us of its 54.
+// block 2 sequences 246 us -> 144, 4 253 -> 157, 8 259 -> 173, 16 290 -> 188; GPT-2 block d768 2 sequences
+// 286 -> 167, 16 323 -> 222; Llama block, 16 sequences behind 1900 positions 522 -> 444, 190 MB of cache per
+// layer in some 37 us of its 52.
 //
 // The order things are sent in is most of the design.  A wavefront's loads return in the order they
 // went out, and a workgroup's stores leave behind what its other wavefronts have asked for: weights are
