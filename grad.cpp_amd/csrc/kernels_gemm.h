@@ -365,7 +365,7 @@ inline void launch_gemm16_as(const GemvParams& p, int M, hipStream_t st) {
             dim3(64 * KW), 0, st, p, M, m_groups);
 }
 
-// Weight tiles per workgroup of the wide kernel: 16000 rows = 250 workgroups.
+// Weight tiles in flight per workgroup of the wide kernel: 16000 rows = 250 workgroups.
 constexpr int kWideTiles = 4;
 
 // Wide projections of a few rows (the tied logits of a decode step: N = vocab,
@@ -374,11 +374,14 @@ constexpr int kWideTiles = 4;
 // times the weights.  Here A is stationary: K is split over the 8 wavefronts of
 // a workgroup, each keeps its K / 8 slice of all M rows in registers in the MFMA
 // operand layout (RMSNorm gain already applied), and the workgroup walks
-// kWideTiles consecutive 16-row weight tiles, all requested at the start, so
-// every weight row crosses the chip once and A once per four tiles.
+// consecutive 16-row weight tiles, kWideTiles of them in flight from the start, so
+// every weight row crosses the chip once and A once per workgroup.
 // KS = K / 128 K-steps of 16 per wavefront; MT 16-row tiles of A.
-template <bool RMS, int MT, int KS>
-__global__ __launch_bounds__(512) void gemm_wide_kernel(const GemvParams p, int M) {
+// LOOP: `each` tiles per workgroup, a tile's registers asked for the tile kWideTiles on as soon as they are
+// used, so that a matrix of more than kWideTiles tiles per compute unit is one stream and not several rounds
+// of workgroups, each with a start, its rows of A and an empty memory system in front of it.
+template <bool RMS, int MT, int KS, bool LOOP>
+__global__ __launch_bounds__(512) void gemm_wide_kernel(const GemvParams p, int M, int each) {
     constexpr int KW = 8, NTILE = kWideTiles;
     __shared__ float red[KW][MT][16 * 16];
     __shared__ float ssq[KW][MT][16];
@@ -396,8 +399,8 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const GemvParams p, int 
             __int_as_float(__builtin_amdgcn_ds_bpermute(from_lane, __float_as_int(v.w))));
     };
     const int n_tiles = (p.N + 15) >> 4;
-    const int tile0 = blockIdx.x * NTILE;
-    const int tile_end = min(tile0 + NTILE, n_tiles);
+    const int tile0 = blockIdx.x * (LOOP ? each : NTILE);
+    const int tile_end = min(tile0 + (LOOP ? each : NTILE), n_tiles);
     if (tile0 >= n_tiles) return;
     // Weights and outputs go through bounded buffer descriptors: an access past the
     // end reads zero / is dropped, so no load or store of the tile loop sits under
@@ -479,13 +482,12 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const GemvParams p, int 
     const int em = et * 16 + ei;
     const bool e_live = e < MT * 128 && em < M;
 
-    // Straight-line code over the tiles: no loop carries loads across a back edge,
-    // so every wait names exactly the tile it needs.  Tiles past the end were read
+    // Straight-line code over the tiles in flight: every wait names exactly the tile it needs.  Tiles past the end were read
     // as zeros and their stores are dropped.
-    {
+    for (int first = tile0; first < tile_end; first += NTILE) {
 #pragma unroll
         for (int f = 0; f < NTILE; f++) {
-            const int tile = tile0 + f;
+            const int tile = first + f;
             v4f acc[MT];
 #pragma unroll
             for (int t = 0; t < MT; t++) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -500,6 +502,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const GemvParams p, int 
                     acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(as[t][s].w, b.w, acc[t], 0, 0, 0);
                 }
             }
+            if (LOOP) fetch_tile(tile + NTILE, wf[f]);
 #pragma unroll
             for (int t = 0; t < MT; t++)
 #pragma unroll
@@ -520,9 +523,9 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const GemvParams p, int 
                     v1 *= r;
                 }
                 const unsigned o = (static_cast<unsigned>(em) * p.out_stride + n) * 4u;
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v0), rs_o, e_live && n < p.N ? o : kPastEnd, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v0), rs_o, e_live && tile < tile_end && n < p.N ? o : kPastEnd, 0, 0);
                 __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v1), rs_o,
-                                                      e_live && n + 1 < p.N ? o + 4u : kPastEnd, 0, 0);
+                                                      e_live && tile < tile_end && n + 1 < p.N ? o + 4u : kPastEnd, 0, 0);
                 if (p.best) {
                     // eight neighbouring lanes hold the tile's 16 columns of one row, in column order
                     const bool has1 = n + 1 < p.N;
@@ -531,12 +534,13 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const GemvParams p, int 
                     first_max_step<0xB1, 0xF>(bv, bn);
                     first_max_step<0x4E, 0xF>(bv, bn);
                     first_max_step<0x141, 0xF>(bv, bn);
-                    if ((e & 7) == 0 && e_live && n < p.N)
+                    if ((e & 7) == 0 && e_live && tile < tile_end && n < p.N)
                         p.best[static_cast<size_t>(em) * p.best_stride + tile] = make_float2(bv, __int_as_float(bn));
                 }
             }
             __syncthreads();  // red is rewritten by the next tile
         }
+        if (!LOOP) break;
     }
     // the launch that makes the logits also ends the step (inference.cpp:256)
     if (p.advance && blockIdx.x == 0 && threadIdx.x == 0) p.advance->pos += 1;
@@ -554,10 +558,24 @@ inline bool gemm_wide_ok(const GemvParams& p, int M) {
     return ks == 4 || ks == 6 || ks == 8;
 }
 
+// The loop where a compute unit holds one workgroup of the other form (more than 128 registers: RMSNorm's gains or
+// a second tile of rows): Llama block, a step of 13 sequences with 32000 / 50257 outputs 196.6 -> 192.4 /
+// 218.4 -> 209.2 us, of 32 320 -> 312 / 350 -> 332; GPT-2 d768, 32 sequences 355 -> 352 / 380 -> 369.  Where two fit, the
+// second one's loads already fill the gaps of the first (GPT-2 d768, 13 sequences: 224.7 against 227.2 in the
+// loop), and two row tiles of 1024 columns would spill.
+template <bool RMS, int MT, int KS>
+inline constexpr bool kWideLoops = KS == 6 ? RMS || MT == 2 : KS == 8 && MT == 1;
+
 template <bool RMS, int MT, int KS>
 inline void launch_gemm_wide_as(const GemvParams& p, int M, hipStream_t st) {
-    const int n_tiles = (p.N + 15) / 16;
-    enqueue(gemm_wide_kernel<RMS, MT, KS>, dim3((n_tiles + kWideTiles - 1) / kWideTiles), dim3(512), 0, st, p, M);
+    const int n_tiles = (p.N + 15) / 16, each = (n_tiles + 255) / 256;
+    if constexpr (kWideLoops<RMS, MT, KS>) {
+        if (each > kWideTiles) {
+            enqueue(gemm_wide_kernel<RMS, MT, KS, true>, dim3((n_tiles + each - 1) / each), dim3(512), 0, st, p, M, each);
+            return;
+        }
+    }
+    enqueue(gemm_wide_kernel<RMS, MT, KS, false>, dim3((n_tiles + kWideTiles - 1) / kWideTiles), dim3(512), 0, st, p, M, kWideTiles);
 }
 
 template <bool RMS, int MT>
