@@ -316,31 +316,56 @@ static __global__ __launch_bounds__(256, 2) void attn_split_kernel(const SplitAt
                          o[db][4 * q4 + 1] * inv, o[db][4 * q4 + 2] * inv, o[db][4 * q4 + 3] * inv);
 }
 
-// Folds the partial results of a query block, in the order of the keys.
+// Folds the partial results of a query block, in the order of the keys.  A chain of trips to memory, one per
+// part (a part's rows were written by another workgroup): so a workgroup takes 32 queries only and a wavefront 8 of
+// their 32 registers, and kMergeAhead parts are requested together.  12 heads x 1999 queries in up to 8 parts: 12.7 us ->
+// 9.3 (4 TB/s), against four times the queries per workgroup, 32 registers per wavefront and a part at a time.
+constexpr int kMergeAhead = 4;
+
 static __global__ __launch_bounds__(256) void attn_split_merge_kernel(const SplitAttnParams p) {
     const int pair = p.first + blockIdx.y, b = pair / p.heads, h = pair - b * p.heads;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h32 = lane >> 5;
-    const int qb = (p.len + kAttnQueries - 1) / kAttnQueries - 1 - static_cast<int>(blockIdx.x);
+    const int lane = threadIdx.x & 63, h32 = lane >> 5;
+    const int r0 = (threadIdx.x >> 6) * 8, rows = blockIdx.x & 3;  // this wavefront's registers, the workgroup's 32 queries
+    const int qb = (p.len + kAttnQueries - 1) / kAttnQueries - 1 - static_cast<int>(blockIdx.x >> 2);
     int first = 0;
     for (int i = qb + 1; i * kAttnQueries < p.len; i++) first += attn_parts(i, p.len, p.pos_base, p.chunk_shift);
-    const int parts = attn_parts(qb, p.len, p.pos_base, p.chunk_shift), t = qb * kAttnQueries + wave * 32 + (lane & 31);
+    const int parts = attn_parts(qb, p.len, p.pos_base, p.chunk_shift), t = qb * kAttnQueries + rows * 32 + (lane & 31);
     if (parts == 1 || t >= p.len) return;
-    const float* part = p.part + (static_cast<size_t>(blockIdx.y) * p.items + first) * kAttnPart + wave * (34 * 64) + lane;
-    float m = -INFINITY, l = 0.0f, o[32];
-    for (int c = 0; c < parts; c++) m = fmaxf(m, part[static_cast<size_t>(c) * kAttnPart]);
+    const float* part = p.part + (static_cast<size_t>(blockIdx.y) * p.items + first) * kAttnPart + rows * (34 * 64) + lane;
+    const auto at = [&](int c) { return part + static_cast<size_t>(min(c, parts - 1)) * kAttnPart; };
+    float m = -INFINITY, l = 0.0f, o[8];
+    for (int c = 0; c < parts; c += 2 * kMergeAhead) {
+        float v[2 * kMergeAhead];
 #pragma unroll
-    for (int r = 0; r < 32; r++) o[r] = 0.0f;
-    for (int c = 0; c < parts; c++) {
-        const float* at = part + static_cast<size_t>(c) * kAttnPart;
-        const float f = __builtin_amdgcn_exp2f(at[0] - m);
-        l += at[64] * f;
+        for (int i = 0; i < 2 * kMergeAhead; i++) v[i] = at(c + i)[0];
 #pragma unroll
-        for (int r = 0; r < 32; r++) o[r] += at[(2 + r) * 64] * f;
+        for (int i = 0; i < 2 * kMergeAhead; i++) m = fmaxf(m, v[i]);
+    }
+#pragma unroll
+    for (int r = 0; r < 8; r++) o[r] = 0.0f;
+    for (int c = 0; c < parts; c += kMergeAhead) {
+        float v[kMergeAhead][10];
+#pragma unroll
+        for (int i = 0; i < kMergeAhead; i++) {
+            v[i][8] = at(c + i)[0];
+            v[i][9] = at(c + i)[64];
+#pragma unroll
+            for (int r = 0; r < 8; r++) v[i][r] = at(c + i)[(2 + r0 + r) * 64];
+        }
+#pragma unroll
+        for (int i = 0; i < kMergeAhead; i++) {
+            if (c + i < parts) {
+                const float f = __builtin_amdgcn_exp2f(v[i][8] - m);
+                l += v[i][9] * f;
+#pragma unroll
+                for (int r = 0; r < 8; r++) o[r] += v[i][r] * f;
+            }
+        }
     }
     const float inv = 1.0f / l;
 #pragma unroll
-    for (int q = 0; q < 8; q++)
-        store_split4(p.out, b * p.len + t, h * 64 + q * 8 + h32 * 4, p.d_model / kSplitCols, o[4 * q] * inv, o[4 * q + 1] * inv,
+    for (int q = 0; q < 2; q++)
+        store_split4(p.out, b * p.len + t, h * 64 + r0 * 2 + q * 8 + h32 * 4, p.d_model / kSplitCols, o[4 * q] * inv, o[4 * q + 1] * inv,
                      o[4 * q + 2] * inv, o[4 * q + 3] * inv);
 }
 

@@ -99,7 +99,8 @@ void split_gemm(SplitGemmParams& p, hipStream_t st) {
 // all their keys) while there are enough of them or the longest has six tiles at most (8
 // sequences of 256 tokens: 18 us, shared 18 and 8 for the merge); below 640 workgroups the keys of the
 // long blocks are shared, as coarsely as reaches 640 and so among 1300 or so at most (12 heads of 1999 tokens: 89 us unshared, 76 in runs of
-// 1024 keys, 47 of 512, 46 of 256, 48 of 128; the merge costs 1, 6, 8, 12, 18 us more).
+// 1024 keys, 47 of 512, 46 of 256, 48 of 128; the merge cost 1, 6, 8, 12, 18 us more, that of
+// 256 keys costs 9 since its loads go out together).
 static int attn_chunk_shift(int pairs, int len, int pos_base) {
     const int blocks = (len + kAttnQueries - 1) / kAttnQueries;
     int shift = 20;
@@ -171,7 +172,7 @@ void split_attention(const PrefillAttnParams& a, int batch, char* kv, size_t kv_
         hipLaunchKernelGGL(attn_split_kernel, dim3((p.pairs + 7) / 8 * 8 * p.items), dim3(256), kAttnLds, st, p);
         check(hipGetLastError(), "attn_split");
         if (p.items > blocks) {
-            hipLaunchKernelGGL(attn_split_merge_kernel, dim3(blocks, p.pairs), dim3(256), 0, st, p);
+            hipLaunchKernelGGL(attn_split_merge_kernel, dim3(4 * blocks, p.pairs), dim3(256), 0, st, p);
             check(hipGetLastError(), "attn_split_merge");
         }
     }
