@@ -73,7 +73,7 @@ def test_more_runs_of_positions_than_halves_of_workgroups():
 
 
 @pytest.mark.parametrize("name", sorted(SHAPES))
-def test_steps_match_the_checker(models, name):
+def test_steps_match_the_oracle(models, name):
     cfg, W, gm = models[name]
     s = G.Session(gm, batch=3)
     tokens = synth.uniform_tokens(18, cfg.vocab, 104).reshape(3, 6)
