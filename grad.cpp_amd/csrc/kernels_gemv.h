@@ -28,7 +28,8 @@ enum Epilogue { EPI_STORE = 0, EPI_QKV = 1, EPI_RESID = 2, EPI_GELU = 3, EPI_SWI
 // sequences at context 2048 516.0 -> 509.5 (the same touches dealt to the workgroups
 // without regard to the XCD, which only fills the memory-side cache: 516.1 -> 513.3).  At 64
 // sequences the launches that carry the touches lose more than the next ones gain, so the
-// engine asks for it up to 48.  blocks == 0: nothing to do.
+// engine asks for it up to 48 (of 2 to 16 sequences, the steps that the resident kernel does not run).
+// blocks == 0: nothing to do.
 struct NextWeights {
     const float* base;
     int chunk_lines;
