@@ -132,10 +132,11 @@ __device__ __forceinline__ void cell_put(Cell* c, float v, unsigned tag) {
 }
 
 // Two cells that follow each other, the first on a boundary of 16 bytes: one store (each cell's value and tag
-// still travel together).
-__device__ __forceinline__ void cell_put_pair(Cell* c, float v0, float v1, unsigned tag) {
+// still travel together).  Through the builtin: a store of 16 bytes needs two wait states in front of whatever
+// next writes its registers, and behind one in inline assembly the compiler leaves none.
+__device__ __forceinline__ void cell_put2(__amdgpu_buffer_rsrc_t rs, int cell, float v0, float v1, unsigned tag) {
     const v4i w = {__float_as_int(v0), static_cast<int>(tag), __float_as_int(v1), static_cast<int>(tag)};
-    asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(c), "v"(w) : "memory");
+    __builtin_amdgcn_raw_buffer_store_b128(w, rs, cell * 8, 0, kAuxDeviceScope);
 }
 
 __device__ __forceinline__ bool cell_get(const Cell* c, unsigned tag, float& v) {
@@ -483,6 +484,9 @@ __global__ __launch_bounds__(kPersistThreads) void persist_decode_kernel(const P
         return ((run << p.kv.page_shift) + slot) * HS;
     };
 
+    // the cells a layer's phases hand on
+    const auto layer_cells = [&] { return make_buffer(p.cells, (6u * D + F) * sizeof(Cell)); };
+
     constexpr int NQKV = 3 * D / 2;  // phase A items: pairs of rows
     const bool has_qkv = wg + G * wave < NQKV;
 
@@ -689,9 +693,9 @@ __global__ __launch_bounds__(kPersistThreads) void persist_decode_kernel(const P
                     }
                     const unsigned t = tag_of(l, 0);
                     if (sec == 0) {
-                        cell_put_pair(p.cells + 2 * D + col, a, c, t);
+                        cell_put2(layer_cells(), 2 * D + col, a, c, t);
                     } else {
-                        cell_put_pair((sec == 1 ? (p.cells + 3 * D) : (p.cells + 4 * D)) + col, a, c, t);
+                        cell_put2(layer_cells(), (sec == 1 ? 3 * D : 4 * D) + col, a, c, t);
                         const int head = col / HS, jj = col - head * HS;
                         float* cr = p.kv.pool + kv_at(l, sec - 1, head, pos) + jj;
                         coherent_store(cr, a);
@@ -1058,7 +1062,7 @@ __global__ __launch_bounds__(kPersistThreads) void persist_decode_kernel(const P
                         if (MODERN) {
                             cell_put((p.cells + 6 * D) + item, c * silu(a), t);
                         } else {
-                            cell_put_pair(p.cells + 6 * D + 2 * item, gelu_tanh(a + fb0), gelu_tanh(c + fb1), t);
+                            cell_put2(layer_cells(), 6 * D + 2 * item, gelu_tanh(a + fb0), gelu_tanh(c + fb1), t);
                         }
                     }
                     item += stride;

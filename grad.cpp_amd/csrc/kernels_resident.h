@@ -71,11 +71,6 @@ __device__ __forceinline__ int operand_cell(int k, int r, int rows) {
     return ((((k >> 4) * 2 + ((k >> 1) & 1)) * 4 + ((k >> 2) & 3)) * rows + r) * 2 + (k & 1);
 }
 
-__device__ __forceinline__ void cell_put2(__amdgpu_buffer_rsrc_t rs, int cell, float v0, float v1, unsigned tag) {
-    const v4i w = {__float_as_int(v0), static_cast<int>(tag), __float_as_int(v1), static_cast<int>(tag)};
-    __builtin_amdgcn_raw_buffer_store_b128(w, rs, cell * 8, 0, kAuxDeviceScope);
-}
-
 // RP: rows a load of operands is dealt for (B <= RP, of 4, 8 and 16).  A product takes row lane % 16, so with few
 // rows most lanes would have nothing to load: 16 / RP units of two columns share a load instead, and
 // move to their lanes inside the registers.
