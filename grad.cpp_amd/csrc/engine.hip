@@ -13,6 +13,7 @@
 #include "rows.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -513,6 +514,12 @@ struct Session {
     unsigned repoch = 1;    // tag base; grows with every launch, re-based by clearing the cells
     unsigned rspin_limit = 1u << 18;
     std::unique_lock<std::mutex> resident_lock;  // this call's hold on g_persist_gate
+    int resident_rest = 0;   // steps to run as launches before the gate is tried again
+    int resident_ahead = 0;  // resident steps enqueued since the last of window_ev was recorded
+    int resident_window = 0; // how often that was, in this hold
+    hipEvent_t window_ev[2] = {nullptr, nullptr};
+    // what is on the stream in front of the next step and may take long: nothing, all of it, or up to ev[1]
+    enum { AHEAD_NONE, AHEAD_STREAM, AHEAD_PROMPT } ahead = AHEAD_NONE;
     float* start_logits = nullptr;  // a copy of the logits that a run of steps began with
 
     void* host_block = nullptr;    // one pinned allocation, which kernels read and write directly:
@@ -560,7 +567,7 @@ struct Session {
             if (e) (void)hipGraphExecDestroy(e);
         for (hipGraph_t g : graph)
             if (g) (void)hipGraphDestroy(g);
-        for (hipEvent_t e : ev)
+        for (hipEvent_t e : {ev[0], ev[1], ev[2], window_ev[0], window_ev[1]})
             if (e) (void)hipEventDestroy(e);
         for (void* p : {block, static_cast<void*>(uniforms), static_cast<void*>(logit_log),
                         static_cast<void*>(pp_x), static_cast<void*>(pp_q), static_cast<void*>(pp_attn),
@@ -579,8 +586,10 @@ struct Session {
 // same time (two sessions on two host threads) could each hold a part of the
 // GPU and wait for the rest for ever.  Every entry point that launches the
 // kernel therefore holds this process-wide lock from before the launch until
-// the stream has been synchronised; sessions on other engines never take it.
+// the stream has been synchronised.  Sessions whose steps may be resident take it when it is free and
+// somebody does not want it (resident_begin); the others never do.
 static std::mutex g_persist_gate;
+static std::atomic<int> g_gate_waiting{0};  // calls of the one-launch engine that are waiting for it
 
 static thread_local int g_gate_depth = 0;
 
@@ -600,7 +609,9 @@ PersistGate::PersistGate(const Session& s) {
     if (g_gate_depth > 0)
         throw ApiError{GH_ERR_RUNTIME, "a persistent-engine call is already running on this thread "
                                        "(token callbacks must not call into persistent-engine sessions)"};
+    g_gate_waiting.fetch_add(1);
     lock = std::unique_lock<std::mutex>(g_persist_gate);
+    g_gate_waiting.fetch_sub(1);
     g_gate_depth++;
 }
 
@@ -849,25 +860,61 @@ static int enqueue_layer(Session& s, int l, bool query_only) {
 
 // ---- all layers of a step in one launch (kernels_resident.h)
 
+// A call whose steps are resident enqueues them far ahead of the GPU, and whoever waits for the gate can have it only
+// when what is enqueued has run.  So no more than two windows of steps are, and a hold begins when what may take
+// long in front of it (a prompt, steps as launches) is done: a call on the one-launch engine waits for at most 2 x 8
+// steps. (One step of a single sequence beside 13 sequences x 600 tokens: 133 ms before there were windows, 2.9 at
+// most with them; beside 16 x 400 behind 1500 positions 189, 6.9. Alone, 48 tokens of 13 sequences 10.76 ms either
+// way, 16 behind 1536 positions 35.47.)
+constexpr int kResidentWindow = 8;
+// Steps as launches behind a hold that was given up to somebody, about what the call got that waited for it.
+constexpr int kResidentRest = 64;
+
+// The stream has been synchronised (or nothing resident is on it).
+static void resident_end(Session& s) {
+    s.ahead = Session::AHEAD_NONE;
+    s.resident_ahead = s.resident_window = 0;
+    if (!s.resident_lock.owns_lock()) return;
+    g_gate_depth--;
+    s.resident_lock.unlock();
+    s.resident_lock = {};
+}
+
 // What this call launches may take the whole GPU from here on: the gate that resident launches share is this
 // session's until resident_end. False, and the step runs as a launch per operation, when another
-// session has it or this thread is inside a callback of one that does: both forms give the same bits.
+// session has it or waits for it or this thread is inside a callback of one that does: both forms give the same bits.
 static bool resident_begin(Session& s) {
-    if (s.resident_lock.owns_lock()) return true;
-    if (g_gate_depth > 0) return false;
+    if (s.resident_lock.owns_lock()) {
+        if (g_gate_waiting.load(std::memory_order_relaxed) == 0) return true;
+        HIP_CHECK(hipStreamSynchronize(s.stream));
+        resident_end(s);
+        s.resident_rest = kResidentRest;
+        return false;
+    }
+    if (s.resident_rest > 0) {
+        s.resident_rest--;
+        return false;
+    }
+    if (g_gate_depth > 0 || g_gate_waiting.load(std::memory_order_relaxed) != 0) return false;
     std::unique_lock<std::mutex> lock(g_persist_gate, std::try_to_lock);
     if (!lock.owns_lock()) return false;
+    if (s.ahead != Session::AHEAD_NONE) {
+        lock.unlock();
+        HIP_CHECK(s.ahead == Session::AHEAD_PROMPT ? hipEventSynchronize(s.ev[1]) : hipStreamSynchronize(s.stream));
+        s.ahead = Session::AHEAD_NONE;
+        if (!lock.try_lock()) return false;
+    }
     s.resident_lock = std::move(lock);
     g_gate_depth++;
     return true;
 }
 
-// The stream has been synchronised (or nothing resident is on it).
-static void resident_end(Session& s) {
-    if (!s.resident_lock.owns_lock()) return;
-    g_gate_depth--;
-    s.resident_lock.unlock();
-    s.resident_lock = {};
+// Behind a resident step: waits until the window before the present one has run.
+static void resident_pace(Session& s) {
+    if (++s.resident_ahead < kResidentWindow) return;
+    s.resident_ahead = 0;
+    HIP_CHECK(hipEventRecord(s.window_ev[s.resident_window & 1], s.stream));
+    if (s.resident_window++ > 0) HIP_CHECK(hipEventSynchronize(s.window_ev[s.resident_window & 1]));
 }
 
 // Ends the call's hold however the call ends; what it launched has left the GPU by then.
@@ -888,7 +935,15 @@ static int resident_items(const Session& s) { return s.B * s.m->shape.heads * (s
 
 // For the next step of this session: can and may it run that way?
 static bool resident_now(Session& s) {
-    return s.resident && resident_kernel_for(s.m->shape, s.B, resident_items(s)) && resident_begin(s);
+    if (!s.resident) return false;
+    if (!resident_kernel_for(s.m->shape, s.B, resident_items(s))) {
+        if (s.resident_lock.owns_lock()) {  // (the context has outgrown the kernel)
+            HIP_CHECK(hipStreamSynchronize(s.stream));
+            resident_end(s);
+        }
+        return false;
+    }
+    return resident_begin(s);
 }
 
 static void launch_resident(Session& s) {
@@ -1278,7 +1333,12 @@ static int record_step(Session& s, StepForm form, hipGraph_t* graph) {
 static void run_step(Session& s, StepForm form = STEP_EMBED) {
     if (resident_now(s)) {
         enqueue_step(s, form, /*resident=*/true);
-    } else if (s.engine == GH_ENGINE_GRAPH) {
+        resident_pace(s);
+        s.pos++;
+        return;
+    }
+    s.ahead = Session::AHEAD_STREAM;
+    if (s.engine == GH_ENGINE_GRAPH) {
         if (!s.exec[form]) {  // (a form's graph is made when it is first wanted)
             if (!s.graph[form]) {
                 const int launches = record_step(s, form, &s.graph[form]);
@@ -1576,6 +1636,8 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
         if (o.engine == GH_ENGINE_AUTO && s.engine == GH_ENGINE_GRAPH && resident_kernel_for(sh, s.B, pairs) && cus >= kResidentGrid
             && table_bytes <= kResidentTableBytes && s.page_shift >= 5 && s.attn_chunk % 128 == 0 && layers_back_to_back(m)) {
             s.resident = true;
+            for (hipEvent_t& e : s.window_ev)  // (nobody reads memory on their word)
+                HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventDisableSystemFence));
             s.rcells_count = resident_cells(d, F, B);
             parts.add(s.rcells, s.rcells_count);
             parts.add(s.rctl, 1);
@@ -3048,6 +3110,7 @@ gh_status gh_session_generate(gh_session* sess, const int32_t* prompts, int32_t 
             HIP_CHECK(hipEventRecord(s.ev[0], s.stream));
             run_prompt(s, prompt_len, log, &steps);
             HIP_CHECK(hipEventRecord(s.ev[1], s.stream));
+            s.ahead = Session::AHEAD_PROMPT;
             std::tie(made, stepped) = run_decode(s, max_tokens, *opt, du, max_tokens, seed, log, &steps);
             HIP_CHECK(hipEventRecord(s.ev[2], s.stream));
 

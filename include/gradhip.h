@@ -14,7 +14,8 @@
  * lock until the launch has finished; results do not depend on the order.
  * Sessions of 2 to 16 sequences run a step's layers as one such launch (AUTO, the
  * same shapes except d_model 1024) when the lock is free, and as a launch per
- * operation when it is not: the results are the same to the bit.
+ * operation when it is not: the results are the same to the bit.  They hand the
+ * lock on, within 16 steps, to a one-launch call that waits for it.
  *
  * There is no CPU fallback: every compute entry point fails with
  * GH_ERR_DEVICE when no gfx950 device is usable.

@@ -2,6 +2,7 @@
 (the graph engine), whatever the batch, the context and the place of the cache pages; and the same
 results when a step has to be given up, when the chip is someone else's, and where the tags start over."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -177,6 +178,52 @@ def test_sessions_on_several_threads(models):
     for t in threads:
         t.join(timeout=60)
     assert not bad and not any(t.is_alive() for t in threads)
+
+
+def _beside_a_batch(gm, vocab, call):
+    """Runs call(session, prompts) of a batch on a thread of its own and 20 steps of a single sequence from 5 ms later
+    on; which of the two ended first, and what both returned."""
+    prompts = synth.uniform_tokens(13 * 12, vocab, 130).reshape(13, 12)
+    tokens = synth.uniform_tokens(20, vocab, 131)
+    batch, single = G.Session(gm, batch=13), G.Session(gm, batch=1)
+    want = call(batch, prompts), [single.step([t]) for t in tokens]  # alone, and everything has been used once
+    batch.reset()
+    single.reset()
+    order, out, started = [], {}, threading.Event()
+
+    def run():
+        started.set()
+        out["batch"] = call(batch, prompts)
+        order.append("batch")
+
+    thread = threading.Thread(target=run)
+    thread.start()
+    started.wait()
+    time.sleep(0.005)
+    out["single"] = [single.step([t]) for t in tokens]
+    order.append("single")
+    thread.join(timeout=60)
+    assert not thread.is_alive()
+    assert out["batch"].tobytes() == want[0].tobytes()
+    assert np.stack(out["single"]).tobytes() == np.stack(want[1]).tobytes()
+    return order
+
+
+@pytest.mark.parametrize("kind", ["generate", "stream"])
+def test_a_single_sequence_does_not_wait_for_a_whole_batched_call(models, kind):
+    """A batch of 900 tokens (some 50 ms) has the chip; 20 single steps (2 ms) that begin 5 ms later end before it."""
+    cfg, _, gm = models["llama-d768"]
+    opt = G.sampling(0.9, 0, 1.0, 1.1, False)
+
+    def call(s, prompts):
+        if kind == "generate":
+            return s.generate(prompts, 900, opt, seed=9)
+        got = []
+        s.prefill(prompts)
+        s.decode_stream(900, opt, lambda ids, i: got.append(np.array(ids)), seed=9)
+        return np.stack(got)
+
+    assert _beside_a_batch(gm, cfg.vocab, call) == ["single", "batch"]
 
 
 def test_a_callback_may_use_any_session(models):
