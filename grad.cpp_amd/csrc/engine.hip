@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -445,6 +446,7 @@ struct Session {
 
     hipStream_t stream = nullptr;
     hipGraph_t graph[kStepForms] = {};
+    int form_launches[kStepForms] = {};
     hipGraphExec_t exec[kStepForms] = {};
     // Batched greedy decoding without a penalty: the logits launch leaves the largest
     // value of every run of 16 columns, and a second form of the step opens with the
@@ -507,12 +509,17 @@ struct Session {
     bool xcd_all_slices = false;  // every workgroup of an XCD takes a slice of the attention at any context
 
     // steps of a few sequences as one launch for all layers (kernels_resident.h)
-    bool resident = false;  // ... is built for this session and has not failed
+    bool resident = false;  // ... is built for this session
     Cell* rcells = nullptr;
     size_t rcells_count = 0;
     ResidentCtl* rctl = nullptr;
     unsigned repoch = 1;    // tag base; grows with every launch, re-based by clearing the cells
     unsigned rspin_limit = 1u << 18;
+    int impatient_from = 0, impatient_n = 0;  // (tests: launches that have spins_impatient looks instead)
+    unsigned spins_impatient = 0;
+    int resident_launches = 0;   // resident launches made so far
+    bool resident_off = false;   // the rest of this call runs as launches
+    int resident_backoff = 1 << 12;  // steps that run as launches behind the next step that gives up
     std::unique_lock<std::mutex> resident_lock;  // this call's hold on g_persist_gate
     int resident_rest = 0;   // steps to run as launches before the gate is tried again
     int resident_ahead = 0;  // resident steps enqueued since the last of window_ev was recorded
@@ -925,6 +932,7 @@ struct ResidentScope {
     ~ResidentScope() {
         if (std::uncaught_exceptions() > exceptions && s.resident_lock.owns_lock()) (void)hipStreamSynchronize(s.stream);
         resident_end(s);
+        s.resident_off = false;
     }
     ResidentScope(const ResidentScope&) = delete;
     ResidentScope& operator=(const ResidentScope&) = delete;
@@ -935,7 +943,7 @@ static int resident_items(const Session& s) { return s.B * s.m->shape.heads * (s
 
 // For the next step of this session: can and may it run that way?
 static bool resident_now(Session& s) {
-    if (!s.resident) return false;
+    if (!s.resident || s.resident_off) return false;
     if (!resident_kernel_for(s.m->shape, s.B, resident_items(s))) {
         if (s.resident_lock.owns_lock()) {  // (the context has outgrown the kernel)
             HIP_CHECK(hipStreamSynchronize(s.stream));
@@ -967,7 +975,9 @@ static void launch_resident(Session& s) {
     p.pos = s.pos;
     p.chunk = s.attn_chunk;
     p.epoch = s.repoch;
-    p.spin_limit = s.rspin_limit;
+    const int launch = s.resident_launches;
+    s.resident_launches = launch < INT_MAX ? launch + 1 : launch;
+    p.spin_limit = launch >= s.impatient_from && launch - s.impatient_from < s.impatient_n ? s.spins_impatient : s.rspin_limit;
     s.repoch += static_cast<unsigned>(sh.layers);
     hipLaunchKernelGGL(resident_kernel_for(sh, s.B, resident_items(s)), dim3(kResidentGrid), dim3(kResidentThreads),
                        static_cast<size_t>(s.B) * s.pages_per_seq * sizeof(int), s.stream, p);
@@ -1333,6 +1343,8 @@ static int record_step(Session& s, StepForm form, hipGraph_t* graph) {
 static void run_step(Session& s, StepForm form = STEP_EMBED) {
     if (resident_now(s)) {
         enqueue_step(s, form, /*resident=*/true);
+        // (embedding, layers, logits; a LayerNorm in front of the logits is a launch of its own)
+        s.launches_per_step = s.m->shape.modern() ? 3 : 4;
         resident_pace(s);
         s.pos++;
         return;
@@ -1340,12 +1352,10 @@ static void run_step(Session& s, StepForm form = STEP_EMBED) {
     s.ahead = Session::AHEAD_STREAM;
     if (s.engine == GH_ENGINE_GRAPH) {
         if (!s.exec[form]) {  // (a form's graph is made when it is first wanted)
-            if (!s.graph[form]) {
-                const int launches = record_step(s, form, &s.graph[form]);
-                if (!s.resident) s.launches_per_step = launches;
-            }
+            if (!s.graph[form]) s.form_launches[form] = record_step(s, form, &s.graph[form]);
             HIP_CHECK(hipGraphInstantiate(&s.exec[form], s.graph[form], nullptr, nullptr, 0));
         }
+        s.launches_per_step = s.form_launches[form];
         HIP_CHECK(hipGraphLaunch(s.exec[form], s.stream));
     } else {
         enqueue_step(s, form);
@@ -1426,17 +1436,29 @@ static void deliver_logits(Session& s) {
     deliver(s, s.logits, 0, 1, s.B * V, s.host_logits);
 }
 
+// After a synchronisation of what deliver() enqueued: did a resident step give up its wait (something else held a part of
+// the GPU for long)? Then the session's next steps are launches, and twice as many the next time.  A wait is
+// given up after 2^18 looks, some tenths of a second: as much as the first rest, 4096 steps, loses, and a few percent of
+// the longest if something is always in the way.
+static bool resident_gave_up(Session& s) {
+    if (!s.resident || *s.host_err == 0) return false;
+    *s.host_err = 0;
+    resident_end(s);
+    HIP_CHECK(hipMemsetAsync(s.rctl, 0, sizeof(ResidentCtl), s.stream));  // (no step in flight, none recorded)
+    s.resident_rest = s.resident_backoff;
+    s.resident_backoff = std::min(2 * s.resident_backoff, 1 << 16);
+    return true;
+}
+
 // Launches of a session whose steps may be resident, up to and with a deliver() and the synchronisation behind it. If a
-// resident step gave up its wait (something else held a part of the GPU for long), the session does
-// without from here on, and the call runs once more from where the session stood: the cache rows below that
-// position, the history and the call's ids are as they were, and what comes after is written again.
+// resident step gave up its wait, the call runs once more, as launches, from where the session stood: the
+// cache rows below that position, the history and the call's ids are as they were, and what comes after is written again.
 template <class Work>
 static void run_resident(Session& s, Work work) {
     const int pos = s.pos, n_hist = s.n_hist, picks = s.picks;
     work();
-    if (!s.resident || *s.host_err == 0) return;
-    s.resident = false;
-    *s.host_err = 0;
+    if (!resident_gave_up(s)) return;
+    s.resident_off = true;  // until the call ends
     s.pos = pos;
     s.n_hist = n_hist;
     s.picks = picks;
@@ -1647,11 +1669,20 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
                     HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, kResidentTableBytes));
             }
-            // (embedding, layers, logits; a LayerNorm in front of the logits is a launch of its own)
             s.launches_per_step = sh.modern() ? 3 : 4;
-            // Test aid: looks at a cell that a wait may take (0: the first look has to succeed).
-            if (const char* spins = std::getenv("GRADHIP_TEST_RESIDENT_SPINS"))
-                s.rspin_limit = static_cast<unsigned>(std::min(std::max(std::strtol(spins, nullptr, 10), 0l), 1l << 18));
+            // Test aid, "looks", "looks,first" or "looks,first,launches": looks at a cell that a wait may take (0: the
+            // first look has to succeed), from which of the session's resident launches on, and in how many.
+            if (const char* spins = std::getenv("GRADHIP_TEST_RESIDENT_SPINS")) {
+                int looks = 0, from = 0, n = INT_MAX;
+                if (std::sscanf(spins, "%d,%d,%d", &looks, &from, &n) >= 1) {
+                    s.spins_impatient = static_cast<unsigned>(std::min(std::max(looks, 0), 1 << 18));
+                    s.impatient_from = std::max(from, 0);
+                    s.impatient_n = std::max(n, 0);
+                }
+            }
+            // ... and how many steps are launches behind the first one that gave up.
+            if (const char* rest = std::getenv("GRADHIP_TEST_RESIDENT_REST"))
+                s.resident_backoff = static_cast<int>(std::min(std::max(std::strtol(rest, nullptr, 10), 1l), 1l << 12));
             // ... and steps until the tags start over (as for the one-launch engine, below).
             if (const char* near = std::getenv("GRADHIP_TEST_NEAR_WRAP")) {
                 const long asked = std::strtol(near, nullptr, 10);
@@ -1713,7 +1744,7 @@ static std::unique_ptr<Session> create_session(const Model& m, const gh_session_
         // nothing to record: one launch runs any number of steps
     } else if (!s.resident) {
         // Counts the launches of a step without running one.
-        s.launches_per_step = record_step(s, STEP_EMBED, &s.graph[STEP_EMBED]);
+        s.launches_per_step = s.form_launches[STEP_EMBED] = record_step(s, STEP_EMBED, &s.graph[STEP_EMBED]);
     }
     return sp;
 }
@@ -2230,7 +2261,7 @@ static void keep_logits(Session& s, bool restore) {
     }
     if (!s.resident) return;
     if (!s.start_logits && !try_alloc(s.start_logits, n)) {
-        s.resident = false;
+        s.resident_off = true;  // for this call
         return;
     }
     HIP_CHECK(hipMemcpyAsync(s.start_logits, s.logits, n * sizeof(float), hipMemcpyDeviceToDevice, s.stream));
@@ -2239,9 +2270,7 @@ static void keep_logits(Session& s, bool restore) {
 // In a streamed run, after a synchronisation: if the last step was resident and gave up, it runs again as launches.
 // picked: a pick made from its logits is to be forgotten.  True if it had to.
 static bool repeat_step(Session& s, bool picked) {
-    if (!s.resident || *s.host_err == 0) return false;
-    s.resident = false;
-    *s.host_err = 0;
+    if (!resident_gave_up(s)) return false;
     s.pos--;
     if (picked) {
         s.n_hist--;
@@ -2928,6 +2957,7 @@ gh_status gh_session_decode(gh_session* sess, int32_t max_tokens, const gh_sampl
         *out_count = made;
         HIP_CHECK(hipEventElapsedTime(&s.timing.decode_ms, s.ev[1], s.ev[2]));
         s.timing.decode_steps = stepped;
+        s.timing.launches_per_step = s.launches_per_step;
     });
 }
 
@@ -3060,6 +3090,7 @@ gh_status gh_session_decode_stream(gh_session* sess, int32_t max_tokens, const g
         *out_count = made;
         HIP_CHECK(hipEventElapsedTime(&s.timing.decode_ms, s.ev[1], s.ev[2]));
         s.timing.decode_steps = stepped;
+        s.timing.launches_per_step = s.launches_per_step;
     });
 }
 
@@ -3131,6 +3162,7 @@ gh_status gh_session_generate(gh_session* sess, const int32_t* prompts, int32_t 
         HIP_CHECK(hipEventElapsedTime(&s.timing.decode_ms, s.ev[1], s.ev[2]));
         s.timing.prompt_steps = prompt_len;
         s.timing.decode_steps = stepped;
+        s.timing.launches_per_step = s.launches_per_step;
     });
 }
 

@@ -343,7 +343,7 @@ typedef struct gh_timing {
     float decode_ms;
     int32_t prompt_steps;
     int32_t decode_steps;
-    int32_t launches_per_step; /* kernel launches (or graph nodes) in one step */
+    int32_t launches_per_step; /* kernel launches (or graph nodes) in a step, as the last one was made */
     /* Persistent engine, since the session was created: picks that one workgroup made from
      * the whole row of logits.  The others (greedy, or 0 < top_k <= 64, after a step of the
      * same launch) were made by every workgroup at once from a few candidates per workgroup. */

@@ -148,6 +148,51 @@ def test_a_step_that_gives_up_runs_as_launches(models, monkeypatch, spins):
         assert res[0].tobytes() == res[2].tobytes() and res[1].tobytes() == res[3].tobytes(), call
 
 
+@pytest.mark.parametrize("name", sorted(SHAPES))
+def test_a_session_that_gave_up_tries_again(models, monkeypatch, name):
+    """The step that gives up is the call's first one or a late one; so many steps later, twice as many the second
+    time, the session's steps are resident again."""
+    cfg, _, gm = models[name]
+    greedy, plain = G.sampling(1.0, 0, 1.0, 1.0, True), G.sampling(0.9, 0, 1.0, 1.1, False)
+    prompt = synth.uniform_tokens(5 * 40, cfg.vocab, 109).reshape(5, 40)
+    monkeypatch.setenv("GRADHIP_TEST_RESIDENT_REST", "4")
+    for first in (0, 17):
+        monkeypatch.setenv("GRADHIP_TEST_RESIDENT_SPINS", f"0,{first},1")
+        s, ref = _both(gm, 5)
+        for x in (s, ref):
+            x.prefill(prompt)  # one pass: nothing resident before the calls
+        for n, opt, resident in ((24, plain, False), (4, plain, False), (3, greedy, True), (9, plain, True)):
+            assert s.decode(n, opt, seed=n).tobytes() == ref.decode(n, opt, seed=n).tobytes(), (first, n)
+            assert (s.last_timing()["launches_per_step"] == RESIDENT[name]) == resident, (first, n)
+        assert s.step(prompt[:, 0]).tobytes() == ref.step(prompt[:, 0]).tobytes()
+    monkeypatch.setenv("GRADHIP_TEST_RESIDENT_SPINS", "0,0,2")
+    s, ref = _both(gm, 5)
+    for x in (s, ref):
+        x.prefill(prompt)
+    for i, resident in enumerate([False] + 4 * [False] + [False] + 8 * [False] + 3 * [True]):
+        assert s.decode(1, plain, seed=i).tobytes() == ref.decode(1, plain, seed=i).tobytes(), i
+        assert (s.last_timing()["launches_per_step"] == RESIDENT[name]) == resident, i
+
+
+@pytest.mark.parametrize("looks", [1, 4, 12, 40])
+@pytest.mark.parametrize("name", ["gpt2-d768", "llama-d768"])
+def test_giving_up_in_a_long_context(models, monkeypatch, name, looks):
+    """Three runs of positions per head: with more or fewer looks it is the rows, q or another workgroup's share
+    that is not waited for, in a streamed run and in single steps."""
+    cfg, _, gm = models[name]
+    plain = G.sampling(0.9, 0, 1.0, 1.1, False)
+    prompt = synth.uniform_tokens(9 * 1050, cfg.vocab, 111).reshape(9, 1050)
+    monkeypatch.setenv("GRADHIP_TEST_RESIDENT_SPINS", f"{looks},3,2")
+    monkeypatch.setenv("GRADHIP_TEST_RESIDENT_REST", "2")
+    out = []
+    for s in _both(gm, 9, shuffle_pages=True):
+        s.prefill(prompt)
+        got = []
+        s.decode_stream(12, plain, lambda ids, i: got.append(np.array(ids)), seed=8)
+        out.append(np.stack(got).tobytes() + b"".join(s.step(prompt[:, t]).tobytes() for t in range(5)))
+    assert out[0] == out[1]
+
+
 def test_tags_start_over(models, monkeypatch):
     cfg, _, gm = models["llama-d768"]
     monkeypatch.setenv("GRADHIP_TEST_NEAR_WRAP", "5")
