@@ -73,6 +73,25 @@ def test_more_runs_of_positions_than_halves_of_workgroups():
         assert one.step(tokens[:, t]).tobytes() == many.step(tokens[:, t]).tobytes(), t
 
 
+@pytest.mark.parametrize("name, batch, behind", [("gpt2-d768", 13, 4096), ("llama-d768", 16, 4096), ("llama-d768", 8, 6144),
+                                                 ("gpt2-d512", 16, 6144)])
+def test_three_and_four_rounds_of_runs_in_two_layers(name, batch, behind):
+    """The cells of the runs are used again in every round and by the next layer; here a step adds a run per head."""
+    shape = SHAPES[name]
+    cfg = synth.Config(shape.arch, 90, shape.d_model, 2, shape.heads, behind + 16)
+    runs = [(p + 511) // 512 for p in (behind, behind + 1)]  # (the runs of contexts this long have 512 positions)
+    assert {-(-batch * cfg.heads * r // 512) for r in runs} <= {2, 3, 4} and -(-batch * cfg.heads * runs[1] // 512) >= 3
+    W = synth.make_weights(cfg, 103, std=lively_std(cfg), norm_noise=0.1)
+    one, many = _both(G.Model.from_tensors(cfg, W), batch, shuffle_pages=True)
+    tokens = synth.uniform_tokens(batch * (behind + 3), cfg.vocab, 112).reshape(batch, -1)
+    for s in (one, many):
+        s.prefill(tokens[:, :behind - 2])
+    for t in range(behind - 2, behind + 3):
+        assert one.step(tokens[:, t]).tobytes() == many.step(tokens[:, t]).tobytes(), t
+    assert one.decode(1, G.sampling(1.0, 0, 1.0, 1.0, True)).shape == (batch, 1)
+    assert one.last_timing()["launches_per_step"] == RESIDENT[name]
+
+
 @pytest.mark.parametrize("name", sorted(SHAPES))
 def test_steps_match_the_oracle(models, name):
     cfg, W, gm = models[name]
