@@ -596,9 +596,10 @@ inline void launch_gemm_wide(const GemvParams& p, int M, hipStream_t st) {
 // of them give the same sums.  A launch costs a start and then, for every workgroup that a
 // compute unit is dealt, a time that grows more slowly than the tiles in it, since more tiles
 // share the rows they read (what is being paid for is operand traffic from the L2s and operand
-// permutes, 2 x 2 tiles having half of both per product).  Measured over 65 to 511 rows against eight
-// matrices (512 to 4096 outputs, 512 to 3072 columns): 1 x 1 tiles 1.7 us per workgroup and 768 columns,
-// two tiles 2.4, 2 x 2 4.0; the rule's pick is the fastest of them or within 15 % of it.
+// permutes, 2 x 2 tiles having half of both per product).  Measured over 65 to 511 rows against thirteen
+// matrices (512 to 4096 outputs, 512 to 4096 columns): 1 x 1 tiles 1.7 us per workgroup and 768 columns,
+// two tiles 2.4, 2 x 2 4.0; the rule's pick is the fastest of them or within 6 % of it in 142 of 143
+// cases, and 11.3 us for 9.8 at 511 x 768 x 768 (profiles/many_row_tilings.md).
 // 1 x 1 for narrow matrices and 4 x 1 for the others, as it was: 100 x 4096 x 768 17.1 us -> 14.3,
 // 244 x 2304 x 768 24.4 -> 17.1, 397 x 4096 x 768 52.5 -> 35.8, 244 x 768 x 2048 12.8 -> 12.2.
 // (Both operands through an LDS ring, 32 x 32 to 64 x 64 outputs per workgroup: 35-36 us at 397 x 4096 x

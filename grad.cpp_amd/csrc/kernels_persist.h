@@ -658,7 +658,8 @@ __global__ __launch_bounds__(kPersistThreads) void persist_decode_kernel(const P
             // workgroups 16, 32, ... places further on are on the same XCD: their wavefronts
             // without an item of phase A touch the rows' 128-byte lines now (greedy tokens behind 300 / 397 /
             // 600: Llama block 117.5 / 122.3 / 138.9 us without, 112.3 / 113.4 / 135.7 with; GPT-2 d768 128.6 /
-            // 133.4 / 145.5, 121.0 / 123.2 / 140.0).  Fewer rows are there in time (Llama behind 33 and 190: 1.5
+            // 133.4 / 145.5, 121.0 / 123.2 / 140.0; GPT-2 d1024 behind 300 / 600 / 1900 171.6 / 186.4 / 192.8, 155.9 /
+            // 176.4 / 186.6).  Fewer rows are there in time (Llama behind 33 and 190: 1.5
             // slower), and so are those of the 512 block, whose weights are fewer (900: 80.4, 87.1).
             if (KD >= 3 && pos >= 256 && wg >= 16 && (wg & 15) < H && first >= NQKV) {
                 const int busy = (NQKV - wg + G - 1) / G, idle = kPersistWaves - busy;
@@ -1080,7 +1081,8 @@ __global__ __launch_bounds__(kPersistThreads) void persist_decode_kernel(const P
             // rows of the next phase before all have stored theirs.  Where that pays was found by trying it behind
             // every phase (greedy tokens at positions 60..124, us): here, d768 GPT-2 117.5 -> 115.9, Llama block
             // 108.3 -> 107.2, d512 67.9 -> 68.0; in front of the FFN1 rows, d512 67.9 -> 67.4, d768
-            // 117.0 -> 126.8, Llama block 108.5 -> 114.8; behind QKV 118.0, 112.0, 68.4.
+            // 117.0 -> 126.8, Llama block 108.5 -> 114.8; behind QKV 118.0, 112.0, 68.4.  d1024: here 152.4 -> 152.6, in
+            // front of the FFN1 rows 152.4 -> 159.6.
             if constexpr (KD == 3) __syncthreads();
             stamp();
 
@@ -1096,7 +1098,8 @@ __global__ __launch_bounds__(kPersistThreads) void persist_decode_kernel(const P
                     for (int i = 0; i < KF; i++) w0[i] = make_float4(0.f, 0.f, 0.f, 0.f);
                 }
                 // A first look that comes a little too early costs a whole round (none / 0.1 / 0.3 us of
-                // patience: Llama block 107.1 / 106.5 / 106.4, the others 115.9 / 115.9 / 116.9 and 67.8 / 67.9 / 68.8).
+                // patience: Llama block 107.1 / 106.5 / 106.4, the others 115.9 / 115.9 / 116.9 and 67.8 / 67.9 / 68.8;
+                // d1024 152.4 / - / 152.3).
                 if constexpr (MODERN) __builtin_amdgcn_s_sleep(4);
                 gather_in_layer((p.cells + 6 * D), F, tag_of(l, 3), vin, p);
                 for (int row = first; row < D; ) {

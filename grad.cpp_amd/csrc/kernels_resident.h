@@ -14,13 +14,18 @@
 // attention attn_decode64_kernel's, the LayerNorm layernorm_rows_kernel's.  So which of the two
 // forms runs a step is a matter of speed alone.  (src/transformer/inference.cpp:184-249)
 //
-// What bounds it: five hand-offs per layer of 0.8 to 1.9 us, and between them chains of a few hundred
-// instructions on eight wavefronts.  One layer of the Llama block d768, 4 sequences behind 64 positions: QKV 3.1 us (1.1
-// of it until the rows are there), attention 2.4, W_o 2.5, FFN1 4.1, FFN2 4.7 (1.7 of it products, 16-row tiles for
-// 4 rows; 128 KB of weights through one compute unit).  Per step, launches -> this, context 200: Llama
-// block 2 sequences 246 us -> 144, 4 253 -> 157, 8 259 -> 173, 16 290 -> 188; GPT-2 block d768 2 sequences
-// 286 -> 167, 16 323 -> 222; Llama block, 16 sequences behind 1900 positions 522 -> 444, 190 MB of cache per
-// layer in some 37 us of its 52.
+// What bounds it: five hand-offs per layer, and between them chains of a few hundred instructions on eight wavefronts.
+// From the last store of a phase to the rows of the next being there / from there to its last store, us, one layer of the
+// Llama block d768, 4 sequences behind 64 positions: QKV 1.1 / 1.8, attention 0.6 / 1.8, W_o 1.8 / 1.1, FFN1 1.2 / 2.8,
+// FFN2 2.2 / 1.6 (0.9 of it products, 16-row tiles for 4 rows; 128 KB of weights through one compute unit), 16.1 in
+// all; 16 sequences behind 200 1.4 / 2.1, 0.9 / 2.8, 2.3 / 1.6, 1.7 / 3.1, 1.7 / 3.7, 21.3.  The matrix cores are busy
+// 8 % of the time at 4 sequences, and the 251 MB that miss the L2s (226 of them weights) go at 1.9 TB/s.  Per step,
+// launches -> this, behind 184 positions: Llama block 2 sequences 249 us -> 144, 4 257 -> 158, 8 276 -> 173, 16 318 -> 193;
+// GPT-2 block d768 2 sequences 289 -> 166, 16 353 -> 222; Llama block, 16 sequences behind 1884 positions 523 -> 444:
+// 188 MB of cache per layer in the 33 us of its 53 that the attention takes.
+// Built for the d512 and d768 shapes.  d1024 / F4096 would fit (64 + 192 workgroups, two FFN1 tiles each) and is
+// launches, 337 us at 2 sequences and 403 at 16 behind 128: not tried.  So are more than 16 sequences (Llama, behind
+// 128: 16 188, 17 324), which need a second tile of rows per product.
 //
 // The order things are sent in is most of the design.  A wavefront's loads return in the order they
 // went out, and a workgroup's stores leave behind what its other wavefronts have asked for: weights are

@@ -5,6 +5,7 @@ namespace gh {
 
 template <int KD, int KF, bool MODERN>
 static ResidentKernel of_rows(int batch, bool rounds) {
+    // (up to 4 sequences a second round begins beyond 5120 positions, where a step of 4 goes from 351 us to 467)
     if (batch <= 4) return rounds ? nullptr : resident_layers_kernel<KD, KF, MODERN, 4, false>;
     if (batch <= 8) return rounds ? resident_layers_kernel<KD, KF, MODERN, 8, true> : resident_layers_kernel<KD, KF, MODERN, 8, false>;
     if (batch > kResidentRows) return nullptr;

@@ -105,7 +105,7 @@ typedef enum gh_engine {
 typedef struct gh_session_opts {
     int32_t batch;       /* independent sequences decoded in lock step (>= 1) */
     int32_t engine;      /* gh_engine */
-    int32_t page_tokens; /* KV-cache page size in positions; 0 = default (64) */
+    int32_t page_tokens; /* KV-cache page size in positions; 0 = default (64); larger than 65536 is 65536 */
     int32_t shuffle_pages; /* non-zero: hand out physical pages in a scrambled order */
     int32_t flags;         /* GH_FLAG_* */
 } gh_session_opts;
