@@ -133,7 +133,9 @@ __device__ __forceinline__ void cell_put(Cell* c, float v, unsigned tag) {
 
 // Two cells that follow each other, the first on a boundary of 16 bytes: one store (each cell's value and tag
 // still travel together).  Through the builtin: a store of 16 bytes needs two wait states in front of whatever
-// next writes its registers, and behind one in inline assembly the compiler leaves none.
+// next writes its registers, and behind one in inline assembly the compiler leaves none.  (Greedy token behind 40
+// positions, as assembly / this: Llama block 101.4 / 101.4 us, GPT-2 d768 109.6 / 108.8, d512 63.8 / 63.3, d1024
+// 152.9 / 151.8; the same assembly with s_nop 1 behind it 101.3, 110.0, 64.1, 153.1.)
 __device__ __forceinline__ void cell_put2(__amdgpu_buffer_rsrc_t rs, int cell, float v0, float v1, unsigned tag) {
     const v4i w = {__float_as_int(v0), static_cast<int>(tag), __float_as_int(v1), static_cast<int>(tag)};
     __builtin_amdgcn_raw_buffer_store_b128(w, rs, cell * 8, 0, kAuxDeviceScope);

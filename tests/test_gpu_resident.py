@@ -92,6 +92,22 @@ def test_three_and_four_rounds_of_runs_in_two_layers(name, batch, behind):
     assert one.last_timing()["launches_per_step"] == RESIDENT[name]
 
 
+@pytest.mark.parametrize("batch, behind", [(4, 5112), (3, 7160)])
+def test_a_run_that_outgrows_the_kernel(batch, behind):
+    """Up to 4 sequences take one round: one call whose first steps are resident and whose later ones are launches."""
+    cfg = synth.Config(synth.ARCH_MODERN, 90, 768, 2, 12, behind + 40)
+    W = synth.make_weights(cfg, 113, std=lively_std(cfg), norm_noise=0.1)
+    one, many = _both(G.Model.from_tensors(cfg, W), batch, shuffle_pages=True)
+    opt = G.sampling(0.9, 0, 1.0, 1.1, False)
+    tokens = synth.uniform_tokens(batch * behind, cfg.vocab, 114).reshape(batch, behind)
+    for s in (one, many):
+        s.prefill(tokens)
+    assert batch * 12 * ((behind + 511) // 512) <= 512 < batch * 12 * ((behind + 30 + 511) // 512)
+    for n, resident in ((5, True), (25, False)):
+        assert one.decode(n, opt, seed=n).tobytes() == many.decode(n, opt, seed=n).tobytes()
+        assert (one.last_timing()["launches_per_step"] == RESIDENT["llama-d768"]) == resident
+
+
 @pytest.mark.parametrize("name", sorted(SHAPES))
 def test_steps_match_the_oracle(models, name):
     cfg, W, gm = models[name]
