@@ -151,12 +151,22 @@ struct SplitLayer {
     char *wqkv, *wo, *w1, *w2;
 };
 
+// The same matrices in pairs (kernels_pair.h), each with its outputs' exponents, and the powers of two that the
+// operands of those products are scaled by: norm(x) in front of QKV, the attention's rows, norm(x) in front of FFN1,
+// the hidden units.
+struct PairLayer {
+    char *wqkv, *wo, *w1, *w2;
+    int *eqkv, *eo, *e1, *e2;
+    int norm1, attn, norm2, hidden;
+};
+
 // One allocation of split matrices.
 struct SplitForm {
     std::mutex mutex;
     char* blob = nullptr;
     bool ready = false;
     bool unfit = false;  // a weight is outside the range of the parts (kSplitTop): fp32 products only
+    bool pairs = false;  // there are pairs (of the layers: beside the three parts; of the logits matrix: in their place)
     ~SplitForm() {
         if (blob) (void)hipFree(blob);
     }
@@ -181,11 +191,14 @@ struct Model {
     float *rope_cos = nullptr, *rope_sin = nullptr;  // (max_len, head_size/2)
     std::vector<Placement> place;                    // file order
 
-    // Split forms of the matrices, six bytes per weight beside the four above, each written by the
-    // first pass that multiplies by it and kept: the layers' (split_layers), and the logits matrix,
-    // which scoring alone needs and at any length (split_logits).
+    // Split forms of the matrices, each written by the first pass that multiplies by it and kept: the layers'
+    // (split_layers; ten bytes per weight beside the four above, six where there are no pairs), and that of the
+    // logits matrix (split_logits; four bytes, or six), which scoring alone needs and at any length.
     mutable SplitForm layers_split, logits_split;
     mutable std::vector<SplitLayer> split_layers;
+    mutable std::vector<PairLayer> pair_layers;
+    mutable int* logits_exponent = nullptr;  // of the logits matrix in pairs, in its allocation
+    mutable int logits_norm = 0;             // the power of two of its operand, norm(x)
 
     // The XCD-sharded persistent kernel reads the weights from a second copy laid
     // out as one contiguous stream per workgroup (kernels_xcd.h); built by the
@@ -284,15 +297,16 @@ static bool rows_shape_ok(const Shape& sh) {
     return sh.head_size() == 64 && sh.d_model % 64 == 0 && sh.d_ff() % 64 == 0;
 }
 
-// Writes a split form, once per model: fill calls place(src, N, K, gate_up) for every matrix and
-// is given the place of its split form.  False: the weights have none, or there is no memory for it
-// now (the next pass asks again).
+// Writes a split form in three parts, once per model: fill calls place(src, N, K, gate_up) for every matrix and
+// is given the place of its split form.  `more`: bytes wanted behind it, given up if there is no memory for both.
+// False: the weights have none, or there is no memory for it now (the next pass asks again).
 template <class Fill>
-static bool make_split_form(SplitForm& f, size_t bytes, Fill fill) {
-    std::lock_guard<std::mutex> lock(f.mutex);
-    if (f.ready || f.unfit) return f.ready;
-    if (!f.blob && !try_alloc(f.blob, bytes + sizeof(int))) return false;
-    int* const beyond = reinterpret_cast<int*>(f.blob + bytes);  // set if any weight is out of range
+static bool make_split_form(SplitForm& f, size_t bytes, size_t& more, Fill fill) {
+    if (!f.blob && !(more && try_alloc(f.blob, bytes + more + sizeof(int)))) {
+        more = 0;
+        if (!try_alloc(f.blob, bytes + sizeof(int))) return false;
+    }
+    int* const beyond = reinterpret_cast<int*>(f.blob + bytes + more);  // set if any weight is out of range
     HIP_CHECK(hipMemset(beyond, 0, sizeof(int)));
     char* at = f.blob;
     fill([&](const float* src, int N, int K, bool gate_up) {
@@ -312,11 +326,105 @@ static bool make_split_form(SplitForm& f, size_t bytes, Fill fill) {
     return f.ready;
 }
 
+// Storage of a matrix in pairs: the blocks, its outputs' exponents, and the 2-norms of its rows.
+struct PairPlace {
+    char* w;
+    int* exponent;
+    float* norm;
+};
+
+static size_t pair_place_bytes(size_t N, size_t K) { return pair_bytes(N, K) + 2 * pair_rows(N) * sizeof(float); }
+
+static PairPlace place_pairs(char*& at, const float* src, int N, int K, bool gate_up) {
+    PairPlace p;
+    p.w = at;
+    p.exponent = reinterpret_cast<int*>(at + pair_bytes(N, K));
+    p.norm = reinterpret_cast<float*>(p.exponent + pair_rows(N));
+    at += pair_place_bytes(N, K);
+    pair_weights(src, N, K, gate_up, p.w, p.exponent, p.norm, nullptr);
+    return p;
+}
+
+// Sizes on the host, of which bounds are made: the largest magnitude of n values, and one that seven of eight of those
+// that are not zero reach (a mean would follow the largest).
+struct Size {
+    double top = 0.0, low = 0.0;
+};
+
+static Size size_of(const float* device, size_t n) {
+    std::vector<float> v(n);
+    HIP_CHECK(hipMemcpy(v.data(), device, n * sizeof(float), hipMemcpyDeviceToHost));
+    std::vector<double> sizes;
+    Size s;
+    bool nan = false;
+    for (const float x : v) {
+        const double size = std::fabs(static_cast<double>(x));
+        nan = nan || std::isnan(size);
+        s.top = std::fmax(s.top, size);
+        if (size > 0.0) sizes.push_back(size);
+    }
+    if (nan && std::isfinite(s.top)) return {std::nan(""), std::nan("")};
+    if (!sizes.empty()) {
+        const auto at = sizes.begin() + sizes.size() / 8;
+        std::nth_element(sizes.begin(), at, sizes.end());
+        s.low = *at;
+    }
+    return s;
+}
+
+// The power of two that takes values of at most `bound` below 2^15, if what most of them reach, `low`, lies within 2^24 of
+// it (a pair is off by 2^-51 of the bound at most); none for a bound that is no number or far from fp32's middle.
+static std::optional<int> pair_exponent(double bound, double low) {
+    if (bound == 0.0) return 0;
+    if (!(bound > 0x1p-90 && bound < 0x1p90) || !(low >= bound * 0x1p-24)) return std::nullopt;
+    return 14 - std::ilogb(bound);
+}
+
+// Largest magnitude and largest 2-norm of a norm's rows, and what most of their values reach.
+struct NormSize {
+    double top, norm, low;
+};
+
+static NormSize norm_size(const Shape& sh, const float* gamma, const float* beta) {
+    const size_t d = sh.d_model;
+    const Size g = size_of(gamma, d), b = sh.modern() ? Size{} : size_of(beta, d);
+    const double root = std::sqrt(static_cast<double>(d));
+    return {root * g.top + b.top, root * (g.top + b.top), g.low};
+}
+
+// The operands' powers of two, from bounds that hold for every input: a row of norm(x) has at most sqrt(d) times the
+// largest gain as its largest value and as its norm (and beta), an output at most that times its row of weights, an
+// average of values at most the largest of them, |gelu(z)| <= |z| and |silu(g) u| <= |g u|.  (fp32 roundings on
+// the way are far from the factor of two that is left to fp16's largest number.)
+static bool pair_bounds(const Shape& sh, const LayerWeights& w, const PairPlace& qkv, const PairPlace& ffn1, PairLayer& l) {
+    const size_t d = sh.d_model, F = sh.d_ff();
+    const NormSize n1 = norm_size(sh, w.g1, w.be1), n2 = norm_size(sh, w.g2, w.be2);
+    const Size wv = size_of(qkv.norm + 2 * d, d), bv = size_of(w.bqkv + 2 * d, d);
+    const Size w1 = size_of(ffn1.norm, (sh.modern() ? 2 : 1) * F), b1 = sh.modern() ? Size{} : size_of(w.b1, F);
+    const double value = wv.top * n1.norm + bv.top, unit = w1.top * n2.norm + b1.top;
+    const double low_value = wv.low * n1.low, low_unit = w1.low * n2.low;
+    const auto norm1 = pair_exponent(n1.top, n1.low), norm2 = pair_exponent(n2.top, n2.low);
+    const auto attn = pair_exponent(value, low_value / 64);  // (an average of many is smaller than one of them)
+    const auto hidden = sh.modern() ? pair_exponent(unit * unit, low_unit * low_unit / 4) : pair_exponent(unit, low_unit / 4);
+    if (!norm1 || !norm2 || !attn || !hidden) return false;
+    l.norm1 = *norm1;
+    l.attn = *attn;
+    l.norm2 = *norm2;
+    l.hidden = *hidden;
+    return true;
+}
+
 static bool split_layers(const Model& m) {
+    std::lock_guard<std::mutex> lock(m.layers_split.mutex);
+    SplitForm& f = m.layers_split;
+    if (f.ready || f.unfit) return f.ready;
     const Shape& sh = m.shape;
     const int d = sh.d_model, F = sh.d_ff(), up = sh.modern() ? 2 : 1;
     const size_t per_layer = split_bytes(3 * d, d) + split_bytes(d, d) + split_bytes(up * F, d) + split_bytes(d, F);
-    return make_split_form(m.layers_split, sh.layers * per_layer, [&](auto place) {
+    const size_t pairs_per_layer =
+        pair_place_bytes(3 * d, d) + pair_place_bytes(d, d) + pair_place_bytes(up * F, d) + pair_place_bytes(d, F);
+    size_t more = d >= kPairMinCols ? sh.layers * pairs_per_layer : 0;
+    const bool made = make_split_form(f, sh.layers * per_layer, more, [&](auto place) {
         m.split_layers.clear();
         for (const LayerWeights& w : m.layers) {
             SplitLayer l;
@@ -327,11 +435,44 @@ static bool split_layers(const Model& m) {
             m.split_layers.push_back(l);
         }
     });
+    if (!made || !more) return made;
+    char* at = f.blob + sh.layers * per_layer;
+    m.pair_layers.clear();
+    bool fit = true;
+    for (const LayerWeights& w : m.layers) {
+        const PairPlace qkv = place_pairs(at, w.wqkv, 3 * d, d, false), o = place_pairs(at, w.wo, d, d, false);
+        const PairPlace ffn1 = place_pairs(at, w.w1, up * F, d, sh.modern()), ffn2 = place_pairs(at, w.w2, d, F, false);
+        PairLayer l{qkv.w, o.w, ffn1.w, ffn2.w, qkv.exponent, o.exponent, ffn1.exponent, ffn2.exponent, 0, 0, 0, 0};
+        // (W_o and FFN2 feed no operand, but an infinite weight has no pair either)
+        fit = fit && std::isfinite(size_of(o.norm, d).top) && std::isfinite(size_of(ffn2.norm, d).top)
+              && std::isfinite(size_of(qkv.norm, 2 * d).top) && pair_bounds(sh, w, qkv, ffn1, l);
+        m.pair_layers.push_back(l);
+    }
+    f.pairs = fit;
+    return true;
 }
 
 static bool split_logits(const Model& m) {
-    return make_split_form(m.logits_split, split_bytes(m.shape.vocab, m.shape.d_model),
-                           [&](auto place) { place(m.E, m.shape.vocab, m.shape.d_model, false); });
+    std::lock_guard<std::mutex> lock(m.logits_split.mutex);
+    SplitForm& f = m.logits_split;
+    if (f.ready || f.unfit) return f.ready;
+    const Shape& sh = m.shape;
+    const int d = sh.d_model, V = sh.vocab;
+    const NormSize n = norm_size(sh, m.gf, m.bf);
+    const std::optional<int> norm = pair_exponent(n.top, n.low);
+    if (d >= kPairMinCols && norm) {
+        if (!try_alloc(f.blob, pair_place_bytes(V, d))) return false;
+        char* at = f.blob;
+        const PairPlace e = place_pairs(at, m.E, V, d, false);
+        m.logits_exponent = e.exponent;
+        m.logits_norm = *norm;
+        f.ready = f.pairs = !std::isinf(size_of(e.norm, V).top);
+        if (f.ready) return true;
+        HIP_CHECK(hipFree(f.blob));
+        f.blob = nullptr;
+    }
+    size_t more = 0;
+    return make_split_form(f, split_bytes(V, d), more, [&](auto place) { place(m.E, V, d, false); });
 }
 
 static std::unique_ptr<Model> upload_model(const Shape& shape, const std::vector<const float*>& t,
@@ -1815,22 +1956,33 @@ static bool prompt_pass_ok(const Session& s, int len) {
 // What that keeps is the replies, not precision: the split sums are the closer ones to float64.
 constexpr int kSplitMinRows = 512, kSplitMinScoreRows = 160;
 
+// Operands of a split pass go in pairs (kernels_pair.h) wherever the model has them, except in front of draws from
+// the whole row, for the reason above: those replies stay what three parts made of their prompts.  (With a
+// cut at k of a flat distribution a draw has k boundaries to fall beside, not 16000.)
+constexpr int kWholeRowTopK = 1024;
+
+static bool draws_from_whole_row(const gh_sampling& o) {
+    return !o.greedy && (o.top_k <= 0 || o.top_k > kWholeRowTopK);
+}
+
 // How a pass over len tokens of every sequence runs: in slices of `slice` tokens (0: token by
 // token), those of split_rows rows and more on the split weights.
 struct RowsPlan {
     int slice;
     int split_rows;
+    bool pairs;  // ... those in two parts each, not in three
 };
 
 // Decided before anything is launched.  Weights without a split form, or no memory for it, leave the small fp32 tiles,
 // in slices below the rows from which the split projections take over (the tiles' buffers hold no
 // more), and for scoring, whose logits come from the split matrix alone, the token-by-token way.
-static RowsPlan plan_rows(const Session& s, int len, bool score) {
-    if (!prompt_pass_ok(s, len) || (score && !split_logits(*s.m))) return {0, 0};
+static RowsPlan plan_rows(const Session& s, int len, bool score, bool whole_row_draws) {
+    if (!prompt_pass_ok(s, len) || (score && !split_logits(*s.m))) return {0, 0, false};
     const int most = static_cast<int>(std::max<size_t>(1, std::min<size_t>(len, kPromptPassRows / s.B)));
     const int split_rows = score ? kSplitMinScoreRows : kSplitMinRows;
-    if (static_cast<long>(most) * s.B < split_rows || split_layers(*s.m)) return {most, split_rows};
-    return {std::min(len, (kSplitMinRows - 1) / s.B), kSplitMinRows};
+    if (static_cast<long>(most) * s.B < split_rows) return {most, split_rows, false};
+    if (split_layers(*s.m)) return {most, split_rows, s.m->layers_split.pairs && !whole_row_draws};
+    return {std::min(len, (kSplitMinRows - 1) / s.B), kSplitMinRows, false};
 }
 
 // One projection over M rows (norm folded in for RMSNorm, a norm kernel for LayerNorm).
@@ -1868,21 +2020,43 @@ static SplitGemmParams split_params(const char* A, const char* W, int M, int N, 
     return g;
 }
 
+// What a product of pairs needs beside its operands: the exponents of W's outputs and the power of two of A.
+static void pair_params(SplitGemmParams& g, const int* exponent, int operand) {
+    g.exponent = exponent;
+    g.operand_exponent = -operand;
+}
+
+template <int EPI>
+static void split_project(Session& s, bool pairs, SplitGemmParams& g) {
+    if (pairs) pair_gemm<EPI>(g, s.stream);
+    else split_gemm<EPI>(g, s.stream);
+}
+
+// norm(pp_x) as an operand.
+static void split_norm(Session& s, bool pairs, const float* gamma, const float* beta, int operand, int M) {
+    const Shape& sh = s.m->shape;
+    if (pairs)
+        norm_pair(sh.modern(), s.pp_x, gamma, beta, s.pp_split, M, sh.d_model, std::ldexp(1.0f, operand), s.stream);
+    else norm_split(sh.modern(), s.pp_x, gamma, beta, s.pp_split, M, sh.d_model, s.stream);
+}
+
 // Final norm, logits and the target's negative log-likelihood for rows
 // pp_x[0 .. M) of a slice (row m = seq * n + t, position t0 + t).  The logits are not
 // stored: every run of outputs leaves its maximum and its sum of exponentials.
 static void score_rows(Session& s, const ScoreSink& sink, int M, int n, int t0, int len) {
     const Model& m = *s.m;
     const Shape& sh = m.shape;
-    norm_split(sh.modern(), s.pp_x, m.gf, m.bf, s.pp_split, M, sh.d_model, s.stream);
+    const bool pairs = m.logits_split.pairs;
+    split_norm(s, pairs, m.gf, m.bf, m.logits_norm, M);
     SplitGemmParams g = split_params(s.pp_split, m.logits_split.blob, M, sh.vocab, sh.d_model);
+    if (pairs) pair_params(g, m.logits_exponent, m.logits_norm);
     g.rows_per_seq = n;
     g.targets = sink.targets;
     g.nll_t0 = t0;
     g.nll_len = len;
     g.nll_part = s.nll_part;
     g.nll_target = s.nll_target;
-    split_gemm<EPI_STORE>(g, s.stream);
+    split_project<EPI_STORE>(s, pairs, g);
     nll_parts(g, sink.nll, s.stream);
 }
 
@@ -1929,20 +2103,23 @@ static void launch_prompt_attn(const Session& s, const PrefillAttnParams& a) {
     HIP_CHECK(hipGetLastError());
 }
 
-// One layer over M = n * B rows of pp_x through the split projections, and with split_attn through the
-// split attention.  keys_only: nothing but the keys and values.
-static void prompt_layer_split(Session& s, int layer, int n, int pos_base, bool split_attn, bool keys_only) {
+// One layer over M = n * B rows of pp_x through the split projections, operands in pairs or in three parts, and with
+// split_attn through the split attention.  keys_only: nothing but the keys and values.
+static void prompt_layer_split(Session& s, int layer, int n, int pos_base, bool pairs, bool split_attn, bool keys_only) {
     const Model& m = *s.m;
     const Shape& sh = m.shape;
     const LayerWeights& w = m.layers[layer];
     const SplitLayer& sw = m.split_layers[layer];
+    const PairLayer pw = pairs ? m.pair_layers[layer] : PairLayer{};
     const int d = sh.d_model, F = sh.d_ff(), M = n * s.B;
     hipStream_t st = s.stream;
 
-    norm_split(sh.modern(), s.pp_x, w.g1, w.be1, s.pp_split, M, d, st);
-    SplitGemmParams g = split_params(s.pp_split, sw.wqkv, M, 3 * d, d);
+    split_norm(s, pairs, w.g1, w.be1, pw.norm1, M);
+    SplitGemmParams g = split_params(s.pp_split, pairs ? pw.wqkv : sw.wqkv, M, 3 * d, d);
+    pair_params(g, pw.eqkv, pw.norm1);
     if (keys_only) {
-        g.W += static_cast<size_t>(d / kSplitRows) * (d / kSplitCols) * kSplitBlockBytes;
+        g.W += static_cast<size_t>(d / kSplitRows) * (d / kSplitCols) * (pairs ? kPairBlockBytes : kSplitBlockBytes);
+        if (pairs) g.exponent += d;
         g.N = 2 * d;
         g.first = d;
     }
@@ -1957,33 +2134,38 @@ static void prompt_layer_split(Session& s, int layer, int n, int pos_base, bool 
     g.rope_sin = m.rope_sin;
     g.rows_per_seq = n;
     g.pos_base = pos_base;
-    split_gemm<EPI_QKV>(g, st);
+    split_project<EPI_QKV>(s, pairs, g);
     if (keys_only) return;
 
     PrefillAttnParams a = prompt_attn_params(s, layer, n, pos_base);
     a.out_split = s.pp_split;
+    a.pair_scale = pairs ? std::ldexp(1.0f, pw.attn) : 0.0f;
     if (split_attn) split_attention(a, s.B, s.pp_kv, s.pp_kv_bytes, s.pp_part, st);
     else launch_prompt_attn(s, a);
 
-    g = split_params(s.pp_split, sw.wo, M, d, d);
+    g = split_params(s.pp_split, pairs ? pw.wo : sw.wo, M, d, d);
+    pair_params(g, pw.eo, pw.attn);
     g.bias = w.bo;
     g.out = s.pp_x;
     g.out_stride = d;
-    split_gemm<EPI_RESID>(g, st);
+    split_project<EPI_RESID>(s, pairs, g);
 
-    norm_split(sh.modern(), s.pp_x, w.g2, w.be2, s.pp_split, M, d, st);
-    g = split_params(s.pp_split, sw.w1, M, sh.modern() ? 2 * F : F, d);
+    split_norm(s, pairs, w.g2, w.be2, pw.norm2, M);
+    g = split_params(s.pp_split, pairs ? pw.w1 : sw.w1, M, sh.modern() ? 2 * F : F, d);
+    pair_params(g, pw.e1, pw.norm2);
+    g.pair_scale = std::ldexp(1.0f, pw.hidden);
     g.bias = sh.modern() ? nullptr : w.b1;
     g.out_split = s.pp_split_hidden;
     g.out_kblocks = F / kSplitCols;
-    if (sh.modern()) split_gemm<EPI_SWIGLU>(g, st);
-    else split_gemm<EPI_GELU>(g, st);
+    if (sh.modern()) split_project<EPI_SWIGLU>(s, pairs, g);
+    else split_project<EPI_GELU>(s, pairs, g);
 
-    g = split_params(s.pp_split_hidden, sw.w2, M, d, F);
+    g = split_params(s.pp_split_hidden, pairs ? pw.w2 : sw.w2, M, d, F);
+    pair_params(g, pw.e2, pw.hidden);
     g.bias = sh.modern() ? nullptr : w.b2;
     g.out = s.pp_x;
     g.out_stride = d;
-    split_gemm<EPI_RESID>(g, st);
+    split_project<EPI_RESID>(s, pairs, g);
 }
 
 // The same layer through the decode step's small fp32 tiles (few rows).
@@ -2145,7 +2327,7 @@ static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSi
         // else at the last position alone, where the decode step's launches are as good.
         const bool trim = split && !sink;
         for (int l = 0; l < sh.layers; l++) {
-            if (split) prompt_layer_split(s, l, n, pos_base, split_attn, trim && l == sh.layers - 1);
+            if (split) prompt_layer_split(s, l, n, pos_base, plan.pairs, split_attn, trim && l == sh.layers - 1);
             else prompt_layer_small(s, l, n, pos_base);
         }
         if (sink) score_rows(s, *sink, M, n, t0, len);
@@ -2170,9 +2352,9 @@ static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSi
 
 // Steps through `len` tokens already staged in the history at n_hist.. (the
 // prompt loop of text_gen.cpp:44-46).  log: per-step logits destination or null.
-static void run_prompt(Session& s, int len, float* log, size_t* steps_logged) {
+static void run_prompt(Session& s, int len, float* log, size_t* steps_logged, bool whole_row_draws = false) {
     const size_t BV = static_cast<size_t>(s.B) * s.m->shape.vocab;
-    const RowsPlan plan = log ? RowsPlan{0, 0} : plan_rows(s, len, /*score=*/false);
+    const RowsPlan plan = log ? RowsPlan{0, 0, false} : plan_rows(s, len, /*score=*/false, whole_row_draws);
     if (plan.slice > 0) {
         prompt_pass(s, len, plan);
         if (steps_logged) *steps_logged += len;
@@ -2826,7 +3008,7 @@ gh_status gh_session_score(gh_session* sess, const int32_t* ids, const int32_t* 
         }
         stage_ids(s, host_targets, len, s.score_targets, len, 0);
         const ScoreSink sink{s.score_targets, s.score_nll};
-        const RowsPlan plan = plan_rows(s, len, /*score=*/true);
+        const RowsPlan plan = plan_rows(s, len, /*score=*/true, /*whole_row_draws=*/false);
         run_resident(s, [&] {
             if (plan.slice > 0) {
                 prompt_pass(s, len, plan, &sink);
@@ -3139,7 +3321,7 @@ gh_status gh_session_generate(gh_session* sess, const int32_t* prompts, int32_t 
         run_resident(s, [&] {
             steps = 0;
             HIP_CHECK(hipEventRecord(s.ev[0], s.stream));
-            run_prompt(s, prompt_len, log, &steps);
+            run_prompt(s, prompt_len, log, &steps, draws_from_whole_row(*opt));
             HIP_CHECK(hipEventRecord(s.ev[1], s.stream));
             s.ahead = Session::AHEAD_PROMPT;
             std::tie(made, stepped) = run_decode(s, max_tokens, *opt, du, max_tokens, seed, log, &steps);

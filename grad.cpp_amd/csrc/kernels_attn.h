@@ -7,7 +7,7 @@
 // softmax_row (:60-67).
 #pragma once
 
-#include "kernels_split.h"
+#include "kernels_pair.h"
 
 namespace gh {
 
@@ -429,7 +429,8 @@ __global__ __launch_bounds__(256) void attn_decode64_kernel(const AttnParams p) 
 struct PrefillAttnParams {
     const float* q;  // [batch * len][d_model], rotated
     float* out;      // [batch * len][d_model]
-    char* out_split;  // when set: the output rows in split form instead (split_offset)
+    char* out_split;  // when set: the output rows as an operand instead (store_operand4)
+    float pair_scale;  // of that operand, 0: in three parts
     KvLayout kv;
     int layer, d_model, len, pos_base;
     float scale;
@@ -560,8 +561,8 @@ static __global__ __launch_bounds__(256) void attn_prefill64_kernel(const Prefil
         if (p.out_split) {
 #pragma unroll
             for (int db = 0; db < 4; db++)
-                store_split4(p.out_split, b * p.len + t, h * HS + db * 16 + g * 4, p.d_model / kSplitCols, o[db][0] * inv,
-                             o[db][1] * inv, o[db][2] * inv, o[db][3] * inv);
+                store_operand4(p.out_split, b * p.len + t, h * HS + db * 16 + g * 4, p.d_model / kSplitCols, o[db][0] * inv,
+                               o[db][1] * inv, o[db][2] * inv, o[db][3] * inv, p.pair_scale);
             return;
         }
         float* orow = p.out + (static_cast<size_t>(b) * p.len + t) * p.d_model + h * HS;
@@ -684,7 +685,8 @@ static __global__ __launch_bounds__(256) void attn_prefill16_kernel(const Prefil
         const float inv = 1.0f / l;
         const int at = h * HS + wave * 16 + g * 4;
         if (p.out_split) {
-            store_split4(p.out_split, b * p.len + t, at, p.d_model / kSplitCols, o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv);
+            store_operand4(p.out_split, b * p.len + t, at, p.d_model / kSplitCols, o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv,
+                           p.pair_scale);
         } else {
             *reinterpret_cast<float4*>(p.out + (static_cast<size_t>(b) * p.len + t) * p.d_model + at) =
                 make_float4(o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv);

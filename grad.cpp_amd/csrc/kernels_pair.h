@@ -1,0 +1,351 @@
+// Projections over many rows on the fp16 matrix cores: every fp32 operand as the sum of two fp16
+// numbers, three products of parts for one fp32 product.
+//
+//   a 2^s = a1 + a2,  a1 = fp16(a 2^s), a2 = fp16(a 2^s - a1)
+//
+// What that costs and what pays for it.  a1 + a2 holds 22 bits and a sign, so a value is at most one unit
+// of its 24th bit away (a quarter of all values are; half a unit rms, where rounding to fp32 leaves 0.29),
+// and a2 b2 (2^-22 of the product at most) is left out: 7.5e-8 of a dot product's size, whatever its length.
+// The six products of the exact three-part form (kernels_split.h) lose nothing there, but their sums are K / 16 terms
+// added one after the other, and those roundings grow with K.  Here every 64 columns are summed from zero and
+// then added to the running sum: 12 and K / 64 roundings.  The matrix cores cut the low bits of what they
+// align, downwards: a bias of 2e-8 (K = 768) to 4e-8 (2048) of the result, the same in every row, which an attention over
+// many positions would not average out; so the weights of every other 64 columns are stored negated and their
+// sums subtracted (what is left is below 1e-9).  Error over the size of the result against float64, 512 x 512
+// outputs, normal operands / gated hidden units times normal weights, three parts -> two: K = 512 1.27e-7 -> 1.26e-7
+// / 1.44e-7 -> 1.28e-7, 768 1.59e-7 -> 1.32e-7 / 1.76e-7 -> 1.33e-7, 2048 2.71e-7 -> 1.55e-7 / 2.90e-7 -> 1.57e-7,
+// 3072 3.39e-7 -> 1.71e-7 / 3.55e-7 -> 1.72e-7 (an fp32 sum of one product after the other: 4.0e-7 to 9.9e-7).  Below K = 512
+// the three parts are the closer ones (256: 0.89e-7 against 1.20e-7), so narrower models keep them (kPairMinCols).
+//
+// The range.  fp16 has exponents -14 to 15 and, below, numbers of fewer bits (the matrix cores take them as
+// they are).  Weights are scaled row by row so that a row's largest lies in [2^14, 2^15).  Activations have one power of two
+// per operand, from a bound that holds for every input (pair_bounds in engine.hip): nothing can
+// overflow, and how far a bound lies above what occurs costs nothing: a2 of an activation is
+// stored 2^11 larger, and meets a1 of the weight 2^-11 smaller, so that an activation keeps its 22 bits down to
+// 2^-29 of the bound, and a weight down to 2^-17 of its row's largest; what is smaller is off by 2^-51 of the
+// bound, or 2^-40 of the row's largest.  Models whose bounds lie further above what occurs than that leaves room
+// for keep the three parts.
+//
+// Why: a third fewer bytes per operand and half the products.  In turn on one box, 128 x 128 tiles, operands of
+// full-length significands: 16384 x 768 x 3072 180 -> 342 TFLOP/s of fp32 products, 24576 x 4096 x 768 180 -> 277,
+// 1999 x 768 x 2048 136 -> 198 (best tile of either).
+#pragma once
+
+#include "kernels_split.h"
+
+namespace gh {
+
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+constexpr int kPairMinCols = 512;
+constexpr int kPairStages = 4;  // of the ring of steps; also the steps of a part
+
+// Storage of a matrix of pairs (rows x K, K a multiple of 16): blocks of 16 rows x 16 columns, 1024
+// contiguous bytes each, row group by row group and inside one along K.  A block is the first parts of columns
+// 0..7 of its 16 rows (16 bytes each), those of columns 8..15, and the second parts likewise: 16 lanes that read
+// an operand's 16 rows read 256 consecutive bytes of LDS.
+constexpr int kPairBlockBytes = 1024, kPairPartBytes = 512, kPairChunkBytes = 256;
+
+// Byte offset of the first part of column k (a multiple of 8) of row r.
+__device__ __forceinline__ size_t pair_offset(int r, int k, int kblocks) {
+    return (static_cast<size_t>(r >> 4) * kblocks + (k >> 4)) * kPairBlockBytes + ((k >> 3) & 1) * kPairChunkBytes + (r & 15) * 16;
+}
+
+// Sign that the weights of block `block` of a row are stored with.
+__host__ __device__ __forceinline__ float pair_sign(int block) { return (block & kPairStages) ? -1.0f : 1.0f; }
+
+constexpr float kPairLift = 2048.0f;  // 2^11, of an activation's second part
+
+__device__ __forceinline__ void to_pair(float x, float lift, _Float16& first, _Float16& second) {
+    first = static_cast<_Float16>(x);
+    second = static_cast<_Float16>((x - static_cast<float>(first)) * lift);
+}
+
+// Eight consecutive columns (k a multiple of 8) of one row of activations.
+__device__ __forceinline__ void store_pair8(char* base, int r, int k, int kblocks, const float (&v)[8], float scale) {
+    v8h p1, p2;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        _Float16 a, b;
+        to_pair(v[i] * scale, kPairLift, a, b);
+        p1[i] = a;
+        p2[i] = b;
+    }
+    char* at = base + pair_offset(r, k, kblocks);
+    *reinterpret_cast<v8h*>(at) = p1;
+    *reinterpret_cast<v8h*>(at + kPairPartBytes) = p2;
+}
+
+// Four consecutive columns (k a multiple of 4).
+__device__ __forceinline__ void store_pair4(char* base, int r, int k, int kblocks, float x, float y, float z, float w, float scale) {
+    typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+    const float v[4] = {x, y, z, w};
+    v4h p1, p2;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        _Float16 a, b;
+        to_pair(v[i] * scale, kPairLift, a, b);
+        p1[i] = a;
+        p2[i] = b;
+    }
+    char* at = base + pair_offset(r, k & ~7, kblocks) + (k & 4) * 2;
+    *reinterpret_cast<v4h*>(at) = p1;
+    *reinterpret_cast<v4h*>(at + kPairPartBytes) = p2;
+}
+
+// Four consecutive columns of a row of activations, in the form that the projection behind reads: pairs scaled by
+// pair_scale, three parts where that is zero.
+__device__ __forceinline__ void store_operand4(char* base, int r, int k, int kblocks, float x, float y, float z, float w,
+                                               float pair_scale) {
+    if (pair_scale != 0.0f) store_pair4(base, r, k, kblocks, x, y, z, w, pair_scale);
+    else store_split4(base, r, k, kblocks, x, y, z, w);
+}
+
+// Writes the pairs of a weight matrix src (N x K, row per output), rows in the order of split_weights_kernel, one
+// wavefront per row, zeros past N.  exponent[j]: the power of two that output j's sum is to be multiplied by, j as the
+// product counts them; norm[n]: the 2-norm of row n of src, infinite if the row has no pairs: a weight is infinite, or
+// more than an eighth of them (zeros aside) lie 2^14 and more below the largest.
+static __global__ __launch_bounds__(256) void pair_weights_kernel(const float* __restrict__ src, int N, int K, int rows,
+                                                                  int gate_up, char* dst, int* exponent, float* norm) {
+    const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const int out = split_output_of_row(row);  // as the product hands it back
+    const int n = gate_up ? (out & ~15) + 2 * (out & 7) + ((out >> 3) & 1) : out;
+    const float* const w = src + static_cast<size_t>(min(n, N - 1)) * K;
+    float top = 0.0f;
+    for (int k = lane * 4; k < K; k += 256) {
+        const float4 a = *reinterpret_cast<const float4*>(w + k);
+        top = fmaxf(fmaxf(top, fmaxf(fabsf(a.x), fabsf(a.y))), fmaxf(fabsf(a.z), fabsf(a.w)));
+    }
+    top = wave_max(top);
+    // the largest goes to [2^14, 2^15)
+    const int s = top > 0.0f && top < INFINITY ? min(14 - ilogbf(top), 126) : 0;
+    const float scale = ldexpf(1.0f, s);
+    float sum = 0.0f, some = 0.0f, most = 0.0f;  // weights that are not zero, and those within 2^14 of the largest
+    for (int k = lane * 4; k < K; k += 256) {
+        const float4 a = *reinterpret_cast<const float4*>(w + k);
+        const float v[4] = {a.x * scale, a.y * scale, a.z * scale, a.w * scale};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            sum += v[i] * v[i];
+            some += v[i] != 0.0f ? 1.0f : 0.0f;
+            most += fabsf(v[i]) >= 1.0f ? 1.0f : 0.0f;
+        }
+    }
+    sum = wave_sum(sum);
+    const bool fit = top < INFINITY && wave_sum(most) * 8.0f >= wave_sum(some) * 7.0f;
+    if (lane == 0) exponent[out] = out < N ? -s : 0;
+    if (lane == 0 && n < N) norm[n] = fit ? ldexpf(sqrtf(sum), -s) : INFINITY;
+    for (int k = lane * 8; k < K; k += 512) {
+        const float factor = scale * pair_sign(k >> 4);
+        v8h p1, p2;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            _Float16 a, b;
+            to_pair(n < N ? w[k + i] * factor : 0.0f, 1.0f, a, b);
+            p1[i] = a;
+            p2[i] = b;
+        }
+        char* at = dst + pair_offset(row, k, K >> 4);
+        *reinterpret_cast<v8h*>(at) = p1;
+        *reinterpret_cast<v8h*>(at + kPairPartBytes) = p2;
+    }
+}
+
+// norm(x) of every row as pairs: norm_split_kernel with its sums, and its rows in registers.
+template <bool RMS, int NI>
+static __global__ __launch_bounds__(1024) void norm_pair_kernel(const float* __restrict__ x, const float* __restrict__ gamma,
+                                                                const float* __restrict__ beta, char* out, int M, int d,
+                                                                float pair_scale) {
+    const int lane = threadIdx.x & 63;
+    const int m = blockIdx.x * 16 + (threadIdx.x >> 6);
+    if (m >= M) return;
+    norm_row<RMS, NI>(x + static_cast<size_t>(m) * d, gamma, beta, d, lane,
+                      [&](int k, const float(&o)[8]) { store_pair8(out, m, k, d / kSplitCols, o, pair_scale); });
+}
+
+template <bool RMS>
+static __global__ __launch_bounds__(1024) void norm_pair_long_kernel(const float* __restrict__ x, const float* __restrict__ gamma,
+                                                                     const float* __restrict__ beta, char* out, int M, int d,
+                                                                     float pair_scale) {
+    const int lane = threadIdx.x & 63;
+    const int m = blockIdx.x * 16 + (threadIdx.x >> 6);
+    if (m >= M) return;
+    norm_long_row<RMS>(x + static_cast<size_t>(m) * d, gamma, beta, d, lane,
+                       [&](int k, const float(&o)[8]) { store_pair8(out, m, k, d / kSplitCols, o, pair_scale); });
+}
+
+struct PairRowsOut {
+    static __device__ __forceinline__ void store8(const SplitGemmParams& p, int m, int k, const float (&v)[8]) {
+        store_pair8(p.out_split, m, k, p.out_kblocks, v, p.pair_scale);
+    }
+};
+
+// C[M,N] = A[M,K] . W[N,K]^T of pairs.  Tiles, workgroup order, LDS ring and epilogues are split_gemm_kernel's.
+// A step of 16 columns is three rounds of products (w1 a2, w2 a1, w1 a1), its fragments read from LDS during the
+// step before into registers of their own (a 64 x 64 wavefront has 128 of its 256 for sums).  Four steps make a
+// 64-column part that starts from zero; it is added to the running sums (or taken from them, the weights of every
+// other part being negative) in front of the next part's first products, one accumulator at a time, so that this
+// runs beside the other accumulators' products.  K / KG is a multiple of 64.
+template <int EPI, int MB, int NB, int WM, int WN, int KG, int PER_CU>
+__global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void pair_gemm_kernel(const SplitGemmParams p) {
+    extern __shared__ __attribute__((aligned(1024))) char lds_pair[];
+    constexpr int kWaves = WM * WN, TM = 32 * MB * WM, TN = 32 * NB * WN, kStages = kPairStages;
+    constexpr int kUnitsA = TM / 16, kUnits = (TM + TN) / 16;  // 1024-byte loads of a step: a block each
+    constexpr int kLoads = kUnits / kWaves;                    // ... per wavefront
+    constexpr int kStage = kUnits * 1024;
+    static_assert(kUnits % kWaves == 0, "every wavefront has as many loads");
+    static_assert((KG - 1) * TM * TN * 4 <= KG * kStages * kStage, "the sums fit in the rings");
+    const int lane = threadIdx.x & 63, wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = wave_id / kWaves, wave = wave_id % kWaves;
+    const int wm = wave / WN, wn = wave % WN;
+    int m_tile, n_tile;
+    if (!split_tile(p, m_tile, n_tile)) return;
+    const int row_blocks = p.K / kSplitCols, kblocks = row_blocks / KG;  // of a row, of this set of wavefronts
+    const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) char*)lds_pair))
+                          + kg * (kStages * kStage);
+    const char* a_base = p.A + (static_cast<size_t>(m_tile) * kUnitsA * row_blocks + kg * kblocks) * kPairBlockBytes;
+    const char* w_base = p.W + (static_cast<size_t>(n_tile) * (kUnits - kUnitsA) * row_blocks + kg * kblocks) * kPairBlockBytes;
+    // this wavefront's loads: units wave, wave + kWaves, ... of a step's image in LDS (the row groups of A, then those of W)
+    unsigned src[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; i++) {
+        const int u = wave + i * kWaves;
+        src[i] = (u < kUnitsA ? u : u - kUnitsA) * (row_blocks * kPairBlockBytes) + lane * 16;
+    }
+    const auto issue_one = [&](int i, int step, int stage) {
+        const int u = wave + i * kWaves;
+        const char* at = (u < kUnitsA ? a_base : w_base) + static_cast<size_t>(step) * kPairBlockBytes;
+        load_to_lds(at, src[i], lds0 + stage * kStage + u * 1024);
+    };
+    // operand reads: row lane % 32 of a 32-row block, columns 8 (lane / 32) .. + 7
+    const int r32 = lane & 31, h32 = lane >> 5;
+    const char* const frag = lds_pair + kg * (kStages * kStage) + (r32 >> 4) * kPairBlockBytes + h32 * kPairChunkBytes + (r32 & 15) * 16;
+    v8h a1[2][MB], a2[2][MB], w1[2][NB], w2[2][NB];  // fragments of even and odd steps
+    const auto read_a = [&](int stage, int part, v8h (&f)[MB]) {
+#pragma unroll
+        for (int x = 0; x < MB; x++)
+            f[x] = *reinterpret_cast<const v8h*>(frag + stage * kStage + part * kPairPartBytes + (wm * MB + x) * 2 * kPairBlockBytes);
+    };
+    const auto read_w = [&](int stage, int part, v8h (&f)[NB]) {
+#pragma unroll
+        for (int x = 0; x < NB; x++)
+            f[x] = *reinterpret_cast<const v8h*>(frag + stage * kStage + part * kPairPartBytes
+                                                 + (kUnitsA + (wn * NB + x) * 2) * kPairBlockBytes);
+    };
+    v16f sum[NB][MB], part[NB][MB], zero;
+#pragma unroll
+    for (int r = 0; r < 16; r++) zero[r] = 0.0f;
+#pragma unroll
+    for (int a = 0; a < NB; a++)
+#pragma unroll
+        for (int b = 0; b < MB; b++) sum[a][b] = part[a][b] = zero;
+    const auto multiply = [&](const v8h (&w)[NB], const v8h (&x)[MB]) {
+#pragma unroll
+        for (int a = 0; a < NB; a++)
+#pragma unroll
+            for (int b = 0; b < MB; b++) part[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[a], x[b], part[a][b], 0, 0, 0);
+    };
+    float sign = 1.0f;  // of the part at hand, then of the one before
+    const auto add_part = [&](v16f& to, const v16f& v) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) to[r] = __builtin_fmaf(v[r], sign, to[r]);
+    };
+
+#pragma unroll
+    for (int s = 0; s < kStages; s++)
+#pragma unroll
+        for (int i = 0; i < kLoads; i++) issue_one(i, s, s);
+    wait_loads<(kStages - 1) * kLoads>();
+    meet();
+    read_w(0, 0, w1[0]);
+    read_a(0, 1, a2[0]);
+    read_w(0, 1, w2[0]);
+    read_a(0, 0, a1[0]);
+    for (int s0 = 0; s0 < kblocks; s0 += kStages) {
+#pragma unroll
+        for (int t = 0; t < kStages; t++) {  // step s0 + t, in place t of the ring
+            constexpr int kPer = (kLoads + 2) / 3;
+            const int c = t & 1, n = c ^ 1, next = (t + 1) % kStages;
+            const bool more = s0 + t + kStages < kblocks;
+            const auto send = [&](int q) {  // a third of the loads of the step that comes to this place next
+                if (more) {
+#pragma unroll
+                    for (int i = q * kPer; i < (q + 1) * kPer; i++)
+                        if (i < kLoads) issue_one(i, s0 + t + kStages, t);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            if (s0 + t + kStages - 1 < kblocks) wait_loads<(kStages - 2) * kLoads>();  // the next step is here
+            else wait_loads<0>();
+            meet();  // ... for everyone, and everyone has read this step's place
+            v8h low[NB];
+#pragma unroll
+            for (int a = 0; a < NB; a++) low[a] = w1[c][a] * static_cast<_Float16>(1.0f / kPairLift);
+#pragma unroll
+            for (int a = 0; a < NB; a++)
+#pragma unroll
+                for (int b = 0; b < MB; b++) {
+                    if (t == 0) add_part(sum[a][b], part[a][b]);
+                    part[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(low[a], a2[c][b], t == 0 ? zero : part[a][b], 0, 0, 0);
+                }
+            if (t == 0) sign = pair_sign(kg * kblocks + s0);
+            read_w(next, 0, w1[n]);
+            read_a(next, 1, a2[n]);
+            send(0);
+            multiply(w2[c], a1[c]);
+            read_w(next, 1, w2[n]);
+            send(1);
+            multiply(w1[c], a1[c]);
+            read_a(next, 0, a1[n]);
+            send(2);
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < NB; a++)
+#pragma unroll
+        for (int b = 0; b < MB; b++) add_part(sum[a][b], part[a][b]);
+    if constexpr (KG > 1) {
+        // the other sets' sums through the LDS the rings no longer need, added in order
+        float* sums = reinterpret_cast<float*>(lds_pair);
+        const auto at = [&](int g, int a, int b) { return sums + (((g - 1) * kWaves + wave) * NB * MB + a * MB + b) * 1024 + lane; };
+        __syncthreads();
+        if (kg > 0) {
+#pragma unroll
+            for (int a = 0; a < NB; a++)
+#pragma unroll
+                for (int b = 0; b < MB; b++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) at(kg, a, b)[r * 64] = sum[a][b][r];
+        }
+        __syncthreads();
+        if (kg > 0) return;
+#pragma unroll
+        for (int g = 1; g < KG; g++)
+#pragma unroll
+            for (int a = 0; a < NB; a++)
+#pragma unroll
+                for (int b = 0; b < MB; b++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) sum[a][b][r] += at(g, a, b)[r * 64];
+    }
+    const int n0 = n_tile * TN + wn * 32 * NB;
+#pragma unroll
+    for (int a = 0; a < NB; a++) {
+        // (storage of exponents for whole tiles, as of the weights)
+        const int4* const e = reinterpret_cast<const int4*>(p.exponent + n0 + 32 * a + 16 * h32);
+        int es[16];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int4 v = e[q];
+            es[4 * q] = v.x, es[4 * q + 1] = v.y, es[4 * q + 2] = v.z, es[4 * q + 3] = v.w;
+        }
+#pragma unroll
+        for (int b = 0; b < MB; b++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) sum[a][b][r] = ldexpf(sum[a][b][r], es[r] + p.operand_exponent);
+    }
+    split_epilogue<PairRowsOut, EPI, MB, NB>(p, sum, m_tile * TM + wm * 32 * MB, n0, n_tile * WN + wn);
+}
+
+}  // namespace gh

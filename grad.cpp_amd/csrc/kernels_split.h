@@ -136,18 +136,11 @@ static __global__ __launch_bounds__(256) void split_weights_kernel(const float* 
     store_split8(dst, row, k, K / kSplitCols, v);
 }
 
-// h = norm(x) of every row in split form (layer_norm_row, inference.cpp:30-58).  One
-// wavefront per row, 16 rows per workgroup: the workgroup writes whole blocks.  A row stays
-// in registers: NI chunks of eight columns per lane, d <= 512 NI.
-template <bool RMS, int NI>
-static __global__ __launch_bounds__(1024) void norm_split_kernel(const float* __restrict__ x,
-                                                                 const float* __restrict__ gamma,
-                                                                 const float* __restrict__ beta, char* out, int M,
-                                                                 int d) {
-    const int lane = threadIdx.x & 63;
-    const int m = blockIdx.x * 16 + (threadIdx.x >> 6);
-    if (m >= M) return;
-    const float* xr = x + static_cast<size_t>(m) * d;
+// norm(x) of a row (layer_norm_row, inference.cpp:30-58) by one wavefront; store(k, v) takes
+// columns k .. k + 7.  The row stays in registers: NI chunks of eight columns per lane, d <= 512 NI.
+template <bool RMS, int NI, class Store>
+__device__ __forceinline__ void norm_row(const float* __restrict__ xr, const float* __restrict__ gamma,
+                                         const float* __restrict__ beta, int d, int lane, Store store) {
     const int chunks = d >> 3;
     float v[NI][8];
     float s = 0.0f;
@@ -190,21 +183,15 @@ static __global__ __launch_bounds__(1024) void norm_split_kernel(const float* __
             o[e] = gamma[c * 8 + e] * v[i][e] * scale;
             if (!RMS) o[e] += beta[c * 8 + e];
         }
-        store_split8(out, m, c * 8, d / kSplitCols, o);
+        store(c * 8, o);
     }
 }
 
-// The same for rows that do not fit the registers: one pass over the row per sum and one to write,
+// The same for a row that does not fit the registers: one pass over it per sum and one to write,
 // the later ones from the L2.
-template <bool RMS>
-static __global__ __launch_bounds__(1024) void norm_split_long_kernel(const float* __restrict__ x,
-                                                                      const float* __restrict__ gamma,
-                                                                      const float* __restrict__ beta, char* out, int M,
-                                                                      int d) {
-    const int lane = threadIdx.x & 63;
-    const int m = blockIdx.x * 16 + (threadIdx.x >> 6);
-    if (m >= M) return;
-    const float* xr = x + static_cast<size_t>(m) * d;
+template <bool RMS, class Store>
+__device__ __forceinline__ void norm_long_row(const float* __restrict__ xr, const float* __restrict__ gamma,
+                                              const float* __restrict__ beta, int d, int lane, Store store) {
     float s = 0.0f;
     for (int k = lane * 4; k < d; k += 256) {
         const float4 a = *reinterpret_cast<const float4*>(xr + k);
@@ -229,8 +216,31 @@ static __global__ __launch_bounds__(1024) void norm_split_long_kernel(const floa
             o[e] = gamma[k + e] * (xr[k + e] - mean) * scale;
             if (!RMS) o[e] += beta[k + e];
         }
-        store_split8(out, m, k, d / kSplitCols, o);
+        store(k, o);
     }
+}
+
+// h = norm(x) of every row in split form, 16 rows per workgroup: it writes whole blocks.
+template <bool RMS, int NI>
+static __global__ __launch_bounds__(1024) void norm_split_kernel(const float* __restrict__ x,
+                                                                 const float* __restrict__ gamma,
+                                                                 const float* __restrict__ beta, char* out, int M,
+                                                                 int d) {
+    const int m = blockIdx.x * 16 + (threadIdx.x >> 6);
+    if (m >= M) return;
+    norm_row<RMS, NI>(x + static_cast<size_t>(m) * d, gamma, beta, d, threadIdx.x & 63,
+                      [&](int k, const float(&o)[8]) { store_split8(out, m, k, d / kSplitCols, o); });
+}
+
+template <bool RMS>
+static __global__ __launch_bounds__(1024) void norm_split_long_kernel(const float* __restrict__ x,
+                                                                      const float* __restrict__ gamma,
+                                                                      const float* __restrict__ beta, char* out, int M,
+                                                                      int d) {
+    const int m = blockIdx.x * 16 + (threadIdx.x >> 6);
+    if (m >= M) return;
+    norm_long_row<RMS>(x + static_cast<size_t>(m) * d, gamma, beta, d, threadIdx.x & 63,
+                       [&](int k, const float(&o)[8]) { store_split8(out, m, k, d / kSplitCols, o); });
 }
 
 struct SplitGemmParams {
@@ -243,6 +253,10 @@ struct SplitGemmParams {
     int out_stride;
     char* out_split;  // EPI_GELU, EPI_SWIGLU: split rows of out_cols columns
     int out_kblocks;
+    // operands in pairs (kernels_pair.h)
+    const int* exponent;   // per output, of the weights
+    int operand_exponent;  // of A
+    float pair_scale;      // of the rows at out_split
     // EPI_QKV (rows of a prompt pass, as in GemvParams); outputs first .. first + N of the fused product
     int first;
     KvLayout kv;
@@ -282,6 +296,143 @@ __device__ __forceinline__ void meet() {
     asm volatile("" ::: "memory");
 }
 
+// The workgroup's tile.  Workgroup ids go round-robin over the eight XCDs: every XCD takes a contiguous run of
+// tiles, eight row tiles deep inside a column of outputs, so that what its workgroups read
+// at about the same time is the same few tiles of both operands.  False: there is none for it.
+__device__ __forceinline__ bool split_tile(const SplitGemmParams& p, int& m_tile, int& n_tile) {
+    const int per = (p.tiles + 7) >> 3, id = blockIdx.x;
+    const int tile = (id & 7) * per + (id >> 3);
+    if ((id >> 3) >= per || tile >= p.tiles) return false;
+    const int m_tiles = p.tiles / p.n_tiles;
+    const int group = tile / (8 * p.n_tiles), rest = tile - group * 8 * p.n_tiles;
+    const int deep = min(8, m_tiles - group * 8);
+    n_tile = rest / deep;
+    m_tile = group * 8 + rest - n_tile * deep;
+    return true;
+}
+
+// How the split projections leave rows of the next one's operand.
+struct SplitRowsOut {
+    static __device__ __forceinline__ void store8(const SplitGemmParams& p, int m, int k, const float (&v)[8]) {
+        store_split8(p.out_split, m, k, p.out_kblocks, v);
+    }
+};
+
+// What becomes of a wavefront's outputs, straight from the accumulators: register r of acc[a][b] is output
+// n0 + 32 a + 16 (lane / 32) + r of row m0 + 32 b + lane % 32.  nll_at: the wavefront's run of outputs (EPI_STORE).
+template <class Rows, int EPI, int MB, int NB>
+__device__ __forceinline__ void split_epilogue(const SplitGemmParams& p, const v16f (&acc)[NB][MB], int m0, int n0, int nll_at) {
+    const int lane = threadIdx.x & 63, r32 = lane & 31, h32 = lane >> 5;
+#pragma unroll
+    for (int b = 0; b < MB; b++) {
+        const int m = m0 + 32 * b + r32;
+        if constexpr (EPI == EPI_STORE) {
+            // scored logits: no store, the row's running maximum and sum of exponentials
+            float mx = -INFINITY;
+            int target = -1;
+            if (m < p.M) {
+                const int seq = m / p.rows_per_seq, t = m - seq * p.rows_per_seq;
+                target = p.targets[static_cast<size_t>(seq) * p.nll_len + p.nll_t0 + t];
+            }
+#pragma unroll
+            for (int a = 0; a < NB; a++) {
+                const int n = n0 + 32 * a + 16 * h32;
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    if (n + r < p.N) mx = fmaxf(mx, acc[a][b][r]);
+                    if (n + r == target) p.nll_target[m] = acc[a][b][r];
+                }
+            }
+            mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+            const float base = mx == -INFINITY ? 0.0f : mx;  // (nothing but -inf here: a mass of 0)
+            float sum = 0.0f;
+#pragma unroll
+            for (int a = 0; a < NB; a++) {
+                const int n = n0 + 32 * a + 16 * h32;
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    if (n + r < p.N) sum += expf(acc[a][b][r] - base);
+            }
+            sum += __shfl_xor(sum, 32, kWave);
+            if (m < p.M && h32 == 0)
+                p.nll_part[static_cast<size_t>(m) * p.nll_stride + nll_at] = make_float2(mx, sum);
+        } else {
+            if (m >= p.M) continue;
+            int pos = 0, page = 0;
+            if constexpr (EPI == EPI_QKV) {
+                const int seq = m / p.rows_per_seq;
+                pos = p.pos_base + (m - seq * p.rows_per_seq);
+                page = p.kv.page_table[seq * p.kv.pages_per_seq + (pos >> p.kv.page_shift)];
+            }
+#pragma unroll
+            for (int a = 0; a < NB; a++) {
+                const int n = n0 + 32 * a + 16 * h32;
+                if (n >= p.N) continue;
+                float v[16];
+#pragma unroll
+                for (int r = 0; r < 16; r++) v[r] = acc[a][b][r];
+                if constexpr (EPI == EPI_RESID) {
+                    // y += b, then y += x @ W (inference.cpp:22-28)
+                    float4* out = reinterpret_cast<float4*>(p.out + static_cast<size_t>(m) * p.out_stride + n);
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        float4 c = out[q];
+                        if (p.bias) {
+                            const float4 bb = *reinterpret_cast<const float4*>(p.bias + n + 4 * q);
+                            c = make_float4(c.x + bb.x, c.y + bb.y, c.z + bb.z, c.w + bb.w);
+                        }
+                        out[q] = make_float4(c.x + v[4 * q], c.y + v[4 * q + 1], c.z + v[4 * q + 2], c.w + v[4 * q + 3]);
+                    }
+                } else if constexpr (EPI == EPI_GELU) {
+                    float o[2][8];
+#pragma unroll
+                    for (int r = 0; r < 16; r++) o[r >> 3][r & 7] = gelu_tanh(v[r] + p.bias[n + r]);
+                    Rows::store8(p, m, n, o[0]);
+                    Rows::store8(p, m, n + 8, o[1]);
+                } else if constexpr (EPI == EPI_SWIGLU) {
+                    float o[8];
+#pragma unroll
+                    for (int r = 0; r < 8; r++) o[r] = v[8 + r] * silu(v[r]);
+                    Rows::store8(p, m, n >> 1, o);
+                } else if constexpr (EPI == EPI_QKV) {
+                    const int sec = (p.first + n) / p.d_model, c = p.first + n - sec * p.d_model, head = c >> 6, j = c & 63;
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const float4 bb = *reinterpret_cast<const float4*>(p.bias + p.first + n + 4 * q);
+                        v[4 * q] += bb.x, v[4 * q + 1] += bb.y, v[4 * q + 2] += bb.z, v[4 * q + 3] += bb.w;
+                    }
+                    if (p.rope && sec < 2) {
+                        const float* cs = p.rope_cos + pos * 32 + (j >> 1);
+                        const float* sn = p.rope_sin + pos * 32 + (j >> 1);
+#pragma unroll
+                        for (int q = 0; q < 2; q++) {
+                            const float4 c4 = *reinterpret_cast<const float4*>(cs + 4 * q);
+                            const float4 s4 = *reinterpret_cast<const float4*>(sn + 4 * q);
+                            const float cc[4] = {c4.x, c4.y, c4.z, c4.w}, ss[4] = {s4.x, s4.y, s4.z, s4.w};
+#pragma unroll
+                            for (int e = 0; e < 4; e++) {
+                                const float x = v[8 * q + 2 * e], y = v[8 * q + 2 * e + 1];
+                                v[8 * q + 2 * e] = x * cc[e] - y * ss[e];
+                                v[8 * q + 2 * e + 1] = x * ss[e] + y * cc[e];
+                            }
+                        }
+                    }
+                    float* dst;
+                    if (sec == 0) {
+                        dst = p.out + static_cast<size_t>(m) * p.out_stride + c;
+                    } else {
+                        const size_t run = ((static_cast<size_t>(p.layer) * p.kv.n_pages + page) * 2 + (sec - 1)) * p.kv.heads + head;
+                        dst = p.kv.pool + ((run << p.kv.page_shift) + (pos & ((1 << p.kv.page_shift) - 1))) * 64 + j;
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        reinterpret_cast<float4*>(dst)[q] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+                }
+            }
+        }
+    }
+}
+
 // C[M,N] = A[M,K] . W[N,K]^T, operands split.  A workgroup of WM x WN wavefronts owns
 // 32 MB WM rows and 32 NB WN outputs, a wavefront 32 MB x 32 NB of them in accumulators of
 // 32 x 32 (outputs along the matrix rows, so a lane holds one row of activations).  Operands
@@ -300,20 +451,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
     const int lane = threadIdx.x & 63, wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kg = wave_id / kWaves, wave = wave_id % kWaves;
     const int wm = wave / WN, wn = wave % WN;
-    // Workgroup ids go round-robin over the eight XCDs: every XCD takes a contiguous run of
-    // tiles, eight row tiles deep inside a column of outputs, so that what its workgroups read
-    // at about the same time is the same few tiles of both operands.
-    const int per = (p.tiles + 7) >> 3, id = blockIdx.x;
-    const int tile = (id & 7) * per + (id >> 3);
-    if ((id >> 3) >= per || tile >= p.tiles) return;
     int m_tile, n_tile;
-    {
-        const int m_tiles = p.tiles / p.n_tiles;
-        const int group = tile / (8 * p.n_tiles), rest = tile - group * 8 * p.n_tiles;
-        const int deep = min(8, m_tiles - group * 8);
-        n_tile = rest / deep;
-        m_tile = group * 8 + rest - n_tile * deep;
-    }
+    if (!split_tile(p, m_tile, n_tile)) return;
     const int row_blocks = p.K / kSplitCols, kblocks = row_blocks / KG;  // of a row, of this set of wavefronts
     const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) char*)lds_split))
                           + kg * (STAGES * kStage);
@@ -452,117 +591,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
                     for (int r = 0; r < 16; r++) acc[a][b][r] += at(g, a, b)[r * 64];
     }
 
-    // Epilogue, straight from the accumulators: register r of acc[a][b] is output
-    // n0 + 32 a + 16 h32 + r of row m0 + 32 b + r32.
-    const int m0 = m_tile * TM + wm * 32 * MB, n0 = n_tile * TN + wn * 32 * NB;
-#pragma unroll
-    for (int b = 0; b < MB; b++) {
-        const int m = m0 + 32 * b + r32;
-        if constexpr (EPI == EPI_STORE) {
-            // scored logits: no store, the row's running maximum and sum of exponentials
-            float mx = -INFINITY;
-            int target = -1;
-            if (m < p.M) {
-                const int seq = m / p.rows_per_seq, t = m - seq * p.rows_per_seq;
-                target = p.targets[static_cast<size_t>(seq) * p.nll_len + p.nll_t0 + t];
-            }
-#pragma unroll
-            for (int a = 0; a < NB; a++) {
-                const int n = n0 + 32 * a + 16 * h32;
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    if (n + r < p.N) mx = fmaxf(mx, acc[a][b][r]);
-                    if (n + r == target) p.nll_target[m] = acc[a][b][r];
-                }
-            }
-            mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-            const float base = mx == -INFINITY ? 0.0f : mx;  // (nothing but -inf here: a mass of 0)
-            float sum = 0.0f;
-#pragma unroll
-            for (int a = 0; a < NB; a++) {
-                const int n = n0 + 32 * a + 16 * h32;
-#pragma unroll
-                for (int r = 0; r < 16; r++)
-                    if (n + r < p.N) sum += expf(acc[a][b][r] - base);
-            }
-            sum += __shfl_xor(sum, 32, kWave);
-            if (m < p.M && h32 == 0)
-                p.nll_part[static_cast<size_t>(m) * p.nll_stride + n_tile * WN + wn] = make_float2(mx, sum);
-        } else {
-            if (m >= p.M) continue;
-            int pos = 0, page = 0;
-            if constexpr (EPI == EPI_QKV) {
-                const int seq = m / p.rows_per_seq;
-                pos = p.pos_base + (m - seq * p.rows_per_seq);
-                page = p.kv.page_table[seq * p.kv.pages_per_seq + (pos >> p.kv.page_shift)];
-            }
-#pragma unroll
-            for (int a = 0; a < NB; a++) {
-                const int n = n0 + 32 * a + 16 * h32;
-                if (n >= p.N) continue;
-                float v[16];
-#pragma unroll
-                for (int r = 0; r < 16; r++) v[r] = acc[a][b][r];
-                if constexpr (EPI == EPI_RESID) {
-                    // y += b, then y += x @ W (inference.cpp:22-28)
-                    float4* out = reinterpret_cast<float4*>(p.out + static_cast<size_t>(m) * p.out_stride + n);
-#pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        float4 c = out[q];
-                        if (p.bias) {
-                            const float4 bb = *reinterpret_cast<const float4*>(p.bias + n + 4 * q);
-                            c = make_float4(c.x + bb.x, c.y + bb.y, c.z + bb.z, c.w + bb.w);
-                        }
-                        out[q] = make_float4(c.x + v[4 * q], c.y + v[4 * q + 1], c.z + v[4 * q + 2], c.w + v[4 * q + 3]);
-                    }
-                } else if constexpr (EPI == EPI_GELU) {
-                    float o[2][8];
-#pragma unroll
-                    for (int r = 0; r < 16; r++) o[r >> 3][r & 7] = gelu_tanh(v[r] + p.bias[n + r]);
-                    store_split8(p.out_split, m, n, p.out_kblocks, o[0]);
-                    store_split8(p.out_split, m, n + 8, p.out_kblocks, o[1]);
-                } else if constexpr (EPI == EPI_SWIGLU) {
-                    float o[8];
-#pragma unroll
-                    for (int r = 0; r < 8; r++) o[r] = v[8 + r] * silu(v[r]);
-                    store_split8(p.out_split, m, n >> 1, p.out_kblocks, o);
-                } else if constexpr (EPI == EPI_QKV) {
-                    const int sec = (p.first + n) / p.d_model, c = p.first + n - sec * p.d_model, head = c >> 6, j = c & 63;
-#pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        const float4 bb = *reinterpret_cast<const float4*>(p.bias + p.first + n + 4 * q);
-                        v[4 * q] += bb.x, v[4 * q + 1] += bb.y, v[4 * q + 2] += bb.z, v[4 * q + 3] += bb.w;
-                    }
-                    if (p.rope && sec < 2) {
-                        const float* cs = p.rope_cos + pos * 32 + (j >> 1);
-                        const float* sn = p.rope_sin + pos * 32 + (j >> 1);
-#pragma unroll
-                        for (int q = 0; q < 2; q++) {
-                            const float4 c4 = *reinterpret_cast<const float4*>(cs + 4 * q);
-                            const float4 s4 = *reinterpret_cast<const float4*>(sn + 4 * q);
-                            const float cc[4] = {c4.x, c4.y, c4.z, c4.w}, ss[4] = {s4.x, s4.y, s4.z, s4.w};
-#pragma unroll
-                            for (int e = 0; e < 4; e++) {
-                                const float x = v[8 * q + 2 * e], y = v[8 * q + 2 * e + 1];
-                                v[8 * q + 2 * e] = x * cc[e] - y * ss[e];
-                                v[8 * q + 2 * e + 1] = x * ss[e] + y * cc[e];
-                            }
-                        }
-                    }
-                    float* dst;
-                    if (sec == 0) {
-                        dst = p.out + static_cast<size_t>(m) * p.out_stride + c;
-                    } else {
-                        const size_t run = ((static_cast<size_t>(p.layer) * p.kv.n_pages + page) * 2 + (sec - 1)) * p.kv.heads + head;
-                        dst = p.kv.pool + ((run << p.kv.page_shift) + (pos & ((1 << p.kv.page_shift) - 1))) * 64 + j;
-                    }
-#pragma unroll
-                    for (int q = 0; q < 4; q++)
-                        reinterpret_cast<float4*>(dst)[q] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
-                }
-            }
-        }
-    }
+    split_epilogue<SplitRowsOut, EPI, MB, NB>(p, acc, m_tile * TM + wm * 32 * MB, n_tile * TN + wn * 32 * NB, n_tile * WN + wn);
 }
 
 // nll of a scored row from what the logits launch left of it: log of the sum of all

@@ -2,7 +2,7 @@
 // projections (kernels_split.h): six bf16 products for one fp32 product, head size 64.
 #pragma once
 
-#include "kernels_split.h"
+#include "kernels_pair.h"
 
 namespace gh {
 
@@ -62,7 +62,8 @@ struct SplitAttnParams {
     const float* q;  // [batch * len][d_model], rotated
     const char* kv;  // split_kv_kernel's tiles
     int tiles;       // ... per pair
-    char* out;       // split rows [batch * len] x d_model
+    char* out;       // operand rows [batch * len] x d_model
+    float pair_scale;  // ... of pairs, 0: in three parts
     float* part;     // partial results of query blocks whose keys are shared among workgroups
     int d_model, heads, len, pos_base;
     int chunk_shift;  // a workgroup takes up to 1 << chunk_shift tiles of keys
@@ -312,8 +313,8 @@ static __global__ __launch_bounds__(256, 2) void attn_split_kernel(const SplitAt
     for (int db = 0; db < 2; db++)
 #pragma unroll
         for (int q4 = 0; q4 < 4; q4++)
-            store_split4(p.out, b * p.len + t, h * 64 + db * 32 + q4 * 8 + h32 * 4, p.d_model / kSplitCols, o[db][4 * q4] * inv,
-                         o[db][4 * q4 + 1] * inv, o[db][4 * q4 + 2] * inv, o[db][4 * q4 + 3] * inv);
+            store_operand4(p.out, b * p.len + t, h * 64 + db * 32 + q4 * 8 + h32 * 4, p.d_model / kSplitCols, o[db][4 * q4] * inv,
+                           o[db][4 * q4 + 1] * inv, o[db][4 * q4 + 2] * inv, o[db][4 * q4 + 3] * inv, p.pair_scale);
 }
 
 // Folds the partial results of a query block, in the order of the keys.  A chain of trips to memory, one per
@@ -365,8 +366,8 @@ static __global__ __launch_bounds__(256) void attn_split_merge_kernel(const Spli
     const float inv = 1.0f / l;
 #pragma unroll
     for (int q = 0; q < 2; q++)
-        store_split4(p.out, b * p.len + t, h * 64 + r0 * 2 + q * 8 + h32 * 4, p.d_model / kSplitCols, o[4 * q] * inv, o[4 * q + 1] * inv,
-                     o[4 * q + 2] * inv, o[4 * q + 3] * inv);
+        store_operand4(p.out, b * p.len + t, h * 64 + r0 * 2 + q * 8 + h32 * 4, p.d_model / kSplitCols, o[4 * q] * inv,
+                       o[4 * q + 1] * inv, o[4 * q + 2] * inv, o[4 * q + 3] * inv, p.pair_scale);
 }
 
 }  // namespace gh

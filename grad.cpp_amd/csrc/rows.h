@@ -23,6 +23,15 @@ void norm_split(bool rms, const float* x, const float* gamma, const float* beta,
 template <int EPI>
 void split_gemm(SplitGemmParams& p, hipStream_t st);
 
+// The same three in pairs (kernels_pair.h); exponents of a matrix: one per row of its storage.
+inline size_t pair_rows(size_t rows) { return (rows + kSplitPad - 1) / kSplitPad * kSplitPad; }
+inline size_t pair_bytes(size_t rows, size_t cols) { return pair_rows(rows) * cols * 4; }
+void pair_weights(const float* src, int N, int K, bool gate_up, char* dst, int* exponent, float* norm, hipStream_t st);
+void norm_pair(bool rms, const float* x, const float* gamma, const float* beta, char* out, int M, int d, float pair_scale,
+               hipStream_t st);
+template <int EPI>
+void pair_gemm(SplitGemmParams& p, hipStream_t st);
+
 // Causal attention of p.len new positions of every sequence over the cache, output rows in split form.
 // kv: scratch of kv_bytes, at least one (sequence, head) pair's keys and values; the pairs go in groups
 // that fit.  split_attention_kv_bytes: what is worth giving for so many filled positions.

@@ -156,6 +156,7 @@ void split_attention(const PrefillAttnParams& a, int batch, char* kv, size_t kv_
     p.kv = kv;
     p.tiles = (positions + 63) / 64;
     p.out = a.out_split;
+    p.pair_scale = a.pair_scale;
     p.part = part;
     p.d_model = a.d_model;
     p.heads = heads;

@@ -19,7 +19,7 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-fno-fast-math", "-Wall", "-Wno-unused-function", *os.environ.get("GRADHIP_EXTRA_FLAGS", "").split(),
 ]
-SOURCES = ["engine.hip", "persist.hip", "xcd.hip", "resident.hip", "rows.hip", "checkpoint.cpp", "tokenizer.cpp"]
+SOURCES = ["engine.hip", "persist.hip", "xcd.hip", "resident.hip", "rows.hip", "pairs.hip", "checkpoint.cpp", "tokenizer.cpp"]
 OBJ_DIR = os.path.join(PKG, "build")
 
 

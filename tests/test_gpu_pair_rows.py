@@ -1,0 +1,125 @@
+"""Passes over many rows whose operands are two fp16 parts each (models of 512 columns and more): every tiling and
+epilogue at row counts that leave ragged tiles, operands at the ends of their range, and models whose weights have
+no such form, against the float64 forward.  The bounds are what fp32 sums give, as for the three-part form."""
+import numpy as np
+import pytest
+
+import gradhip as G
+import ref_forward
+from gradhip import synth
+from helpers import lively_std
+
+pytestmark = pytest.mark.gpu
+
+
+def _loss(ref, targets):
+    top = ref.max(axis=1)
+    return np.log(np.exp(ref - top[:, None]).sum(axis=1)) + top - ref[np.arange(len(targets)), targets]
+
+
+def _check(cfg, W, B, n, seed, sequences=None):
+    tokens = synth.uniform_tokens(B * (n + 1), cfg.vocab, seed).reshape(B, n + 1)
+    gm = G.Model.from_tensors(cfg, W)
+    nll = G.Session(gm, batch=B).score(tokens[:, :-1], tokens[:, 1:])
+    last = G.Session(gm, batch=B).prefill(tokens[:, :-1])
+    for b in sequences or sorted({0, B - 1}):
+        with np.errstate(over="ignore"):
+            ref = ref_forward.forward(cfg, W, tokens[b, :-1])
+        want = _loss(ref, tokens[b, 1:])
+        assert np.abs(nll[b] - want).max() <= 2e-5 * max(1.0, np.abs(want).max()), b
+        assert np.abs(last[b] - ref[-1]).max() <= 1e-5 * np.abs(ref[-1]).max(), b
+
+
+CASES = {
+    # name: (width, vocab, sequences, tokens)
+    "32-wide tiles, K in four sets": (512, 130, 1, 161),
+    "64-wide tiles, K in four sets": (512, 1001, 3, 171),
+    "64-wide tiles, one row past a tile": (768, 515, 1, 577),
+    "no whole parts for four sets of K": (576, 130, 1, 161),  # 36 blocks of 16 columns
+    "nine parts, one set of K": (576, 301, 5, 193),
+    "128 x 64 tiles, a nearly empty one": (768, 130, 3, 449),
+    "128-wide tiles, several rounds": (768, 301, 11, 487),
+}
+
+
+@pytest.mark.parametrize("arch", [synth.ARCH_GPT2, synth.ARCH_MODERN])
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_rows_match_the_float64_forward(name, arch):
+    d, vocab, B, n = CASES[name]
+    cfg = synth.Config(arch, vocab, d, 1, d // 64, 600)
+    _check(cfg, synth.make_weights(cfg, 101, std=lively_std(cfg), norm_noise=0.1), B, n, 102)
+
+
+@pytest.mark.parametrize("arch", [synth.ARCH_GPT2, synth.ARCH_MODERN])
+def test_rows_of_one_large_element_reach_the_bound_of_the_norm(arch):
+    """norm(x) of a row with one element that outweighs the rest is sqrt(d) there: the largest an operand can be."""
+    cfg = synth.Config(arch, 67, 512, 2, 8, 600)
+    W = synth.make_weights(cfg, 103, std=lively_std(cfg), norm_noise=0.1)
+    W[0][np.arange(67), np.arange(67) * 7] += 1e4
+    _check(cfg, W, 1, 530, 104)
+
+
+def test_operands_far_below_their_bound():
+    """Gains of 1/50 to 50 in one norm: what most operands hold lies 2^-10 and more below the bound."""
+    cfg = synth.Config(synth.ARCH_GPT2, 67, 512, 2, 8, 600)
+    W = synth.make_weights(cfg, 105, std=lively_std(cfg), norm_noise=0.1)
+    names = [what[0] for what in synth.tensor_specs(cfg)]
+    for layer in range(2):
+        W[names.index(f"layer {layer} norm2 gamma")][0, :] = np.geomspace(0.02, 3.0, 512)
+        W[names.index(f"layer {layer} norm2 gamma")][0, 5] = 50.0
+    _check(cfg, W, 1, 530, 106)
+
+
+@pytest.mark.parametrize("gain", [1e6, 1e30])
+def test_a_gain_too_far_above_the_others_for_two_parts(gain):
+    """One gain so large that bounds say nothing about the rest (the weights behind it are zero): three parts."""
+    cfg = synth.Config(synth.ARCH_MODERN, 67, 512, 1, 8, 600)
+    W = synth.make_weights(cfg, 107, std=lively_std(cfg), norm_noise=0.1)
+    names = [what[0] for what in synth.tensor_specs(cfg)]
+    W[names.index("layer 0 norm2 gamma")][0, 5] = gain
+    W[names.index("layer 0 FFN gate")][5, :] = 0.0
+    W[names.index("layer 0 FFN up")][5, :] = 0.0
+    _check(cfg, W, 1, 530, 108)
+
+
+def test_weights_at_both_ends_of_the_range():
+    """A row of weights below fp32's normal numbers, one of zeros, one of 1e12 (what comes of it is not used, but bounds
+    have to count with it), and a weight 2^20 times the rest of its row."""
+    cfg = synth.Config(synth.ARCH_GPT2, 67, 512, 1, 8, 600)
+    W = synth.make_weights(cfg, 109, std=lively_std(cfg), norm_noise=0.1)
+    names = [what[0] for what in synth.tensor_specs(cfg)]
+    up, down = names.index("layer 0 FFN W1"), names.index("layer 0 FFN W2")
+    W[up][:, 3] = 1e-40
+    W[up][:, 4] = 0.0
+    W[up][:, 6] = 1e12
+    W[down][6, :] = 0.0
+    W[up][9, 7] *= 2.0 ** 20
+    W[down][7, :] *= 2.0 ** -20
+    _check(cfg, W, 1, 530, 110)
+
+
+def test_infinite_and_nan_weights_keep_their_meaning():
+    cfg = synth.Config(synth.ARCH_GPT2, 301, 512, 1, 8, 200)
+    W = synth.make_weights(cfg, 111, std=lively_std(cfg), norm_noise=0.1)
+    W[0][300, 5] = -np.inf
+    W[-1][0, 5] = 30.0  # beta of the final norm: that logit is -inf at every position
+    tokens = synth.uniform_tokens(172, 300, 112)
+    want = _loss(ref_forward.forward(cfg, W, tokens[:-1]), tokens[1:])
+    nll = G.Session(G.Model.from_tensors(cfg, W)).score(tokens[:-1], tokens[1:])[0]
+    assert np.abs(nll - want).max() <= 2e-5 * max(1.0, np.abs(want).max())
+    W[0][300, 5] = np.nan
+    assert np.isnan(G.Session(G.Model.from_tensors(cfg, W)).score(tokens[:-1], tokens[1:])).all()
+
+
+def test_a_prompt_in_front_of_draws_from_the_whole_row():
+    """Its operands stay in three parts; prefill's are two.  Both are within fp32 sums of one another: greedy picks,
+    with margins far above that, are the same behind either."""
+    cfg = synth.Config(synth.ARCH_MODERN, 130, 512, 2, 8, 640)
+    gm = G.Model.from_tensors(cfg, synth.make_weights(cfg, 113, std=lively_std(cfg), norm_noise=0.1))
+    prompt = synth.uniform_tokens(600, cfg.vocab, 114)
+    for opt in (G.sampling(1e-3, 0, 1.0, 1.0), G.sampling(1.0, 0, 1.0, 1.0, True)):  # temperature 1e-3: the arg-max
+        picks, s = [], G.Session(gm)
+        s.prefill(prompt)
+        s.decode_stream(12, opt, lambda ids, index: picks.append(ids[0]), seed=5)
+        tokens = G.Session(gm).generate(prompt, 12, opt, seed=5)
+        assert np.array_equal(np.asarray(tokens)[0, 600:], picks)
