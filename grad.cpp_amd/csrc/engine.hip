@@ -152,12 +152,12 @@ struct SplitLayer {
 };
 
 // The same matrices in pairs (kernels_pair.h), each with its outputs' exponents, and the powers of two that the
-// operands of those products are scaled by: norm(x) in front of QKV, the attention's rows, norm(x) in front of FFN1,
-// the hidden units.
+// operands of those products are scaled by: norm(x) in front of QKV, keys, values and the attention's rows, norm(x) in front
+// of FFN1, the hidden units.
 struct PairLayer {
     char *wqkv, *wo, *w1, *w2;
     int *eqkv, *eo, *e1, *e2;
-    int norm1, attn, norm2, hidden;
+    int norm1, keys, attn, norm2, hidden;
 };
 
 // One allocation of split matrices.
@@ -401,13 +401,17 @@ static bool pair_bounds(const Shape& sh, const LayerWeights& w, const PairPlace&
     const NormSize n1 = norm_size(sh, w.g1, w.be1), n2 = norm_size(sh, w.g2, w.be2);
     const Size wv = size_of(qkv.norm + 2 * d, d), bv = size_of(w.bqkv + 2 * d, d);
     const Size w1 = size_of(ffn1.norm, (sh.modern() ? 2 : 1) * F), b1 = sh.modern() ? Size{} : size_of(w.b1, F);
+    const Size wk = size_of(qkv.norm + d, d), bk = size_of(w.bqkv + d, d);
+    const double key = std::sqrt(2.0) * (wk.top * n1.norm + bk.top);  // (a rotated pair is as long as it was)
     const double value = wv.top * n1.norm + bv.top, unit = w1.top * n2.norm + b1.top;
-    const double low_value = wv.low * n1.low, low_unit = w1.low * n2.low;
+    const double low_key = wk.low * n1.low, low_value = wv.low * n1.low, low_unit = w1.low * n2.low;
     const auto norm1 = pair_exponent(n1.top, n1.low), norm2 = pair_exponent(n2.top, n2.low);
+    const auto keys = pair_exponent(key, low_key);
     const auto attn = pair_exponent(value, low_value / 64);  // (an average of many is smaller than one of them)
     const auto hidden = sh.modern() ? pair_exponent(unit * unit, low_unit * low_unit / 4) : pair_exponent(unit, low_unit / 4);
-    if (!norm1 || !norm2 || !attn || !hidden) return false;
+    if (!norm1 || !norm2 || !keys || !attn || !hidden) return false;
     l.norm1 = *norm1;
+    l.keys = *keys;
     l.attn = *attn;
     l.norm2 = *norm2;
     l.hidden = *hidden;
@@ -442,7 +446,7 @@ static bool split_layers(const Model& m) {
     for (const LayerWeights& w : m.layers) {
         const PairPlace qkv = place_pairs(at, w.wqkv, 3 * d, d, false), o = place_pairs(at, w.wo, d, d, false);
         const PairPlace ffn1 = place_pairs(at, w.w1, up * F, d, sh.modern()), ffn2 = place_pairs(at, w.w2, d, F, false);
-        PairLayer l{qkv.w, o.w, ffn1.w, ffn2.w, qkv.exponent, o.exponent, ffn1.exponent, ffn2.exponent, 0, 0, 0, 0};
+        PairLayer l{qkv.w, o.w, ffn1.w, ffn2.w, qkv.exponent, o.exponent, ffn1.exponent, ffn2.exponent, 0, 0, 0, 0, 0};
         // (W_o and FFN2 feed no operand, but an infinite weight has no pair either)
         fit = fit && std::isfinite(size_of(o.norm, d).top) && std::isfinite(size_of(ffn2.norm, d).top)
               && std::isfinite(size_of(qkv.norm, 2 * d).top) && pair_bounds(sh, w, qkv, ffn1, l);
@@ -2140,6 +2144,7 @@ static void prompt_layer_split(Session& s, int layer, int n, int pos_base, bool 
     PrefillAttnParams a = prompt_attn_params(s, layer, n, pos_base);
     a.out_split = s.pp_split;
     a.pair_scale = pairs ? std::ldexp(1.0f, pw.attn) : 0.0f;
+    a.key_scale = std::ldexp(1.0f, pw.keys);
     if (split_attn) split_attention(a, s.B, s.pp_kv, s.pp_kv_bytes, s.pp_part, st);
     else launch_prompt_attn(s, a);
 

@@ -431,6 +431,7 @@ struct PrefillAttnParams {
     float* out;      // [batch * len][d_model]
     char* out_split;  // when set: the output rows as an operand instead (store_operand4)
     float pair_scale;  // of that operand, 0: in three parts
+    float key_scale;   // split attention in pairs: a power of two that no key exceeds fp16 with
     KvLayout kv;
     int layer, d_model, len, pos_base;
     float scale;

@@ -56,41 +56,44 @@ __host__ __device__ __forceinline__ float pair_sign(int block) { return (block &
 
 constexpr float kPairLift = 2048.0f;  // 2^11, of an activation's second part
 
-__device__ __forceinline__ void to_pair(float x, float lift, _Float16& first, _Float16& second) {
-    first = static_cast<_Float16>(x);
-    second = static_cast<_Float16>((x - static_cast<float>(first)) * lift);
+// Two values as two words of two fp16 each (low half: the first value's part).  The first parts are hidden from the
+// compiler once they are made: it would form them a second time, by an instruction that rounds halves the other way, for
+// the subtraction.
+__device__ __forceinline__ void to_pairs(float x, float y, float lift, unsigned& first, unsigned& second) {
+    typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+    first = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f{x, y}), v2h));
+    asm("" : "+v"(first));
+    const v2h f = __builtin_bit_cast(v2h, first);
+    second = __builtin_bit_cast(
+        unsigned, __builtin_convertvector((v2f{(x - static_cast<float>(f[0])) * lift, (y - static_cast<float>(f[1])) * lift}), v2h));
 }
 
 // Eight consecutive columns (k a multiple of 8) of one row of activations.
 __device__ __forceinline__ void store_pair8(char* base, int r, int k, int kblocks, const float (&v)[8], float scale) {
-    v8h p1, p2;
+    v4u p1, p2;
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        _Float16 a, b;
-        to_pair(v[i] * scale, kPairLift, a, b);
+    for (int i = 0; i < 4; i++) {
+        unsigned a, b;
+        to_pairs(v[2 * i] * scale, v[2 * i + 1] * scale, kPairLift, a, b);
         p1[i] = a;
         p2[i] = b;
     }
     char* at = base + pair_offset(r, k, kblocks);
-    *reinterpret_cast<v8h*>(at) = p1;
-    *reinterpret_cast<v8h*>(at + kPairPartBytes) = p2;
+    *reinterpret_cast<v4u*>(at) = p1;
+    *reinterpret_cast<v4u*>(at + kPairPartBytes) = p2;
 }
 
 // Four consecutive columns (k a multiple of 4).
 __device__ __forceinline__ void store_pair4(char* base, int r, int k, int kblocks, float x, float y, float z, float w, float scale) {
-    typedef _Float16 v4h __attribute__((ext_vector_type(4)));
-    const float v[4] = {x, y, z, w};
-    v4h p1, p2;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        _Float16 a, b;
-        to_pair(v[i] * scale, kPairLift, a, b);
-        p1[i] = a;
-        p2[i] = b;
-    }
+    v2u p1, p2;
+    unsigned a, b;
+    to_pairs(x * scale, y * scale, kPairLift, a, b);
+    p1[0] = a, p2[0] = b;
+    to_pairs(z * scale, w * scale, kPairLift, a, b);
+    p1[1] = a, p2[1] = b;
     char* at = base + pair_offset(r, k & ~7, kblocks) + (k & 4) * 2;
-    *reinterpret_cast<v4h*>(at) = p1;
-    *reinterpret_cast<v4h*>(at + kPairPartBytes) = p2;
+    *reinterpret_cast<v2u*>(at) = p1;
+    *reinterpret_cast<v2u*>(at + kPairPartBytes) = p2;
 }
 
 // Four consecutive columns of a row of activations, in the form that the projection behind reads: pairs scaled by
@@ -138,17 +141,18 @@ static __global__ __launch_bounds__(256) void pair_weights_kernel(const float* _
     if (lane == 0 && n < N) norm[n] = fit ? ldexpf(sqrtf(sum), -s) : INFINITY;
     for (int k = lane * 8; k < K; k += 512) {
         const float factor = scale * pair_sign(k >> 4);
-        v8h p1, p2;
+        v4u p1, p2;
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            _Float16 a, b;
-            to_pair(n < N ? w[k + i] * factor : 0.0f, 1.0f, a, b);
+        for (int i = 0; i < 4; i++) {
+            const float x = w[k + 2 * i], y = w[k + 2 * i + 1];
+            unsigned a, b;
+            to_pairs(n < N ? x * factor : 0.0f, n < N ? y * factor : 0.0f, 1.0f, a, b);
             p1[i] = a;
             p2[i] = b;
         }
         char* at = dst + pair_offset(row, k, K >> 4);
-        *reinterpret_cast<v8h*>(at) = p1;
-        *reinterpret_cast<v8h*>(at + kPairPartBytes) = p2;
+        *reinterpret_cast<v4u*>(at) = p1;
+        *reinterpret_cast<v4u*>(at + kPairPartBytes) = p2;
     }
 }
 
@@ -192,9 +196,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
     extern __shared__ __attribute__((aligned(1024))) char lds_pair[];
     constexpr int kWaves = WM * WN, TM = 32 * MB * WM, TN = 32 * NB * WN, kStages = kPairStages;
     constexpr int kUnitsA = TM / 16, kUnits = (TM + TN) / 16;  // 1024-byte loads of a step: a block each
-    constexpr int kLoads = kUnits / kWaves;                    // ... per wavefront
+    constexpr int kLoads = (kUnits + kWaves - 1) / kWaves;     // ... per wavefront
     constexpr int kStage = kUnits * 1024;
-    static_assert(kUnits % kWaves == 0, "every wavefront has as many loads");
     static_assert((KG - 1) * TM * TN * 4 <= KG * kStages * kStage, "the sums fit in the rings");
     const int lane = threadIdx.x & 63, wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kg = wave_id / kWaves, wave = wave_id % kWaves;
@@ -210,11 +213,11 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
     unsigned src[kLoads];
 #pragma unroll
     for (int i = 0; i < kLoads; i++) {
-        const int u = wave + i * kWaves;
+        const int u = min(wave + i * kWaves, kUnits - 1);  // (a load too many brings the last unit again)
         src[i] = (u < kUnitsA ? u : u - kUnitsA) * (row_blocks * kPairBlockBytes) + lane * 16;
     }
     const auto issue_one = [&](int i, int step, int stage) {
-        const int u = wave + i * kWaves;
+        const int u = min(wave + i * kWaves, kUnits - 1);
         const char* at = (u < kUnitsA ? a_base : w_base) + static_cast<size_t>(step) * kPairBlockBytes;
         load_to_lds(at, src[i], lds0 + stage * kStage + u * 1024);
     };

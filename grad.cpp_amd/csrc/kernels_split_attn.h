@@ -21,15 +21,24 @@ struct SplitKvParams {
     int first;      // pair of workgroups y = 0
     int positions;  // filled positions of every sequence
     char* out;      // [pairs of the launch][ceil(positions / 64)][kAttnTile]
+    float key_scale, value_scale;  // in two parts (kernels_pair_attn.h): their powers of two
 };
 
 // One workgroup per tile; rows past the last position become zeros (their scores are masked,
 // and a weight of zero times what an earlier pass left must stay zero).
+// PARTS: 3, or 2 in the same order (tiles of 32 KB).
+template <int PARTS>
 static __global__ __launch_bounds__(256) void split_kv_kernel(const SplitKvParams p) {
+    constexpr int kOperand = PARTS == 3 ? kAttnOperand : 64 * 4 * kPairBlockBytes / 16;
+    constexpr int kStep = PARTS == 3 ? 4 * kSplitBlockBytes : 4 * kPairBlockBytes;  // 16 keys of V^T
+    const auto store = [](char* at, int row, int k, int kblocks, const float(&v)[8], float scale) {
+        if constexpr (PARTS == 3) store_split8(at, row, k, kblocks, v);
+        else store_pair8(at, row, k, kblocks, v, scale);
+    };
     __shared__ float vs[64][65];
     const int tile = blockIdx.x, tid = threadIdx.x;
     const int pair = p.first + blockIdx.y, b = pair / p.kv.heads, h = pair - b * p.kv.heads;
-    char* out = p.out + (static_cast<size_t>(blockIdx.y) * gridDim.x + tile) * kAttnTile;
+    char* out = p.out + (static_cast<size_t>(blockIdx.y) * gridDim.x + tile) * (2 * kOperand);
 #pragma unroll
     for (int i = 0; i < 2; i++) {
         const int row = (tid >> 3) + 32 * i, k = (tid & 7) * 8, pos = tile * 64 + row;
@@ -43,7 +52,7 @@ static __global__ __launch_bounds__(256) void split_kv_kernel(const SplitKvParam
             va = *reinterpret_cast<const float4*>(vr);
             vb = *reinterpret_cast<const float4*>(vr + 4);
         }
-        store_split8(out, row, k, 4, kx);
+        store(out, row, k, 4, kx, p.key_scale);
         vs[row][k] = va.x, vs[row][k + 1] = va.y, vs[row][k + 2] = va.z, vs[row][k + 3] = va.w;
         vs[row][k + 4] = vb.x, vs[row][k + 5] = vb.y, vs[row][k + 6] = vb.z, vs[row][k + 7] = vb.w;
     }
@@ -54,7 +63,7 @@ static __global__ __launch_bounds__(256) void split_kv_kernel(const SplitKvParam
         float v[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) v[j] = vs[16 * s + 4 * c + (j & 3) + 8 * (j >> 2)][dim];
-        store_split8(out + kAttnOperand + s * 4 * kSplitBlockBytes, dim, 8 * c, 1, v);
+        store(out + kOperand + s * kStep, dim, 8 * c, 1, v, p.value_scale);
     }
 }
 
@@ -70,6 +79,7 @@ struct SplitAttnParams {
     int items;        // workgroups per pair
     int first, pairs;  // the pairs of this launch
     float scale;
+    float key_unit;  // in two parts: what a key's unit is worth, a power of two
 };
 
 // Workgroup ids go round-robin over the eight XCDs.  With many (sequence, head) pairs all

@@ -2,7 +2,7 @@
 // their own.
 #include "rows.h"
 
-#include "kernels_split_attn.h"
+#include "kernels_pair_attn.h"
 
 #include <algorithm>
 #include <stdexcept>
@@ -148,6 +148,7 @@ void split_attention(const PrefillAttnParams& a, int batch, char* kv, size_t kv_
     static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_split_kernel),
                                                          hipFuncAttributeMaxDynamicSharedMemorySize, kAttnLds);
     check(raised, "hipFuncSetAttribute");
+    const bool in_pairs = a.pair_scale != 0.0f;
     const int heads = a.kv.heads, pairs = batch * heads, positions = a.pos_base + a.len;
     const int group = attn_group(pairs, positions, kv_bytes);
     const int blocks = (a.len + kAttnQueries - 1) / kAttnQueries;
@@ -156,7 +157,8 @@ void split_attention(const PrefillAttnParams& a, int batch, char* kv, size_t kv_
     p.kv = kv;
     p.tiles = (positions + 63) / 64;
     p.out = a.out_split;
-    p.pair_scale = a.pair_scale;
+    p.pair_scale = in_pairs ? 1.0f / kPairWeightScale : 0.0f;  // of merged parts (values carry that of the rows)
+    p.key_unit = in_pairs ? 1.0f / a.key_scale : 0.0f;
     p.part = part;
     p.d_model = a.d_model;
     p.heads = heads;
@@ -167,10 +169,11 @@ void split_attention(const PrefillAttnParams& a, int batch, char* kv, size_t kv_
         p.pairs = std::min(group, pairs - p.first);
         p.chunk_shift = attn_chunk_shift(p.pairs, a.len, a.pos_base);
         p.items = attn_items(a.len, a.pos_base, p.chunk_shift);
-        const SplitKvParams k{a.kv, a.layer, p.first, positions, kv};
-        hipLaunchKernelGGL(split_kv_kernel, dim3(p.tiles, p.pairs), dim3(256), 0, st, k);
+        const SplitKvParams k{a.kv, a.layer, p.first, positions, kv, a.key_scale, a.pair_scale};
+        hipLaunchKernelGGL(in_pairs ? split_kv_kernel<2> : split_kv_kernel<3>, dim3(p.tiles, p.pairs), dim3(256), 0, st, k);
         check(hipGetLastError(), "split_kv");
-        hipLaunchKernelGGL(attn_split_kernel, dim3((p.pairs + 7) / 8 * 8 * p.items), dim3(256), kAttnLds, st, p);
+        hipLaunchKernelGGL(in_pairs ? attn_pair_kernel : attn_split_kernel, dim3((p.pairs + 7) / 8 * 8 * p.items), dim3(256),
+                           in_pairs ? kPairAttnLds : kAttnLds, st, p);
         check(hipGetLastError(), "attn_split");
         if (p.items > blocks) {
             hipLaunchKernelGGL(attn_split_merge_kernel, dim3(4 * blocks, p.pairs), dim3(256), 0, st, p);
