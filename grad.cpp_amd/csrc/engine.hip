@@ -151,12 +151,12 @@ struct SplitLayer {
     char *wqkv, *wo, *w1, *w2;
 };
 
-// The same matrices in pairs (kernels_pair.h), each with its outputs' exponents, and the powers of two that the
+// The same matrices in pairs (kernels_pair.h), each with its outputs' units, and the powers of two that the
 // operands of those products are scaled by: norm(x) in front of QKV, keys, values and the attention's rows, norm(x) in front
 // of FFN1, the hidden units.
 struct PairLayer {
     char *wqkv, *wo, *w1, *w2;
-    int *eqkv, *eo, *e1, *e2;
+    float *uqkv, *uo, *u1, *u2;
     int norm1, keys, attn, norm2, hidden;
 };
 
@@ -197,7 +197,7 @@ struct Model {
     mutable SplitForm layers_split, logits_split;
     mutable std::vector<SplitLayer> split_layers;
     mutable std::vector<PairLayer> pair_layers;
-    mutable int* logits_exponent = nullptr;  // of the logits matrix in pairs, in its allocation
+    mutable float* logits_unit = nullptr;  // of the logits matrix in pairs, in its allocation
     mutable int logits_norm = 0;             // the power of two of its operand, norm(x)
 
     // The XCD-sharded persistent kernel reads the weights from a second copy laid
@@ -326,10 +326,10 @@ static bool make_split_form(SplitForm& f, size_t bytes, size_t& more, Fill fill)
     return f.ready;
 }
 
-// Storage of a matrix in pairs: the blocks, its outputs' exponents, and the 2-norms of its rows.
+// Storage of a matrix in pairs: the blocks, its outputs' units, and the 2-norms of its rows.
 struct PairPlace {
     char* w;
-    int* exponent;
+    float* unit;
     float* norm;
 };
 
@@ -338,10 +338,10 @@ static size_t pair_place_bytes(size_t N, size_t K) { return pair_bytes(N, K) + 2
 static PairPlace place_pairs(char*& at, const float* src, int N, int K, bool gate_up) {
     PairPlace p;
     p.w = at;
-    p.exponent = reinterpret_cast<int*>(at + pair_bytes(N, K));
-    p.norm = reinterpret_cast<float*>(p.exponent + pair_rows(N));
+    p.unit = reinterpret_cast<float*>(at + pair_bytes(N, K));
+    p.norm = p.unit + pair_rows(N);
     at += pair_place_bytes(N, K);
-    pair_weights(src, N, K, gate_up, p.w, p.exponent, p.norm, nullptr);
+    pair_weights(src, N, K, gate_up, p.w, p.unit, p.norm, nullptr);
     return p;
 }
 
@@ -376,7 +376,7 @@ static Size size_of(const float* device, size_t n) {
 // it (a pair is off by 2^-51 of the bound at most); none for a bound that is no number or far from fp32's middle.
 static std::optional<int> pair_exponent(double bound, double low) {
     if (bound == 0.0) return 0;
-    if (!(bound > 0x1p-90 && bound < 0x1p90) || !(low >= bound * 0x1p-24)) return std::nullopt;
+    if (!(bound > 0x1p-40 && bound < 0x1p40) || !(low >= bound * 0x1p-24)) return std::nullopt;
     return 14 - std::ilogb(bound);
 }
 
@@ -446,7 +446,7 @@ static bool split_layers(const Model& m) {
     for (const LayerWeights& w : m.layers) {
         const PairPlace qkv = place_pairs(at, w.wqkv, 3 * d, d, false), o = place_pairs(at, w.wo, d, d, false);
         const PairPlace ffn1 = place_pairs(at, w.w1, up * F, d, sh.modern()), ffn2 = place_pairs(at, w.w2, d, F, false);
-        PairLayer l{qkv.w, o.w, ffn1.w, ffn2.w, qkv.exponent, o.exponent, ffn1.exponent, ffn2.exponent, 0, 0, 0, 0, 0};
+        PairLayer l{qkv.w, o.w, ffn1.w, ffn2.w, qkv.unit, o.unit, ffn1.unit, ffn2.unit, 0, 0, 0, 0, 0};
         // (W_o and FFN2 feed no operand, but an infinite weight has no pair either)
         fit = fit && std::isfinite(size_of(o.norm, d).top) && std::isfinite(size_of(ffn2.norm, d).top)
               && std::isfinite(size_of(qkv.norm, 2 * d).top) && pair_bounds(sh, w, qkv, ffn1, l);
@@ -468,7 +468,7 @@ static bool split_logits(const Model& m) {
         if (!try_alloc(f.blob, pair_place_bytes(V, d))) return false;
         char* at = f.blob;
         const PairPlace e = place_pairs(at, m.E, V, d, false);
-        m.logits_exponent = e.exponent;
+        m.logits_unit = e.unit;
         m.logits_norm = *norm;
         f.ready = f.pairs = !std::isinf(size_of(e.norm, V).top);
         if (f.ready) return true;
@@ -2024,10 +2024,10 @@ static SplitGemmParams split_params(const char* A, const char* W, int M, int N, 
     return g;
 }
 
-// What a product of pairs needs beside its operands: the exponents of W's outputs and the power of two of A.
-static void pair_params(SplitGemmParams& g, const int* exponent, int operand) {
-    g.exponent = exponent;
-    g.operand_exponent = -operand;
+// What a product of pairs needs beside its operands: the units of W's outputs and of A.
+static void pair_params(SplitGemmParams& g, const float* unit, int operand) {
+    g.unit = unit;
+    g.operand_unit = std::ldexp(1.0f, -operand);
 }
 
 template <int EPI>
@@ -2053,7 +2053,7 @@ static void score_rows(Session& s, const ScoreSink& sink, int M, int n, int t0, 
     const bool pairs = m.logits_split.pairs;
     split_norm(s, pairs, m.gf, m.bf, m.logits_norm, M);
     SplitGemmParams g = split_params(s.pp_split, m.logits_split.blob, M, sh.vocab, sh.d_model);
-    if (pairs) pair_params(g, m.logits_exponent, m.logits_norm);
+    if (pairs) pair_params(g, m.logits_unit, m.logits_norm);
     g.rows_per_seq = n;
     g.targets = sink.targets;
     g.nll_t0 = t0;
@@ -2120,10 +2120,10 @@ static void prompt_layer_split(Session& s, int layer, int n, int pos_base, bool 
 
     split_norm(s, pairs, w.g1, w.be1, pw.norm1, M);
     SplitGemmParams g = split_params(s.pp_split, pairs ? pw.wqkv : sw.wqkv, M, 3 * d, d);
-    pair_params(g, pw.eqkv, pw.norm1);
+    pair_params(g, pw.uqkv, pw.norm1);
     if (keys_only) {
         g.W += static_cast<size_t>(d / kSplitRows) * (d / kSplitCols) * (pairs ? kPairBlockBytes : kSplitBlockBytes);
-        if (pairs) g.exponent += d;
+        if (pairs) g.unit += d;
         g.N = 2 * d;
         g.first = d;
     }
@@ -2149,7 +2149,7 @@ static void prompt_layer_split(Session& s, int layer, int n, int pos_base, bool 
     else launch_prompt_attn(s, a);
 
     g = split_params(s.pp_split, pairs ? pw.wo : sw.wo, M, d, d);
-    pair_params(g, pw.eo, pw.attn);
+    pair_params(g, pw.uo, pw.attn);
     g.bias = w.bo;
     g.out = s.pp_x;
     g.out_stride = d;
@@ -2157,7 +2157,7 @@ static void prompt_layer_split(Session& s, int layer, int n, int pos_base, bool 
 
     split_norm(s, pairs, w.g2, w.be2, pw.norm2, M);
     g = split_params(s.pp_split, pairs ? pw.w1 : sw.w1, M, sh.modern() ? 2 * F : F, d);
-    pair_params(g, pw.e1, pw.norm2);
+    pair_params(g, pw.u1, pw.norm2);
     g.pair_scale = std::ldexp(1.0f, pw.hidden);
     g.bias = sh.modern() ? nullptr : w.b1;
     g.out_split = s.pp_split_hidden;
@@ -2166,7 +2166,7 @@ static void prompt_layer_split(Session& s, int layer, int n, int pos_base, bool 
     else split_project<EPI_GELU>(s, pairs, g);
 
     g = split_params(s.pp_split_hidden, pairs ? pw.w2 : sw.w2, M, d, F);
-    pair_params(g, pw.e2, pw.hidden);
+    pair_params(g, pw.u2, pw.hidden);
     g.bias = sh.modern() ? nullptr : w.b2;
     g.out = s.pp_x;
     g.out_stride = d;

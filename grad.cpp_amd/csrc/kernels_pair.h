@@ -105,11 +105,11 @@ __device__ __forceinline__ void store_operand4(char* base, int r, int k, int kbl
 }
 
 // Writes the pairs of a weight matrix src (N x K, row per output), rows in the order of split_weights_kernel, one
-// wavefront per row, zeros past N.  exponent[j]: the power of two that output j's sum is to be multiplied by, j as the
-// product counts them; norm[n]: the 2-norm of row n of src, infinite if the row has no pairs: a weight is infinite, or
-// more than an eighth of them (zeros aside) lie 2^14 and more below the largest.
+// wavefront per row, zeros past N.  unit[j]: the power of two that output j's sum is to be multiplied by, j as the
+// product counts them; norm[n]: the 2-norm of row n of src, infinite if the row has no pairs: a weight is 2^40 or more
+// (units stay far inside fp32), or more than an eighth of them (zeros aside) lie 2^14 and more below the largest.
 static __global__ __launch_bounds__(256) void pair_weights_kernel(const float* __restrict__ src, int N, int K, int rows,
-                                                                  int gate_up, char* dst, int* exponent, float* norm) {
+                                                                  int gate_up, char* dst, float* unit, float* norm) {
     const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
     const int out = split_output_of_row(row);  // as the product hands it back
@@ -121,9 +121,9 @@ static __global__ __launch_bounds__(256) void pair_weights_kernel(const float* _
         top = fmaxf(fmaxf(top, fmaxf(fabsf(a.x), fabsf(a.y))), fmaxf(fabsf(a.z), fabsf(a.w)));
     }
     top = wave_max(top);
-    // the largest goes to [2^14, 2^15)
-    const int s = top > 0.0f && top < INFINITY ? min(14 - ilogbf(top), 126) : 0;
-    const float scale = ldexpf(1.0f, s);
+    // the largest goes to [2^14, 2^15); a row below 2^-40 stays lower, and is off by 2^-79 at most
+    const int s = top > 0.0f && top < INFINITY ? min(14 - ilogbf(top), 54) : 0;
+    const float scale = ldexpf(1.0f, s), high = ldexpf(top, s - 14);
     float sum = 0.0f, some = 0.0f, most = 0.0f;  // weights that are not zero, and those within 2^14 of the largest
     for (int k = lane * 4; k < K; k += 256) {
         const float4 a = *reinterpret_cast<const float4*>(w + k);
@@ -132,12 +132,12 @@ static __global__ __launch_bounds__(256) void pair_weights_kernel(const float* _
         for (int i = 0; i < 4; i++) {
             sum += v[i] * v[i];
             some += v[i] != 0.0f ? 1.0f : 0.0f;
-            most += fabsf(v[i]) >= 1.0f ? 1.0f : 0.0f;
+            most += fabsf(v[i]) >= high ? 1.0f : 0.0f;
         }
     }
     sum = wave_sum(sum);
-    const bool fit = top < INFINITY && wave_sum(most) * 8.0f >= wave_sum(some) * 7.0f;
-    if (lane == 0) exponent[out] = out < N ? -s : 0;
+    const bool fit = top < 0x1p40f && wave_sum(most) * 8.0f >= wave_sum(some) * 7.0f;
+    if (lane == 0) unit[out] = out < N ? ldexpf(1.0f, -s) : 0.0f;
     if (lane == 0 && n < N) norm[n] = fit ? ldexpf(sqrtf(sum), -s) : INFINITY;
     for (int k = lane * 8; k < K; k += 512) {
         const float factor = scale * pair_sign(k >> 4);
@@ -179,7 +179,19 @@ static __global__ __launch_bounds__(1024) void norm_pair_long_kernel(const float
                        [&](int k, const float(&o)[8]) { store_pair8(out, m, k, d / kSplitCols, o, pair_scale); });
 }
 
+// The epilogues' functions by the hardware's 2^x and reciprocal: five vector instructions beside the two, where tanhf
+// makes 66 of the GELU (two thirds of what a 768-column FFN1 tile issued).  As x over 1 + exp(-2 u) the GELU of a negative
+// argument loses nothing to 1 + tanh(u).  Infinities and NaN come out as of the functions themselves.
 struct PairRowsOut {
+    static __device__ __forceinline__ float gelu(float x) {
+        // 0.5 x (1 + tanh(u)) = x / (1 + exp(-2 u)), u = sqrt(2 / pi) (x + 0.044715 x^3)
+        constexpr float k = -2.0f * 0.79788456f * 1.44269504f;
+        return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * __builtin_fmaf(x * x, 0.044715f * k, k)));
+    }
+    static __device__ __forceinline__ float silu(float x) {
+        return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.44269504f));
+    }
+    static __device__ __forceinline__ float exp_of(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504f); }
     static __device__ __forceinline__ void store8(const SplitGemmParams& p, int m, int k, const float (&v)[8]) {
         store_pair8(p.out_split, m, k, p.out_kblocks, v, p.pair_scale);
     }
@@ -188,9 +200,9 @@ struct PairRowsOut {
 // C[M,N] = A[M,K] . W[N,K]^T of pairs.  Tiles, workgroup order, LDS ring and epilogues are split_gemm_kernel's.
 // A step of 16 columns is three rounds of products (w1 a2, w2 a1, w1 a1), its fragments read from LDS during the
 // step before into registers of their own (a 64 x 64 wavefront has 128 of its 256 for sums).  Four steps make a
-// 64-column part that starts from zero; it is added to the running sums (or taken from them, the weights of every
-// other part being negative) in front of the next part's first products, one accumulator at a time, so that this
-// runs beside the other accumulators' products.  K / KG is a multiple of 64.
+// 64-column part that starts from zero and is then added to the running sums (or taken from them, the weights of every
+// other part being negative).  (Added in front of the next part's products instead, accumulator by accumulator, the
+// compiler copies every part first.)  K / KG is a multiple of 64.
 template <int EPI, int MB, int NB, int WM, int WN, int KG, int PER_CU>
 __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void pair_gemm_kernel(const SplitGemmParams p) {
     extern __shared__ __attribute__((aligned(1024))) char lds_pair[];
@@ -242,19 +254,13 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
 #pragma unroll
     for (int a = 0; a < NB; a++)
 #pragma unroll
-        for (int b = 0; b < MB; b++) sum[a][b] = part[a][b] = zero;
+        for (int b = 0; b < MB; b++) sum[a][b] = zero;
     const auto multiply = [&](const v8h (&w)[NB], const v8h (&x)[MB]) {
 #pragma unroll
         for (int a = 0; a < NB; a++)
 #pragma unroll
             for (int b = 0; b < MB; b++) part[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[a], x[b], part[a][b], 0, 0, 0);
     };
-    float sign = 1.0f;  // of the part at hand, then of the one before
-    const auto add_part = [&](v16f& to, const v16f& v) {
-#pragma unroll
-        for (int r = 0; r < 16; r++) to[r] = __builtin_fmaf(v[r], sign, to[r]);
-    };
-
 #pragma unroll
     for (int s = 0; s < kStages; s++)
 #pragma unroll
@@ -288,11 +294,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
 #pragma unroll
             for (int a = 0; a < NB; a++)
 #pragma unroll
-                for (int b = 0; b < MB; b++) {
-                    if (t == 0) add_part(sum[a][b], part[a][b]);
+                for (int b = 0; b < MB; b++)
                     part[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(low[a], a2[c][b], t == 0 ? zero : part[a][b], 0, 0, 0);
-                }
-            if (t == 0) sign = pair_sign(kg * kblocks + s0);
             read_w(next, 0, w1[n]);
             read_a(next, 1, a2[n]);
             send(0);
@@ -303,11 +306,14 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
             read_a(next, 0, a1[n]);
             send(2);
         }
+        const float sign = pair_sign(kg * kblocks + s0);
+#pragma unroll
+        for (int a = 0; a < NB; a++)
+#pragma unroll
+            for (int b = 0; b < MB; b++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) sum[a][b][r] = __builtin_fmaf(part[a][b][r], sign, sum[a][b][r]);
     }
-#pragma unroll
-    for (int a = 0; a < NB; a++)
-#pragma unroll
-        for (int b = 0; b < MB; b++) add_part(sum[a][b], part[a][b]);
     if constexpr (KG > 1) {
         // the other sets' sums through the LDS the rings no longer need, added in order
         float* sums = reinterpret_cast<float*>(lds_pair);
@@ -335,18 +341,20 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
     const int n0 = n_tile * TN + wn * 32 * NB;
 #pragma unroll
     for (int a = 0; a < NB; a++) {
-        // (storage of exponents for whole tiles, as of the weights)
-        const int4* const e = reinterpret_cast<const int4*>(p.exponent + n0 + 32 * a + 16 * h32);
-        int es[16];
+        // (storage of units for whole tiles, as of the weights)
+        const float4* const u = reinterpret_cast<const float4*>(p.unit + n0 + 32 * a + 16 * h32);
+        float units[16];
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const int4 v = e[q];
-            es[4 * q] = v.x, es[4 * q + 1] = v.y, es[4 * q + 2] = v.z, es[4 * q + 3] = v.w;
+            const float4 v = u[q];
+            units[4 * q] = v.x, units[4 * q + 1] = v.y, units[4 * q + 2] = v.z, units[4 * q + 3] = v.w;
         }
 #pragma unroll
-        for (int b = 0; b < MB; b++)
+        for (int r = 0; r < 16; r++) {
+            const float f = units[r] * p.operand_unit;
 #pragma unroll
-            for (int r = 0; r < 16; r++) sum[a][b][r] = ldexpf(sum[a][b][r], es[r] + p.operand_exponent);
+            for (int b = 0; b < MB; b++) sum[a][b][r] *= f;
+        }
     }
     split_epilogue<PairRowsOut, EPI, MB, NB>(p, sum, m_tile * TM + wm * 32 * MB, n0, n_tile * WN + wn);
 }

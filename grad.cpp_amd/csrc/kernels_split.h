@@ -254,9 +254,9 @@ struct SplitGemmParams {
     char* out_split;  // EPI_GELU, EPI_SWIGLU: split rows of out_cols columns
     int out_kblocks;
     // operands in pairs (kernels_pair.h)
-    const int* exponent;   // per output, of the weights
-    int operand_exponent;  // of A
-    float pair_scale;      // of the rows at out_split
+    const float* unit;   // per output: what a sum's unit is worth, of W
+    float operand_unit;  // ... of A
+    float pair_scale;    // of the rows at out_split
     // EPI_QKV (rows of a prompt pass, as in GemvParams); outputs first .. first + N of the fused product
     int first;
     KvLayout kv;
@@ -311,8 +311,11 @@ __device__ __forceinline__ bool split_tile(const SplitGemmParams& p, int& m_tile
     return true;
 }
 
-// How the split projections leave rows of the next one's operand.
+// What the split projections make of their outputs, and how they leave rows of the next one's operand.
 struct SplitRowsOut {
+    static __device__ __forceinline__ float gelu(float x) { return gelu_tanh(x); }
+    static __device__ __forceinline__ float silu(float x) { return gh::silu(x); }
+    static __device__ __forceinline__ float exp_of(float x) { return expf(x); }
     static __device__ __forceinline__ void store8(const SplitGemmParams& p, int m, int k, const float (&v)[8]) {
         store_split8(p.out_split, m, k, p.out_kblocks, v);
     }
@@ -351,7 +354,7 @@ __device__ __forceinline__ void split_epilogue(const SplitGemmParams& p, const v
                 const int n = n0 + 32 * a + 16 * h32;
 #pragma unroll
                 for (int r = 0; r < 16; r++)
-                    if (n + r < p.N) sum += expf(acc[a][b][r] - base);
+                    if (n + r < p.N) sum += Rows::exp_of(acc[a][b][r] - base);
             }
             sum += __shfl_xor(sum, 32, kWave);
             if (m < p.M && h32 == 0)
@@ -386,13 +389,13 @@ __device__ __forceinline__ void split_epilogue(const SplitGemmParams& p, const v
                 } else if constexpr (EPI == EPI_GELU) {
                     float o[2][8];
 #pragma unroll
-                    for (int r = 0; r < 16; r++) o[r >> 3][r & 7] = gelu_tanh(v[r] + p.bias[n + r]);
+                    for (int r = 0; r < 16; r++) o[r >> 3][r & 7] = Rows::gelu(v[r] + p.bias[n + r]);
                     Rows::store8(p, m, n, o[0]);
                     Rows::store8(p, m, n + 8, o[1]);
                 } else if constexpr (EPI == EPI_SWIGLU) {
                     float o[8];
 #pragma unroll
-                    for (int r = 0; r < 8; r++) o[r] = v[8 + r] * silu(v[r]);
+                    for (int r = 0; r < 8; r++) o[r] = v[8 + r] * Rows::silu(v[r]);
                     Rows::store8(p, m, n >> 1, o);
                 } else if constexpr (EPI == EPI_QKV) {
                     const int sec = (p.first + n) / p.d_model, c = p.first + n - sec * p.d_model, head = c >> 6, j = c & 63;

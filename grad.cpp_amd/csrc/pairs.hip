@@ -10,10 +10,9 @@ static void check(hipError_t e, const char* what) {
     if (e != hipSuccess) throw std::runtime_error(std::string("HIP error in ") + what + ": " + hipGetErrorString(e));
 }
 
-void pair_weights(const float* src, int N, int K, bool gate_up, char* dst, int* exponent, float* norm, hipStream_t st) {
+void pair_weights(const float* src, int N, int K, bool gate_up, char* dst, float* unit, float* norm, hipStream_t st) {
     const int rows = static_cast<int>(pair_rows(N));
-    hipLaunchKernelGGL(pair_weights_kernel, dim3(rows / 4), dim3(256), 0, st, src, N, K, rows, gate_up ? 1 : 0, dst, exponent,
-                       norm);
+    hipLaunchKernelGGL(pair_weights_kernel, dim3(rows / 4), dim3(256), 0, st, src, N, K, rows, gate_up ? 1 : 0, dst, unit, norm);
     check(hipGetLastError(), "pair_weights");
 }
 

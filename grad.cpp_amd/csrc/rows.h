@@ -23,10 +23,10 @@ void norm_split(bool rms, const float* x, const float* gamma, const float* beta,
 template <int EPI>
 void split_gemm(SplitGemmParams& p, hipStream_t st);
 
-// The same three in pairs (kernels_pair.h); exponents of a matrix: one per row of its storage.
+// The same three in pairs (kernels_pair.h); units of a matrix: one per row of its storage.
 inline size_t pair_rows(size_t rows) { return (rows + kSplitPad - 1) / kSplitPad * kSplitPad; }
 inline size_t pair_bytes(size_t rows, size_t cols) { return pair_rows(rows) * cols * 4; }
-void pair_weights(const float* src, int N, int K, bool gate_up, char* dst, int* exponent, float* norm, hipStream_t st);
+void pair_weights(const float* src, int N, int K, bool gate_up, char* dst, float* unit, float* norm, hipStream_t st);
 void norm_pair(bool rms, const float* x, const float* gamma, const float* beta, char* out, int M, int d, float pair_scale,
                hipStream_t st);
 template <int EPI>
