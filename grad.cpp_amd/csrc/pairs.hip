@@ -1,6 +1,8 @@
 // The many-row projections in pairs: variants and the rule that picks one, in a translation unit of their own.
 #include "rows.h"
 
+#include <algorithm>
+#include <cmath>
 #include <stdexcept>
 #include <string>
 
@@ -32,18 +34,43 @@ void norm_pair(bool rms, const float* x, const float* gamma, const float* beta, 
     else norm_pair_as<false>(x, gamma, beta, out, M, d, pair_scale, st);
 }
 
-enum Tiling { TILE_32_K4, TILE_64_K4, TILE_64, TILE_128x64, TILE_128 };
+// The tilings, and what a launch takes with each: with n tiles on the fullest of 256 compute units and K in thousands
+//   start + max(chain K, n step K) + n out
+// us, fitted to 231 launches (160 to 16384 rows against the ten matrices of models 512 and 768 columns wide: W_o,
+// QKV, both FFN1 and FFN2), medians off by 6 to 9 %.  A lone workgroup is a chain of K steps (64 x 64 tiles with K shared by four
+// sets of wavefronts, and 32 x 32 ones, are the shorter chains); beside others its chain hides, and what counts is what the unit
+// moves through LDS and multiplies; `out` is the epilogue, of a residual (queries, keys, values and logits counted
+// like it), a GELU or a SwiGLU.  Taking the least by this rule, those launches take 1.2 % longer than with the
+// best of eleven tilings each (at most 12 %), 1.3 with the same seven and no line between epilogues, 8.0 with the three-part form's rule
+// (at most 48 %).  1999 x 768 x 768 15.9 -> 13.3 us, 1999 x 768 x 2048 31.3 -> 25.2, 1999 x 2304 x 768 33.4 -> 30.5, 1999 x 3072 x 768
+// 44.7 -> 39.4.
+struct Tiling {
+    int m, n, sets;  // rows, outputs, sets of wavefronts that share K
+    float start, chain, step, out[3];
+};
+enum { TILE_128, TILE_128x64, TILE_64, TILE_64_K2, TILE_64x96_K2, TILE_64x96_K4, TILE_32_K4, TILINGS };
+constexpr Tiling kTilings[TILINGS] = {
+    {128, 128, 1, 2.94f, 22.28f, 18.05f, {5.93f, 9.24f, 4.43f}}, {128, 64, 1, 2.39f, 13.85f, 10.60f, {3.23f, 4.09f, 1.92f}},
+    {64, 64, 1, 2.49f, 9.47f, 6.43f, {1.56f, 1.75f, 0.87f}},     {64, 64, 2, 1.96f, 4.74f, 6.25f, {2.14f, 2.64f, 1.37f}},
+    {64, 96, 2, 1.75f, 10.33f, 8.38f, {3.33f, 6.61f, 2.86f}},    {64, 96, 4, 0.50f, 0.49f, 8.40f, {5.86f, 12.77f, 5.47f}},
+    {32, 32, 4, 1.93f, 2.93f, 2.57f, {0.89f, 2.14f, 0.95f}},
+};
 
-static Tiling pick_tiling(int M, int N, int K) {
-    const auto tiles = [&](int t) { return static_cast<long>((M + t - 1) / t) * ((N + t - 1) / t); };
-    const auto rounds = [&](int t) { return (tiles(t) + 255) / 256; };
-    if (K % 256 == 0) {
-        if (rounds(32) <= 2) return TILE_32_K4;
-        if (rounds(64) == 1) return TILE_64_K4;
+static int pick_tiling(int M, int N, int K, int epilogue) {
+    const int out = epilogue == EPI_GELU ? 1 : epilogue == EPI_SWIGLU ? 2 : 0;
+    int best = TILE_128;
+    float least = INFINITY;
+    for (int i = 0; i < TILINGS; i++) {
+        const Tiling& t = kTilings[i];
+        if (K % (64 * t.sets) != 0) continue;  // (whole parts per set)
+        const float tiles = static_cast<float>((M + t.m - 1) / t.m) * ((N + t.n - 1) / t.n), n = std::ceil(tiles / 256.0f);
+        const float us = t.start + std::max(t.chain, n * t.step) * K * 1e-3f + n * t.out[out];
+        if (us < least) {
+            least = us;
+            best = i;
+        }
     }
-    const long tall = static_cast<long>((M + 127) / 128) * ((N + 63) / 64);
-    if (rounds(64) == 2 && tall <= 256 && K >= 768) return TILE_128x64;
-    return rounds(128) * 28 < rounds(64) * 10 ? TILE_128 : TILE_64;
+    return best;
 }
 
 template <int EPI, int MB, int NB, int WM, int WN, int KG, int PER_CU>
@@ -64,12 +91,14 @@ static void launch(SplitGemmParams& p, hipStream_t st) {
 
 template <int EPI>
 void pair_gemm(SplitGemmParams& p, hipStream_t st) {
-    switch (pick_tiling(p.M, p.N, p.K)) {
-        case TILE_32_K4: launch<EPI, 1, 1, 1, 1, 4, 2>(p, st); break;
-        case TILE_64_K4: launch<EPI, 1, 1, 2, 2, 4, 1>(p, st); break;
-        case TILE_64: launch<EPI, 1, 1, 2, 2, 1, 4>(p, st); break;
-        case TILE_128x64: launch<EPI, 2, 1, 2, 2, 1, 2>(p, st); break;
+    switch (pick_tiling(p.M, p.N, p.K, EPI)) {
         case TILE_128: launch<EPI, 2, 2, 2, 2, 1, 2>(p, st); break;
+        case TILE_128x64: launch<EPI, 2, 1, 2, 2, 1, 2>(p, st); break;
+        case TILE_64: launch<EPI, 1, 1, 2, 2, 1, 4>(p, st); break;
+        case TILE_64_K2: launch<EPI, 1, 1, 2, 2, 2, 2>(p, st); break;
+        case TILE_64x96_K2: launch<EPI, 1, 3, 2, 1, 2, 2>(p, st); break;
+        case TILE_64x96_K4: launch<EPI, 1, 3, 2, 1, 4, 1>(p, st); break;
+        case TILE_32_K4: launch<EPI, 1, 1, 1, 1, 4, 2>(p, st); break;
     }
 }
 

@@ -24,7 +24,8 @@ template <int EPI>
 void split_gemm(SplitGemmParams& p, hipStream_t st);
 
 // The same three in pairs (kernels_pair.h); units of a matrix: one per row of its storage.
-inline size_t pair_rows(size_t rows) { return (rows + kSplitPad - 1) / kSplitPad * kSplitPad; }
+// (whole tiles of 96 outputs, also from a row behind the first)
+inline size_t pair_rows(size_t rows) { return (rows + 95 + kSplitPad - 1) / kSplitPad * kSplitPad; }
 inline size_t pair_bytes(size_t rows, size_t cols) { return pair_rows(rows) * cols * 4; }
 void pair_weights(const float* src, int N, int K, bool gate_up, char* dst, float* unit, float* norm, hipStream_t st);
 void norm_pair(bool rms, const float* x, const float* gamma, const float* beta, char* out, int M, int d, float pair_scale,

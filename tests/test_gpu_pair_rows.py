@@ -31,14 +31,20 @@ def _check(cfg, W, B, n, seed, sequences=None):
 
 
 CASES = {
-    # name: (width, vocab, sequences, tokens)
-    "32-wide tiles, K in four sets": (512, 130, 1, 161),
-    "64-wide tiles, K in four sets": (512, 1001, 3, 171),
-    "64-wide tiles, one row past a tile": (768, 515, 1, 577),
-    "no whole parts for four sets of K": (576, 130, 1, 161),  # 36 blocks of 16 columns
-    "nine parts, one set of K": (576, 301, 5, 193),
-    "128 x 64 tiles, a nearly empty one": (768, 130, 3, 449),
-    "128-wide tiles, several rounds": (768, 301, 11, 487),
+    # rows reach: name: (width, vocab, sequences, tokens)
+    "32 x 32 tiles, one row past a tile": (512, 130, 1, 161),
+    "64 x 64 of two sets of K": (512, 1001, 3, 171),
+    "64 x 96 of two sets, q, k, v; keys and values from the middle of the matrix": (512, 130, 3, 449),
+    "128 x 64, both FFN1; a nearly empty tile": (512, 130, 3, 667),
+    "128 x 128 at 512 columns": (512, 515, 11, 487),
+    "64 x 96 of four sets, q, k, v and SwiGLU": (768, 130, 2, 150),
+    "64 x 64 of one set, FFN1; four sets of 64 x 96, q, k, v": (768, 515, 1, 449),
+    "64 x 64 of two sets, W_o": (768, 1001, 3, 334),
+    "64 x 96 of four sets, W_o, FFN2 and logits": (768, 515, 4, 501),
+    "64 x 96 of two sets, W_o and FFN2": (768, 515, 6, 500),
+    "128 x 128, all": (768, 515, 19, 474),
+    "nine parts of K: one set": (576, 130, 1, 161),
+    "nine parts of K: one set, FFN2 in four": (576, 301, 3, 667),
 }
 
 
