@@ -52,7 +52,7 @@ CASES = {
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_rows_match_the_float64_forward(name, arch):
     d, vocab, B, n = CASES[name]
-    cfg = synth.Config(arch, vocab, d, 1, d // 64, 600)
+    cfg = synth.Config(arch, vocab, d, 1, d // 64, 700)
     _check(cfg, synth.make_weights(cfg, 101, std=lively_std(cfg), norm_noise=0.1), B, n, 102)
 
 
