@@ -2282,7 +2282,7 @@ static bool reserve_score_rows(Session& s, size_t rows) {
 // the session's whole context can use, so that it is allocated once (nothing in it is read that the
 // pass has not written, so it is not cleared); partial results grow in steps of 8 MB, up to some 45.
 // False: there is no memory, or too little work; the fp32 kernel, which needs none, does it.
-static bool reserve_split_attention(Session& s, int n, int pos_base) {
+static bool reserve_split_attention(Session& s, int n, int pos_base, bool pairs) {
     if (n <= kSplitAttnMin) return false;
     const int heads = s.m->shape.heads;
     if (!s.pp_kv) {
@@ -2290,7 +2290,7 @@ static bool reserve_split_attention(Session& s, int n, int pos_base) {
         if (!try_alloc(s.pp_kv, bytes)) return false;
         s.pp_kv_bytes = bytes;
     }
-    const size_t need = split_attention_part_floats(s.B, heads, n, pos_base, s.pp_kv_bytes);
+    const size_t need = split_attention_part_floats(s.B, heads, n, pos_base, s.pp_kv_bytes, pairs);
     if (s.pp_part_floats < need) {
         if (s.pp_part) HIP_CHECK(hipFree(s.pp_part));
         s.pp_part_floats = 0;
@@ -2324,7 +2324,7 @@ static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSi
         const int M = n * B;
         const int pos_base = s.pos + t0;
         const bool split = M >= plan.split_rows;
-        const bool split_attn = split && reserve_split_attention(s, n, pos_base);
+        const bool split_attn = split && reserve_split_attention(s, n, pos_base, plan.pairs);
         hipLaunchKernelGGL(embed_rows_kernel, dim3((d + 255) / 256, M), dim3(256), 0, st, m.E, m.P, s.hist,
                            s.hist_stride, s.n_hist + t0, n, pos_base, s.pp_x, d);
         HIP_CHECK(hipGetLastError());

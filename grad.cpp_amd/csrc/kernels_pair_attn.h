@@ -10,19 +10,25 @@ namespace gh {
 // keys, each 64 rows (dims) x 16 columns; second parts 2^11 larger.
 constexpr int kPairAttnOperand = 16 * kPairBlockBytes;
 constexpr int kPairAttnTile = 2 * kPairAttnOperand;
-constexpr int kPairAttnLds = kAttnRing * kPairAttnOperand;
+constexpr int kPairAttnRing = 4;
+constexpr int kPairAttnLds = kPairAttnRing * kPairAttnOperand;
 constexpr float kPairWeightScale = 16384.0f;  // of the probabilities: fp16's upper end
 
-// attn_split_kernel's work and order: 128 queries per workgroup against a run of key tiles, both products transposed,
-// operands through a ring of three in LDS.  What differs:
+// attn_split_kernel's work and order: 128 queries per workgroup against a run of key tiles, both products transposed.
+// What differs:
 // - A query is scaled by a power of two of its own, from its largest element, and its scores come back with it (in the
 //   multiply-add that takes off the maximum).  Probabilities are split 2^14 larger; values carry the power of
 //   two of the rows that leave.
 // - Of a tile's twelve products per 32 x 32 block the eight small ones go first, over all of K = 64, then the four of the first
 //   parts: four roundings of a full-sized sum, where three parts had 24.  (Sums of 64 terms against float64, over the
 //   size of the result: 0.98e-7 with the small products apart, 1.09e-7 with the six of three parts in turn.)
-// 16 x 12 heads, us, three parts -> two: 1024 tokens 206 -> 142, 1536 400 -> 272; 1 x 12 x 1999 48 -> 36; with
-// split_kv_kernel's part 52 -> 35, 68 -> 49, 7.8 -> 6.2.
+// - The workgroup meets once per tile, its ring four operands deep, and a product's fragments are all read well ahead: values
+//   in front of the softmax, the next keys behind the products with them.  The softmax takes one kind of step over all 32 scores
+//   after the other (pair by pair each step waited for the one before).
+// 16 x 12 heads, us, three parts -> two in that kernel's form -> as it is: 1024 tokens 206 -> 110 -> 106, 1536 400 -> 221 -> 215;
+// 1 x 12 x 1999 48 -> 36 -> 34 (the first with each form's best order of workgroups).  What bounds it: 48 products and 290 vector
+// instructions per wavefront and tile, two wavefronts per SIMD.  The next tile's scores formed beside the softmax, a product
+// every 8, 12 or 16 instructions: 7 % slower; a ring of five, one of them a tile further ahead: no faster.
 static __global__ __launch_bounds__(256, 2) void attn_pair_kernel(const SplitAttnParams p) {
     extern __shared__ __attribute__((aligned(1024))) char lds_pair_attn[];
     int pair, b, h, item;
@@ -47,14 +53,15 @@ static __global__ __launch_bounds__(256, 2) void attn_pair_kernel(const SplitAtt
     constexpr int kLoads = kPairAttnOperand / 1024 / 4;  // per wavefront and operand: one in front of each step
     const int operands = 2 * (tile1 - tile0);
     // load i of operand j: K (even) or V^T (odd) of tile tile0 + j / 2
-    const auto issue = [&](int j, int slot, int i) {
+    const auto issue = [&](int j, int i) {
         const char* at = src + static_cast<size_t>(2 * tile0 + j) * kPairAttnOperand;
-        load_to_lds(at, (wave * kLoads + i) * 1024 + lane * 16, lds0 + slot * kPairAttnOperand + (wave * kLoads + i) * 1024);
+        load_to_lds(at, (wave * kLoads + i) * 1024 + lane * 16,
+                    lds0 + (j & (kPairAttnRing - 1)) * kPairAttnOperand + (wave * kLoads + i) * 1024);
     };
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int j = 0; j < 3; j++)
 #pragma unroll
-        for (int i = 0; i < kLoads; i++) issue(j, j, i);
+        for (int i = 0; i < kLoads; i++) issue(min(j, operands - 1), i);
 
     // Q^T: dims 16 c + 8 (lane / 32) .. + 7 of the lane's query, in units of ln 2
     v8h q1[4], q2[4];
@@ -98,27 +105,27 @@ static __global__ __launch_bounds__(256, 2) void attn_pair_kernel(const SplitAtt
 
     const int row_at = (n32 & 15) * 16 + h32 * kPairChunkBytes;
     const int k_at = (n32 >> 4) * 4 * kPairBlockBytes + row_at, v_at = (n32 >> 4) * kPairBlockBytes + row_at;
-    // a tile's product: fragments of step c at at + c * step, of two 32-row blocks `far` bytes apart
-    const auto product = [&](const char* at, int step, int far, const v8h (&g1)[4], const v8h (&g2)[4], v16f (&out)[2], auto send) {
-        v8h f1[4][2], f2[2][2];
-        const auto read = [&](int c, int part, v8h (&f)[2]) {
+    const auto place = [&](int j) { return lds_pair_attn + (j & (kPairAttnRing - 1)) * kPairAttnOperand; };
+    // A tile's product: fragments of its four steps of two 32-row blocks, read all at once and well ahead.
+    v8h f1[4][2], f2[4][2];
+    const auto fetch = [&](const char* at, int step, int far) {
 #pragma unroll
-            for (int i = 0; i < 2; i++) f[i] = *reinterpret_cast<const v8h*>(at + c * step + i * far + part * kPairPartBytes);
-        };
-        read(0, 1, f2[0]);
-        read(0, 0, f1[0]);
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                f2[c][i] = *reinterpret_cast<const v8h*>(at + c * step + i * far + kPairPartBytes);
+                f1[c][i] = *reinterpret_cast<const v8h*>(at + c * step + i * far);
+            }
+    };
+    const auto fetch_keys = [&](int j) { fetch(place(j) + k_at, kPairBlockBytes, 8 * kPairBlockBytes); };
+    const auto fetch_values = [&](int j) { fetch(place(j) + v_at, 4 * kPairBlockBytes, 2 * kPairBlockBytes); };
+    const auto product = [&](const v8h (&g1)[4], const v8h (&g2)[4], v16f (&out)[2]) {
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            if (c < 3) {
-                read(c + 1, 1, f2[(c + 1) & 1]);
-                read(c + 1, 0, f1[c + 1]);
-            }
-            send(c);
-            __builtin_amdgcn_sched_barrier(0);  // the reads and loads go out before the products
             const v8h low = g1[c] * down;
 #pragma unroll
             for (int i = 0; i < 2; i++)
-                out[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f2[c & 1][i], low, c == 0 ? zero : out[i], 0, 0, 0);
+                out[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f2[c][i], low, c == 0 ? zero : out[i], 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < 2; i++) out[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f1[c][i], g2[c], out[i], 0, 0, 0);
         }
@@ -128,83 +135,85 @@ static __global__ __launch_bounds__(256, 2) void attn_pair_kernel(const SplitAtt
             for (int i = 0; i < 2; i++) out[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f1[c][i], g1[c], out[i], 0, 0, 0);
     };
 
-    int slot = 0;  // of the operand being multiplied
-    const auto arrive = [&](int j) {  // operand j has landed everywhere, and everyone is done with operand j - 1
-        if (j + 1 < operands) wait_loads<kLoads>();
-        else wait_loads<0>();
-        meet();
-    };
-    const auto send = [&](int j, int i) {  // load i of operand j + 2 sets out, to the place of operand j - 1
-        if (j + 2 < operands) issue(j + 2, slot == 0 ? 2 : slot - 1, i);
-    };
+    wait_loads<2 * kLoads>();  // the first tile's keys
+    meet();
+    fetch_keys(0);
     for (int kt = tile0; kt < tile1; kt++) {
         const int j = 2 * (kt - tile0), kh = kt * 64;
         const bool future = kh > wave_last;  // every key of the tile lies behind this wavefront's queries
-        arrive(j);
-        v8h p1[4], p2[4];
-        float f = 1.0f;
-        if (!future) {
-            v16f sc[2];
-            product(lds_pair_attn + slot * kPairAttnOperand + k_at, kPairBlockBytes, 8 * kPairBlockBytes, q1, q2, sc,
-                    [&](int c) { send(j, c); });
-            // causal mask (keys up to the query's own position) and the tile's maximum per query
-            if (kh + 63 > wave_first) {  // only the tiles on the diagonal need the comparisons
+        v16f sc[2];
+        if (!future) product(q1, q2, sc);
+        // this tile's values and the next one's keys are here, and everyone is done with the operands before them
+        wait_loads<0>();
+        meet();
+        if (j + 3 < operands) {
 #pragma unroll
-                for (int kb = 0; kb < 2; kb++)
+            for (int i = 0; i < kLoads; i++) issue(j + 3, i);
+            if (j + 4 < operands) {
 #pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        const int key = kh + kb * 32 + 8 * (r >> 2) + 4 * h32 + (r & 3);
-                        sc[kb][r] = (key <= qpos) ? sc[kb][r] : -INFINITY;
-                    }
+                for (int i = 0; i < kLoads; i++) issue(j + 4, i);
             }
-            float mb = -INFINITY;
+        }
+        if (future) continue;
+        fetch_values(j + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        // causal mask (keys up to the query's own position)
+        if (kh + 63 > wave_first) {  // only the tiles on the diagonal need the comparisons
 #pragma unroll
             for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) mb = fmaxf(mb, sc[kb][r]);
-            mb = fmaxf(mb, __shfl_xor(mb, 32, kWave)) * unit;  // the two halves of a wavefront hold different keys of a query
-            const float mn = fmaxf(m, mb);
-            const float base = mn == -INFINITY ? 0.0f : mn;  // (a query may have no key in this run of tiles yet)
-            f = __builtin_amdgcn_exp2f(m - base);            // 0 on the first tile
-            float psum = 0.0f;
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                v4u a, b;
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int r = (s & 1) * 8 + 2 * i;
-                    const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[s >> 1][r], unit, -base));
-                    const float y = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[s >> 1][r + 1], unit, -base));
-                    psum += x + y;
-                    unsigned first, second;
-                    to_pairs(x * kPairWeightScale, y * kPairWeightScale, 1.0f, first, second);
-                    a[i] = first, b[i] = second;
+                for (int r = 0; r < 16; r++) {
+                    const int key = kh + kb * 32 + 8 * (r >> 2) + 4 * h32 + (r & 3);
+                    sc[kb][r] = (key <= qpos) ? sc[kb][r] : -INFINITY;
                 }
-                p1[s] = __builtin_bit_cast(v8h, a);
-                p2[s] = __builtin_bit_cast(v8h, b);
+        }
+        float mb = -INFINITY;
+#pragma unroll
+        for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) mb = fmaxf(mb, sc[kb][r]);
+        mb = fmaxf(mb, __shfl_xor(mb, 32, kWave)) * unit;  // the two halves of a wavefront hold different keys of a query
+        const float mn = fmaxf(m, mb);
+        const float base = mn == -INFINITY ? 0.0f : mn;   // (a query may have no key in this run of tiles yet)
+        const float f = __builtin_amdgcn_exp2f(m - base);  // 0 on the first tile
+        // (one kind of step over all of them after the other: pair by pair every step waits for the one before)
+#pragma unroll
+        for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) sc[kb][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kb][r], unit, -base));
+        __builtin_amdgcn_sched_barrier(0);
+        float sums[4] = {0.f, 0.f, 0.f, 0.f};
+        v8h p1[4], p2[4];
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            v4u a, b;
+            float x[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                x[i] = sc[s >> 1][(s & 1) * 8 + i];
+                sums[i & 3] += x[i];
+                x[i] *= kPairWeightScale;
             }
-            psum += __shfl_xor(psum, 32, kWave);
-            l = l * f + psum;
-            m = mn;
-        } else {
 #pragma unroll
-            for (int i = 0; i < kLoads; i++) send(j, i);
+            for (int i = 0; i < 4; i++) {
+                unsigned first, second;
+                to_pairs(x[2 * i], x[2 * i + 1], 1.0f, first, second);
+                a[i] = first, b[i] = second;
+            }
+            p1[s] = __builtin_bit_cast(v8h, a);
+            p2[s] = __builtin_bit_cast(v8h, b);
         }
-        slot = slot == kAttnRing - 1 ? 0 : slot + 1;
-        arrive(j + 1);
-        if (!future) {
-            v16f tile[2];
-            product(lds_pair_attn + slot * kPairAttnOperand + v_at, 4 * kPairBlockBytes, 2 * kPairBlockBytes, p1, p2, tile,
-                    [&](int c) { send(j + 1, c); });
+        float psum = (sums[0] + sums[1]) + (sums[2] + sums[3]);
+        psum += __shfl_xor(psum, 32, kWave);
+        l = l * f + psum;
+        m = mn;
+        v16f tile[2];
+        product(p1, p2, tile);
+        fetch_keys(j + 2);  // (past the last tile: of whatever lies there, not used)
 #pragma unroll
-            for (int db = 0; db < 2; db++)
+        for (int db = 0; db < 2; db++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) o[db][r] = o[db][r] * f + tile[db][r];
-        } else {
-#pragma unroll
-            for (int i = 0; i < kLoads; i++) send(j + 1, i);
-        }
-        slot = slot == kAttnRing - 1 ? 0 : slot + 1;
+            for (int r = 0; r < 16; r++) o[db][r] = o[db][r] * f + tile[db][r];
     }
     if (parts > 1) {
         float* part = p.part + (static_cast<size_t>(pair) * p.items + item) * kAttnPart + wave * (34 * 64) + lane;

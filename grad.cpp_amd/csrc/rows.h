@@ -38,7 +38,7 @@ void pair_gemm(SplitGemmParams& p, hipStream_t st);
 // that fit.  split_attention_kv_bytes: what is worth giving for so many filled positions.
 // part: scratch of the size split_attention_part_floats names for the call.
 size_t split_attention_kv_bytes(int batch, int heads, int positions);
-size_t split_attention_part_floats(int batch, int heads, int len, int pos_base, size_t kv_bytes);
+size_t split_attention_part_floats(int batch, int heads, int len, int pos_base, size_t kv_bytes, bool in_pairs);
 void split_attention(const PrefillAttnParams& p, int batch, char* kv, size_t kv_bytes, float* part, hipStream_t st);
 
 // Widest run of partial results per row that split_gemm<EPI_STORE> leaves.

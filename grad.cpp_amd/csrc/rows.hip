@@ -101,7 +101,9 @@ void split_gemm(SplitGemmParams& p, hipStream_t st) {
 // long blocks are shared, as coarsely as reaches 640 and so among 1300 or so at most (12 heads of 1999 tokens: 89 us unshared, 76 in runs of
 // 1024 keys, 47 of 512, 46 of 256, 48 of 128; the merge cost 1, 6, 8, 12, 18 us more, that of
 // 256 keys costs 9 since its loads go out together).
-static int attn_chunk_shift(int pairs, int len, int pos_base) {
+// attn_pair_kernel: 480 instead of 640 (12 heads of 1999 tokens with the merge: 44.6 us in runs of 256 keys, 42.3 of 512,
+// 57.8 of 1024; 48 heads of 1024: 41.1 unshared, 39.9 of 512, 46.6 of 256).
+static int attn_chunk_shift(int pairs, int len, int pos_base, bool in_pairs) {
     const int blocks = (len + kAttnQueries - 1) / kAttnQueries;
     int shift = 20;
     const auto workgroups = [&](int sh) {
@@ -109,8 +111,9 @@ static int attn_chunk_shift(int pairs, int len, int pos_base) {
         for (int i = 0; i < blocks; i++) n += attn_parts(i, len, pos_base, sh);
         return static_cast<long>(n) * pairs;
     };
-    if (workgroups(20) >= 640 || attn_key_tiles(blocks - 1, len, pos_base) <= 6) return 20;
-    for (shift = 14; shift > 1 && workgroups(shift) < 640; shift--) {
+    const int enough = in_pairs ? 480 : 640;
+    if (workgroups(20) >= enough || attn_key_tiles(blocks - 1, len, pos_base) <= 6) return 20;
+    for (shift = 14; shift > 1 && workgroups(shift) < enough; shift--) {
     }
     return shift;
 }
@@ -134,11 +137,11 @@ size_t split_attention_kv_bytes(int batch, int heads, int positions) {
     return std::max(pair, std::min(pair * batch * heads, size_t{256} << 20));
 }
 
-size_t split_attention_part_floats(int batch, int heads, int len, int pos_base, size_t kv_bytes) {
+size_t split_attention_part_floats(int batch, int heads, int len, int pos_base, size_t kv_bytes, bool in_pairs) {
     size_t need = 0;
     const int pairs = batch * heads, group = attn_group(pairs, pos_base + len, kv_bytes);
     for (const int n : {group, pairs % group}) {
-        const int shift = n ? attn_chunk_shift(n, len, pos_base) : 20;
+        const int shift = n ? attn_chunk_shift(n, len, pos_base, in_pairs) : 20;
         if (shift != 20) need = std::max(need, static_cast<size_t>(n) * attn_items(len, pos_base, shift) * kAttnPart);
     }
     return need;
@@ -167,7 +170,7 @@ void split_attention(const PrefillAttnParams& a, int batch, char* kv, size_t kv_
     p.scale = a.scale;
     for (p.first = 0; p.first < pairs; p.first += group) {
         p.pairs = std::min(group, pairs - p.first);
-        p.chunk_shift = attn_chunk_shift(p.pairs, a.len, a.pos_base);
+        p.chunk_shift = attn_chunk_shift(p.pairs, a.len, a.pos_base, in_pairs);
         p.items = attn_items(a.len, a.pos_base, p.chunk_shift);
         const SplitKvParams k{a.kv, a.layer, p.first, positions, kv, a.key_scale, a.pair_scale};
         hipLaunchKernelGGL(in_pairs ? split_kv_kernel<2> : split_kv_kernel<3>, dim3(p.tiles, p.pairs), dim3(256), 0, st, k);
