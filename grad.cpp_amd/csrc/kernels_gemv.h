@@ -135,7 +135,7 @@ __device__ __forceinline__ EpiOperands epi_fetch(const GemvParams& p, int b, int
         if (p.rope && row < 2 * p.d_model) {
             // head_size is even under RoPE, so (row, row+1) is one rotation pair.
             const int hs = p.kv.head_size;
-            const int j = ((row % p.d_model) % hs) >> 1;
+            const int j = (hs == 64 ? row & 63 : (row % p.d_model) % hs) >> 1;  // (a row of 64-wide heads is a multiple of 64)
             o.cs = p.rope_cos[o.pos * (hs >> 1) + j];
             o.sn = p.rope_sin[o.pos * (hs >> 1) + j];
         }
@@ -164,6 +164,25 @@ __device__ __forceinline__ void store_qkv(const GemvParams& p, int m, int row, f
             (((static_cast<size_t>(p.layer) * p.kv.n_pages + page) * 2 + (sec - 1)) * p.kv.heads + head);
         p.kv.pool[((run << p.kv.page_shift) + slot) * hs + j] = v;
     }
+}
+
+// Both values of a pair (row even) with 64-wide heads: they lie side by side, and nothing has to be divided
+// (beside fp32 matrix products every vector instruction counts).
+__device__ __forceinline__ void store_qkv_pair64(const GemvParams& p, int m, int row, float v0, float v1, const EpiOperands& o) {
+    const int d = p.d_model;
+    const int sec = (row >= d) + (row >= 2 * d), c = row - sec * d;
+    float* to;
+    if (sec == 0) {
+        to = p.out + static_cast<size_t>(m) * p.out_stride + c;
+    } else {
+        const int slot = o.pos & ((1 << p.kv.page_shift) - 1);
+        int page = o.page;  // (see store_qkv)
+        asm volatile("" : "+v"(page));
+        const size_t run =
+            (((static_cast<size_t>(p.layer) * p.kv.n_pages + page) * 2 + (sec - 1)) * p.kv.heads + (c >> 6));
+        to = p.kv.pool + ((run << p.kv.page_shift) + slot) * 64 + (c & 63);
+    }
+    *reinterpret_cast<float2*>(to) = make_float2(v0, v1);
 }
 
 template <int EPI>
@@ -195,8 +214,11 @@ __device__ __forceinline__ void epi_apply(const GemvParams& p, int b, int row, f
             a = ra;
             c = rc;
         }
-        store_qkv(p, b, row, a, o);
-        if (has1) store_qkv(p, b, row + 1, c, o);
+        if (p.kv.head_size == 64 && has1) store_qkv_pair64(p, b, row, a, c, o);
+        else {
+            store_qkv(p, b, row, a, o);
+            if (has1) store_qkv(p, b, row + 1, c, o);
+        }
     }
 }
 
