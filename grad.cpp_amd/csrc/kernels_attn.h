@@ -7,7 +7,7 @@
 // softmax_row (:60-67).
 #pragma once
 
-#include "kernels_pair.h"
+#include "operand_format.h"
 
 namespace gh {
 

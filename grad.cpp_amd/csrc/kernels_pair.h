@@ -35,74 +35,10 @@
 
 namespace gh {
 
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-
-constexpr int kPairMinCols = 512;
 constexpr int kPairStages = 4;  // of the ring of steps; also the steps of a part
-
-// Storage of a matrix of pairs (rows x K, K a multiple of 16): blocks of 16 rows x 16 columns, 1024
-// contiguous bytes each, row group by row group and inside one along K.  A block is the first parts of columns
-// 0..7 of its 16 rows (16 bytes each), those of columns 8..15, and the second parts likewise: 16 lanes that read
-// an operand's 16 rows read 256 consecutive bytes of LDS.
-constexpr int kPairBlockBytes = 1024, kPairPartBytes = 512, kPairChunkBytes = 256;
-
-// Byte offset of the first part of column k (a multiple of 8) of row r.
-__device__ __forceinline__ size_t pair_offset(int r, int k, int kblocks) {
-    return (static_cast<size_t>(r >> 4) * kblocks + (k >> 4)) * kPairBlockBytes + ((k >> 3) & 1) * kPairChunkBytes + (r & 15) * 16;
-}
 
 // Sign that the weights of block `block` of a row are stored with.
 __host__ __device__ __forceinline__ float pair_sign(int block) { return (block & kPairStages) ? -1.0f : 1.0f; }
-
-constexpr float kPairLift = 2048.0f;  // 2^11, of an activation's second part
-
-// Two values as two words of two fp16 each (low half: the first value's part).  The first parts are hidden from the
-// compiler once they are made: it would form them a second time, by an instruction that rounds halves the other way, for
-// the subtraction.
-__device__ __forceinline__ void to_pairs(float x, float y, float lift, unsigned& first, unsigned& second) {
-    typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-    first = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f{x, y}), v2h));
-    asm("" : "+v"(first));
-    const v2h f = __builtin_bit_cast(v2h, first);
-    second = __builtin_bit_cast(
-        unsigned, __builtin_convertvector((v2f{(x - static_cast<float>(f[0])) * lift, (y - static_cast<float>(f[1])) * lift}), v2h));
-}
-
-// Eight consecutive columns (k a multiple of 8) of one row of activations.
-__device__ __forceinline__ void store_pair8(char* base, int r, int k, int kblocks, const float (&v)[8], float scale) {
-    v4u p1, p2;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        unsigned a, b;
-        to_pairs(v[2 * i] * scale, v[2 * i + 1] * scale, kPairLift, a, b);
-        p1[i] = a;
-        p2[i] = b;
-    }
-    char* at = base + pair_offset(r, k, kblocks);
-    *reinterpret_cast<v4u*>(at) = p1;
-    *reinterpret_cast<v4u*>(at + kPairPartBytes) = p2;
-}
-
-// Four consecutive columns (k a multiple of 4).
-__device__ __forceinline__ void store_pair4(char* base, int r, int k, int kblocks, float x, float y, float z, float w, float scale) {
-    v2u p1, p2;
-    unsigned a, b;
-    to_pairs(x * scale, y * scale, kPairLift, a, b);
-    p1[0] = a, p2[0] = b;
-    to_pairs(z * scale, w * scale, kPairLift, a, b);
-    p1[1] = a, p2[1] = b;
-    char* at = base + pair_offset(r, k & ~7, kblocks) + (k & 4) * 2;
-    *reinterpret_cast<v2u*>(at) = p1;
-    *reinterpret_cast<v2u*>(at + kPairPartBytes) = p2;
-}
-
-// Four consecutive columns of a row of activations, in the form that the projection behind reads: pairs scaled by
-// pair_scale, three parts where that is zero.
-__device__ __forceinline__ void store_operand4(char* base, int r, int k, int kblocks, float x, float y, float z, float w,
-                                               float pair_scale) {
-    if (pair_scale != 0.0f) store_pair4(base, r, k, kblocks, x, y, z, w, pair_scale);
-    else store_split4(base, r, k, kblocks, x, y, z, w);
-}
 
 // Writes the pairs of a weight matrix src (N x K, row per output), rows in the order of split_weights_kernel, one
 // wavefront per row, zeros past N.  unit[j]: the power of two that output j's sum is to be multiplied by, j as the

@@ -26,79 +26,9 @@
 #pragma once
 
 #include "kernels_gemv.h"
+#include "operand_format.h"
 
 namespace gh {
-
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef float v2f __attribute__((ext_vector_type(2)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef unsigned v2u __attribute__((ext_vector_type(2)));
-typedef unsigned v4u __attribute__((ext_vector_type(4)));
-
-// Two floats as three words of two bf16 each (low half: the first float's part).
-__device__ __forceinline__ void split_pair(float x, float y, unsigned& p1, unsigned& p2, unsigned& p3) {
-    const auto pack = [](float a, float b) {
-        return __builtin_bit_cast(unsigned, __builtin_convertvector((v2f{a, b}), v2bf));
-    };
-    const auto lo = [](unsigned w) { return __uint_as_float(w << 16); };
-    const auto hi = [](unsigned w) { return __uint_as_float(w & 0xFFFF0000u); };
-    p1 = pack(x, y);
-    x -= lo(p1);
-    y -= hi(p1);
-    p2 = pack(x, y);
-    p3 = pack(x - lo(p2), y - hi(p2));
-}
-
-constexpr unsigned kSplitTop = 0x7F7F8000u;  // bits of the smallest magnitude that rounds to an infinite bf16
-
-// Storage of a split matrix (rows x K, K a multiple of 16): blocks of 16 rows x 16 columns,
-// 1536 contiguous bytes each, row group by row group and inside one along K.  In a block a
-// row is 96 bytes: the 16 first parts, the 16 second, the 16 third, each as two 16-byte
-// chunks of eight columns, in the other order in rows 8..15.  A block is copied into LDS as
-// it is; that exchange of chunks makes the 16-byte operand reads of 16 rows fall on all 64
-// banks once.
-constexpr int kSplitRows = 16, kSplitCols = 16;
-constexpr int kSplitPartBytes = kSplitCols * 2;  // from one part of a row to the next
-constexpr int kSplitRowBytes = 3 * kSplitPartBytes;
-constexpr int kSplitBlockBytes = kSplitRows * kSplitRowBytes;
-
-// Byte offset of the first part of column k (a multiple of 8: the start of a chunk) of row r.
-__device__ __forceinline__ size_t split_offset(int r, int k, int kblocks) {
-    return (static_cast<size_t>(r >> 4) * kblocks + (k >> 4)) * kSplitBlockBytes + (r & 15) * kSplitRowBytes
-           + ((((k >> 3) & 1) ^ ((r >> 3) & 1)) << 4);
-}
-
-// Eight consecutive columns (k a multiple of 8) of one row.
-__device__ __forceinline__ void store_split8(char* base, int r, int k, int kblocks, const float (&v)[8]) {
-    v4u p1, p2, p3;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        unsigned a, b, c;
-        split_pair(v[2 * i], v[2 * i + 1], a, b, c);
-        p1[i] = a;
-        p2[i] = b;
-        p3[i] = c;
-    }
-    char* at = base + split_offset(r, k, kblocks);
-    *reinterpret_cast<v4u*>(at) = p1;
-    *reinterpret_cast<v4u*>(at + kSplitPartBytes) = p2;
-    *reinterpret_cast<v4u*>(at + 2 * kSplitPartBytes) = p3;
-}
-
-// Four consecutive columns (k a multiple of 4).
-__device__ __forceinline__ void store_split4(char* base, int r, int k, int kblocks, float x, float y, float z, float w) {
-    v2u p1, p2, p3;
-    unsigned a, b, c;
-    split_pair(x, y, a, b, c);
-    p1[0] = a, p2[0] = b, p3[0] = c;
-    split_pair(z, w, a, b, c);
-    p1[1] = a, p2[1] = b, p3[1] = c;
-    char* at = base + split_offset(r, k & ~7, kblocks) + (k & 4) * 2;
-    *reinterpret_cast<v2u*>(at) = p1;
-    *reinterpret_cast<v2u*>(at + kSplitPartBytes) = p2;
-    *reinterpret_cast<v2u*>(at + 2 * kSplitPartBytes) = p3;
-}
 
 // Rows of weights are stored in the order in which the accumulator hands outputs back: of
 // every 32 outputs, lane half h of a 32 x 32 product holds matrix rows 8 q + 4 h + e (q, e in

@@ -2,7 +2,7 @@
 // projections (kernels_split.h): six bf16 products for one fp32 product, head size 64.
 #pragma once
 
-#include "kernels_pair.h"
+#include "kernels_split.h"
 
 namespace gh {
 

@@ -1,6 +1,8 @@
 // The many-row projections in pairs: variants and the rule that picks one, in a translation unit of their own.
 #include "rows.h"
 
+#include "kernels_pair.h"
+
 #include <algorithm>
 #include <cmath>
 #include <stdexcept>

@@ -23,7 +23,10 @@ void norm_split(bool rms, const float* x, const float* gamma, const float* beta,
 template <int EPI>
 void split_gemm(SplitGemmParams& p, hipStream_t st);
 
-// The same three in pairs (kernels_pair.h); units of a matrix: one per row of its storage.
+// Narrower models have no pairs (kernels_pair.h).
+constexpr int kPairMinCols = 512;
+
+// The same three in pairs; units of a matrix: one per row of its storage.
 // (whole tiles of 96 outputs, also from a row behind the first)
 inline size_t pair_rows(size_t rows) { return (rows + 95 + kSplitPad - 1) / kSplitPad * kSplitPad; }
 inline size_t pair_bytes(size_t rows, size_t cols) { return pair_rows(rows) * cols * 4; }
