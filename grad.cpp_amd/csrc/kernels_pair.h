@@ -133,6 +133,81 @@ struct PairRowsOut {
     }
 };
 
+// EPI_RESID and EPI_QKV leave in strips of 8 rows x 32 outputs (lane / 8 the row, four outputs per lane), after a turn of
+// a 32 x 32 block through LDS.  A lane of the accumulators holds 16 outputs of one row: from there an instruction
+// touched 64 lines for 16 bytes each, a strip is eight whole lines.  What a strip reads, of memory that nobody else writes
+// meanwhile, is requested in front of the products.  Where sets share K, all of them add and store strips,
+// instead of the first set alone.  Same sums in the same order.  us per launch, before -> after: W_o and FFN2 of 16384
+// rows 159 -> 155 (768 columns wide, GPT), 191 -> 176 (Llama, 16000 rows), QKV 197 -> 181 and 287 -> 267, 2048 rows' W_o and FFN2 23.0 -> 21.5;
+// over 160 to 16384 rows 4 to 11 % less.  A residual's bias and units held the same way from the start were slower (128 x 128:
+// 253 registers, 0.995 of before instead of 0.945); QKV's are held where the wavefront's sums are its own (0.95 -> 0.91).
+constexpr int kTurnStride = 36, kTurnFloats = 32 * kTurnStride;  // of a block of 32 x 32
+
+__device__ __forceinline__ void turn_block(float* lds, const v16f& v) {
+    const int lane = threadIdx.x & 63;
+    float* const to = lds + (lane & 31) * kTurnStride + 16 * (lane >> 5);
+#pragma unroll
+    for (int q = 0; q < 4; q++) *reinterpret_cast<float4*>(to + 4 * q) = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+}
+
+__device__ __forceinline__ float4 turned_strip(const float* lds, int i) {
+    const int lane = threadIdx.x & 63;
+    return *reinterpret_cast<const float4*>(lds + (8 * i + (lane >> 3)) * kTurnStride + (lane & 7) * 4);
+}
+
+struct StripRow {  // EPI_QKV
+    int pos, page;
+};
+
+struct StripColumns {  // EPI_QKV: of the lane's four outputs
+    float4 unit, bias;
+};
+
+__device__ __forceinline__ StripColumns strip_columns(const SplitGemmParams& p, int n) {
+    // (storage of units for whole tiles, as of the weights)
+    return {*reinterpret_cast<const float4*>(p.unit + n),
+            n < p.N ? *reinterpret_cast<const float4*>(p.bias + p.first + n) : make_float4(0.f, 0.f, 0.f, 0.f)};
+}
+
+__device__ __forceinline__ StripRow strip_row(const SplitGemmParams& p, int m) {
+    const int row = min(m, p.M - 1), seq = row / p.rows_per_seq, pos = p.pos_base + (row - seq * p.rows_per_seq);
+    return {pos, p.kv.page_table[seq * p.kv.pages_per_seq + (pos >> p.kv.page_shift)]};
+}
+
+__device__ __forceinline__ float4 strip_operand(const SplitGemmParams& p, int m, int n) {  // EPI_RESID
+    return m < p.M && n < p.N ? *reinterpret_cast<const float4*>(p.out + static_cast<size_t>(m) * p.out_stride + n)
+                              : make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+// Outputs n .. n + 3 of row m.
+__device__ __forceinline__ void strip_resid(const SplitGemmParams& p, int m, int n, const float4& y, const float4& v) {
+    // y += b, then y += x @ W (inference.cpp:22-28)
+    float4 c = y;
+    if (p.bias) {
+        const float4 bb = *reinterpret_cast<const float4*>(p.bias + n);
+        c = make_float4(c.x + bb.x, c.y + bb.y, c.z + bb.z, c.w + bb.w);
+    }
+    *reinterpret_cast<float4*>(p.out + static_cast<size_t>(m) * p.out_stride + n) = make_float4(c.x + v.x, c.y + v.y, c.z + v.z, c.w + v.w);
+}
+
+__device__ __forceinline__ void strip_qkv(const SplitGemmParams& p, int m, int n, const StripRow& r, const float4& bb, const float4& v) {
+    const int of = p.first + n, sec = (of >= p.d_model) + (of >= 2 * p.d_model), c = of - sec * p.d_model, j = c & 63;
+    float4 o = make_float4(v.x + bb.x, v.y + bb.y, v.z + bb.z, v.w + bb.w);
+    if (p.rope && sec < 2) {
+        const float2 cs = *reinterpret_cast<const float2*>(p.rope_cos + r.pos * 32 + (j >> 1));
+        const float2 sn = *reinterpret_cast<const float2*>(p.rope_sin + r.pos * 32 + (j >> 1));
+        o = make_float4(o.x * cs.x - o.y * sn.x, o.x * sn.x + o.y * cs.x, o.z * cs.y - o.w * sn.y, o.z * sn.y + o.w * cs.y);
+    }
+    float* dst;
+    if (sec == 0) {
+        dst = p.out + static_cast<size_t>(m) * p.out_stride + c;
+    } else {
+        const size_t run = ((static_cast<size_t>(p.layer) * p.kv.n_pages + r.page) * 2 + (sec - 1)) * p.kv.heads + (c >> 6);
+        dst = p.kv.pool + ((run << p.kv.page_shift) + (r.pos & ((1 << p.kv.page_shift) - 1))) * 64 + j;
+    }
+    *reinterpret_cast<float4*>(dst) = o;
+}
+
 // C[M,N] = A[M,K] . W[N,K]^T of pairs.  Tiles, workgroup order, LDS ring and epilogues are split_gemm_kernel's.
 // A step of 16 columns is three rounds of products (w1 a2, w2 a1, w1 a1), its fragments read from LDS during the
 // step before into registers of their own (a 64 x 64 wavefront has 128 of its 256 for sums).  Four steps make a
@@ -197,6 +272,38 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
 #pragma unroll
             for (int b = 0; b < MB; b++) part[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[a], x[b], part[a][b], 0, 0, 0);
     };
+    // Strips: of the wavefront's own blocks, or, where sets share K, every kAll-th of the tile's.
+    // (QKV's 64 x 96 tiles with K shared by two sets are as fast without, 37.9 us against 38.9 for 2048 x 2304 x 768.)
+    constexpr bool kStrips = EPI == EPI_RESID || (EPI == EPI_QKV && !(NB == 3 && KG == 2));
+    constexpr int kAll = kWaves * KG, kCount = KG == 1 ? MB * NB * 4 : TM * TN / 256 / kAll;
+    static_assert(!kStrips || kCount * 256 * kAll == TM * TN, "whole rounds of strips");
+    const int col = (lane & 7) * 4;
+    const auto strip_block = [&](int i) { return KG == 1 ? i >> 2 : (wave_id + i * kAll) >> 2; };  // a * MB + b; of the tile: row by row
+    const auto strip_at = [&](int i) { return KG == 1 ? i & 3 : (wave_id + i * kAll) & 3; };
+    const auto strip_m = [&](int i) {
+        const int block = strip_block(i);
+        return m_tile * TM + (KG == 1 ? (wm * MB + block % MB) * 32 : block / (TN / 32) * 32) + strip_at(i) * 8 + (lane >> 3);
+    };
+    const auto strip_n = [&](int i) {
+        const int block = strip_block(i);
+        return n_tile * TN + (KG == 1 ? (wn * NB + block / MB) * 32 : block % (TN / 32) * 32) + col;
+    };
+    constexpr bool kColumnsEarly = EPI == EPI_QKV && KG == 1;
+    StripColumns cols[kColumnsEarly ? NB : 1];
+    if constexpr (kColumnsEarly) {
+#pragma unroll
+        for (int a = 0; a < NB; a++) cols[a] = strip_columns(p, strip_n(a * MB * 4));
+    }
+    float4 y[EPI == EPI_RESID ? kCount : 1];
+    StripRow row[EPI == EPI_QKV && kStrips ? (KG == 1 ? MB * 4 : kCount) : 1];
+    if constexpr (EPI == EPI_RESID) {
+#pragma unroll
+        for (int i = 0; i < kCount; i++) y[i] = strip_operand(p, strip_m(i), strip_n(i));
+    }
+    if constexpr (EPI == EPI_QKV && kStrips) {
+#pragma unroll
+        for (int i = 0; i < (KG == 1 ? MB * 4 : kCount); i++) row[i] = strip_row(p, strip_m(i));
+    }
 #pragma unroll
     for (int s = 0; s < kStages; s++)
 #pragma unroll
@@ -250,6 +357,46 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
 #pragma unroll
                 for (int r = 0; r < 16; r++) sum[a][b][r] = __builtin_fmaf(part[a][b][r], sign, sum[a][b][r]);
     }
+    const auto scaled = [&](const float4& v, const float4& unit) {
+        const float f = p.operand_unit;
+        return make_float4(v.x * (unit.x * f), v.y * (unit.y * f), v.z * (unit.z * f), v.w * (unit.w * f));
+    };
+    const auto strip_out = [&](int i, const float4& v) {
+        const int m = strip_m(i), n = strip_n(i);
+        if (m >= p.M || n >= p.N) return;
+        if constexpr (EPI == EPI_RESID) {
+            strip_resid(p, m, n, y[i], v);
+        } else if constexpr (kColumnsEarly) {
+            const StripColumns& c = cols[i / (MB * 4)];
+            strip_qkv(p, m, n, row[i % (MB * 4)], c.bias, scaled(v, c.unit));
+        } else if constexpr (EPI == EPI_QKV) {
+            strip_qkv(p, m, n, row[i], *reinterpret_cast<const float4*>(p.bias + p.first + n), v);
+        }
+    };
+    if constexpr (KG > 1 && kStrips) {
+        // Every set leaves its sums in the LDS that the rings no longer need; a strip's are added in the sets' order.
+        constexpr int kBlocks = TM * TN / 1024;
+        static_assert(KG * kBlocks * kTurnFloats * 4 <= KG * kStages * kStage, "they fit in the rings");
+        float* const sums = reinterpret_cast<float*>(lds_pair);
+        __syncthreads();
+#pragma unroll
+        for (int a = 0; a < NB; a++)
+#pragma unroll
+            for (int b = 0; b < MB; b++)
+                turn_block(sums + (kg * kBlocks + (wm * MB + b) * (TN / 32) + wn * NB + a) * kTurnFloats, sum[a][b]);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kCount; i++) {
+            float4 v = turned_strip(sums + strip_block(i) * kTurnFloats, strip_at(i));
+#pragma unroll
+            for (int g = 1; g < KG; g++) {
+                const float4 w = turned_strip(sums + (g * kBlocks + strip_block(i)) * kTurnFloats, strip_at(i));
+                v = make_float4(v.x + w.x, v.y + w.y, v.z + w.z, v.w + w.w);
+            }
+            strip_out(i, scaled(v, *reinterpret_cast<const float4*>(p.unit + strip_n(i))));
+        }
+        return;
+    }
     if constexpr (KG > 1) {
         // the other sets' sums through the LDS the rings no longer need, added in order
         float* sums = reinterpret_cast<float*>(lds_pair);
@@ -275,24 +422,40 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
                     for (int r = 0; r < 16; r++) sum[a][b][r] += at(g, a, b)[r * 64];
     }
     const int n0 = n_tile * TN + wn * 32 * NB;
+    if constexpr (!kColumnsEarly) {
 #pragma unroll
-    for (int a = 0; a < NB; a++) {
-        // (storage of units for whole tiles, as of the weights)
-        const float4* const u = reinterpret_cast<const float4*>(p.unit + n0 + 32 * a + 16 * h32);
-        float units[16];
+        for (int a = 0; a < NB; a++) {
+            // (storage of units for whole tiles, as of the weights)
+            const float4* const u = reinterpret_cast<const float4*>(p.unit + n0 + 32 * a + 16 * h32);
+            float units[16];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const float4 v = u[q];
-            units[4 * q] = v.x, units[4 * q + 1] = v.y, units[4 * q + 2] = v.z, units[4 * q + 3] = v.w;
-        }
+            for (int q = 0; q < 4; q++) {
+                const float4 v = u[q];
+                units[4 * q] = v.x, units[4 * q + 1] = v.y, units[4 * q + 2] = v.z, units[4 * q + 3] = v.w;
+            }
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const float f = units[r] * p.operand_unit;
+            for (int r = 0; r < 16; r++) {
+                const float f = units[r] * p.operand_unit;
 #pragma unroll
-            for (int b = 0; b < MB; b++) sum[a][b][r] *= f;
+                for (int b = 0; b < MB; b++) sum[a][b][r] *= f;
+            }
         }
     }
-    split_epilogue<PairRowsOut, EPI, MB, NB>(p, sum, m_tile * TM + wm * 32 * MB, n0, n_tile * WN + wn);
+    if constexpr (kStrips) {
+        // (every wavefront has its last step's fragments, so the rings' places are free, one block's to each)
+        static_assert(kWaves * kTurnFloats * 4 <= kStages * kStage, "they fit in the ring");
+        float* const block = reinterpret_cast<float*>(lds_pair) + wave * kTurnFloats;
+#pragma unroll
+        for (int a = 0; a < NB; a++)
+#pragma unroll
+            for (int b = 0; b < MB; b++) {
+                turn_block(block, sum[a][b]);
+#pragma unroll
+                for (int i = 0; i < 4; i++) strip_out((a * MB + b) * 4 + i, turned_strip(block, i));
+            }
+    } else {
+        split_epilogue<PairRowsOut, EPI, MB, NB>(p, sum, m_tile * TM + wm * 32 * MB, n0, n_tile * WN + wn);
+    }
 }
 
 }  // namespace gh

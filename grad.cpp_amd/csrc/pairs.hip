@@ -38,24 +38,24 @@ void norm_pair(bool rms, const float* x, const float* gamma, const float* beta, 
 
 // The tilings, and what a launch takes with each: with n tiles on the fullest of 256 compute units and K in thousands
 //   start + max(chain K, n step K) + n out
-// us, fitted to 231 launches (160 to 16384 rows against the ten matrices of models 512 and 768 columns wide: W_o,
-// QKV, both FFN1 and FFN2), medians off by 6 to 9 %.  A lone workgroup is a chain of K steps (64 x 64 tiles with K shared by four
-// sets of wavefronts, and 32 x 32 ones, are the shorter chains); beside others its chain hides, and what counts is what the unit
+// us, fitted to 230 launches (160 to 16384 rows against the ten matrices of models 512 and 768 columns wide: W_o,
+// QKV, both FFN1 and FFN2), medians off by 2 to 5 %.  A lone workgroup is a chain of K steps (64 x 64 tiles with K shared by
+// two sets of wavefronts, and 32 x 32 ones by four, are the shorter chains); beside others its chain hides, and what counts is what the unit
 // moves through LDS and multiplies; `out` is the epilogue, of a residual (queries, keys, values and logits counted
-// like it), a GELU or a SwiGLU.  Taking the least by this rule, those launches take 1.2 % longer than with the
-// best of eleven tilings each (at most 12 %), 1.3 with the same seven and no line between epilogues, 8.0 with the three-part form's rule
-// (at most 48 %).  1999 x 768 x 768 15.9 -> 13.3 us, 1999 x 768 x 2048 31.3 -> 25.2, 1999 x 2304 x 768 33.4 -> 30.5, 1999 x 3072 x 768
-// 44.7 -> 39.4.
+// like it), a GELU or a SwiGLU.  Taking the least by this rule, those launches take 0.8 % longer than with the
+// best of the seven tilings each (at most 18 %), by the three-part form's rule 5.1 (at most 44 %): 1999 x 768 x 768
+// 14.0 -> 11.4 us, 1999 x 768 x 2048 31.9 -> 24.2, 1999 x 2304 x 768 31.8 -> 31.1, 1999 x 3072 x 768 37.5 -> 34.8.  (Four tilings more, among them 96 x 192, 192 x 64
+// and 128 x 96, were the best by less than 1 % together.)
 struct Tiling {
     int m, n, sets;  // rows, outputs, sets of wavefronts that share K
     float start, chain, step, out[3];
 };
 enum { TILE_128, TILE_128x64, TILE_64, TILE_64_K2, TILE_64x96_K2, TILE_64x96_K4, TILE_32_K4, TILINGS };
 constexpr Tiling kTilings[TILINGS] = {
-    {128, 128, 1, 2.94f, 22.28f, 18.05f, {5.93f, 9.24f, 4.43f}}, {128, 64, 1, 2.39f, 13.85f, 10.60f, {3.23f, 4.09f, 1.92f}},
-    {64, 64, 1, 2.49f, 9.47f, 6.43f, {1.56f, 1.75f, 0.87f}},     {64, 64, 2, 1.96f, 4.74f, 6.25f, {2.14f, 2.64f, 1.37f}},
-    {64, 96, 2, 1.75f, 10.33f, 8.38f, {3.33f, 6.61f, 2.86f}},    {64, 96, 4, 0.50f, 0.49f, 8.40f, {5.86f, 12.77f, 5.47f}},
-    {32, 32, 4, 1.93f, 2.93f, 2.57f, {0.89f, 2.14f, 0.95f}},
+    {128, 128, 1, 1.64f, 21.42f, 18.17f, {4.43f, 4.01f, 3.31f}}, {128, 64, 1, 2.15f, 13.10f, 10.78f, {1.94f, 1.80f, 1.20f}},
+    {64, 64, 1, 1.90f, 9.58f, 6.45f, {1.00f, 0.80f, 0.58f}},     {64, 64, 2, 1.61f, 6.59f, 6.31f, {1.18f, 1.18f, 1.01f}},
+    {64, 96, 2, 2.37f, 10.21f, 8.57f, {2.15f, 2.14f, 1.44f}},    {64, 96, 4, 0.50f, 2.40f, 8.44f, {3.72f, 4.87f, 3.85f}},
+    {32, 32, 4, 2.14f, 2.68f, 2.53f, {0.46f, 0.81f, 0.62f}},
 };
 
 static int pick_tiling(int M, int N, int K, int epilogue) {
