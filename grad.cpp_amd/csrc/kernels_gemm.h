@@ -324,6 +324,10 @@ __global__ __launch_bounds__(64 * KW) void gemm16_kernel(const GemvParams p, int
         epi_at(e, m, n, t, u, at);
         if (m >= M || n >= p.N) continue;
         const int i = at >> 4;
+        const bool has1 = n + 1 < p.N;
+        // (in front of the sums, so that one block holds sums and epilogue in every tiling and they are rounded alike)
+        EpiOperands epi = first_epi;
+        if (kEpiElems > 64 * KW && e != static_cast<int>(threadIdx.x)) epi = epi_fetch<EPI>(p, m, n, has1);
         float v0 = 0.0f, v1 = 0.0f;
 #pragma unroll
         for (int w = 0; w < KW; w++) {
@@ -338,9 +342,7 @@ __global__ __launch_bounds__(64 * KW) void gemm16_kernel(const GemvParams p, int
             v0 *= r;
             v1 *= r;
         }
-        const bool has1 = n + 1 < p.N;
-        if (e == static_cast<int>(threadIdx.x)) epi_apply<EPI>(p, m, n, v0, v1, has1, first_epi);
-        else gemv_epilogue<EPI>(p, m, n, v0, v1, has1);
+        epi_apply<EPI>(p, m, n, v0, v1, has1, epi);
         if constexpr (EPI == EPI_STORE) {
             if (p.best) {
                 // eight neighbouring lanes hold the 16 columns of one row of one tile, in
@@ -598,8 +600,13 @@ inline void launch_gemm_wide(const GemvParams& p, int M, hipStream_t st) {
 // share the rows they read (what is being paid for is operand traffic from the L2s and operand
 // permutes, 2 x 2 tiles having half of both per product).  Measured over 65 to 511 rows against thirteen
 // matrices (512 to 4096 outputs, 512 to 4096 columns): 1 x 1 tiles 1.7 us per workgroup and 768 columns,
-// two tiles 2.4, 2 x 2 4.0; the rule's pick is the fastest of them or within 6 % of it in 142 of 143
-// cases, and 11.3 us for 9.8 at 511 x 768 x 768 (profiles/many_row_tilings.md).
+// two tiles 2.4, 2 x 2 4.0; the rule's pick of these four is the fastest or within 6 % of it in 142 of 143
+// cases, and 11.3 us for 9.8 at 511 x 768 x 768 (profiles/many_row_tilings.md).  3 x 2 tiles 5.9 and 2 x 3 6.2, for
+// the row counts where four tiles leave a last workgroup to few compute units: over 22 row counts and 13 matrices the
+// rule with them is faster by more than 2 % in 69 of 286 cases (384 x 1024 x 768 11.9 us -> 9.0, 511 x 768 x 768
+// 11.2 -> 9.5, 397 x 768 x 2048 19.5 -> 18.0, 244 x 4096 x 768 unchanged at 22.4) and slower by that much in one (3 %); 2.2 %
+// in the mean.  Queries, keys and values stay with four: six tiles are a second round of their epilogue, whose reads
+// (position, page, rotation) nothing hides (244 x 2304 x 768 in a prompt 20.2 us -> 23.4).
 // 1 x 1 for narrow matrices and 4 x 1 for the others, as it was: 100 x 4096 x 768 17.1 us -> 14.3,
 // 244 x 2304 x 768 24.4 -> 17.1, 397 x 4096 x 768 52.5 -> 35.8, 244 x 768 x 2048 12.8 -> 12.2.
 // (Both operands through an LDS ring, 32 x 32 to 64 x 64 outputs per workgroup: 35-36 us at 397 x 4096 x
@@ -612,7 +619,12 @@ inline void launch_gemm16_many(const GemvParams& p, int M, hipStream_t st) {
     };
     const bool wide = p.N > 1024;
     const long c11 = cost(1, 1, 17), c12 = cost(1, 2, wide ? 24 : 25), c21 = cost(2, 1, wide ? 25 : 24), c22 = cost(2, 2, 40);
-    const long least = std::min(std::min(c11, c12), std::min(c21, c22));
+    const long least = std::min({c11, c12, c21, c22});
+    if constexpr (EPI != EPI_QKV) {
+        const long c32 = cost(3, 2, 59), c23 = cost(2, 3, 62);
+        if (c32 < least && c32 <= c23) return launch_gemm16_as<EPI, RMS, 3, 2, 8>(p, M, st);
+        if (c23 < least) return launch_gemm16_as<EPI, RMS, 2, 3, 8>(p, M, st);
+    }
     if (c22 == least) launch_gemm16_as<EPI, RMS, 2, 2, 8>(p, M, st);
     else if (c12 == least) launch_gemm16_as<EPI, RMS, 1, 2, 8>(p, M, st);
     else if (c21 == least) launch_gemm16_as<EPI, RMS, 2, 1, 8>(p, M, st);

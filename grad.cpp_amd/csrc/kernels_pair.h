@@ -138,7 +138,7 @@ struct PairRowsOut {
 // touched 64 lines for 16 bytes each, a strip is eight whole lines.  What a strip reads, of memory that nobody else writes
 // meanwhile, is requested in front of the products.  Where sets share K, all of them add and store strips,
 // instead of the first set alone.  Same sums in the same order.  us per launch, before -> after: W_o and FFN2 of 16384
-// rows 159 -> 155 (768 columns wide, GPT), 191 -> 176 (Llama, 16000 rows), QKV 197 -> 181 and 287 -> 267, 2048 rows' W_o and FFN2 23.0 -> 21.5;
+// rows 159 -> 155 (a GPT of 768 columns), of 24576 191 -> 176 (a Llama of 768), QKV 197 -> 181 and 287 -> 267, 2048 rows' W_o and FFN2 23.0 -> 21.5;
 // over 160 to 16384 rows 4 to 11 % less.  A residual's bias and units held the same way from the start were slower (128 x 128:
 // 253 registers, 0.995 of before instead of 0.945); QKV's are held where the wavefront's sums are its own (0.95 -> 0.91).
 constexpr int kTurnStride = 36, kTurnFloats = 32 * kTurnStride;  // of a block of 32 x 32

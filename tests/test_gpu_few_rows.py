@@ -44,6 +44,25 @@ def test_tiles_do_not_change_a_pass(arch, d):
                 assert got[b].tobytes() == last.tobytes(), (batch, b)
 
 
+@pytest.mark.parametrize("arch, d", [(synth.ARCH_GPT2, 512), (synth.ARCH_MODERN, 768), (synth.ARCH_GPT2, 1024)])
+def test_tiles_do_not_change_the_cache(arch, d):
+    """Rows around whole tiles of 48 and 32: what a prompt leaves of its first positions is the same after any number
+    of rows behind them, tiles of 3 x 2 and 2 x 3 among them (matrices whose outputs are no multiple of 48 too)."""
+    cfg = synth.Config(arch, 201, d, 2, d // 64, 520)
+    W = synth.make_weights(cfg, 99, std=lively_std(cfg), norm_noise=0.1)
+    gm = G.Model.from_tensors(cfg, W)
+    tokens = synth.uniform_tokens(511, cfg.vocab, 100)
+    kept = None
+    for n in (96, 160, 192, 193, 255, 257, 336, 384, 385, 432, 433, 511):
+        s = G.Session(gm)
+        got = s.prefill(tokens[:n])
+        if n in (193, 384, 511):
+            assert_logits_close(got, ref_forward.forward(cfg, W, tokens[:n])[-1], what=f"cache {d} {n}")
+        rows = [s.read_kv(0, 1, kv, pos).tobytes() for kv in (0, 1) for pos in (0, 31, 47, 95)]
+        kept = kept or rows
+        assert rows == kept, n
+
+
 def test_tiles_do_not_change_a_batched_step():
     """33 to 64 sequences: up to 48 the FFN's first matrix goes tile by tile, beyond in pairs of tiles."""
     cfg = synth.Config(synth.ARCH_MODERN, 201, 768, 1, 12, 16)
