@@ -214,8 +214,8 @@ __device__ __forceinline__ void strip_qkv(const SplitGemmParams& p, int m, int n
 // 64-column part that starts from zero and is then added to the running sums (or taken from them, the weights of every
 // other part being negative).  (Added in front of the next part's products instead, accumulator by accumulator, the
 // compiler copies every part first.)  K / KG is a multiple of 64.
-template <int EPI, int MB, int NB, int WM, int WN, int KG, int PER_CU>
-__global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void pair_gemm_kernel(const SplitGemmParams p) {
+template <int EPI, int MB, int NB, int WM, int WN, int KG>
+__device__ __forceinline__ void pair_tile(const SplitGemmParams& p, int m_tile, int n_tile) {
     extern __shared__ __attribute__((aligned(1024))) char lds_pair[];
     constexpr int kWaves = WM * WN, TM = 32 * MB * WM, TN = 32 * NB * WN, kStages = kPairStages;
     constexpr int kUnitsA = TM / 16, kUnits = (TM + TN) / 16;  // 1024-byte loads of a step: a block each
@@ -225,8 +225,6 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
     const int lane = threadIdx.x & 63, wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kg = wave_id / kWaves, wave = wave_id % kWaves;
     const int wm = wave / WN, wn = wave % WN;
-    int m_tile, n_tile;
-    if (!split_tile(p, m_tile, n_tile)) return;
     const int row_blocks = p.K / kSplitCols, kblocks = row_blocks / KG;  // of a row, of this set of wavefronts
     const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) char*)lds_pair))
                           + kg * (kStages * kStage);
@@ -455,6 +453,33 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
             }
     } else {
         split_epilogue<PairRowsOut, EPI, MB, NB>(p, sum, m_tile * TM + wm * 32 * MB, n0, n_tile * WN + wn);
+    }
+}
+
+template <int EPI, int MB, int NB, int WM, int WN, int KG, int PER_CU>
+__global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void pair_gemm_kernel(const SplitGemmParams p) {
+    int m_tile, n_tile;
+    if (split_tile(p, m_tile, n_tile)) pair_tile<EPI, MB, NB, WM, WN, KG>(p, m_tile, n_tile);
+}
+
+// Tiles of 128 x 128, those behind the first `whole` (whole rounds of 256 compute units) in quarters of 64 x 64, dealt
+// over the XCDs the same way.  Bound by the LDS reads and products of a compute unit's whole tiles and its quarter; sums are those of either
+// tiling.  Figures and the line at pick_tiling.
+template <int EPI>
+__global__ __launch_bounds__(256, 2) void pair_mixed_kernel(const SplitGemmParams p, int whole) {
+    const int id = blockIdx.x;
+    int m_tile, n_tile;
+    if (id < whole) {
+        split_place(p, (id & 7) * (whole >> 3) + (id >> 3), m_tile, n_tile);
+        pair_tile<EPI, 2, 2, 2, 2, 1>(p, m_tile, n_tile);
+    } else {
+        const int per = (p.tiles - whole + 7) >> 3, slot = (id - whole) >> 3, quarter = slot & 3;
+        const int tile = whole + (id & 7) * per + (slot >> 2);
+        if ((slot >> 2) >= per || tile >= p.tiles) return;
+        split_place(p, tile, m_tile, n_tile);
+        m_tile = 2 * m_tile + (quarter >> 1);
+        n_tile = 2 * n_tile + (quarter & 1);
+        if (m_tile * 64 < p.M && n_tile * 64 < p.N) pair_tile<EPI, 1, 1, 2, 2, 1>(p, m_tile, n_tile);
     }
 }
 

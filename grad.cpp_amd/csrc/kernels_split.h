@@ -238,18 +238,23 @@ __device__ __forceinline__ void meet() {
     asm volatile("" ::: "memory");
 }
 
-// The workgroup's tile.  Workgroup ids go round-robin over the eight XCDs: every XCD takes a contiguous run of
-// tiles, eight row tiles deep inside a column of outputs, so that what its workgroups read
-// at about the same time is the same few tiles of both operands.  False: there is none for it.
-__device__ __forceinline__ bool split_tile(const SplitGemmParams& p, int& m_tile, int& n_tile) {
-    const int per = (p.tiles + 7) >> 3, id = blockIdx.x;
-    const int tile = (id & 7) * per + (id >> 3);
-    if ((id >> 3) >= per || tile >= p.tiles) return false;
+// The place of the tile-th tile: eight row tiles deep inside a column of outputs, so that what workgroups with
+// neighbouring tiles read at about the same time is the same few tiles of both operands.
+__device__ __forceinline__ void split_place(const SplitGemmParams& p, int tile, int& m_tile, int& n_tile) {
     const int m_tiles = p.tiles / p.n_tiles;
     const int group = tile / (8 * p.n_tiles), rest = tile - group * 8 * p.n_tiles;
     const int deep = min(8, m_tiles - group * 8);
     n_tile = rest / deep;
     m_tile = group * 8 + rest - n_tile * deep;
+}
+
+// The workgroup's tile.  Workgroup ids go round-robin over the eight XCDs: every XCD takes a contiguous run of
+// tiles.  False: there is none for it.
+__device__ __forceinline__ bool split_tile(const SplitGemmParams& p, int& m_tile, int& n_tile) {
+    const int per = (p.tiles + 7) >> 3, id = blockIdx.x;
+    const int tile = (id & 7) * per + (id >> 3);
+    if ((id >> 3) >= per || tile >= p.tiles) return false;
+    split_place(p, tile, m_tile, n_tile);
     return true;
 }
 

@@ -34,17 +34,25 @@ CASES = {
     # rows reach: name: (width, vocab, sequences, tokens)
     "32 x 32 tiles, one row past a tile": (512, 130, 1, 161),
     "64 x 64 of two sets of K": (512, 1001, 3, 171),
-    "64 x 96 of two sets, q, k, v; keys and values from the middle of the matrix": (512, 130, 3, 449),
+    "64 x 64 of one set, q, k, v; 64 x 96 of four, keys and values from the middle of the matrix": (512, 130, 3, 449),
     "128 x 64, both FFN1; a nearly empty tile": (512, 130, 3, 667),
     "128 x 128 at 512 columns": (512, 515, 11, 487),
-    "64 x 96 of four sets, q, k, v and SwiGLU": (768, 130, 2, 150),
+    "64 x 96 of four sets, SwiGLU": (768, 130, 2, 150),
     "64 x 64 of one set, FFN1; four sets of 64 x 96, q, k, v": (768, 515, 1, 449),
     "64 x 64 of two sets, W_o": (768, 1001, 3, 334),
     "64 x 96 of four sets, W_o, FFN2 and logits": (768, 515, 4, 501),
-    "64 x 96 of two sets, W_o and FFN2": (768, 515, 6, 500),
+    "64 x 96 of two sets, FFN2; 128 x 128 and quarters, GELU, keys and values": (768, 515, 6, 500),
     "128 x 128, all": (768, 515, 19, 474),
     "nine parts of K: one set": (576, 130, 1, 161),
     "nine parts of K: one set, FFN2 in four": (576, 301, 3, 667),
+    "64 x 96 of two sets, q, k, v and GELU": (640, 130, 2, 260),
+    "64 x 96 of two sets, SwiGLU": (768, 130, 2, 260),
+    "128 x 64, q, k, v": (512, 130, 9, 377),
+    "128 x 64, W_o": (576, 130, 17, 390),
+    "128 x 128 and quarters, q, k, v": (768, 130, 5, 400),
+    "128 x 128 and quarters, SwiGLU": (768, 130, 2, 520),
+    "128 x 128 and quarters, W_o; a nearly empty row of tiles": (512, 130, 20, 410),
+    "128 x 128 and quarters, q, k, v; quarters past the last row and the last output": (576, 130, 6, 405),
 }
 
 
