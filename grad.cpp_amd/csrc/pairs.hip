@@ -61,10 +61,10 @@ constexpr Tiling kTilings[TILINGS] = {
 // TILE_MIXED: 128 x 128 tiles in whole rounds of 256 and the rest, at most 64 of them, as 64 x 64 quarters in the same
 // launch, at most one for each compute unit, beside its last whole tile (both fit it).  2000 x 2304 outputs are 288
 // tiles: 32 compute units had two and the others waited.  Of 230 launches (160 to 16384 rows) the rule gives it 18, all
-// of them faster than what they took before, by 7 to 22 % (1999 x 2304 x 768 33.0 -> 28.6 us, in a prompt 37.5 -> 32.4, 6000 x 768 x 2048 67.8 ->
-// 61.3, 1280 x 4096 x 768 32.2 -> 27.1, 7000 x 3072 x 768 111.0 -> 101.3); with more than one quarter for a compute
-// unit it is as often the slower one (2600 x 3072 x 768 42.4 -> 48.6, 1800 x 4096 x 768 38.2 -> 44.0).  Not for scored
-// logits, whose sums of exponentials are kept for 64 columns at a time.
+// of them faster than what they took before, by 7 to 22 % (1999 x 2304 x 768 33.0 -> 28.6 us, in a prompt 37.5 -> 32.4,
+// 6000 x 768 x 2048 67.8 -> 61.3, 1280 x 4096 x 768 32.2 -> 27.1, 7000 x 3072 x 768 111.0 -> 101.3); with more than one
+// quarter for a compute unit it is the slower one in 32 of 45 (2600 x 3072 x 768 42.4 -> 48.6, 1800 x 4096 x 768 38.2
+// -> 44.0).  Not for scored logits, whose sums of exponentials are kept for 64 columns at a time.
 constexpr int kMixedRest = 64;
 
 static int pick_tiling(int M, int N, int K, int epilogue) {
