@@ -80,7 +80,9 @@ static __global__ __launch_bounds__(256, 2) void attn_pair_kernel(const SplitAtt
             for (int i = 0; i < 8; i++) top = fmaxf(top, fabsf(v[c][i]));
         }
         top = fmaxf(top, __shfl_xor(top, 32, kWave));
-        const int s = top > 0.0f && top < INFINITY ? min(14 - ilogbf(top), 126) : 0;  // the largest goes to [2^14, 2^15)
+        // the largest goes to [2^14, 2^15), a query below 2^-112, or one near that against small keys, stays lower: its unit has to
+        // be a number other than zero, or a masked score were none (and its scores differ by less than 2^-60)
+        const int s = top > 0.0f && top < INFINITY ? min(14 - ilogbf(top), 126 + min(ilogbf(p.key_unit), 0)) : 0;
         const float up = ldexpf(1.0f, s);
         unit = ldexpf(p.key_unit, -s);
 #pragma unroll

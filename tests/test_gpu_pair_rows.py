@@ -137,3 +137,21 @@ def test_a_prompt_in_front_of_draws_from_the_whole_row():
         s.decode_stream(12, opt, lambda ids, index: picks.append(ids[0]), seed=5)
         tokens = G.Session(gm).generate(prompt, 12, opt, seed=5)
         assert np.array_equal(np.asarray(tokens)[0, 600:], picks)
+
+
+@pytest.mark.parametrize("arch", [synth.ARCH_GPT2, synth.ARCH_MODERN])
+def test_queries_so_small_that_their_unit_leaves_fp32(arch):
+    """A token whose norm(x) is zero leaves a query of the bias alone, 1e-35; behind keys of 1e-4 the unit of its scores was
+    2^-150 and its masked scores not numbers.  (GPT-2: position and token cancel.)"""
+    cfg = synth.Config(arch, 67, 512, 2, 8, 600)
+    W = synth.make_weights(cfg, 115, std=lively_std(cfg), norm_noise=0.1)
+    names = [what[0] for what in synth.tensor_specs(cfg)]
+    W[0][:4] = 0.0
+    if arch == synth.ARCH_GPT2:
+        W[1][:] = 0.0
+        W[names.index("layer 0 norm1 beta")][:] = 0.0
+    for layer in range(2):
+        W[names.index(f"layer {layer} b_q")][:] = 1e-35
+        W[names.index(f"layer {layer} W_k")] *= np.float32(1e-6)
+        W[names.index(f"layer {layer} b_k")] *= np.float32(1e-6)
+    _check(cfg, W, 1, 530, 116)
