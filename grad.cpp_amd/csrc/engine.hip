@@ -374,9 +374,9 @@ static Size size_of(const float* device, size_t n) {
 
 // The power of two that takes values of at most `bound` below 2^15, if what most of them reach, `low`, lies within 2^24 of
 // it (a pair is off by 2^-51 of the bound at most); none for a bound that is no number or far from fp32's middle.
-static std::optional<int> pair_exponent(double bound, double low) {
+static std::optional<int> pair_exponent(double bound, double low, double room = 0x1p-24) {
     if (bound == 0.0) return 0;
-    if (!(bound > 0x1p-40 && bound < 0x1p40) || !(low >= bound * 0x1p-24)) return std::nullopt;
+    if (!(bound > 0x1p-40 && bound < 0x1p40) || !(low >= bound * room)) return std::nullopt;
     return 14 - std::ilogb(bound);
 }
 
@@ -401,7 +401,8 @@ static bool pair_bounds(const Shape& sh, const LayerWeights& w, const PairPlace&
     const NormSize n1 = norm_size(sh, w.g1, w.be1), n2 = norm_size(sh, w.g2, w.be2);
     const Size wv = size_of(qkv.norm + 2 * d, d), bv = size_of(w.bqkv + 2 * d, d);
     const Size w1 = size_of(ffn1.norm, (sh.modern() ? 2 : 1) * F), b1 = sh.modern() ? Size{} : size_of(w.b1, F);
-    const Size wk = size_of(qkv.norm + d, d), bk = size_of(w.bqkv + d, d);
+    const Size wq = size_of(qkv.norm, d), bq = size_of(w.bqkv, d), wk = size_of(qkv.norm + d, d), bk = size_of(w.bqkv + d, d);
+    const double query = std::sqrt(2.0) * (wq.top * n1.norm + bq.top), low_query = wq.low * n1.low;
     const double key = std::sqrt(2.0) * (wk.top * n1.norm + bk.top);  // (a rotated pair is as long as it was)
     const double value = wv.top * n1.norm + bv.top, unit = w1.top * n2.norm + b1.top;
     const double low_key = wk.low * n1.low, low_value = wv.low * n1.low, low_unit = w1.low * n2.low;
@@ -409,7 +410,10 @@ static bool pair_bounds(const Shape& sh, const LayerWeights& w, const PairPlace&
     const auto keys = pair_exponent(key, low_key);
     const auto attn = pair_exponent(value, low_value / 64);  // (an average of many is smaller than one of them)
     const auto hidden = sh.modern() ? pair_exponent(unit * unit, low_unit * low_unit / 4) : pair_exponent(unit, low_unit / 4);
-    if (!norm1 || !norm2 || !keys || !attn || !hidden) return false;
+    // (A query's power of two is its own, attn_pair_kernel's, and its second part is not lifted: one power serves the whole
+    // row while most of it lies within 2^16 of the largest it can hold, off by 2^-39 of that.)
+    const bool queries = pair_exponent(query, low_query, 0x1p-16).has_value();
+    if (!norm1 || !norm2 || !queries || !keys || !attn || !hidden) return false;
     l.norm1 = *norm1;
     l.keys = *keys;
     l.attn = *attn;
@@ -449,7 +453,7 @@ static bool split_layers(const Model& m) {
         PairLayer l{qkv.w, o.w, ffn1.w, ffn2.w, qkv.unit, o.unit, ffn1.unit, ffn2.unit, 0, 0, 0, 0, 0};
         // (W_o and FFN2 feed no operand, but an infinite weight has no pair either)
         fit = fit && std::isfinite(size_of(o.norm, d).top) && std::isfinite(size_of(ffn2.norm, d).top)
-              && std::isfinite(size_of(qkv.norm, 2 * d).top) && pair_bounds(sh, w, qkv, ffn1, l);
+              && pair_bounds(sh, w, qkv, ffn1, l);
         m.pair_layers.push_back(l);
     }
     f.pairs = fit;

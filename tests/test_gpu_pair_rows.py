@@ -155,3 +155,15 @@ def test_queries_so_small_that_their_unit_leaves_fp32(arch):
         W[names.index(f"layer {layer} W_k")] *= np.float32(1e-6)
         W[names.index(f"layer {layer} b_k")] *= np.float32(1e-6)
     _check(cfg, W, 1, 530, 116)
+
+
+@pytest.mark.parametrize("bias", [1e6, 1e20, 1e30])
+def test_a_query_too_far_above_the_others_for_two_parts(bias):
+    """An element of every query so large that one power of two cannot serve the rest of its row (its keys are zero)."""
+    cfg = synth.Config(synth.ARCH_GPT2, 67, 512, 2, 8, 600)
+    W = synth.make_weights(cfg, 117, std=lively_std(cfg), norm_noise=0.1)
+    names = [what[0] for what in synth.tensor_specs(cfg)]
+    W[names.index("layer 1 b_q")][0, 70] = bias
+    W[names.index("layer 1 W_k")][:, 70] = 0.0
+    W[names.index("layer 1 b_k")][0, 70] = 0.0
+    _check(cfg, W, 1, 530, 118)
