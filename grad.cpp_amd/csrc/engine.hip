@@ -160,16 +160,23 @@ struct PairLayer {
     int norm1, keys, attn, norm2, hidden;
 };
 
-// One allocation of split matrices.
+// Device memory that is given back, also where making what it is for throws.
+struct DeviceBlob {
+    char* at = nullptr;
+    DeviceBlob() = default;
+    DeviceBlob(const DeviceBlob&) = delete;
+    DeviceBlob& operator=(const DeviceBlob&) = delete;
+    ~DeviceBlob() {
+        if (at) (void)hipFree(at);
+    }
+};
+
+// Split matrices in one allocation: there is one once they are ready.
 struct SplitForm {
     std::mutex mutex;
-    char* blob = nullptr;
+    DeviceBlob blob;
     bool ready = false;
-    bool unfit = false;  // a weight is outside the range of the parts (kSplitTop): fp32 products only
-    bool pairs = false;  // there are pairs (of the layers: beside the three parts; of the logits matrix: in their place)
-    ~SplitForm() {
-        if (blob) (void)hipFree(blob);
-    }
+    bool unfit = false;  // the weights have no such form
 };
 
 // Where tensor i of the file lives on the device.
@@ -191,10 +198,10 @@ struct Model {
     float *rope_cos = nullptr, *rope_sin = nullptr;  // (max_len, head_size/2)
     std::vector<Placement> place;                    // file order
 
-    // Split forms of the matrices, each written by the first pass that multiplies by it and kept: the layers'
-    // (split_layers; ten bytes per weight beside the four above, six where there are no pairs), and that of the
-    // logits matrix (split_logits; four bytes, or six), which scoring alone needs and at any length.
-    mutable SplitForm layers_split, logits_split;
+    // Split forms of the matrices, each written by the first pass that multiplies by it and kept: in pairs (four bytes
+    // per weight beside the four above) or in three parts (six); the layers', and that of the logits matrix, which
+    // scoring alone needs and at any length.
+    mutable SplitForm layers_split, layers_pairs, logits_split, logits_pairs;
     mutable std::vector<SplitLayer> split_layers;
     mutable std::vector<PairLayer> pair_layers;
     mutable float* logits_unit = nullptr;  // of the logits matrix in pairs, in its allocation
@@ -297,33 +304,39 @@ static bool rows_shape_ok(const Shape& sh) {
     return sh.head_size() == 64 && sh.d_model % 64 == 0 && sh.d_ff() % 64 == 0;
 }
 
-// Writes a split form in three parts, once per model: fill calls place(src, N, K, gate_up) for every matrix and
-// is given the place of its split form.  `more`: bytes wanted behind it, given up if there is no memory for both.
-// False: the weights have none, or there is no memory for it now (the next pass asks again).
-template <class Fill>
-static bool make_split_form(SplitForm& f, size_t bytes, size_t& more, Fill fill) {
-    if (!f.blob && !(more && try_alloc(f.blob, bytes + more + sizeof(int)))) {
-        more = 0;
-        if (!try_alloc(f.blob, bytes + sizeof(int))) return false;
-    }
-    int* const beyond = reinterpret_cast<int*>(f.blob + bytes + more);  // set if any weight is out of range
-    HIP_CHECK(hipMemset(beyond, 0, sizeof(int)));
-    char* at = f.blob;
-    fill([&](const float* src, int N, int K, bool gate_up) {
-        split_weights(src, N, K, gate_up, at, beyond, nullptr);
-        char* const here = at;
-        at += split_bytes(N, K);
-        return here;
-    });
-    int found = 0;
-    HIP_CHECK(hipMemcpy(&found, beyond, sizeof(int), hipMemcpyDeviceToHost));
-    f.unfit = found != 0;
-    f.ready = !f.unfit;
-    if (f.unfit) {
-        HIP_CHECK(hipFree(f.blob));
-        f.blob = nullptr;
+// Writes a split form once per model: make(blob) fills an allocation of so many bytes and says whether the weights have
+// the form.  False: they have none, or there is no memory for it now (the next pass asks again).
+template <class Make>
+static bool make_form(SplitForm& f, size_t bytes, Make make) {
+    std::lock_guard<std::mutex> lock(f.mutex);
+    if (f.ready || f.unfit) return f.ready;
+    DeviceBlob blob;
+    if (!try_alloc(blob.at, bytes)) return false;
+    if (make(blob.at)) {
+        f.ready = true;
+        std::swap(f.blob.at, blob.at);
+    } else {
+        f.unfit = true;
     }
     return f.ready;
+}
+
+// In three parts: fill calls place(src, N, K, gate_up) for every matrix and is given the place of its split form.
+template <class Fill>
+static bool make_split_form(SplitForm& f, size_t bytes, Fill fill) {
+    return make_form(f, bytes + sizeof(int), [&](char* at) {
+        int* const beyond = reinterpret_cast<int*>(at + bytes);  // set if any weight is out of range
+        HIP_CHECK(hipMemset(beyond, 0, sizeof(int)));
+        fill([&](const float* src, int N, int K, bool gate_up) {
+            split_weights(src, N, K, gate_up, at, beyond, nullptr);
+            char* const here = at;
+            at += split_bytes(N, K);
+            return here;
+        });
+        int found = 0;
+        HIP_CHECK(hipMemcpy(&found, beyond, sizeof(int), hipMemcpyDeviceToHost));
+        return found == 0;
+    });
 }
 
 // Storage of a matrix in pairs: the blocks, its outputs' units, and the 2-norms of its rows.
@@ -423,16 +436,10 @@ static bool pair_bounds(const Shape& sh, const LayerWeights& w, const PairPlace&
 }
 
 static bool split_layers(const Model& m) {
-    std::lock_guard<std::mutex> lock(m.layers_split.mutex);
-    SplitForm& f = m.layers_split;
-    if (f.ready || f.unfit) return f.ready;
     const Shape& sh = m.shape;
     const int d = sh.d_model, F = sh.d_ff(), up = sh.modern() ? 2 : 1;
     const size_t per_layer = split_bytes(3 * d, d) + split_bytes(d, d) + split_bytes(up * F, d) + split_bytes(d, F);
-    const size_t pairs_per_layer =
-        pair_place_bytes(3 * d, d) + pair_place_bytes(d, d) + pair_place_bytes(up * F, d) + pair_place_bytes(d, F);
-    size_t more = d >= kPairMinCols ? sh.layers * pairs_per_layer : 0;
-    const bool made = make_split_form(f, sh.layers * per_layer, more, [&](auto place) {
+    return make_split_form(m.layers_split, sh.layers * per_layer, [&](auto place) {
         m.split_layers.clear();
         for (const LayerWeights& w : m.layers) {
             SplitLayer l;
@@ -443,44 +450,53 @@ static bool split_layers(const Model& m) {
             m.split_layers.push_back(l);
         }
     });
-    if (!made || !more) return made;
-    char* at = f.blob + sh.layers * per_layer;
-    m.pair_layers.clear();
-    bool fit = true;
-    for (const LayerWeights& w : m.layers) {
-        const PairPlace qkv = place_pairs(at, w.wqkv, 3 * d, d, false), o = place_pairs(at, w.wo, d, d, false);
-        const PairPlace ffn1 = place_pairs(at, w.w1, up * F, d, sh.modern()), ffn2 = place_pairs(at, w.w2, d, F, false);
-        PairLayer l{qkv.w, o.w, ffn1.w, ffn2.w, qkv.unit, o.unit, ffn1.unit, ffn2.unit, 0, 0, 0, 0, 0};
-        // (W_o and FFN2 feed no operand, but an infinite weight has no pair either)
-        fit = fit && std::isfinite(size_of(o.norm, d).top) && std::isfinite(size_of(ffn2.norm, d).top)
-              && pair_bounds(sh, w, qkv, ffn1, l);
-        m.pair_layers.push_back(l);
-    }
-    f.pairs = fit;
-    return true;
 }
 
-static bool split_logits(const Model& m) {
-    std::lock_guard<std::mutex> lock(m.logits_split.mutex);
-    SplitForm& f = m.logits_split;
-    if (f.ready || f.unfit) return f.ready;
+static bool layers_in_pairs(const Model& m) {
     const Shape& sh = m.shape;
-    const int d = sh.d_model, V = sh.vocab;
-    const NormSize n = norm_size(sh, m.gf, m.bf);
-    const std::optional<int> norm = pair_exponent(n.top, n.low);
-    if (d >= kPairMinCols && norm) {
-        if (!try_alloc(f.blob, pair_place_bytes(V, d))) return false;
-        char* at = f.blob;
-        const PairPlace e = place_pairs(at, m.E, V, d, false);
-        m.logits_unit = e.unit;
-        m.logits_norm = *norm;
-        f.ready = f.pairs = !std::isinf(size_of(e.norm, V).top);
-        if (f.ready) return true;
-        HIP_CHECK(hipFree(f.blob));
-        f.blob = nullptr;
+    const int d = sh.d_model, F = sh.d_ff(), up = sh.modern() ? 2 : 1;
+    const size_t per_layer =
+        pair_place_bytes(3 * d, d) + pair_place_bytes(d, d) + pair_place_bytes(up * F, d) + pair_place_bytes(d, F);
+    return make_form(m.layers_pairs, sh.layers * per_layer, [&](char* at) {
+        m.pair_layers.clear();
+        for (const LayerWeights& w : m.layers) {
+            const PairPlace qkv = place_pairs(at, w.wqkv, 3 * d, d, false), o = place_pairs(at, w.wo, d, d, false);
+            const PairPlace ffn1 = place_pairs(at, w.w1, up * F, d, sh.modern()), ffn2 = place_pairs(at, w.w2, d, F, false);
+            PairLayer l{qkv.w, o.w, ffn1.w, ffn2.w, qkv.unit, o.unit, ffn1.unit, ffn2.unit, 0, 0, 0, 0, 0};
+            // (W_o and FFN2 feed no operand, but an infinite weight has no pair either)
+            if (!std::isfinite(size_of(o.norm, d).top) || !std::isfinite(size_of(ffn2.norm, d).top)
+                || !pair_bounds(sh, w, qkv, ffn1, l))
+                return false;
+            m.pair_layers.push_back(l);
+        }
+        return true;
+    });
+}
+
+// The form that a pass takes: pairs where the model has them, three parts where it does not.
+enum SplitKind { SPLIT_NONE, SPLIT_PAIRS, SPLIT_PARTS };
+
+static SplitKind layers_kind(const Model& m, bool pairs) {
+    if (pairs && m.shape.d_model >= kPairMinCols && layers_in_pairs(m)) return SPLIT_PAIRS;
+    return split_layers(m) ? SPLIT_PARTS : SPLIT_NONE;
+}
+
+static SplitKind logits_kind(const Model& m) {
+    const int d = m.shape.d_model, V = m.shape.vocab;
+    if (d >= kPairMinCols) {
+        const bool pairs = make_form(m.logits_pairs, pair_place_bytes(V, d), [&](char* at) {
+            const NormSize n = norm_size(m.shape, m.gf, m.bf);
+            const std::optional<int> norm = pair_exponent(n.top, n.low);
+            if (!norm) return false;
+            const PairPlace e = place_pairs(at, m.E, V, d, false);
+            m.logits_unit = e.unit;
+            m.logits_norm = *norm;
+            return !std::isinf(size_of(e.norm, V).top);
+        });
+        if (pairs) return SPLIT_PAIRS;
     }
-    size_t more = 0;
-    return make_split_form(f, split_bytes(V, d), more, [&](auto place) { place(m.E, V, d, false); });
+    const bool parts = make_split_form(m.logits_split, split_bytes(V, d), [&](auto place) { place(m.E, V, d, false); });
+    return parts ? SPLIT_PARTS : SPLIT_NONE;
 }
 
 static std::unique_ptr<Model> upload_model(const Shape& shape, const std::vector<const float*>& t,
@@ -1978,19 +1994,20 @@ static bool draws_from_whole_row(const gh_sampling& o) {
 struct RowsPlan {
     int slice;
     int split_rows;
-    bool pairs;  // ... those in two parts each, not in three
+    SplitKind kind;  // ... of those
 };
 
 // Decided before anything is launched.  Weights without a split form, or no memory for it, leave the small fp32 tiles,
 // in slices below the rows from which the split projections take over (the tiles' buffers hold no
 // more), and for scoring, whose logits come from the split matrix alone, the token-by-token way.
 static RowsPlan plan_rows(const Session& s, int len, bool score, bool whole_row_draws) {
-    if (!prompt_pass_ok(s, len) || (score && !split_logits(*s.m))) return {0, 0, false};
+    if (!prompt_pass_ok(s, len) || (score && logits_kind(*s.m) == SPLIT_NONE)) return {0, 0, SPLIT_NONE};
     const int most = static_cast<int>(std::max<size_t>(1, std::min<size_t>(len, kPromptPassRows / s.B)));
     const int split_rows = score ? kSplitMinScoreRows : kSplitMinRows;
-    if (static_cast<long>(most) * s.B < split_rows) return {most, split_rows, false};
-    if (split_layers(*s.m)) return {most, split_rows, s.m->layers_split.pairs && !whole_row_draws};
-    return {std::min(len, (kSplitMinRows - 1) / s.B), kSplitMinRows, false};
+    if (static_cast<long>(most) * s.B < split_rows) return {most, split_rows, SPLIT_NONE};
+    const SplitKind kind = layers_kind(*s.m, !whole_row_draws);
+    if (kind != SPLIT_NONE) return {most, split_rows, kind};
+    return {std::min(len, (kSplitMinRows - 1) / s.B), kSplitMinRows, SPLIT_NONE};
 }
 
 // One projection over M rows (norm folded in for RMSNorm, a norm kernel for LayerNorm).
@@ -2054,9 +2071,9 @@ static void split_norm(Session& s, bool pairs, const float* gamma, const float* 
 static void score_rows(Session& s, const ScoreSink& sink, int M, int n, int t0, int len) {
     const Model& m = *s.m;
     const Shape& sh = m.shape;
-    const bool pairs = m.logits_split.pairs;
+    const bool pairs = m.logits_pairs.ready;  // (as the pass's plan found or made it)
     split_norm(s, pairs, m.gf, m.bf, m.logits_norm, M);
-    SplitGemmParams g = split_params(s.pp_split, m.logits_split.blob, M, sh.vocab, sh.d_model);
+    SplitGemmParams g = split_params(s.pp_split, (pairs ? m.logits_pairs : m.logits_split).blob.at, M, sh.vocab, sh.d_model);
     if (pairs) pair_params(g, m.logits_unit, m.logits_norm);
     g.rows_per_seq = n;
     g.targets = sink.targets;
@@ -2117,7 +2134,7 @@ static void prompt_layer_split(Session& s, int layer, int n, int pos_base, bool 
     const Model& m = *s.m;
     const Shape& sh = m.shape;
     const LayerWeights& w = m.layers[layer];
-    const SplitLayer& sw = m.split_layers[layer];
+    const SplitLayer sw = pairs ? SplitLayer{} : m.split_layers[layer];
     const PairLayer pw = pairs ? m.pair_layers[layer] : PairLayer{};
     const int d = sh.d_model, F = sh.d_ff(), M = n * s.B;
     hipStream_t st = s.stream;
@@ -2328,7 +2345,8 @@ static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSi
         const int M = n * B;
         const int pos_base = s.pos + t0;
         const bool split = M >= plan.split_rows;
-        const bool split_attn = split && reserve_split_attention(s, n, pos_base, plan.pairs);
+        const bool pairs = plan.kind == SPLIT_PAIRS;
+        const bool split_attn = split && reserve_split_attention(s, n, pos_base, pairs);
         hipLaunchKernelGGL(embed_rows_kernel, dim3((d + 255) / 256, M), dim3(256), 0, st, m.E, m.P, s.hist,
                            s.hist_stride, s.n_hist + t0, n, pos_base, s.pp_x, d);
         HIP_CHECK(hipGetLastError());
@@ -2336,7 +2354,7 @@ static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSi
         // else at the last position alone, where the decode step's launches are as good.
         const bool trim = split && !sink;
         for (int l = 0; l < sh.layers; l++) {
-            if (split) prompt_layer_split(s, l, n, pos_base, plan.pairs, split_attn, trim && l == sh.layers - 1);
+            if (split) prompt_layer_split(s, l, n, pos_base, pairs, split_attn, trim && l == sh.layers - 1);
             else prompt_layer_small(s, l, n, pos_base);
         }
         if (sink) score_rows(s, *sink, M, n, t0, len);
@@ -2363,7 +2381,7 @@ static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSi
 // prompt loop of text_gen.cpp:44-46).  log: per-step logits destination or null.
 static void run_prompt(Session& s, int len, float* log, size_t* steps_logged, bool whole_row_draws = false) {
     const size_t BV = static_cast<size_t>(s.B) * s.m->shape.vocab;
-    const RowsPlan plan = log ? RowsPlan{0, 0, false} : plan_rows(s, len, /*score=*/false, whole_row_draws);
+    const RowsPlan plan = log ? RowsPlan{0, 0, SPLIT_NONE} : plan_rows(s, len, /*score=*/false, whole_row_draws);
     if (plan.slice > 0) {
         prompt_pass(s, len, plan);
         if (steps_logged) *steps_logged += len;
