@@ -329,8 +329,8 @@ static __global__ __launch_bounds__(256, 2) void attn_split_kernel(const SplitAt
     for (int db = 0; db < 2; db++)
 #pragma unroll
         for (int q4 = 0; q4 < 4; q4++)
-            store_operand4(p.out, b * p.len + t, h * 64 + db * 32 + q4 * 8 + h32 * 4, p.d_model / kSplitCols, o[db][4 * q4] * inv,
-                           o[db][4 * q4 + 1] * inv, o[db][4 * q4 + 2] * inv, o[db][4 * q4 + 3] * inv, p.pair_scale);
+            store_split4(p.out, b * p.len + t, h * 64 + db * 32 + q4 * 8 + h32 * 4, p.d_model / kSplitCols, o[db][4 * q4] * inv,
+                         o[db][4 * q4 + 1] * inv, o[db][4 * q4 + 2] * inv, o[db][4 * q4 + 3] * inv);
 }
 
 // Folds the partial results of a query block, in the order of the keys.  A chain of trips to memory, one per
