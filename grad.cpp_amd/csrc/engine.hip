@@ -473,11 +473,12 @@ static bool layers_in_pairs(const Model& m) {
     });
 }
 
-// The form that a pass takes: pairs where the model has them, three parts where it does not.
+// The form that a pass takes: pairs (kernels_pair.h) where the model has them, three parts where it does not.  Nothing
+// else decides: what a prompt leaves must not depend on the call it came by, nor on what is drawn behind it.
 enum SplitKind { SPLIT_NONE, SPLIT_PAIRS, SPLIT_PARTS };
 
-static SplitKind layers_kind(const Model& m, bool pairs) {
-    if (pairs && m.shape.d_model >= kPairMinCols && layers_in_pairs(m)) return SPLIT_PAIRS;
+static SplitKind layers_kind(const Model& m) {
+    if (m.shape.d_model >= kPairMinCols && layers_in_pairs(m)) return SPLIT_PAIRS;
     return split_layers(m) ? SPLIT_PARTS : SPLIT_NONE;
 }
 
@@ -1980,15 +1981,6 @@ static bool prompt_pass_ok(const Session& s, int len) {
 // What that keeps is the replies, not precision: the split sums are the closer ones to float64.
 constexpr int kSplitMinRows = 512, kSplitMinScoreRows = 160;
 
-// Operands of a split pass go in pairs (kernels_pair.h) wherever the model has them, except in front of draws from
-// the whole row, for the reason above: those replies stay what three parts made of their prompts.  (With a
-// cut at k of a flat distribution a draw has k boundaries to fall beside, not 16000.)
-constexpr int kWholeRowTopK = 1024;
-
-static bool draws_from_whole_row(const gh_sampling& o) {
-    return !o.greedy && (o.top_k <= 0 || o.top_k > kWholeRowTopK);
-}
-
 // How a pass over len tokens of every sequence runs: in slices of `slice` tokens (0: token by
 // token), those of split_rows rows and more on the split weights.
 struct RowsPlan {
@@ -2000,12 +1992,12 @@ struct RowsPlan {
 // Decided before anything is launched.  Weights without a split form, or no memory for it, leave the small fp32 tiles,
 // in slices below the rows from which the split projections take over (the tiles' buffers hold no
 // more), and for scoring, whose logits come from the split matrix alone, the token-by-token way.
-static RowsPlan plan_rows(const Session& s, int len, bool score, bool whole_row_draws) {
+static RowsPlan plan_rows(const Session& s, int len, bool score) {
     if (!prompt_pass_ok(s, len) || (score && logits_kind(*s.m) == SPLIT_NONE)) return {0, 0, SPLIT_NONE};
     const int most = static_cast<int>(std::max<size_t>(1, std::min<size_t>(len, kPromptPassRows / s.B)));
     const int split_rows = score ? kSplitMinScoreRows : kSplitMinRows;
     if (static_cast<long>(most) * s.B < split_rows) return {most, split_rows, SPLIT_NONE};
-    const SplitKind kind = layers_kind(*s.m, !whole_row_draws);
+    const SplitKind kind = layers_kind(*s.m);
     if (kind != SPLIT_NONE) return {most, split_rows, kind};
     return {std::min(len, (kSplitMinRows - 1) / s.B), kSplitMinRows, SPLIT_NONE};
 }
@@ -2379,9 +2371,9 @@ static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSi
 
 // Steps through `len` tokens already staged in the history at n_hist.. (the
 // prompt loop of text_gen.cpp:44-46).  log: per-step logits destination or null.
-static void run_prompt(Session& s, int len, float* log, size_t* steps_logged, bool whole_row_draws = false) {
+static void run_prompt(Session& s, int len, float* log, size_t* steps_logged) {
     const size_t BV = static_cast<size_t>(s.B) * s.m->shape.vocab;
-    const RowsPlan plan = log ? RowsPlan{0, 0, SPLIT_NONE} : plan_rows(s, len, /*score=*/false, whole_row_draws);
+    const RowsPlan plan = log ? RowsPlan{0, 0, SPLIT_NONE} : plan_rows(s, len, /*score=*/false);
     if (plan.slice > 0) {
         prompt_pass(s, len, plan);
         if (steps_logged) *steps_logged += len;
@@ -3035,7 +3027,7 @@ gh_status gh_session_score(gh_session* sess, const int32_t* ids, const int32_t* 
         }
         stage_ids(s, host_targets, len, s.score_targets, len, 0);
         const ScoreSink sink{s.score_targets, s.score_nll};
-        const RowsPlan plan = plan_rows(s, len, /*score=*/true, /*whole_row_draws=*/false);
+        const RowsPlan plan = plan_rows(s, len, /*score=*/true);
         run_resident(s, [&] {
             if (plan.slice > 0) {
                 prompt_pass(s, len, plan, &sink);
@@ -3348,7 +3340,7 @@ gh_status gh_session_generate(gh_session* sess, const int32_t* prompts, int32_t 
         run_resident(s, [&] {
             steps = 0;
             HIP_CHECK(hipEventRecord(s.ev[0], s.stream));
-            run_prompt(s, prompt_len, log, &steps, draws_from_whole_row(*opt));
+            run_prompt(s, prompt_len, log, &steps);
             HIP_CHECK(hipEventRecord(s.ev[1], s.stream));
             s.ahead = Session::AHEAD_PROMPT;
             std::tie(made, stepped) = run_decode(s, max_tokens, *opt, du, max_tokens, seed, log, &steps);

@@ -126,8 +126,7 @@ def test_infinite_and_nan_weights_keep_their_meaning():
 
 
 def test_a_prompt_in_front_of_draws_from_the_whole_row():
-    """Its operands stay in three parts; prefill's are two.  Both are within fp32 sums of one another: greedy picks,
-    with margins far above that, are the same behind either."""
+    """Greedy picks, and draws that come to the same, are the same behind generate's prompt and behind prefill's."""
     cfg = synth.Config(synth.ARCH_MODERN, 130, 512, 2, 8, 640)
     gm = G.Model.from_tensors(cfg, synth.make_weights(cfg, 113, std=lively_std(cfg), norm_noise=0.1))
     prompt = synth.uniform_tokens(600, cfg.vocab, 114)
@@ -167,3 +166,29 @@ def test_a_query_too_far_above_the_others_for_two_parts(bias):
     W[names.index("layer 1 W_k")][:, 70] = 0.0
     W[names.index("layer 1 b_k")][0, 70] = 0.0
     _check(cfg, W, 1, 530, 118)
+
+
+@pytest.mark.parametrize("opt", [(0.8, 0, 1.0, 1.2), (1.0, 0, 0.95, 1.1), (0.8, 40, 0.9, 1.1), (0.9, 2000, 1.0, 1.0), (1.0, 0, 1.0, 1.0, True)])
+@pytest.mark.parametrize("batch, n", [(1, 600), (5, 130)])
+def test_a_prompt_leaves_the_same_bits_whatever_the_call_and_the_sampler(opt, batch, n):
+    """generate, and prefill with the same reply streamed or decoded behind it: the same cache and tokens."""
+    cfg = synth.Config(synth.ARCH_MODERN, 5000, 512, 2, 8, 640)
+    gm = G.Model.from_tensors(cfg, synth.make_weights(cfg, 119, std=lively_std(cfg), norm_noise=0.1))
+    prompt = synth.uniform_tokens(batch * n, cfg.vocab, 120).reshape(batch, n)
+
+    def cache(s):
+        return [s.read_kv(b, layer, kv, pos).tobytes() for b in (0, batch - 1) for layer in (0, 1) for kv in (0, 1)
+                for pos in (0, 77, n - 1)]
+
+    s = G.Session(gm, batch=batch)
+    s.prefill(prompt)
+    kept = cache(s)
+    picks = np.asarray(s.decode(16, G.sampling(*opt), seed=9))
+    streamed, s = [], G.Session(gm, batch=batch)
+    s.prefill(prompt)
+    s.decode_stream(16, G.sampling(*opt), lambda ids, index: streamed.append(np.array(ids)), seed=9)
+    assert np.array_equal(np.stack(streamed, axis=1), picks)
+    s = G.Session(gm, batch=batch)
+    tokens = np.asarray(s.generate(prompt, 16, G.sampling(*opt), seed=9))
+    assert cache(s) == kept
+    assert np.array_equal(tokens[:, n:], picks)
