@@ -31,6 +31,7 @@
 // 1999 x 768 x 2048 136 -> 198 (best tile of either).
 #pragma once
 
+#include "epilogue_math.h"
 #include "kernels_split.h"
 
 namespace gh {
@@ -115,19 +116,14 @@ static __global__ __launch_bounds__(1024) void norm_pair_long_kernel(const float
                        [&](int k, const float(&o)[8]) { store_pair8(out, m, k, d / kSplitCols, o, pair_scale); });
 }
 
-// The epilogues' functions by the hardware's 2^x and reciprocal: five vector instructions beside the two, where tanhf
-// makes 66 of the GELU (two thirds of what a 768-column FFN1 tile issued).  As x over 1 + exp(-2 u) the GELU of a negative
-// argument loses nothing to 1 + tanh(u).  Infinities and NaN come out as of the functions themselves.
-struct PairRowsOut {
-    static __device__ __forceinline__ float gelu(float x) {
-        // 0.5 x (1 + tanh(u)) = x / (1 + exp(-2 u)), u = sqrt(2 / pi) (x + 0.044715 x^3)
-        constexpr float k = -2.0f * 0.79788456f * 1.44269504f;
-        return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * __builtin_fmaf(x * x, 0.044715f * k, k)));
-    }
-    static __device__ __forceinline__ float silu(float x) {
-        return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.44269504f));
-    }
-    static __device__ __forceinline__ float exp_of(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504f); }
+// The epilogues' functions: figures in epilogue_math.h.
+struct DeviceUnit {
+    static __device__ __forceinline__ float exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+    static __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
+    static __device__ __forceinline__ float med3(float x, float lo, float hi) { return __builtin_amdgcn_fmed3f(x, lo, hi); }
+};
+
+struct PairRowsOut : EpilogueMath<DeviceUnit> {
     static __device__ __forceinline__ void store8(const SplitGemmParams& p, int m, int k, const float (&v)[8]) {
         store_pair8(p.out_split, m, k, p.out_kblocks, v, p.pair_scale);
     }
