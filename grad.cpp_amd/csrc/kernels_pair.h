@@ -3,19 +3,22 @@
 //
 //   a 2^s = a1 + a2,  a1 = fp16(a 2^s), a2 = fp16(a 2^s - a1)
 //
+// (Two half-precision parts, the second lifted by 2^11 and the sums taken out of the matrix core against its truncation: as
+// published by Ootomo and Yokota, 2022.)
+//
 // What that costs and what pays for it.  a1 + a2 holds 22 bits and a sign, so a value is at most one unit
 // of its 24th bit away (a quarter of all values are; half a unit rms, where rounding to fp32 leaves 0.29),
 // and a2 b2 (2^-22 of the product at most) is left out: 7.5e-8 of a dot product's size, whatever its length.
 // The six products of the exact three-part form (kernels_split.h) lose nothing there, but their sums are K / 16 terms
 // added one after the other, and those roundings grow with K.  Here every 64 columns are summed from zero and
-// then added to the running sum: 12 and K / 64 roundings.  The matrix cores cut the low bits of what they
+// then added to the running sum: 4 (or 12, see pair_tile) and K / 64 roundings.  The matrix cores cut the low bits of what they
 // align, downwards: a bias of 2e-8 (K = 768) to 4e-8 (2048) of the result, the same in every row, which an attention over
 // many positions would not average out; so the weights of every other 64 columns are stored negated and their
-// sums subtracted (what is left is below 1e-9).  Error over the size of the result against float64, 512 x 512
-// outputs, normal operands / gated hidden units times normal weights, three parts -> two: K = 512 1.27e-7 -> 1.26e-7
-// / 1.44e-7 -> 1.28e-7, 768 1.59e-7 -> 1.32e-7 / 1.76e-7 -> 1.33e-7, 2048 2.71e-7 -> 1.55e-7 / 2.90e-7 -> 1.57e-7,
-// 3072 3.39e-7 -> 1.71e-7 / 3.55e-7 -> 1.72e-7 (an fp32 sum of one product after the other: 4.0e-7 to 9.9e-7).  Below K = 512
-// the three parts are the closer ones (256: 0.89e-7 against 1.20e-7), so narrower models keep them (kPairMinCols).
+// sums subtracted (what is left is below 1e-9).  Error over the size of the result against float64, normal operands, three
+// parts with K in one set / in four -> two: K = 512 1.28 / 0.77e-7 -> 1.09 to 1.26, 768 1.59 / 0.88 -> 1.12 to 1.32, 1024
+// 1.86 / 0.98 -> 1.14 to 1.37, 2048 2.72 / 1.34 -> 1.19 to 1.27, 3072 3.40 / 1.63 -> 1.25 to 1.38 (the upper end 128 x 128 tiles; an
+// fp32 sum of one product after the other: 4.0 to 9.9).  Below K = 512 the three parts are the closer ones, so narrower
+// models keep them (kPairMinCols).
 //
 // The range.  fp16 has exponents -14 to 15 and, below, numbers of fewer bits (the matrix cores take them as
 // they are).  Weights are scaled row by row so that a row's largest lies in [2^14, 2^15).  Activations have one power of two
@@ -209,7 +212,10 @@ __device__ __forceinline__ void strip_qkv(const SplitGemmParams& p, int m, int n
 // step before into registers of their own (a 64 x 64 wavefront has 128 of its 256 for sums).  Four steps make a
 // 64-column part that starts from zero and is then added to the running sums (or taken from them, the weights of every
 // other part being negative).  (Added in front of the next part's products instead, accumulator by accumulator, the
-// compiler copies every part first.)  K / KG is a multiple of 64.
+// compiler copies every part first.)  The small products of a part (those with a second part) have a sum of their own,
+// except in wavefronts of 64 x 64: a full-sized sum is then cut four times a part instead of twelve (error of K = 512
+// 1.26 -> 1.09e-7, 768 1.32 -> 1.12, 2048 1.55 -> 1.20 or, in one set, 1.27, 3072 1.71 -> 1.25, 1.37; prompts of 2000 rows of a
+// Llama of 768 columns 0.5 % slower by its 16 additions per block and part).  K / KG is a multiple of 64.
 template <int EPI, int MB, int NB, int WM, int WN, int KG>
 __device__ __forceinline__ void pair_tile(const SplitGemmParams& p, int m_tile, int n_tile) {
     extern __shared__ __attribute__((aligned(1024))) char lds_pair[];
@@ -253,18 +259,19 @@ __device__ __forceinline__ void pair_tile(const SplitGemmParams& p, int m_tile, 
             f[x] = *reinterpret_cast<const v8h*>(frag + stage * kStage + part * kPairPartBytes
                                                  + (kUnitsA + (wn * NB + x) * 2) * kPairBlockBytes);
     };
-    v16f sum[NB][MB], part[NB][MB], zero;
+    constexpr bool kApart = MB * NB < 4;  // small products in sums of their own: 2 x 2 blocks have no registers for them
+    v16f sum[NB][MB], part[NB][MB], small[kApart ? NB : 1][kApart ? MB : 1], zero;
 #pragma unroll
     for (int r = 0; r < 16; r++) zero[r] = 0.0f;
 #pragma unroll
     for (int a = 0; a < NB; a++)
 #pragma unroll
         for (int b = 0; b < MB; b++) sum[a][b] = zero;
-    const auto multiply = [&](const v8h (&w)[NB], const v8h (&x)[MB]) {
+    const auto multiply = [&](const v8h (&w)[NB], const v8h (&x)[MB], auto& to, bool first) {
 #pragma unroll
         for (int a = 0; a < NB; a++)
 #pragma unroll
-            for (int b = 0; b < MB; b++) part[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[a], x[b], part[a][b], 0, 0, 0);
+            for (int b = 0; b < MB; b++) to[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[a], x[b], first ? zero : to[a][b], 0, 0, 0);
     };
     // Strips: of the wavefront's own blocks, or, where sets share K, every kAll-th of the tile's.
     // (QKV's 64 x 96 tiles with K shared by two sets are as fast without, 37.9 us against 38.9 for 2048 x 2304 x 768.)
@@ -328,18 +335,16 @@ __device__ __forceinline__ void pair_tile(const SplitGemmParams& p, int m_tile, 
             v8h low[NB];
 #pragma unroll
             for (int a = 0; a < NB; a++) low[a] = w1[c][a] * static_cast<_Float16>(1.0f / kPairLift);
-#pragma unroll
-            for (int a = 0; a < NB; a++)
-#pragma unroll
-                for (int b = 0; b < MB; b++)
-                    part[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(low[a], a2[c][b], t == 0 ? zero : part[a][b], 0, 0, 0);
+            if constexpr (kApart) multiply(low, a2[c], small, t == 0);
+            else multiply(low, a2[c], part, t == 0);
             read_w(next, 0, w1[n]);
             read_a(next, 1, a2[n]);
             send(0);
-            multiply(w2[c], a1[c]);
+            if constexpr (kApart) multiply(w2[c], a1[c], small, false);
+            else multiply(w2[c], a1[c], part, false);
             read_w(next, 1, w2[n]);
             send(1);
-            multiply(w1[c], a1[c]);
+            multiply(w1[c], a1[c], part, kApart && t == 0);
             read_a(next, 0, a1[n]);
             send(2);
         }
@@ -349,7 +354,11 @@ __device__ __forceinline__ void pair_tile(const SplitGemmParams& p, int m_tile, 
 #pragma unroll
             for (int b = 0; b < MB; b++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) sum[a][b][r] = __builtin_fmaf(part[a][b][r], sign, sum[a][b][r]);
+                for (int r = 0; r < 16; r++) {
+                    float v = part[a][b][r];
+                    if constexpr (kApart) v += small[a][b][r];
+                    sum[a][b][r] = __builtin_fmaf(v, sign, sum[a][b][r]);
+                }
     }
     const auto scaled = [&](const float4& v, const float4& unit) {
         const float f = p.operand_unit;

@@ -192,3 +192,32 @@ def test_a_prompt_leaves_the_same_bits_whatever_the_call_and_the_sampler(opt, ba
     tokens = np.asarray(s.generate(prompt, 16, G.sampling(*opt), seed=9))
     assert cache(s) == kept
     assert np.array_equal(tokens[:, n:], picks)
+
+
+#: (arch, width, tokens): what a pass leaves of the second layer's values is no further from float64 than with three parts
+CLOSENESS = [(synth.ARCH_GPT2, 512, 513), (synth.ARCH_GPT2, 512, 1000), (synth.ARCH_MODERN, 512, 641), (synth.ARCH_GPT2, 640, 385),
+             (synth.ARCH_GPT2, 768, 321), (synth.ARCH_GPT2, 768, 1000), (synth.ARCH_MODERN, 768, 300), (synth.ARCH_GPT2, 1024, 160)]
+
+
+@pytest.mark.parametrize("arch, d, n", CLOSENESS)
+def test_errors_are_no_larger_than_those_of_three_parts(arch, d, n):
+    """The same layers with one gain, in front of weights of zero, that leaves them no pairs."""
+    cfg = synth.Config(arch, 1009, d, 2, d // 64, 1001)
+    names = [what[0] for what in synth.tensor_specs(cfg)]
+    errors = [[], []]
+    for seed in (121, 123):
+        W = synth.make_weights(cfg, seed, std=0.02, norm_noise=0.1)
+        for name in ("FFN W1",) if arch == synth.ARCH_GPT2 else ("FFN gate", "FFN up"):
+            W[names.index(f"layer 0 {name}")][5, :] = 0.0
+        tokens = synth.uniform_tokens(n + 1, cfg.vocab, seed + 1)
+        _, kv = ref_forward.forward(cfg, W, tokens[:-1], return_kv=True)
+        at = range(0, n, 8)  # (values: keys carry the rounding of their angles too)
+        want = np.stack([kv[1][1][pos] for pos in at])
+        for form, gain in enumerate((1.0, 1e9)):
+            W[names.index("layer 0 norm2 gamma")][0, 5] = gain
+            s = G.Session(G.Model.from_tensors(cfg, W))
+            s.score(tokens[:-1], tokens[1:])
+            got = np.stack([s.read_kv(0, 1, 1, pos) for pos in at])
+            errors[form].append(np.linalg.norm(got - want) / np.linalg.norm(want))
+    pairs, parts = np.mean(errors, axis=1)
+    assert pairs <= 1.01 * parts, (pairs, parts)  # (40000 values and more: the figures' own spread is 0.5 %)
