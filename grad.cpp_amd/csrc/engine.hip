@@ -473,18 +473,30 @@ static bool layers_in_pairs(const Model& m) {
     });
 }
 
-// The form that a pass takes: pairs (kernels_pair.h) where the model has them, three parts where it does not.  Nothing
-// else decides: what a prompt leaves must not depend on the call it came by, nor on what is drawn behind it.
+// The form that a pass takes: pairs (kernels_pair.h) where the model has them and they are no further from float64 than
+// three parts, which a pass of the other rows takes.  Nothing else decides: what a prompt leaves must not depend on the call
+// it came by, nor on what is drawn behind it.
 enum SplitKind { SPLIT_NONE, SPLIT_PAIRS, SPLIT_PARTS };
 
-static SplitKind layers_kind(const Model& m) {
-    if (m.shape.d_model >= kPairMinCols && layers_in_pairs(m)) return SPLIT_PAIRS;
+// Three parts whose products of few rows are shared among four sets have the smaller errors up to 1024 columns (K = 512
+// 0.77e-7 against 1.09, 768 0.88 / 1.12, 1024 0.98 / 1.14; in one set 1.28, 1.59, 1.86), those of longer K never (2048 1.34 /
+// 1.20).  Over a layer the wider of its products decide: error of the second layer's values, pairs over three parts, below
+// the line and above: GPT-2 512 wide 1.10 (512 rows), 0.98 (513), 768 1.03 (320), 0.88 (321), Llama 768 1.05 (256), 0.98 (300);
+// from 1024 on pairs are closer with any rows (160: 0.95).  Below 640 columns q, k, v count too (Llama 512 wide: 1.03 at 640
+// rows, 0.97 at 641).
+static bool parts_are_closer(const Shape& sh, long rows) {
+    const int d = sh.d_model, up = sh.modern() ? 2 : 1;
+    return d < 1024 && (split_in_four_sets(rows, up * sh.d_ff()) || (d < 640 && split_in_four_sets(rows, 3 * d)));
+}
+
+static SplitKind layers_kind(const Model& m, long rows) {
+    if (m.shape.d_model >= kPairMinCols && !parts_are_closer(m.shape, rows) && layers_in_pairs(m)) return SPLIT_PAIRS;
     return split_layers(m) ? SPLIT_PARTS : SPLIT_NONE;
 }
 
-static SplitKind logits_kind(const Model& m) {
+static SplitKind logits_kind(const Model& m, long rows) {
     const int d = m.shape.d_model, V = m.shape.vocab;
-    if (d >= kPairMinCols) {
+    if (d >= kPairMinCols && !(d <= 1024 && split_in_four_sets(rows, V))) {
         const bool pairs = make_form(m.logits_pairs, pair_place_bytes(V, d), [&](char* at) {
             const NormSize n = norm_size(m.shape, m.gf, m.bf);
             const std::optional<int> norm = pair_exponent(n.top, n.low);
@@ -1984,22 +1996,26 @@ constexpr int kSplitMinRows = 512, kSplitMinScoreRows = 160;
 // How a pass over len tokens of every sequence runs: in slices of `slice` tokens (0: token by
 // token), those of split_rows rows and more on the split weights.
 struct RowsPlan {
-    int slice;
-    int split_rows;
-    SplitKind kind;  // ... of those
+    int slice = 0;
+    int split_rows = 0;
+    SplitKind kind = SPLIT_NONE;    // ... of those
+    SplitKind logits = SPLIT_NONE;  // scored
 };
 
 // Decided before anything is launched.  Weights without a split form, or no memory for it, leave the small fp32 tiles,
 // in slices below the rows from which the split projections take over (the tiles' buffers hold no
 // more), and for scoring, whose logits come from the split matrix alone, the token-by-token way.
 static RowsPlan plan_rows(const Session& s, int len, bool score) {
-    if (!prompt_pass_ok(s, len) || (score && logits_kind(*s.m) == SPLIT_NONE)) return {0, 0, SPLIT_NONE};
+    if (!prompt_pass_ok(s, len)) return {};
     const int most = static_cast<int>(std::max<size_t>(1, std::min<size_t>(len, kPromptPassRows / s.B)));
+    const long rows = static_cast<long>(most) * s.B;
+    const SplitKind logits = score ? logits_kind(*s.m, rows) : SPLIT_NONE;
+    if (score && logits == SPLIT_NONE) return {};
     const int split_rows = score ? kSplitMinScoreRows : kSplitMinRows;
-    if (static_cast<long>(most) * s.B < split_rows) return {most, split_rows, SPLIT_NONE};
-    const SplitKind kind = layers_kind(*s.m);
-    if (kind != SPLIT_NONE) return {most, split_rows, kind};
-    return {std::min(len, (kSplitMinRows - 1) / s.B), kSplitMinRows, SPLIT_NONE};
+    if (rows < split_rows) return {most, split_rows, SPLIT_NONE, logits};
+    const SplitKind kind = layers_kind(*s.m, rows);
+    if (kind != SPLIT_NONE) return {most, split_rows, kind, logits};
+    return {std::min(len, (kSplitMinRows - 1) / s.B), kSplitMinRows, SPLIT_NONE, logits};
 }
 
 // One projection over M rows (norm folded in for RMSNorm, a norm kernel for LayerNorm).
@@ -2060,10 +2076,9 @@ static void split_norm(Session& s, bool pairs, const float* gamma, const float* 
 // Final norm, logits and the target's negative log-likelihood for rows
 // pp_x[0 .. M) of a slice (row m = seq * n + t, position t0 + t).  The logits are not
 // stored: every run of outputs leaves its maximum and its sum of exponentials.
-static void score_rows(Session& s, const ScoreSink& sink, int M, int n, int t0, int len) {
+static void score_rows(Session& s, const ScoreSink& sink, bool pairs, int M, int n, int t0, int len) {
     const Model& m = *s.m;
     const Shape& sh = m.shape;
-    const bool pairs = m.logits_pairs.ready;  // (as the pass's plan found or made it)
     split_norm(s, pairs, m.gf, m.bf, m.logits_norm, M);
     SplitGemmParams g = split_params(s.pp_split, (pairs ? m.logits_pairs : m.logits_split).blob.at, M, sh.vocab, sh.d_model);
     if (pairs) pair_params(g, m.logits_unit, m.logits_norm);
@@ -2337,7 +2352,12 @@ static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSi
         const int M = n * B;
         const int pos_base = s.pos + t0;
         const bool split = M >= plan.split_rows;
-        const bool pairs = plan.kind == SPLIT_PAIRS;
+        // (a shorter slice's form is its own, the others' if there is no memory for it)
+        const auto of_slice = [&](SplitKind planned, auto kind_of) {
+            const SplitKind kind = n == plan.slice ? planned : kind_of(m, M);
+            return kind == SPLIT_NONE ? planned : kind;
+        };
+        const bool pairs = split && of_slice(plan.kind, layers_kind) == SPLIT_PAIRS;
         const bool split_attn = split && reserve_split_attention(s, n, pos_base, pairs);
         hipLaunchKernelGGL(embed_rows_kernel, dim3((d + 255) / 256, M), dim3(256), 0, st, m.E, m.P, s.hist,
                            s.hist_stride, s.n_hist + t0, n, pos_base, s.pp_x, d);
@@ -2349,7 +2369,7 @@ static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSi
             if (split) prompt_layer_split(s, l, n, pos_base, pairs, split_attn, trim && l == sh.layers - 1);
             else prompt_layer_small(s, l, n, pos_base);
         }
-        if (sink) score_rows(s, *sink, M, n, t0, len);
+        if (sink) score_rows(s, *sink, of_slice(plan.logits, logits_kind) == SPLIT_PAIRS, M, n, t0, len);
         if (t0 + n == len) {
             hipLaunchKernelGGL(take_last_rows_kernel, dim3((d + 255) / 256, B), dim3(256), 0, st, s.pp_x, n,
                                s.x, d);
@@ -2373,7 +2393,7 @@ static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSi
 // prompt loop of text_gen.cpp:44-46).  log: per-step logits destination or null.
 static void run_prompt(Session& s, int len, float* log, size_t* steps_logged) {
     const size_t BV = static_cast<size_t>(s.B) * s.m->shape.vocab;
-    const RowsPlan plan = log ? RowsPlan{0, 0, SPLIT_NONE} : plan_rows(s, len, /*score=*/false);
+    const RowsPlan plan = log ? RowsPlan{} : plan_rows(s, len, /*score=*/false);
     if (plan.slice > 0) {
         prompt_pass(s, len, plan);
         if (steps_logged) *steps_logged += len;

@@ -62,7 +62,7 @@ static Tiling pick_tiling(int M, int N, int K) {
     const auto tiles = [&](int t) { return static_cast<long>((M + t - 1) / t) * ((N + t - 1) / t); };
     const auto rounds = [&](int t) { return (tiles(t) + 255) / 256; };
     if (rounds(32) <= 2) return TILE_32_K4;
-    if (rounds(64) == 1) return TILE_64_K4;
+    if (split_in_four_sets(M, N)) return TILE_64_K4;
     const long tall = static_cast<long>((M + 127) / 128) * ((N + 63) / 64);
     if (rounds(64) == 2 && tall <= 256 && K >= 768) return TILE_128x64;
     return rounds(128) * 28 < rounds(64) * 10 ? TILE_128 : TILE_64;

@@ -195,8 +195,11 @@ def test_a_prompt_leaves_the_same_bits_whatever_the_call_and_the_sampler(opt, ba
 
 
 #: (arch, width, tokens): what a pass leaves of the second layer's values is no further from float64 than with three parts
-CLOSENESS = [(synth.ARCH_GPT2, 512, 513), (synth.ARCH_GPT2, 512, 1000), (synth.ARCH_MODERN, 512, 641), (synth.ARCH_GPT2, 640, 385),
-             (synth.ARCH_GPT2, 768, 321), (synth.ARCH_GPT2, 768, 1000), (synth.ARCH_MODERN, 768, 300), (synth.ARCH_GPT2, 1024, 160)]
+CLOSENESS = [(synth.ARCH_GPT2, 512, 160), (synth.ARCH_GPT2, 512, 512), (synth.ARCH_GPT2, 512, 641), (synth.ARCH_GPT2, 512, 1000),
+             (synth.ARCH_MODERN, 512, 400), (synth.ARCH_MODERN, 512, 640), (synth.ARCH_MODERN, 512, 641), (synth.ARCH_GPT2, 576, 400),
+             (synth.ARCH_GPT2, 640, 384), (synth.ARCH_GPT2, 640, 385), (synth.ARCH_GPT2, 768, 320), (synth.ARCH_GPT2, 768, 321),
+             (synth.ARCH_GPT2, 768, 1000), (synth.ARCH_MODERN, 768, 160), (synth.ARCH_MODERN, 768, 256), (synth.ARCH_MODERN, 768, 300),
+             (synth.ARCH_MODERN, 896, 160), (synth.ARCH_GPT2, 1024, 160)]
 
 
 @pytest.mark.parametrize("arch, d, n", CLOSENESS)
