@@ -478,25 +478,14 @@ static bool layers_in_pairs(const Model& m) {
 // it came by, nor on what is drawn behind it.
 enum SplitKind { SPLIT_NONE, SPLIT_PAIRS, SPLIT_PARTS };
 
-// Three parts whose products of few rows are shared among four sets have the smaller errors up to 1024 columns (K = 512
-// 0.77e-7 against 1.09, 768 0.88 / 1.12, 1024 0.98 / 1.14; in one set 1.28, 1.59, 1.86), those of longer K never (2048 1.34 /
-// 1.20).  Over a layer the wider of its products decide: error of the second layer's values, pairs over three parts, below
-// the line and above: GPT-2 512 wide 1.10 (512 rows), 0.98 (513), 768 1.03 (320), 0.88 (321), Llama 768 1.05 (256), 0.98 (300);
-// from 1024 on pairs are closer with any rows (160: 0.95).  Below 640 columns q, k, v count too (Llama 512 wide: 1.03 at 640
-// rows, 0.97 at 641).
-static bool parts_are_closer(const Shape& sh, long rows) {
-    const int d = sh.d_model, up = sh.modern() ? 2 : 1;
-    return d < 1024 && (split_in_four_sets(rows, up * sh.d_ff()) || (d < 640 && split_in_four_sets(rows, 3 * d)));
-}
-
 static SplitKind layers_kind(const Model& m, long rows) {
-    if (m.shape.d_model >= kPairMinCols && !parts_are_closer(m.shape, rows) && layers_in_pairs(m)) return SPLIT_PAIRS;
+    if (m.shape.d_model >= kPairMinCols && !parts_are_closer(m.shape.d_model, (m.shape.modern() ? 2 : 1) * m.shape.d_ff(), rows) && layers_in_pairs(m)) return SPLIT_PAIRS;
     return split_layers(m) ? SPLIT_PARTS : SPLIT_NONE;
 }
 
 static SplitKind logits_kind(const Model& m, long rows) {
     const int d = m.shape.d_model, V = m.shape.vocab;
-    if (d >= kPairMinCols && !(d <= 1024 && split_in_four_sets(rows, V))) {
+    if (d >= kPairMinCols && !logits_parts_are_closer(d, V, rows)) {
         const bool pairs = make_form(m.logits_pairs, pair_place_bytes(V, d), [&](char* at) {
             const NormSize n = norm_size(m.shape, m.gf, m.bf);
             const std::optional<int> norm = pair_exponent(n.top, n.low);

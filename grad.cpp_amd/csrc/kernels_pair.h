@@ -469,7 +469,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
 
 // Tiles of 128 x 128, those behind the first `whole` (whole rounds of 256 compute units) in quarters of 64 x 64, dealt
 // over the XCDs the same way.  Bound by the LDS reads and products of a compute unit's whole tiles and its quarter; sums are those of either
-// tiling.  Figures and the line at pick_tiling.
+// tiling.  Figures and the line at pair_tiling.
 template <int EPI>
 __global__ __launch_bounds__(256, 2) void pair_mixed_kernel(const SplitGemmParams p, int whole) {
     const int id = blockIdx.x;

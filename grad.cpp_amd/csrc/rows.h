@@ -3,6 +3,7 @@
 
 #include "kernels_attn.h"
 #include "kernels_split.h"
+#include "tilings.h"
 
 namespace gh {
 
@@ -19,15 +20,9 @@ void split_weights(const float* src, int N, int K, bool gate_up, char* dst, int*
 // norm(x) of M rows in split form.
 void norm_split(bool rms, const float* x, const float* gamma, const float* beta, char* out, int M, int d, hipStream_t st);
 
-// Products of so many rows and outputs of which split_gemm shares K among four sets of wavefronts (one round of 64 x 64 tiles).
-inline bool split_in_four_sets(long rows, long outputs) { return (rows + 63) / 64 * ((outputs + 63) / 64) <= 256; }
-
 // One projection; p.n_tiles, p.tiles (and p.nll_stride) are filled in.  EPI_STORE: scoring.
 template <int EPI>
 void split_gemm(SplitGemmParams& p, hipStream_t st);
-
-// Narrower models have no pairs (kernels_pair.h).
-constexpr int kPairMinCols = 512;
 
 // The same three in pairs; units of a matrix: one per row of its storage.
 // (whole tiles of 96 outputs, also from a row behind the first)

@@ -36,38 +36,6 @@ void norm_split(bool rms, const float* x, const float* gamma, const float* beta,
     else norm_split_as<false>(x, gamma, beta, out, M, d, st);
 }
 
-// Which tiling.  Measured over 14 row counts from 160 to 8192 against five matrices (768
-// columns: 768, 2304, 4096 outputs; 2048 columns: 768, 512 outputs), the rule takes the fastest
-// tiling or one within 6 % of it:
-// - With two 32 x 32 tiles per compute unit at most they win, K shared by four sets of
-//   wavefronts, and after them 64 x 64 tiles with K shared the same way: such a launch is a chain
-//   of K steps of about 250 ns each (load, LDS, registers, product), so the shorter chain is what
-//   counts (1001 x 768 x 2048: 25 us against 35 with K in one set; 160 x 768 x 2048: 11 against 21).
-// - With more tiles than compute units the chains hide behind each other.  Tiles are dealt to 256
-//   compute units in whole rounds, and a round of 128 x 128 tiles costs 2.8 times one of 64 x 64
-//   (four times the products, half the operand bytes per product): the cheaper one
-//   (6000 x 768 x 2048: 120 us against 126; 8192 x 4096 x 768: 247, i.e. 208 TFLOP/s of fp32 products
-//   or 1.25 PFLOP/s of bf16, against 303).
-// - Two rounds of 64 x 64 tiles that are one round of 128 x 64 ones are taken as those, a
-//   tile's four stages in flight: a wavefront reads three fragments from LDS for two products
-//   instead of four, and no compute unit is left with two tiles where its neighbour has one.  Same
-//   sums in the same order.  280 to 510 tiles of 64 x 64, 40 launches (2231 x 768 x 768: 22.2 to
-//   20.6 us; 1999 x 768 x 2048: 43.4 to 41.3; 2231 x 768 x 3072: 66.2 to 60.8; 695 x 2304 x 768:
-//   21.2 to 20.5): 2 to 8 % faster from 768 columns on, between 11 % slower and 4 % faster at 512, where
-//   filling the longer ring is a larger part.  With more tiles than one each they lose (2807 x 768 x 2048:
-//   67.8 against 61.3), as do 128 x 64 tiles of eight wavefronts.
-enum Tiling { TILE_32_K4, TILE_64_K4, TILE_64, TILE_128x64, TILE_128 };
-
-static Tiling pick_tiling(int M, int N, int K) {
-    const auto tiles = [&](int t) { return static_cast<long>((M + t - 1) / t) * ((N + t - 1) / t); };
-    const auto rounds = [&](int t) { return (tiles(t) + 255) / 256; };
-    if (rounds(32) <= 2) return TILE_32_K4;
-    if (split_in_four_sets(M, N)) return TILE_64_K4;
-    const long tall = static_cast<long>((M + 127) / 128) * ((N + 63) / 64);
-    if (rounds(64) == 2 && tall <= 256 && K >= 768) return TILE_128x64;
-    return rounds(128) * 28 < rounds(64) * 10 ? TILE_128 : TILE_64;
-}
-
 template <int EPI, int MB, int NB, int WM, int WN, int KG, int STAGES, int PER_CU>
 static void launch(SplitGemmParams& p, hipStream_t st) {
     constexpr int TM = 32 * MB * WM, TN = 32 * NB * WN;
@@ -86,12 +54,12 @@ static void launch(SplitGemmParams& p, hipStream_t st) {
 
 template <int EPI>
 void split_gemm(SplitGemmParams& p, hipStream_t st) {
-    switch (pick_tiling(p.M, p.N, p.K)) {
-        case TILE_32_K4: launch<EPI, 1, 1, 1, 1, 4, 3, 2>(p, st); break;
-        case TILE_64_K4: launch<EPI, 1, 1, 2, 2, 4, 3, 1>(p, st); break;
-        case TILE_64: launch<EPI, 1, 1, 2, 2, 1, 3, 4>(p, st); break;
-        case TILE_128x64: launch<EPI, 2, 1, 2, 2, 1, 4, 2>(p, st); break;
-        case TILE_128: launch<EPI, 2, 2, 2, 2, 1, 3, 2>(p, st); break;
+    switch (split_tiling(p.M, p.N, p.K)) {
+        case SPLIT_32_K4: launch<EPI, 1, 1, 1, 1, 4, 3, 2>(p, st); break;
+        case SPLIT_64_K4: launch<EPI, 1, 1, 2, 2, 4, 3, 1>(p, st); break;
+        case SPLIT_64: launch<EPI, 1, 1, 2, 2, 1, 3, 4>(p, st); break;
+        case SPLIT_128x64: launch<EPI, 2, 1, 2, 2, 1, 4, 2>(p, st); break;
+        case SPLIT_128: launch<EPI, 2, 2, 2, 2, 1, 3, 2>(p, st); break;
     }
 }
 

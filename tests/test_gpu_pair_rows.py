@@ -1,6 +1,7 @@
 """Passes over many rows whose operands are two fp16 parts each (models of 512 columns and more): every tiling and
-epilogue at row counts that leave ragged tiles, operands at the ends of their range, and models whose weights have
-no such form, against the float64 forward.  The bounds are what fp32 sums give, as for the three-part form."""
+epilogue at row counts that leave ragged tiles, operands at the ends of their range, models whose weights have
+no such form and rows that are closer in three parts, against the float64 forward.  The bounds are what fp32 sums give, as
+for the three-part form; which form was taken is told from the bits, and how close it is from the same pass in three parts."""
 import numpy as np
 import pytest
 
@@ -30,37 +31,38 @@ def _check(cfg, W, B, n, seed, sequences=None):
         assert np.abs(last[b] - ref[-1]).max() <= 1e-5 * np.abs(ref[-1]).max(), b
 
 
-CASES = {
-    # rows reach: name: (width, vocab, sequences, tokens)
-    "32 x 32 tiles, one row past a tile": (512, 130, 1, 161),
-    "64 x 64 of two sets of K": (512, 1001, 3, 171),
-    "64 x 64 of one set, q, k, v; 64 x 96 of four, keys and values from the middle of the matrix": (512, 130, 3, 449),
-    "128 x 64, both FFN1; a nearly empty tile": (512, 130, 3, 667),
-    "128 x 128 at 512 columns": (512, 515, 11, 487),
-    "64 x 96 of four sets, SwiGLU": (768, 130, 2, 150),
-    "64 x 64 of one set, FFN1; four sets of 64 x 96, q, k, v": (768, 515, 1, 449),
-    "64 x 64 of two sets, W_o": (768, 1001, 3, 334),
-    "64 x 96 of four sets, W_o, FFN2 and logits": (768, 515, 4, 501),
-    "64 x 96 of two sets, FFN2; 128 x 128 and quarters, GELU, keys and values": (768, 515, 6, 500),
-    "128 x 128, all": (768, 515, 19, 474),
-    "nine parts of K: one set": (576, 130, 1, 161),
-    "nine parts of K: one set, FFN2 in four": (576, 301, 3, 667),
-    "64 x 96 of two sets, q, k, v and GELU": (640, 130, 2, 260),
-    "64 x 96 of two sets, SwiGLU": (768, 130, 2, 260),
-    "128 x 64, q, k, v": (512, 130, 9, 377),
-    "128 x 64, W_o": (576, 130, 17, 390),
-    "128 x 128 and quarters, q, k, v": (768, 130, 5, 400),
-    "128 x 128 and quarters, SwiGLU": (768, 130, 2, 520),
-    "128 x 128 and quarters, W_o; a nearly empty row of tiles": (512, 130, 20, 410),
-    "128 x 128 and quarters, q, k, v; quarters past the last row and the last output": (576, 130, 6, 405),
-}
+#: (width, vocabulary, sequences, tokens), both blocks.  Which launches they come to: test_tilings.py.
+CASES = [
+    (512, 130, 1, 161), (512, 1001, 3, 171), (512, 130, 3, 449), (512, 130, 3, 667), (512, 515, 11, 487),
+    (768, 130, 2, 150), (768, 515, 1, 449), (768, 1001, 3, 334), (768, 515, 4, 501), (768, 515, 6, 500),
+    (768, 515, 19, 474), (576, 130, 1, 161), (576, 301, 3, 667), (640, 130, 2, 260), (768, 130, 2, 260),
+    (512, 130, 9, 377), (576, 130, 17, 390), (768, 130, 5, 400), (768, 130, 2, 520), (512, 130, 20, 410),
+    (576, 130, 6, 405),
+]
+#: (arch, width, vocabulary, sequences, tokens): the launches that those leave out, and scored logits of whole vocabularies
+MORE_CASES = [
+    (synth.ARCH_GPT2, 512, 5000, 32, 33), (synth.ARCH_GPT2, 512, 50257, 1, 171), (synth.ARCH_GPT2, 640, 1001, 32, 33),
+    (synth.ARCH_MODERN, 768, 16000, 2, 130), (synth.ARCH_MODERN, 768, 16000, 4, 100), (synth.ARCH_MODERN, 768, 50257, 1, 97),
+    (synth.ARCH_GPT2, 1024, 130, 4, 40), (synth.ARCH_GPT2, 1280, 130, 9, 20),
+]
+
+
+def _case_id(case):
+    return "x".join(str(v) for v in case)
 
 
 @pytest.mark.parametrize("arch", [synth.ARCH_GPT2, synth.ARCH_MODERN])
-@pytest.mark.parametrize("name", sorted(CASES))
-def test_rows_match_the_float64_forward(name, arch):
-    d, vocab, B, n = CASES[name]
+@pytest.mark.parametrize("case", CASES, ids=_case_id)
+def test_rows_match_the_float64_forward(case, arch):
+    d, vocab, B, n = case
     cfg = synth.Config(arch, vocab, d, 1, d // 64, 700)
+    _check(cfg, synth.make_weights(cfg, 101, std=lively_std(cfg), norm_noise=0.1), B, n, 102)
+
+
+@pytest.mark.parametrize("case", MORE_CASES, ids=_case_id)
+def test_more_rows_match_the_float64_forward(case):
+    arch, d, vocab, B, n = case
+    cfg = synth.Config(arch, vocab, d, 1, d // 64, 200)
     _check(cfg, synth.make_weights(cfg, 101, std=lively_std(cfg), norm_noise=0.1), B, n, 102)
 
 
@@ -98,7 +100,7 @@ def test_a_gain_too_far_above_the_others_for_two_parts(gain):
 
 def test_weights_at_both_ends_of_the_range():
     """A row of weights below fp32's normal numbers, one of zeros, one of 1e12 (what comes of it is not used, but bounds
-    have to count with it), and a weight 2^20 times the rest of its row."""
+    have to count with it: three parts), and a weight 2^20 times the rest of its row."""
     cfg = synth.Config(synth.ARCH_GPT2, 67, 512, 1, 8, 600)
     W = synth.make_weights(cfg, 109, std=lively_std(cfg), norm_noise=0.1)
     names = [what[0] for what in synth.tensor_specs(cfg)]
@@ -202,25 +204,114 @@ CLOSENESS = [(synth.ARCH_GPT2, 512, 160), (synth.ARCH_GPT2, 512, 512), (synth.AR
              (synth.ARCH_MODERN, 896, 160), (synth.ARCH_GPT2, 1024, 160)]
 
 
+def _zero_behind_a_gain(cfg, W):
+    """Weights of zero behind element 5 of layer 0's second norm: its gain makes no difference to what comes of a pass, but
+    with 1e9 (_gain) the layers have no pairs."""
+    names = [what[0] for what in synth.tensor_specs(cfg)]
+    for name in ("FFN gate", "FFN up") if cfg.modern else ("FFN W1",):
+        W[names.index(f"layer 0 {name}")][5, :] = 0.0
+
+
+def _gain(cfg, W, value):
+    names = [what[0] for what in synth.tensor_specs(cfg)]
+    W[names.index("layer 0 norm2 gamma")][0, 5] = value
+
+
 @pytest.mark.parametrize("arch, d, n", CLOSENESS)
 def test_errors_are_no_larger_than_those_of_three_parts(arch, d, n):
-    """The same layers with one gain, in front of weights of zero, that leaves them no pairs."""
     cfg = synth.Config(arch, 1009, d, 2, d // 64, 1001)
-    names = [what[0] for what in synth.tensor_specs(cfg)]
     errors = [[], []]
     for seed in (121, 123):
         W = synth.make_weights(cfg, seed, std=0.02, norm_noise=0.1)
-        for name in ("FFN W1",) if arch == synth.ARCH_GPT2 else ("FFN gate", "FFN up"):
-            W[names.index(f"layer 0 {name}")][5, :] = 0.0
+        _zero_behind_a_gain(cfg, W)
         tokens = synth.uniform_tokens(n + 1, cfg.vocab, seed + 1)
         _, kv = ref_forward.forward(cfg, W, tokens[:-1], return_kv=True)
         at = range(0, n, 8)  # (values: keys carry the rounding of their angles too)
         want = np.stack([kv[1][1][pos] for pos in at])
         for form, gain in enumerate((1.0, 1e9)):
-            W[names.index("layer 0 norm2 gamma")][0, 5] = gain
+            _gain(cfg, W, gain)
             s = G.Session(G.Model.from_tensors(cfg, W))
             s.score(tokens[:-1], tokens[1:])
             got = np.stack([s.read_kv(0, 1, 1, pos) for pos in at])
             errors[form].append(np.linalg.norm(got - want) / np.linalg.norm(want))
     pairs, parts = np.mean(errors, axis=1)
     assert pairs <= 1.01 * parts, (pairs, parts)  # (40000 values and more: the figures' own spread is 0.5 %)
+
+
+def _small_rows(W, names):
+    up = W[names.index("layer 0 FFN W1")]
+    up[:, 3], up[:, 4], up[:, 8] = 1e-40, 0.0, 1e-25  # (rows of the product: its columns here)
+
+
+def _one_row_of(value):
+    def change(W, names):
+        W[names.index("layer 0 FFN W1")][:, 6] = value
+        W[names.index("layer 0 FFN W2")][6, :] = 0.0
+    return change
+
+
+def _outlier(W, names):
+    W[names.index("layer 0 FFN W1")][9, 7] *= 2.0 ** 20
+    W[names.index("layer 0 FFN W2")][7, :] *= 2.0 ** -20
+
+
+def _query(W, names):
+    W[names.index("layer 0 b_q")][0, 70] = 1e6
+    W[names.index("layer 0 W_k")][:, 70] = 0.0
+    W[names.index("layer 0 b_k")][0, 70] = 0.0
+
+
+#: name: (width, tokens, whether the pass is in pairs, what is done to the weights of a GPT-2 block)
+FORMS = {
+    "ordinary weights": (512, 641, True, None),
+    "rows of weights below fp32's normal numbers, of zeros and of 1e-25": (512, 641, True, _small_rows),
+    "a row of 1e12": (512, 641, False, _one_row_of(1e12)),
+    "a row a hundred times the others": (512, 641, True, _one_row_of(100.0)),
+    "a weight 2^20 times its row": (512, 641, False, _outlier),
+    "a query's element 1e6 times the others": (512, 641, False, _query),
+    "rows that are closer in three parts, 512 wide": (512, 640, False, None),
+    "rows that are closer in three parts, 768 wide": (768, 320, False, None),
+    "one row more": (768, 321, True, None),
+    "few rows of a wide model": (1024, 160, True, None),
+}
+
+
+@pytest.mark.parametrize("name", sorted(FORMS))
+def test_which_form_a_pass_takes(name):
+    """The values that layer 0 leaves are those of three parts, bit for bit, or they are not."""
+    d, n, in_pairs, change = FORMS[name]
+    cfg = synth.Config(synth.ARCH_GPT2, 301, d, 1, d // 64, n + 1)
+    W = synth.make_weights(cfg, 125, std=lively_std(cfg), norm_noise=0.1)
+    _zero_behind_a_gain(cfg, W)
+    if change:
+        change(W, [what[0] for what in synth.tensor_specs(cfg)])
+    tokens = synth.uniform_tokens(n + 1, cfg.vocab, 126)
+    want = _loss(ref_forward.forward(cfg, W, tokens[:-1]), tokens[1:])
+    bits = []
+    for gain in (1.0, 1e9):
+        _gain(cfg, W, gain)
+        s = G.Session(G.Model.from_tensors(cfg, W))
+        nll = s.score(tokens[:-1], tokens[1:])[0]
+        assert np.abs(nll - want).max() <= 2e-5 * max(1.0, np.abs(want).max())
+        bits.append([s.read_kv(0, 0, 1, pos).tobytes() for pos in range(0, n, 40)])
+    differ = bits[0] != bits[1]
+    assert differ == in_pairs
+
+
+@pytest.mark.parametrize("bytes_per_weight", [3, 8])
+def test_a_shortage_of_memory_does_not_settle_the_form(bytes_per_weight, monkeypatch):
+    """A pass that finds no memory for pairs, or for them alone, is followed by passes that take them."""
+    cfg = synth.Config(synth.ARCH_GPT2, 301, 512, 2, 8, 700)
+    W = synth.make_weights(cfg, 127, std=lively_std(cfg), norm_noise=0.1)
+    tokens = synth.uniform_tokens(700, cfg.vocab, 128)
+
+    def cache(gm):
+        s = G.Session(gm)
+        s.prefill(tokens)
+        return [s.read_kv(0, 1, kv, pos).tobytes() for kv in (0, 1) for pos in range(0, 700, 50)]
+
+    gm = G.Model.from_tensors(cfg, W)
+    monkeypatch.setenv("GRADHIP_TEST_SPARE_BYTES", str(bytes_per_weight * 24 * 512 * 512))
+    cache(gm)
+    monkeypatch.delenv("GRADHIP_TEST_SPARE_BYTES")
+    assert cache(gm) == cache(G.Model.from_tensors(cfg, W))
