@@ -2114,14 +2114,21 @@ constexpr int kSplitAttnMin = 128;
 // 3.9, 1 x 397 31.5 / 17.6, 13 x 77 15.2 / 9.6, 3 x 333 31.5 / 19.4, 8 x 61 behind 500 48 / 27); beyond, keys read
 // once for 64 queries (64 x 64 17.2 / 22.1, 64 x 128 46.8 / 65.3), unless most of a 64-query block would be
 // empty (64 x 31 13.3 / 11.2, 64 x 8 behind 900 180 / 67).
-static void launch_prompt_attn(const Session& s, const PrefillAttnParams& a) {
+template <int ROWS>
+static void launch_prompt_attn_as(const Session& s, const PrefillAttnParams& a) {
     const long pairs = static_cast<long>(s.m->shape.heads) * s.B;
     const long wide = (a.len + 63) / 64 * pairs, narrow = (a.len + 15) / 16 * pairs;
     if (s.page_shift >= 6 && (narrow <= 800 || narrow <= 2 * wide))
-        hipLaunchKernelGGL(attn_prefill16_kernel, dim3((a.len + 15) / 16, s.m->shape.heads, s.B), dim3(256), 0, s.stream, a);
+        hipLaunchKernelGGL(attn_prefill16_kernel<ROWS>, dim3((a.len + 15) / 16, s.m->shape.heads, s.B), dim3(256), 0, s.stream, a);
     else
-        hipLaunchKernelGGL(attn_prefill64_kernel, dim3((a.len + 63) / 64, s.m->shape.heads, s.B), dim3(256), 0, s.stream, a);
+        hipLaunchKernelGGL(attn_prefill64_kernel<ROWS>, dim3((a.len + 63) / 64, s.m->shape.heads, s.B), dim3(256), 0, s.stream, a);
     HIP_CHECK(hipGetLastError());
+}
+
+static void launch_prompt_attn(const Session& s, const PrefillAttnParams& a) {
+    if (!a.out_split) launch_prompt_attn_as<ROWS_FP32>(s, a);
+    else if (a.pair_scale != 0.0f) launch_prompt_attn_as<ROWS_PAIRS>(s, a);
+    else launch_prompt_attn_as<ROWS_PARTS>(s, a);
 }
 
 // One layer over M = n * B rows of pp_x through the split projections, operands in pairs or in three parts, and with

@@ -426,11 +426,13 @@ __global__ __launch_bounds__(256) void attn_decode64_kernel(const AttnParams p) 
 // through LDS in tiles of 64 positions; four threads share a query, each takes
 // every fourth key of a tile and keeps its own running softmax, and the four
 // are merged with quad permutations at the end.
+enum AttnRows { ROWS_FP32, ROWS_PARTS, ROWS_PAIRS };  // what the prompt attention leaves
+
 struct PrefillAttnParams {
     const float* q;  // [batch * len][d_model], rotated
     float* out;      // [batch * len][d_model]
-    char* out_split;  // when set: the output rows as an operand instead (store_operand4)
-    float pair_scale;  // of that operand, 0: in three parts
+    char* out_split;  // ROWS_PARTS, ROWS_PAIRS: the output rows as an operand instead
+    float pair_scale;  // of that operand in pairs, 0: in three parts
     float key_scale;   // split attention in pairs: a power of two that no key exceeds fp16 with
     KvLayout kv;
     int layer, d_model, len, pos_base;
@@ -449,6 +451,7 @@ struct PrefillAttnParams {
 // inference.cpp:211-225 computes the same numbers one query at a time.
 typedef float attn_v4f __attribute__((ext_vector_type(4)));
 
+template <int ROWS>
 static __global__ __launch_bounds__(256) void attn_prefill64_kernel(const PrefillAttnParams p) {
     constexpr int HS = 64, TILE = 64, LDK = HS + 4, LDV = TILE + 4;  // padded rows: float4 reads of 16 rows hit 64 banks
     __shared__ float Ks[TILE * LDK];  // [key][dim]
@@ -559,18 +562,19 @@ static __global__ __launch_bounds__(256) void attn_prefill64_kernel(const Prefil
     }
     if (live) {
         const float inv = 1.0f / l;
-        if (p.out_split) {
+        if constexpr (ROWS != ROWS_FP32) {
 #pragma unroll
             for (int db = 0; db < 4; db++)
-                store_operand4(p.out_split, b * p.len + t, h * HS + db * 16 + g * 4, p.d_model / kSplitCols, o[db][0] * inv,
-                               o[db][1] * inv, o[db][2] * inv, o[db][3] * inv, p.pair_scale);
-            return;
-        }
-        float* orow = p.out + (static_cast<size_t>(b) * p.len + t) * p.d_model + h * HS;
+                store_operand4<ROWS == ROWS_PAIRS>(p.out_split, b * p.len + t, h * HS + db * 16 + g * 4,
+                                                   p.d_model / kSplitCols, o[db][0] * inv, o[db][1] * inv, o[db][2] * inv,
+                                                   o[db][3] * inv, p.pair_scale);
+        } else {
+            float* orow = p.out + (static_cast<size_t>(b) * p.len + t) * p.d_model + h * HS;
 #pragma unroll
-        for (int db = 0; db < 4; db++)
-            *reinterpret_cast<float4*>(orow + db * 16 + g * 4) =
-                make_float4(o[db][0] * inv, o[db][1] * inv, o[db][2] * inv, o[db][3] * inv);
+            for (int db = 0; db < 4; db++)
+                *reinterpret_cast<float4*>(orow + db * 16 + g * 4) =
+                    make_float4(o[db][0] * inv, o[db][1] * inv, o[db][2] * inv, o[db][3] * inv);
+        }
     }
 }
 
@@ -579,6 +583,7 @@ static __global__ __launch_bounds__(256) void attn_prefill64_kernel(const Prefil
 // the outputs of dims 16 w .. + 15; the maxima and the probabilities meet in LDS.  Keys and
 // values go from memory to the operand registers of the one wavefront that uses them, a tile
 // ahead.  For pages of 64 positions and more (a tile sits in one page).
+template <int ROWS>
 static __global__ __launch_bounds__(256) void attn_prefill16_kernel(const PrefillAttnParams p) {
     constexpr int HS = 64, TILE = 64;
     __shared__ float peak[2][4][16];         // [tile parity][wavefront][query]
@@ -685,9 +690,9 @@ static __global__ __launch_bounds__(256) void attn_prefill16_kernel(const Prefil
     if (live) {
         const float inv = 1.0f / l;
         const int at = h * HS + wave * 16 + g * 4;
-        if (p.out_split) {
-            store_operand4(p.out_split, b * p.len + t, at, p.d_model / kSplitCols, o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv,
-                           p.pair_scale);
+        if constexpr (ROWS != ROWS_FP32) {
+            store_operand4<ROWS == ROWS_PAIRS>(p.out_split, b * p.len + t, at, p.d_model / kSplitCols, o[0] * inv, o[1] * inv,
+                                               o[2] * inv, o[3] * inv, p.pair_scale);
         } else {
             *reinterpret_cast<float4*>(p.out + (static_cast<size_t>(b) * p.len + t) * p.d_model + at) =
                 make_float4(o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv);

@@ -72,7 +72,7 @@ struct SplitAttnParams {
     const char* kv;  // split_kv_kernel's tiles
     int tiles;       // ... per pair
     char* out;       // operand rows [batch * len] x d_model
-    float pair_scale;  // ... of pairs, 0: in three parts
+    float pair_scale;  // ... of pairs
     float* part;     // partial results of query blocks whose keys are shared among workgroups
     int d_model, heads, len, pos_base;
     int chunk_shift;  // a workgroup takes up to 1 << chunk_shift tiles of keys
@@ -339,6 +339,7 @@ static __global__ __launch_bounds__(256, 2) void attn_split_kernel(const SplitAt
 // 9.3 (4 TB/s), against four times the queries per workgroup, 32 registers per wavefront and a part at a time.
 constexpr int kMergeAhead = 4;
 
+template <bool PAIRS>
 static __global__ __launch_bounds__(256) void attn_split_merge_kernel(const SplitAttnParams p) {
     const int pair = p.first + blockIdx.y, b = pair / p.heads, h = pair - b * p.heads;
     const int lane = threadIdx.x & 63, h32 = lane >> 5;
@@ -382,8 +383,8 @@ static __global__ __launch_bounds__(256) void attn_split_merge_kernel(const Spli
     const float inv = 1.0f / l;
 #pragma unroll
     for (int q = 0; q < 2; q++)
-        store_operand4(p.out, b * p.len + t, h * 64 + r0 * 2 + q * 8 + h32 * 4, p.d_model / kSplitCols, o[4 * q] * inv,
-                       o[4 * q + 1] * inv, o[4 * q + 2] * inv, o[4 * q + 3] * inv, p.pair_scale);
+        store_operand4<PAIRS>(p.out, b * p.len + t, h * 64 + r0 * 2 + q * 8 + h32 * 4, p.d_model / kSplitCols, o[4 * q] * inv,
+                              o[4 * q + 1] * inv, o[4 * q + 2] * inv, o[4 * q + 3] * inv, p.pair_scale);
 }
 
 }  // namespace gh

@@ -132,11 +132,13 @@ __device__ __forceinline__ void store_pair4(char* base, int r, int k, int kblock
     *reinterpret_cast<v2u*>(at + kPairPartBytes) = p2;
 }
 
-// Four consecutive columns of a row of activations, in the form that the projection behind reads: pairs scaled by
-// pair_scale, three parts where that is zero.
+// Four consecutive columns of a row of activations, in the form that the projection behind reads: three parts, or pairs
+// scaled by pair_scale.  A kernel is made for either: a condition here would part the values' products from the
+// subtractions behind them, and their rounding would go into the parts.
+template <bool PAIRS>
 __device__ __forceinline__ void store_operand4(char* base, int r, int k, int kblocks, float x, float y, float z, float w,
                                                float pair_scale) {
-    if (pair_scale != 0.0f) store_pair4(base, r, k, kblocks, x, y, z, w, pair_scale);
+    if constexpr (PAIRS) store_pair4(base, r, k, kblocks, x, y, z, w, pair_scale);
     else store_split4(base, r, k, kblocks, x, y, z, w);
 }
 

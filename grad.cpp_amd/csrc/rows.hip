@@ -147,7 +147,7 @@ void split_attention(const PrefillAttnParams& a, int batch, char* kv, size_t kv_
                            in_pairs ? kPairAttnLds : kAttnLds, st, p);
         check(hipGetLastError(), "attn_split");
         if (p.items > blocks) {
-            hipLaunchKernelGGL(attn_split_merge_kernel, dim3(4 * blocks, p.pairs), dim3(256), 0, st, p);
+            hipLaunchKernelGGL(in_pairs ? attn_split_merge_kernel<true> : attn_split_merge_kernel<false>, dim3(4 * blocks, p.pairs), dim3(256), 0, st, p);
             check(hipGetLastError(), "attn_split_merge");
         }
     }

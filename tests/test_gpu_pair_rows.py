@@ -315,3 +315,9 @@ def test_a_shortage_of_memory_does_not_settle_the_form(bytes_per_weight, monkeyp
     cache(gm)
     monkeypatch.delenv("GRADHIP_TEST_SPARE_BYTES")
     assert cache(gm) == cache(G.Model.from_tensors(cfg, W))
+
+
+def test_a_short_last_slice_takes_its_own_form():
+    """33280 rows: a slice of 512 tokens of every sequence in pairs, the 512 rows of the last 8 in three parts."""
+    cfg = synth.Config(synth.ARCH_GPT2, 301, 512, 2, 8, 521)
+    _check(cfg, synth.make_weights(cfg, 129, std=lively_std(cfg), norm_noise=0.1), 64, 520, 130)
