@@ -16,7 +16,7 @@
 // many positions would not average out; so the weights of every other 64 columns are stored negated and their
 // sums subtracted (what is left is below 1e-9).  Error over the size of the result against float64, normal operands, three
 // parts with K in one set / in four -> two: K = 512 1.28 / 0.77e-7 -> 1.09 to 1.26, 768 1.59 / 0.88 -> 1.12 to 1.32, 1024
-// 1.86 / 0.98 -> 1.14 to 1.37, 2048 2.72 / 1.34 -> 1.19 to 1.27, 3072 3.40 / 1.63 -> 1.25 to 1.38 (the upper end 128 x 128 tiles; an
+// 1.86 / 0.98 -> 1.14 to 1.37, 2048 2.72 / 1.34 -> 1.19 to 1.27, 3072 3.40 / 1.63 -> 1.25 to 1.38 (the upper end 128 x 128 and 128 x 64 tiles; an
 // fp32 sum of one product after the other: 4.0 to 9.9).  Below K = 512 the three parts are the closer ones, so narrower
 // models keep them (kPairMinCols).
 //
@@ -207,15 +207,17 @@ __device__ __forceinline__ void strip_qkv(const SplitGemmParams& p, int m, int n
     *reinterpret_cast<float4*>(dst) = o;
 }
 
-// C[M,N] = A[M,K] . W[N,K]^T of pairs.  Tiles, workgroup order, LDS ring and epilogues are split_gemm_kernel's.
-// A step of 16 columns is three rounds of products (w1 a2, w2 a1, w1 a1), its fragments read from LDS during the
-// step before into registers of their own (a 64 x 64 wavefront has 128 of its 256 for sums).  Four steps make a
-// 64-column part that starts from zero and is then added to the running sums (or taken from them, the weights of every
-// other part being negative).  (Added in front of the next part's products instead, accumulator by accumulator, the
-// compiler copies every part first.)  The small products of a part (those with a second part) have a sum of their own,
-// except in wavefronts of 64 x 64: a full-sized sum is then cut four times a part instead of twelve (error of K = 512
-// 1.26 -> 1.09e-7, 768 1.32 -> 1.12, 2048 1.55 -> 1.20 or, in one set, 1.27, 3072 1.71 -> 1.25, 1.37; prompts of 2000 rows of a
-// Llama of 768 columns 0.5 % slower by its 16 additions per block and part).  K / KG is a multiple of 64.
+// C[M,N] = A[M,K] . W[N,K]^T of pairs.  Tiles, workgroup order, LDS ring and epilogues are split_gemm_kernel's. A step
+// of 16 columns is three rounds of products (w1 a2, w2 a1, w1 a1), its fragments read from LDS during the step before
+// into registers of their own (a 64 x 64 wavefront has 128 of its 256 for sums).  Four steps make a 64-column part that
+// starts from zero and is then added to the running sums (or taken from them, the weights of every other part being
+// negative).  (Added in front of the next part's products instead, accumulator by accumulator, the compiler copies every
+// part first.)  In wavefronts of 32 rows the small products of a part (those with a second part) have a sum of their
+// own: a full-sized sum is then cut four times a part instead of twelve (error of K = 512 1.26 -> 1.09e-7, 768 1.32 ->
+// 1.12, 2048 1.55 -> 1.20 to 1.27, 3072 1.71 -> 1.25 to 1.38; 2000 rows of 768 columns 21.2 -> 21.8 us by its 16
+// additions per block and part).  Those of 64 rows, which take the larger passes, are the closer ones without it and pay
+// more for it (128 x 64 tiles, 8192 rows of W_o and FFN2 61.6 -> 68.5 us; 64 x 64 wavefronts have no registers left).  K
+// / KG is a multiple of 64.
 template <int EPI, int MB, int NB, int WM, int WN, int KG>
 __device__ __forceinline__ void pair_tile(const SplitGemmParams& p, int m_tile, int n_tile) {
     extern __shared__ __attribute__((aligned(1024))) char lds_pair[];
@@ -259,7 +261,7 @@ __device__ __forceinline__ void pair_tile(const SplitGemmParams& p, int m_tile, 
             f[x] = *reinterpret_cast<const v8h*>(frag + stage * kStage + part * kPairPartBytes
                                                  + (kUnitsA + (wn * NB + x) * 2) * kPairBlockBytes);
     };
-    constexpr bool kApart = MB * NB < 4;  // small products in sums of their own: 2 x 2 blocks have no registers for them
+    constexpr bool kApart = MB == 1;  // small products in sums of their own
     v16f sum[NB][MB], part[NB][MB], small[kApart ? NB : 1][kApart ? MB : 1], zero;
 #pragma unroll
     for (int r = 0; r < 16; r++) zero[r] = 0.0f;
@@ -274,7 +276,8 @@ __device__ __forceinline__ void pair_tile(const SplitGemmParams& p, int m_tile, 
             for (int b = 0; b < MB; b++) to[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[a], x[b], first ? zero : to[a][b], 0, 0, 0);
     };
     // Strips: of the wavefront's own blocks, or, where sets share K, every kAll-th of the tile's.
-    // (QKV's 64 x 96 tiles with K shared by two sets are as fast without, 37.9 us against 38.9 for 2048 x 2304 x 768.)
+    // (QKV's 64 x 96 tiles with K shared by two sets are as fast without: 700 x 1920 x 640 13.9 us against 14.0, 700 and 1000 x 3072 x
+    // 1024 24.9 and 29.3 against 25.1 and 29.4.)
     constexpr bool kStrips = EPI == EPI_RESID || (EPI == EPI_QKV && !(NB == 3 && KG == 2));
     constexpr int kAll = kWaves * KG, kCount = KG == 1 ? MB * NB * 4 : TM * TN / 256 / kAll;
     static_assert(!kStrips || kCount * 256 * kAll == TM * TN, "whole rounds of strips");

@@ -82,14 +82,15 @@ struct SplitAttnParams {
     float key_unit;  // in two parts: what a key's unit is worth, a power of two
 };
 
-// Workgroup ids go round-robin over the eight XCDs.  With many (sequence, head) pairs all
-// workgroups of one sit on one XCD, whose L2 then serves its keys and values to every query
-// block after the first (192 pairs: 1024 tokens 247 -> 198 us, 1536 tokens 411 -> 388); with few the pairs would
-// not spread evenly (12 pairs, 1999 tokens: 47 -> 57 us) and ids are dealt as they come.  On an XCD the longest query
-// blocks of up to kAttnGroup pairs go first, then the next longest: pair by pair, a last pair's longest
-// block began when the others were nearly done (192 pairs, attn_pair_kernel: 1024 tokens 140 -> 106 us, 1536 264 -> 220; in
-// groups of 4, 8, 12 pairs 116, 116, 109 and 225, 222, 219).  pair: counted from the launch's first.  False for an id
-// past the last pair.
+// Workgroup ids go round-robin over the eight XCDs.  With many (sequence, head) pairs all workgroups of one sit on one
+// XCD (192 pairs, three parts, pair by pair: 1024 tokens 247 -> 198 us, 1536 tokens 411 -> 388); with few the pairs
+// would not spread evenly (12 pairs, 1999 tokens: 47 -> 57 us) and ids are dealt as they come.  On an XCD the longest
+// query blocks of up to kAttnGroup pairs go first, then the next longest: pair by pair, a last pair's longest block
+// began when the others were nearly done (192 pairs, attn_pair_kernel: 1024 tokens 140 -> 106 us, 1536 264 -> 220),
+// which counts for more than an L2 of 4 MB that holds four pairs' tiles instead of 24.  us in groups of 4 / 12 / 24 / 48
+// / 96: 96 pairs x 1024 61 / 55 / 55 / 55 / 55, 192 x 2000 411 / 384 / 384 / 385 / 385, 384 x 1000 219 / 215 / 212 / 212
+// / 212, 768 x 500 133 / 135 / 131 / 135 / 137, 768 x 256 48 / 47 / 45 / 46 / 48. pair: counted from the launch's first.
+// False for an id past the last pair.
 constexpr int kAttnGroup = 24;
 
 __device__ __forceinline__ bool attn_place(const SplitAttnParams& p, int& pair, int& b, int& h, int& item) {
