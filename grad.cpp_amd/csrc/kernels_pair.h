@@ -16,8 +16,9 @@
 // many positions would not average out; so the weights of every other 64 columns are stored negated and their
 // sums subtracted (what is left is below 1e-9).  Error over the size of the result against float64, normal operands, three
 // parts with K in one set / in four -> two: K = 512 1.28 / 0.77e-7 -> 1.09 to 1.26, 768 1.59 / 0.88 -> 1.12 to 1.32, 1024
-// 1.86 / 0.98 -> 1.14 to 1.37, 2048 2.72 / 1.34 -> 1.19 to 1.27, 3072 3.40 / 1.63 -> 1.25 to 1.38 (the upper end 128 x 128 and 128 x 64 tiles; an
-// fp32 sum of one product after the other: 4.0 to 9.9).  Below K = 512 the three parts are the closer ones, so narrower
+// 1.86 / 0.98 -> 1.14 to 1.37, 2048 2.72 / 1.34 -> 1.19 to 1.27, 3072 3.40 / 1.63 -> 1.25 to 1.38 (the upper end 128 x 128
+// and 128 x 64 tiles; an fp32 sum of one product after the other: 4.0 to 9.9).  Few rows whose products four sets would
+// share take three parts (parts_are_closer in tilings.h).  Below K = 512 the three parts are the closer ones, so narrower
 // models keep them (kPairMinCols).
 //
 // The range.  fp16 has exponents -14 to 15 and, below, numbers of fewer bits (the matrix cores take them as
@@ -471,8 +472,9 @@ __global__ __launch_bounds__(64 * WM * WN * KG, PER_CU * WM * WN * KG / 4) void 
 }
 
 // Tiles of 128 x 128, those behind the first `whole` (whole rounds of 256 compute units) in quarters of 64 x 64, dealt
-// over the XCDs the same way.  Bound by the LDS reads and products of a compute unit's whole tiles and its quarter; sums are those of either
-// tiling.  Figures and the line at pair_tiling.
+// over the XCDs the same way; sums are those of either tiling.  Its time is one whole tile's chain of steps and epilogue
+// with a quarter beside it: the matrix cores' share is a quarter of it (2000 x 2304 x 768).  Figures and the line at
+// pair_tiling.
 template <int EPI>
 __global__ __launch_bounds__(256, 2) void pair_mixed_kernel(const SplitGemmParams p, int whole) {
     const int id = blockIdx.x;
