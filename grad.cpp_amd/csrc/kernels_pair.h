@@ -124,7 +124,6 @@ static __global__ __launch_bounds__(1024) void norm_pair_long_kernel(const float
 struct DeviceUnit {
     static __device__ __forceinline__ float exp2(float x) { return __builtin_amdgcn_exp2f(x); }
     static __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-    static __device__ __forceinline__ float med3(float x, float lo, float hi) { return __builtin_amdgcn_fmed3f(x, lo, hi); }
 };
 
 struct PairRowsOut : EpilogueMath<DeviceUnit> {
