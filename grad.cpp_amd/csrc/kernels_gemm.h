@@ -7,6 +7,7 @@
 #pragma once
 
 #include "kernels_gemv.h"
+#include "tilings.h"
 
 #include <algorithm>
 
@@ -595,40 +596,21 @@ inline void launch_gemm_wide(const GemvParams& p, int M, hipStream_t st) {
 }
 
 // More than 64 rows on eight wavefronts a workgroup: the tiles per workgroup that finish first.  All
-// of them give the same sums.  A launch costs a start and then, for every workgroup that a
-// compute unit is dealt, a time that grows more slowly than the tiles in it, since more tiles
-// share the rows they read (what is being paid for is operand traffic from the L2s and operand
-// permutes, 2 x 2 tiles having half of both per product).  Measured over 65 to 511 rows against thirteen
-// matrices (512 to 4096 outputs, 512 to 4096 columns): 1 x 1 tiles 1.7 us per workgroup and 768 columns,
-// two tiles 2.4, 2 x 2 4.0; the rule's pick of these four is the fastest or within 6 % of it in 142 of 143
-// cases, and 11.3 us for 9.8 at 511 x 768 x 768 (profiles/many_row_tilings.md).  3 x 2 tiles 5.9 and 2 x 3 6.2, for
-// the row counts where four tiles leave a last workgroup to few compute units: over 22 row counts and 13 matrices the
-// rule with them is faster by more than 2 % in 69 of 286 cases (384 x 1024 x 768 11.9 us -> 9.0, 511 x 768 x 768
-// 11.2 -> 9.5, 397 x 768 x 2048 19.5 -> 18.0, 244 x 4096 x 768 unchanged at 22.4) and slower by that much in one (3 %); 2.2 %
-// in the mean.  Queries, keys and values stay with four: six tiles are a second round of their epilogue, whose reads
-// (position, page, rotation) nothing hides (244 x 2304 x 768 in a prompt 20.2 us -> 23.4).
-// 1 x 1 for narrow matrices and 4 x 1 for the others, as it was: 100 x 4096 x 768 17.1 us -> 14.3,
-// 244 x 2304 x 768 24.4 -> 17.1, 397 x 4096 x 768 52.5 -> 35.8, 244 x 768 x 2048 12.8 -> 12.2.
-// (Both operands through an LDS ring, 32 x 32 to 64 x 64 outputs per workgroup: 35-36 us at 397 x 4096 x
-// 768, slower than this at every narrower shape.)
+// of them give the same sums.
 template <int EPI, bool RMS>
 inline void launch_gemm16_many(const GemvParams& p, int M, hipStream_t st) {
-    const auto cost = [&](int mt, int nt, int each) {
-        const long groups = static_cast<long>((M + 16 * mt - 1) / (16 * mt)) * ((p.N + 16 * nt - 1) / (16 * nt));
-        return (groups + 255) / 256 * each;
-    };
-    const bool wide = p.N > 1024;
-    const long c11 = cost(1, 1, 17), c12 = cost(1, 2, wide ? 24 : 25), c21 = cost(2, 1, wide ? 25 : 24), c22 = cost(2, 2, 40);
-    const long least = std::min({c11, c12, c21, c22});
-    if constexpr (EPI != EPI_QKV) {
-        const long c32 = cost(3, 2, 59), c23 = cost(2, 3, 62);
-        if (c32 < least && c32 <= c23) return launch_gemm16_as<EPI, RMS, 3, 2, 8>(p, M, st);
-        if (c23 < least) return launch_gemm16_as<EPI, RMS, 2, 3, 8>(p, M, st);
+    switch (rows_tiles(M, p.N, EPI != EPI_QKV)) {
+        case ROWS_1x1: launch_gemm16_as<EPI, RMS, 1, 1, 8>(p, M, st); break;
+        case ROWS_1x2: launch_gemm16_as<EPI, RMS, 1, 2, 8>(p, M, st); break;
+        case ROWS_2x1: launch_gemm16_as<EPI, RMS, 2, 1, 8>(p, M, st); break;
+        case ROWS_2x2: launch_gemm16_as<EPI, RMS, 2, 2, 8>(p, M, st); break;
+        case ROWS_3x2:
+            if constexpr (EPI != EPI_QKV) launch_gemm16_as<EPI, RMS, 3, 2, 8>(p, M, st);
+            break;
+        case ROWS_2x3:
+            if constexpr (EPI != EPI_QKV) launch_gemm16_as<EPI, RMS, 2, 3, 8>(p, M, st);
+            break;
     }
-    if (c22 == least) launch_gemm16_as<EPI, RMS, 2, 2, 8>(p, M, st);
-    else if (c12 == least) launch_gemm16_as<EPI, RMS, 1, 2, 8>(p, M, st);
-    else if (c21 == least) launch_gemm16_as<EPI, RMS, 2, 1, 8>(p, M, st);
-    else launch_gemm16_as<EPI, RMS, 1, 1, 8>(p, M, st);
 }
 
 // At 64 rows (0.4575 ms per step with 2 x 1 tiles on 8 wavefronts for the wide projections and

@@ -110,4 +110,42 @@ inline PairTiling pair_tiling(int M, int N, int K, PairOut what) {
     return best;
 }
 
+// fp32 products of 65 to 511 rows in tiles of 16 x 16 (gemm16_kernel on eight wavefronts): how many of them, rows x outputs, a
+// workgroup takes.  A launch costs a start and then, for every workgroup that a compute unit is dealt, a time that grows
+// more slowly than the tiles in it, since more tiles share the rows they read (what is being paid for is operand traffic
+// from the L2s and operand permutes, 2 x 2 tiles having half of both per product): per workgroup and 768 columns 1 x 1
+// tiles 1.7 us, two 2.4 or 2.5, 2 x 2 4.0, 3 x 2 5.9, 2 x 3 6.2.  Runs of outputs are dealt to the eight XCDs in turn,
+// each with all its rows (the weights stay in that L2), so what counts is the XCD with the most of them over its 32
+// compute units: 511 x 576 in 3 x 2 tiles are 198 workgroups and yet two rounds on an XCD that has 3 of the 18 runs
+// (K = 2304 32.9 us; 2 x 3 20.4).  Over 784 launches (16 row counts against W_o, FFN1 and FFN2 of 13 widths from 512 to 1536) the
+// rule takes 1.3 % longer than the best of the six each; with the workgroups counted over the whole chip 3.8 %, 62 % at most
+// (397 x 896 x 3584 48.5 us against 29.9), and 4.7 % without 3 x 2 and 2 x 3, which are there for row counts where
+// four tiles leave a last workgroup to few compute units (511 x 768 x 768 11.2 -> 9.5, 397 x 768 x 2048 19.5 -> 18.0).
+// Queries, keys and values stay with four: six tiles are a second round of their epilogue, whose reads (position,
+// page, rotation) nothing hides (244 x 2304 x 768 in a prompt 20.2 us -> 23.4).
+// (profiles/many_row_tilings.md.  Both operands through an LDS ring, 32 x 32 to 64 x 64 outputs per workgroup: 35-36 us at
+// 397 x 4096 x 768, slower than this at every narrower shape.)
+enum RowsTiles { ROWS_1x1, ROWS_1x2, ROWS_2x1, ROWS_2x2, ROWS_3x2, ROWS_2x3 };
+struct RowsTilesTime {
+    int rows, outputs, each;  // 16-row tiles, 16-output tiles, a workgroup's time
+};
+
+inline RowsTiles rows_tiles(int M, int N, bool six) {
+    const bool wide = N > 1024;
+    const RowsTilesTime tiles[] = {{1, 1, 17}, {1, 2, wide ? 24 : 25}, {2, 1, wide ? 25 : 24}, {2, 2, 40}, {3, 2, 59}, {2, 3, 62}};
+    const auto cost = [&](RowsTiles t) {
+        const long row_groups = (M + 16 * tiles[t].rows - 1) / (16 * tiles[t].rows);
+        const long runs = (N + 16 * tiles[t].outputs - 1) / (16 * tiles[t].outputs);
+        return ((runs + 7) / 8 * row_groups + 31) / 32 * tiles[t].each;
+    };
+    RowsTiles best = ROWS_2x2;  // (of equals the more tiles, but four before six)
+    for (const RowsTiles t : {ROWS_1x2, ROWS_2x1, ROWS_1x1})
+        if (cost(t) < cost(best)) best = t;
+    if (six) {
+        for (const RowsTiles t : {ROWS_3x2, ROWS_2x3})
+            if (cost(t) < cost(best)) best = t;
+    }
+    return best;
+}
+
 }  // namespace gh

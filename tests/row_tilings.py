@@ -15,6 +15,11 @@ def compile_rules(path):
     return exe
 
 
+def ask(exe, lines):
+    return subprocess.run([exe], input="\n".join(lines) + "\n", capture_output=True, text=True, check=True,
+                          timeout=60).stdout.splitlines()
+
+
 def launches(exe, cases):
     """Of every (arch, width, vocabulary, sequences, tokens, whether the weights have pairs), scored and as a prompt: the set of
     (form, epilogue, tiling) it runs; keys: keys and values alone, of the last layer of a prompt."""
@@ -27,8 +32,7 @@ def launches(exe, cases):
         wanted.append([("qkv", 3 * d, d), ("keys", 2 * d, d), ("resid", d, d), (act, ffn1, d), ("resid", d, F), ("logits", vocab, d)])
         for what, N, K in wanted[-1]:
             lines += [f"parts {M} {N} {K}", f"pairs {M} {N} {K} {what if what in ('gelu', 'swiglu', 'logits') else 'rows'}"]
-    out = iter(subprocess.run([exe], input="\n".join(lines) + "\n", capture_output=True, text=True, check=True,
-                              timeout=60).stdout.split("\n"))
+    out = iter(ask(exe, lines))
     found = []
     for (arch, d, vocab, B, n, fit), products in zip(cases, wanted):
         layers, logits = next(out), next(out)

@@ -53,3 +53,26 @@ def test_forms_change_where_the_gpu_tests_say(rules):
         if change is None:
             taken, = row_tilings.launches(rules, [(synth.ARCH_GPT2, d, 301, 1, n, True)])
             assert {form for form, what, _ in taken if what != "logits"} == {"pairs" if in_pairs else "parts"}, (d, n)
+
+
+def _rounds(M, N, rows, outputs):
+    """Of the XCD that is dealt the most workgroups, by the kernel's map of ids (gemm16_kernel), on its 32 compute units."""
+    row_groups, runs = -(-M // (16 * rows)), -(-N // (16 * outputs))
+    dealt = [0] * 8
+    for at in range(-(-runs // 8) * 8 * row_groups):
+        xcd, slot = at & 7, at >> 3
+        dealt[xcd] += xcd + 8 * (slot // row_groups) < runs
+    return -(-max(dealt) // 32)
+
+
+def test_few_rows_take_the_tiles_that_the_fullest_xcd_ends_first_with(rules):
+    """Widths whose runs of outputs are no multiple of eight among them: 511 x 576 in 3 x 2 tiles were two rounds taken for one."""
+    sizes = [(M, N, six) for M in (65, 96, 150, 200, 256, 333, 397, 420, 511) for N in (512, 576, 640, 832, 896, 1152, 1408, 2304, 5504)
+             for six in (0, 1)]
+    out = row_tilings.ask(rules, [f"few {M} {N} {six}" for M, N, six in sizes])
+    for (M, N, six), got in zip(sizes, out):
+        each = {"2x2": 40, "1x2": 24 if N > 1024 else 25, "2x1": 25 if N > 1024 else 24, "1x1": 17}
+        if six:
+            each.update({"3x2": 59, "2x3": 62})
+        cost = {name: _rounds(M, N, *map(int, name.split("x"))) * us for name, us in each.items()}
+        assert got == min(cost, key=cost.get), (M, N, six, cost)  # (the first of equals)
