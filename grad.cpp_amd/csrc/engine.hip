@@ -358,32 +358,11 @@ static PairPlace place_pairs(char*& at, const float* src, int N, int K, bool gat
     return p;
 }
 
-// Sizes on the host, of which bounds are made: the largest magnitude of n values, and one that seven of eight of those
-// that are not zero reach (a mean would follow the largest).
+// Sizes of runs of values, in double.
 struct Size {
     double top = 0.0, low = 0.0;
+    Size(const Sizes& s) : top(s.top), low(s.low) {}
 };
-
-static Size size_of(const float* device, size_t n) {
-    std::vector<float> v(n);
-    HIP_CHECK(hipMemcpy(v.data(), device, n * sizeof(float), hipMemcpyDeviceToHost));
-    std::vector<double> sizes;
-    Size s;
-    bool nan = false;
-    for (const float x : v) {
-        const double size = std::fabs(static_cast<double>(x));
-        nan = nan || std::isnan(size);
-        s.top = std::fmax(s.top, size);
-        if (size > 0.0) sizes.push_back(size);
-    }
-    if (nan && std::isfinite(s.top)) return {std::nan(""), std::nan("")};
-    if (!sizes.empty()) {
-        const auto at = sizes.begin() + sizes.size() / 8;
-        std::nth_element(sizes.begin(), at, sizes.end());
-        s.low = *at;
-    }
-    return s;
-}
 
 // The power of two that takes values of at most `bound` below 2^15, if what most of them reach, `low`, lies within 2^24 of
 // it (a pair is off by 2^-51 of the bound at most); none for a bound that is no number or far from fp32's middle.
@@ -398,23 +377,26 @@ struct NormSize {
     double top, norm, low;
 };
 
-static NormSize norm_size(const Shape& sh, const float* gamma, const float* beta) {
-    const size_t d = sh.d_model;
-    const Size g = size_of(gamma, d), b = sh.modern() ? Size{} : size_of(beta, d);
+static NormSize norm_size(size_t d, const Size& g, const Size& b) {
     const double root = std::sqrt(static_cast<double>(d));
     return {root * g.top + b.top, root * (g.top + b.top), g.low};
 }
+
+// The runs of a layer's vectors and of its rows' 2-norms that bounds are made of (of a vector that the block has not, none).
+enum LayerRun { RUN_WQ, RUN_WK, RUN_WV, RUN_WO, RUN_W1, RUN_W2, RUN_BQ, RUN_BK, RUN_BV, RUN_B1, RUN_G1, RUN_BE1, RUN_G2, RUN_BE2, LAYER_RUNS };
+static_assert(LAYER_RUNS <= kSizeRuns, "one launch");
 
 // The operands' powers of two, from bounds that hold for every input: a row of norm(x) has at most sqrt(d) times the
 // largest gain as its largest value and as its norm (and beta), an output at most that times its row of weights, an
 // average of values at most the largest of them, |gelu(z)| <= |z| and |silu(g) u| <= |g u|.  (fp32 roundings on
 // the way are far from the factor of two that is left to fp16's largest number.)
-static bool pair_bounds(const Shape& sh, const LayerWeights& w, const PairPlace& qkv, const PairPlace& ffn1, PairLayer& l) {
-    const size_t d = sh.d_model, F = sh.d_ff();
-    const NormSize n1 = norm_size(sh, w.g1, w.be1), n2 = norm_size(sh, w.g2, w.be2);
-    const Size wv = size_of(qkv.norm + 2 * d, d), bv = size_of(w.bqkv + 2 * d, d);
-    const Size w1 = size_of(ffn1.norm, (sh.modern() ? 2 : 1) * F), b1 = sh.modern() ? Size{} : size_of(w.b1, F);
-    const Size wq = size_of(qkv.norm, d), bq = size_of(w.bqkv, d), wk = size_of(qkv.norm + d, d), bk = size_of(w.bqkv + d, d);
+static bool pair_bounds(const Shape& sh, const Sizes* run, PairLayer& l) {
+    const size_t d = sh.d_model;
+    const NormSize n1 = norm_size(d, run[RUN_G1], run[RUN_BE1]), n2 = norm_size(d, run[RUN_G2], run[RUN_BE2]);
+    const Size wq = run[RUN_WQ], wk = run[RUN_WK], wv = run[RUN_WV], w1 = run[RUN_W1];
+    const Size bq = run[RUN_BQ], bk = run[RUN_BK], bv = run[RUN_BV], b1 = run[RUN_B1];
+    // (W_o and FFN2 feed no operand, but an infinite weight has no pair either)
+    if (!std::isfinite(run[RUN_WO].top) || !std::isfinite(run[RUN_W2].top)) return false;
     const double query = std::sqrt(2.0) * (wq.top * n1.norm + bq.top), low_query = wq.low * n1.low;
     const double key = std::sqrt(2.0) * (wk.top * n1.norm + bk.top);  // (a rotated pair is as long as it was)
     const double value = wv.top * n1.norm + bv.top, unit = w1.top * n2.norm + b1.top;
@@ -457,18 +439,27 @@ static bool layers_in_pairs(const Model& m) {
     const int d = sh.d_model, F = sh.d_ff(), up = sh.modern() ? 2 : 1;
     const size_t per_layer =
         pair_place_bytes(3 * d, d) + pair_place_bytes(d, d) + pair_place_bytes(up * F, d) + pair_place_bytes(d, F);
-    return make_form(m.layers_pairs, sh.layers * per_layer, [&](char* at) {
+    const size_t sizes_at = sh.layers * per_layer;
+    return make_form(m.layers_pairs, sizes_at + sh.layers * kSizeRuns * sizeof(Sizes), [&](char* at) {
+        Sizes* const device = reinterpret_cast<Sizes*>(at + sizes_at);
         m.pair_layers.clear();
         for (const LayerWeights& w : m.layers) {
             const PairPlace qkv = place_pairs(at, w.wqkv, 3 * d, d, false), o = place_pairs(at, w.wo, d, d, false);
             const PairPlace ffn1 = place_pairs(at, w.w1, up * F, d, sh.modern()), ffn2 = place_pairs(at, w.w2, d, F, false);
-            PairLayer l{qkv.w, o.w, ffn1.w, ffn2.w, qkv.unit, o.unit, ffn1.unit, ffn2.unit, 0, 0, 0, 0, 0};
-            // (W_o and FFN2 feed no operand, but an infinite weight has no pair either)
-            if (!std::isfinite(size_of(o.norm, d).top) || !std::isfinite(size_of(ffn2.norm, d).top)
-                || !pair_bounds(sh, w, qkv, ffn1, l))
-                return false;
-            m.pair_layers.push_back(l);
+            SizeRuns runs{};
+            const auto run = [&](LayerRun r, const float* values, int n) { runs.at[r] = values, runs.n[r] = n; };
+            run(RUN_WQ, qkv.norm, d), run(RUN_WK, qkv.norm + d, d), run(RUN_WV, qkv.norm + 2 * d, d);
+            run(RUN_WO, o.norm, d), run(RUN_W1, ffn1.norm, up * F), run(RUN_W2, ffn2.norm, d);
+            run(RUN_BQ, w.bqkv, d), run(RUN_BK, w.bqkv + d, d), run(RUN_BV, w.bqkv + 2 * d, d);
+            run(RUN_G1, w.g1, d), run(RUN_G2, w.g2, d);
+            if (!sh.modern()) run(RUN_B1, w.b1, F), run(RUN_BE1, w.be1, d), run(RUN_BE2, w.be2, d);
+            sizes_of(runs, device + m.pair_layers.size() * kSizeRuns, nullptr);
+            m.pair_layers.push_back({qkv.w, o.w, ffn1.w, ffn2.w, qkv.unit, o.unit, ffn1.unit, ffn2.unit, 0, 0, 0, 0, 0});
         }
+        std::vector<Sizes> sizes(m.pair_layers.size() * kSizeRuns);
+        HIP_CHECK(hipMemcpy(sizes.data(), device, sizes.size() * sizeof(Sizes), hipMemcpyDeviceToHost));
+        for (size_t i = 0; i < m.pair_layers.size(); i++)
+            if (!pair_bounds(sh, &sizes[i * kSizeRuns], m.pair_layers[i])) return false;
         return true;
     });
 }
@@ -479,21 +470,29 @@ static bool layers_in_pairs(const Model& m) {
 enum SplitKind { SPLIT_NONE, SPLIT_PAIRS, SPLIT_PARTS };
 
 static SplitKind layers_kind(const Model& m, long rows) {
-    if (m.shape.d_model >= kPairMinCols && !parts_are_closer(m.shape.d_model, (m.shape.modern() ? 2 : 1) * m.shape.d_ff(), rows) && layers_in_pairs(m)) return SPLIT_PAIRS;
+    const Shape& sh = m.shape;
+    const int ffn1 = (sh.modern() ? 2 : 1) * sh.d_ff();
+    if (sh.d_model >= kPairMinCols && !parts_are_closer(sh.d_model, ffn1, rows) && layers_in_pairs(m)) return SPLIT_PAIRS;
     return split_layers(m) ? SPLIT_PARTS : SPLIT_NONE;
 }
 
 static SplitKind logits_kind(const Model& m, long rows) {
     const int d = m.shape.d_model, V = m.shape.vocab;
     if (d >= kPairMinCols && !logits_parts_are_closer(d, V, rows)) {
-        const bool pairs = make_form(m.logits_pairs, pair_place_bytes(V, d), [&](char* at) {
-            const NormSize n = norm_size(m.shape, m.gf, m.bf);
+        const size_t sizes_at = pair_place_bytes(V, d);
+        const bool pairs = make_form(m.logits_pairs, sizes_at + kSizeRuns * sizeof(Sizes), [&](char* at) {
+            Sizes* const device = reinterpret_cast<Sizes*>(at + sizes_at);
+            const PairPlace e = place_pairs(at, m.E, V, d, false);
+            SizeRuns runs{{e.norm, m.gf, m.bf}, {V, d, m.shape.modern() ? 0 : d}};
+            sizes_of(runs, device, nullptr);
+            Sizes sizes[3];
+            HIP_CHECK(hipMemcpy(sizes, device, sizeof(sizes), hipMemcpyDeviceToHost));
+            const NormSize n = norm_size(d, sizes[1], sizes[2]);
             const std::optional<int> norm = pair_exponent(n.top, n.low);
             if (!norm) return false;
-            const PairPlace e = place_pairs(at, m.E, V, d, false);
             m.logits_unit = e.unit;
             m.logits_norm = *norm;
-            return !std::isinf(size_of(e.norm, V).top);
+            return !std::isinf(sizes[0].top);
         });
         if (pairs) return SPLIT_PAIRS;
     }

@@ -29,6 +29,18 @@ void split_gemm(SplitGemmParams& p, hipStream_t st);
 inline size_t pair_rows(size_t rows) { return (rows + 95 + kSplitPad - 1) / kSplitPad * kSplitPad; }
 inline size_t pair_bytes(size_t rows, size_t cols) { return pair_rows(rows) * cols * 4; }
 void pair_weights(const float* src, int N, int K, bool gate_up, char* dst, float* unit, float* norm, hipStream_t st);
+// Sizes of runs of values, of which the bounds of operands in pairs are made: the largest magnitude, and one that seven of eight
+// of those that are not zero reach (a mean would follow the largest); not numbers where one of the values is none and the
+// largest is finite.
+struct Sizes {
+    float top, low;
+};
+constexpr int kSizeRuns = 16;
+struct SizeRuns {
+    const float* at[kSizeRuns];
+    int n[kSizeRuns];  // 0: no values, sizes of 0
+};
+void sizes_of(const SizeRuns& runs, Sizes* out, hipStream_t st);  // kSizeRuns of them
 void norm_pair(bool rms, const float* x, const float* gamma, const float* beta, char* out, int M, int d, float pair_scale,
                hipStream_t st);
 template <int EPI>
