@@ -98,3 +98,21 @@ def test_query_blocks_do_not_change_a_pass(batch, n, before):
     assert got[1].tobytes() == got[0].tobytes() and got[2].tobytes() == got[0].tobytes()
     ref = ref_forward.forward(cfg, W, tokens[batch - 1])[-1]
     assert_logits_close(got[1][batch - 1], ref, what=f"queries {batch} x {n}")
+
+
+@pytest.mark.parametrize("arch, d", [(synth.ARCH_GPT2, 576), (synth.ARCH_MODERN, 896), (synth.ARCH_GPT2, 1152)])
+def test_widths_dealt_unevenly_to_the_xcds(arch, d):
+    """Runs of outputs that are no multiple of eight: the same first positions behind any number of rows, whatever tiles those take."""
+    cfg = synth.Config(arch, 201, d, 2, d // 64, 520)
+    W = synth.make_weights(cfg, 135, std=lively_std(cfg), norm_noise=0.1)
+    gm = G.Model.from_tensors(cfg, W)
+    tokens = synth.uniform_tokens(511, cfg.vocab, 136)
+    kept = None
+    for n in (66, 200, 300, 333, 397, 420, 511):
+        s = G.Session(gm)
+        got = s.prefill(tokens[:n])
+        if n in (66, 397):
+            assert_logits_close(got, ref_forward.forward(cfg, W, tokens[:n])[-1], what=f"uneven {d} {n}")
+        rows = [s.read_kv(0, 1, kv, pos).tobytes() for kv in (0, 1) for pos in (0, 31, 47, 65)]
+        kept = kept or rows
+        assert rows == kept, n
