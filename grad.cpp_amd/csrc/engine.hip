@@ -2342,17 +2342,22 @@ static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSi
         if (slice == 1 || slice * B < kSplitMinRows) throw ApiError{GH_ERR_DEVICE, "out of device memory for a prompt pass"};
         slice = (slice + 1) / 2;
     }
+    // Whether the layers and the scored logits of n tokens go in pairs: a shorter slice's form is its own, the others' if there is
+    // no memory for it.  Made, like the plan's, before anything is launched.
+    const auto in_pairs = [&](int n) {
+        const auto kind = [&](SplitKind planned, auto kind_of) {
+            const SplitKind own = n == plan.slice ? planned : kind_of(m, static_cast<long>(n) * B);
+            return (own == SPLIT_NONE ? planned : own) == SPLIT_PAIRS;
+        };
+        return std::make_pair(n * B >= plan.split_rows && kind(plan.kind, layers_kind), sink && kind(plan.logits, logits_kind));
+    };
+    const auto whole = in_pairs(slice), last = in_pairs((len - 1) % slice + 1);
     for (int t0 = 0; t0 < len; t0 += slice) {
         const int n = std::min(slice, len - t0);
         const int M = n * B;
         const int pos_base = s.pos + t0;
         const bool split = M >= plan.split_rows;
-        // (a shorter slice's form is its own, the others' if there is no memory for it)
-        const auto of_slice = [&](SplitKind planned, auto kind_of) {
-            const SplitKind kind = n == plan.slice ? planned : kind_of(m, M);
-            return kind == SPLIT_NONE ? planned : kind;
-        };
-        const bool pairs = split && of_slice(plan.kind, layers_kind) == SPLIT_PAIRS;
+        const bool pairs = split && (n == slice ? whole : last).first;
         const bool split_attn = split && reserve_split_attention(s, n, pos_base, pairs);
         hipLaunchKernelGGL(embed_rows_kernel, dim3((d + 255) / 256, M), dim3(256), 0, st, m.E, m.P, s.hist,
                            s.hist_stride, s.n_hist + t0, n, pos_base, s.pp_x, d);
@@ -2364,7 +2369,7 @@ static void prompt_pass(Session& s, int len, const RowsPlan& plan, const ScoreSi
             if (split) prompt_layer_split(s, l, n, pos_base, pairs, split_attn, trim && l == sh.layers - 1);
             else prompt_layer_small(s, l, n, pos_base);
         }
-        if (sink) score_rows(s, *sink, of_slice(plan.logits, logits_kind) == SPLIT_PAIRS, M, n, t0, len);
+        if (sink) score_rows(s, *sink, (n == slice ? whole : last).second, M, n, t0, len);
         if (t0 + n == len) {
             hipLaunchKernelGGL(take_last_rows_kernel, dim3((d + 255) / 256, B), dim3(256), 0, st, s.pp_x, n,
                                s.x, d);
